@@ -56,6 +56,8 @@ inline size_t vi_box_count(const DevGeom& d) {
 // enter and leave the FOV within a few slabs of each other (the waves walk
 // slabs or samples in lockstep).
 constexpr int kProjTileU = 32, kProjTileV = 8;
+// Tile of the z-column copies: kColTile x by kColTile words of their columns, one y.
+constexpr int kColTile = 64;
 
 struct BatchItem {
     DevGeom g;
@@ -91,6 +93,10 @@ constexpr int32_t kItemBF16 = 0x10;
 // Item flag bit of the BF16 copy and RS launches: the copies are A-pair
 // copies (zpair.hpp), read with one load per RS sample.
 constexpr int32_t kItemApair = 0x20;
+
+// Item flag bit of the copy launches: the z-column copy (one item; BF16 pairs
+// with kItemBF16).
+constexpr int32_t kItemZcol = 0x40;
 
 // Per-problem scalars of the gradient loop, FP64, in `slot`.
 enum GdSlot {
@@ -143,7 +149,7 @@ __device__ __forceinline__ int batch_find(const BatchTable* t, uint32_t tile) {
 // The state is FP32 throughout; operator copies are FP32 or BF16 (kItemBF16).
 hipError_t launch_batch_zpair_x(const BatchTable* t, hipStream_t s);   // in volume -> out qx (FP32/BF16)
 hipError_t launch_batch_zpair_y(const BatchTable* t, hipStream_t s);   // in volume -> out qy (FP32/BF16)
-hipError_t launch_batch_siddon(BatchTable* t, hipStream_t s);          // in qx, in2 qy -> out sinogram
+hipError_t launch_batch_siddon(BatchTable* t, hipStream_t s);          // in z-column copy -> out sinogram
 hipError_t launch_batch_rs(BatchTable* t, hipStream_t s);              // in qx, in2 qy -> out; flags bit0 cube
 // Grids of the shared launches whose workgroups take more registers than
 // kBatchGrid resident workgroups allow (RS): the number the device holds at

@@ -39,8 +39,7 @@ struct SidRay {
 // out of the grid there and then stops, so no index range test is needed in
 // the loops below.
 __device__ __forceinline__ SidRay sid_setup(const DevGeom& g, int p, int m, int n) {
-    SidRay r;
-    r.ok = false;
+    SidRay r{};
     const double* vw = g.view + (size_t)p * kViewStride;
     const double ca = vw[0], sa = vw[1], dl = (double)g.delta;
     const double s = ((double)m - (double)g.cu) * (double)g.du;
@@ -152,23 +151,6 @@ template <> struct VolReader<float, true> {
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, lin * 4u, 0, 0));
     }
 };
-template <> struct VolReader<__half, true> {
-    __amdgpu_buffer_rsrc_t r;
-    float inv;
-    __device__ __forceinline__ float operator()(unsigned lin) const {
-        const unsigned short b = __builtin_amdgcn_raw_buffer_load_b16(r, lin * 2u, 0, 0);
-        return __half2float(__builtin_bit_cast(__half, b)) * inv;
-    }
-};
-template <> struct VolReader<__hip_bfloat16, true> {
-    __amdgpu_buffer_rsrc_t r;
-    float inv;
-    __device__ __forceinline__ float operator()(unsigned lin) const {
-        const unsigned short b = __builtin_amdgcn_raw_buffer_load_b16(r, lin * 2u, 0, 0);
-        return __uint_as_float((unsigned)b << 16) * inv;
-    }
-};
-
 template <typename TV, bool BUF>
 __device__ __forceinline__ VolReader<TV, BUF> make_reader(const TV* p, unsigned bytes, float inv) {
     VolReader<TV, BUF> v;
@@ -226,254 +208,197 @@ __device__ __forceinline__ void sid_step(SidState& s, const SidRay& r, const RD&
     s.live = s.t < r.tmax;
 }
 
-// Slab walk on the z-pair copy.  Per slab one load gives the current voxel
-// V0, its B neighbour Vb, its z neighbour Vz and Vbz (in the step directions).
-// The wave was admitted only if, for each of its rays, consecutive crossings
-// of B and of z are spaced more than two ulps of tmax beyond the slab
-// length, so a slab holds at most one crossing of each; its segments are
-//   [t, e1] V0,  [e1, e2] Vb or Vz (whichever comes first),  [e2, tA] Vb, Vz or Vbz
-// with e1 <= e2 the interior crossings (tA when absent), every end clipped to
-// tmax.  These are the segments of the general step in the same order; an
-// absent one has zero length and adds exactly 0.  ZNEG: the wave's rays go
-// down in z (rows on one side of the detector centre, one sign).
-// Quad reads of a z-pair copy: a buffer resource with a 32-bit byte offset
-// (copies below 4 GiB; the walk carries the offset in bytes) or a plain
-// global load by element index.
-template <typename TV, bool BUF> struct QuadReader;
-// A byte offset past every copy the buffer path reads (copies stay below it):
-// a read there returns zeros without touching memory.
+// Column walk on the z-column copy (zpair.hpp: z varies fastest).  A lane walks
+// the in-plane cells (x, y) its ray crosses, one per iteration; a cell's
+// segments are
+//   [t, c1] V(z),  [c1, te] V(z + dz)
+// with te the nearer of the cell's x and y crossing and tmax and c1 the z
+// crossing (te when it comes later).  The wave was admitted only if, for each
+// of its rays, consecutive z crossings are spaced more than two ulps of tmax
+// beyond the longest stretch in one cell, so a cell holds at most one.  These
+// are the segments of the general step in the same order; an absent one has
+// zero length and adds exactly 0 (x and y crossed at once are two steps with an
+// empty cell between them).
+//
+// Why columns: all rows of a detector column cross the same in-plane cells
+// (the source, the column and the z axis span a vertical plane), so the lanes
+// of a wave -- rows of one column, or of a few neighbouring ones -- read one
+// contiguous run of z per cell.  A gather of 8 or 16 bytes a lane takes the
+// texture path 4 lanes a cycle (16.5 cycles a wave measured), a second pass for
+// each four lanes that straddle two rows of the copy, and 2 cycles per 128-byte
+// line from L2.  With lanes along the detector rows, four lanes straddle z rows
+// often and a wave touches 10-13 lines: 31 cycles per 16-byte gather of a slab's
+// (B, z) quad, 46.1 ms at 512^3 / 512 views.  Along the columns a cell's
+// 8 bytes take two to four lines, from one copy of the volume (the quads took
+// four volumes).
 constexpr uint32_t kSidOutside = 0xfffffff0u;
-template <typename TV> struct QuadReader<TV, false> {
-    static constexpr uint32_t kUnit = 1;  // element index
-    static constexpr bool kAnyOffset = false;  // only a live lane's offset may be read
-    const TV* p;
-    float inv;
-    __device__ __forceinline__ float4 operator()(uint32_t e) const { return Storage<TV>::load4(p, e, inv); }
-};
-template <typename TV> struct QuadReader<TV, true> {
-    static constexpr uint32_t kUnit = sizeof(TV);  // byte offset
-    static constexpr bool kAnyOffset = true;  // an offset past the copy reads zeros
+
+// Reads V(z), V(z + 1) of a column.  BUF: by byte offset through a buffer
+// resource; an offset past its end reads 0 without touching memory.
+// Otherwise by element index.  FP32 elements are single voxels, 16-bit ones
+// (z, z + 1) pairs, one 4-byte word.
+template <typename TV, bool BUF> struct ColumnReader {
+    static constexpr uint32_t kUnit = BUF ? 4u : 1u;
+    static constexpr uint32_t kIdle = BUF ? kSidOutside : 0u;
     __amdgpu_buffer_rsrc_t r;
-    float inv;
-    __device__ __forceinline__ float4 operator()(uint32_t off) const { return BufLoad4<TV>::load(r, off, 0u, inv); }
+    const uint32_t* p;
+    __device__ __forceinline__ float2 operator()(uint32_t o) const {
+        if constexpr (sizeof(TV) == 4) {
+            uint32_t w[2];
+            if constexpr (BUF) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)o, 0, 0);
+                w[0] = v[0];
+                w[1] = v[1];
+            } else {
+                __builtin_memcpy(w, p + o, 8);
+            }
+            return make_float2(__uint_as_float(w[0]), __uint_as_float(w[1]));
+        } else {
+            const uint32_t w = BUF ? __builtin_amdgcn_raw_buffer_load_b32(r, (int)o, 0, 0) : p[o];
+            return make_float2(Unpack16<TV>::lo(w), Unpack16<TV>::hi(w));
+        }
+    }
+    // one voxel (the general step)
+    __device__ __forceinline__ float one(uint32_t o) const { return (*this)(o).x; }
 };
-template <typename TV, bool BUF>
-__device__ __forceinline__ QuadReader<TV, BUF> make_quad_reader(const TV* p, uint32_t bytes, float inv) {
-    QuadReader<TV, BUF> q;
-    if constexpr (BUF) q.r = buffer_rsrc(p, bytes);
-    else q.p = p;
-    q.inv = inv;
-    return q;
+
+// The ray as its lane walks it; e: offset of V(z), or of V(z - 1) when the ray
+// goes down in z (the pair below), dX, dY, dZ its signed steps.
+struct ColumnRay {
+    float fx, ix, fy, iy, fz, iz, tmax;
+    uint32_t e, dX, dY, dZ;
+    bool down;
+};
+
+// DIR: 0 / 1 when every ray of the wave goes up / down in z, 2 when they differ.
+template <int DIR, typename CR>
+__device__ __forceinline__ float sid_walk_columns(const ColumnRay& r, const CR& rd, int trips) {
+    float tx = r.fx, ty = r.fy, tz = r.fz, k = 0.0f, cx = 0.0f, cz = 0.0f, t = 0.0f, acc = 0.0f;
+    uint32_t e = r.e;
+    // A lane past its last cell has t = tmax: every later time lies at tmax or
+    // beyond, so its segments have no length, and its loads go to kIdle.
+    struct Cell {
+        float d1, d2;
+        float2 v;
+    };
+    auto next = [&]() __attribute__((always_inline)) {
+        Cell c;
+        c.v = rd(t < r.tmax ? e : CR::kIdle);
+        const float te = min_nn(min_nn(tx, ty), r.tmax);
+        const float c1 = min_nn(tz, te);
+        c.d1 = c1 - t;
+        c.d2 = te - c1;
+        const bool sx = tx <= ty, sz = tz <= te;
+        e += (sx ? r.dX : r.dY) + (sz ? r.dZ : 0u);
+        t = te;
+        k += 1.0f;
+        cx += sx ? 1.0f : 0.0f;
+        cz += sz ? 1.0f : 0.0f;
+        tx = fmaf(cx, r.ix, r.fx);
+        ty = fmaf(k - cx, r.iy, r.fy);
+        tz = fmaf(cz, r.iz, r.fz);
+        return c;
+    };
+    auto add = [&](const Cell& c) __attribute__((always_inline)) {
+        const bool down = DIR == 2 ? r.down : DIR == 1;
+        acc = fmaf(c.d1, down ? c.v.y : c.v.x, acc);
+        acc = fmaf(c.d2, down ? c.v.x : c.v.y, acc);
+    };
+    // kAhead cells are loaded before the oldest is summed
+    constexpr int kAhead = 3;
+    Cell q[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) q[j] = next();
+    for (int i = 0; i < trips; i += kAhead) {
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            add(q[j]);
+            q[j] = next();
+        }
+    }
+    return acc;
 }
 
-// BNEG: 0 / 1 when every ray of the wave steps up / down along B, 2 when
-// the wave mixes both (per-lane selects).
-template <int A, bool ZNEG, int BNEG, typename QR>
-__device__ __forceinline__ void sid_walk_quads(const SidRay& r, const QR& rd, int nA, int nB, int nz, bool live,
-                                               float& acc_out) {
-    constexpr int B = 1 - A;
-    const int sA = r.step[A], sB = r.step[B];
-    const bool bneg = BNEG == 2 ? sB < 0 : BNEG == 1;
-    float tA = r.first[A], tB = r.first[B], tz = r.first[2];
-    float cA = 0.0f, cB = 0.0f, cz = 0.0f;
-    int iA = r.idx[A];
-    float t = 0.0f, acc = 0.0f;
-    // Offset of the block corner (A = iA, B = iB or iB - 1, z = iz or
-    // iz - 1), carried by the steps.  A live lane's voxel is inside the grid
-    // (tmax stops at the first crossing that leaves it), so the corner is in
-    // the copy; the offset of a finished lane is never used.
-    constexpr uint32_t u = QR::kUnit;
-    const uint32_t sz_e = 2u * (uint32_t)(nB + 2), sa_e = sz_e * (uint32_t)(nz + 1);
-    uint32_t e = 0u;
-    if (live) {
-        const int bb = (bneg ? r.idx[B] - 1 : r.idx[B]) + 1;
-        const int zz = (ZNEG ? r.idx[2] - 1 : r.idx[2]) + 1;
-        e = ((uint32_t)iA * sa_e + (uint32_t)zz * sz_e + 2u * (uint32_t)bb) * u;
-    }
-    const uint32_t dA = (uint32_t)sA * sa_e * u, dB = 2u * (uint32_t)sB * u, dZ = (uint32_t)r.step[2] * sz_e * u;
-    // Lockstep: the wave's slab starts at the first slab of its lanes (in
-    // each lane's direction along A) and advances one slab per iteration; a
-    // lane joins at iteration lag = |iA - I| and then takes one slab per
-    // iteration while it is live.
-    const int I = sA > 0 ? wave_min(live ? iA : 0x7fffffff) : wave_max(live ? iA : -0x7fffffff);
-    const int lag = abs(iA - I);
-    // The wave's iterations, counted once (a scalar loop instead of a vote
-    // per slab): a lane's slabs are at iterations lag .. lag + K, K the first
-    // count with fma(K, inc, first) >= tmax (its last slab); the estimate
-    // below, a rounded quotient of two FP32 times, is off by less than one,
-    // and the count adds a margin of two.  Extra iterations find no live lane
-    // and skip the body.
-    int span = 0;
-    if (live) {
-        const float kf = ceilf((r.tmax - r.first[A]) * __builtin_amdgcn_rcpf(r.inc[A]));
-        span = lag + (int)fminf(fmaxf(kf, 0.0f), 1.0e6f) + 3;
-    }
-    const int trips = __builtin_amdgcn_readfirstlane(min(wave_max(span), nA + 2));
-    // One slab in two halves: advance() takes the slab's segment ends and
-    // steps the walk to the next slab (its block offset follows from the
-    // crossing times alone, not from the voxels); accumulate() adds the
-    // slab's segments, given its block.
-    struct Slab {
-        bool act, stepB, stepZ, bfirst;
-        float t0, c1, c2, c3;
-    };
-    auto advance = [&](int outer) __attribute__((always_inline)) {
-        Slab sl;
-        sl.act = live && outer >= lag;
-        // Segment ends: c3 = min(tA, tmax) closes the slab; the interior
-        // crossings are c1 = min(tB, tz, c3) and c2 = min(max(tB, tz), c3)
-        // (min(x, tA) of each crossing, in order, clipped to tmax).  The
-        // middle segment's voxel is Vb when B is crossed first and Vz when z
-        // is; the last one's is the voxel after the crossings taken (tB <= tA:
-        // B stepped).  Where these choices differ from the general step's (a
-        // tie, or a crossing exactly at tA) the segment has zero length and
-        // adds exactly 0.
-        sl.stepB = tB <= tA;
-        sl.stepZ = tz <= tA;
-        sl.bfirst = tB < tz;
-        sl.c3 = min_nn(tA, r.tmax);
-        sl.c1 = min_nn(min_nn(tB, tz), sl.c3);
-        sl.c2 = min_nn(max_nn(tB, tz), sl.c3);
-        sl.t0 = t;
-        if (sl.act) {
-            t = sl.c3;
-            // the next crossing times follow from the counts (an axis not
-            // stepped recomputes the same time)
-            e += (sl.stepB ? dB : 0u) + (sl.stepZ ? dZ : 0u) + dA;
-            cB += sl.stepB ? 1.0f : 0.0f;
-            cz += sl.stepZ ? 1.0f : 0.0f;
-            tB = fmaf(cB, r.inc[B], r.first[B]);
-            tz = fmaf(cz, r.inc[2], r.first[2]);
-            cA += 1.0f;
-            tA = fmaf(cA, r.inc[A], r.first[A]);
-            live = t < r.tmax;
-        }
-        return sl;
-    };
-    auto accumulate = [&](const Slab& sl, const float4& v) __attribute__((always_inline)) {
-        if (!sl.act) return;
-        // v = (b, z), (b, z+1), (b+1, z), (b+1, z+1) of the block's corner
-        const float V0 = bneg ? (ZNEG ? v.w : v.z) : (ZNEG ? v.y : v.x);
-        const float Vb = bneg ? (ZNEG ? v.y : v.x) : (ZNEG ? v.w : v.z);
-        const float Vz = bneg ? (ZNEG ? v.z : v.w) : (ZNEG ? v.x : v.y);
-        const float Vbz = bneg ? (ZNEG ? v.x : v.y) : (ZNEG ? v.z : v.w);
-        const float V1 = sl.bfirst ? Vb : Vz;
-        const float V2 = sl.stepB ? (sl.stepZ ? Vbz : Vb) : (sl.stepZ ? Vz : V0);
-        acc = fmaf(sl.c1 - sl.t0, V0, acc);
-        acc = fmaf(sl.c2 - sl.c1, V1, acc);
-        acc = fmaf(sl.c3 - sl.c2, V2, acc);
-    };
-    if constexpr (QR::kAnyOffset) {
-        // Copies read through the buffer path: the next slab's block is
-        // loaded before this slab's segments are summed, into two alternating
-        // registers.  Every lane issues the load (a load guarded per lane is a
-        // branch, at whose end the compiler waits for it, and so is a copy of
-        // the prefetched value); a lane that will not use it reads past the
-        // copy (zeros, no memory access), its offset formed with a mask.  At
-        // 512^3 / 512 views: FP32 48.5 -> 46.5 ms, FP16 46.0 -> 42.7 ms; with
-        // every lane reading its stale offset instead, the idle lanes' lines
-        // cost FP32 what the prefetch gained.  The 64-bit index reads (copies
-        // of 4 GiB or more) keep the direct form below: at 1024^3 the walk is
-        // bound by the memory traffic, and the same prefetch (idle lanes
-        // reading the copy's first block) took FP32 from 482 to 520 ms.
-        auto next_off = [&](int outer_next) __attribute__((always_inline)) {
-            const uint32_t keep = 0u - (uint32_t)(live && outer_next >= lag);
-            return (e & keep) | (kSidOutside & ~keep);
-        };
-        float4 va = rd(next_off(0)), vb = va;
-        for (int outer = 0; outer < trips; outer += 2) {
-            Slab sl = advance(outer);
-            vb = rd(next_off(outer + 1));
-            accumulate(sl, va);
-            if (outer + 1 < trips) {
-                sl = advance(outer + 1);
-                va = rd(next_off(outer + 2));
-                accumulate(sl, vb);
-            }
-        }
-    } else {
-        for (int outer = 0; outer < trips; ++outer) {
-            if (live && outer >= lag) {
-                const float4 v = rd(e);
-                const Slab sl = advance(outer);
-                accumulate(sl, v);
-            }
-        }
-    }
-    acc_out = acc;
-}
-
-template <int A, bool ZNEG, typename QR>
-__device__ __forceinline__ void sid_walk_quads_b(const SidRay& r, const QR& rd, int nA, int nB, int nz, bool live,
-                                                 float& acc) {
-    const bool pos_all = __ballot(live && r.step[1 - A] < 0) == 0ull;
-    const bool neg_all = __ballot(live && r.step[1 - A] >= 0) == 0ull;
-    if (pos_all) sid_walk_quads<A, ZNEG, 0>(r, rd, nA, nB, nz, live, acc);
-    else if (neg_all) sid_walk_quads<A, ZNEG, 1>(r, rd, nA, nB, nz, live, acc);
-    else sid_walk_quads<A, ZNEG, 2>(r, rd, nA, nB, nz, live, acc);
+// The column group of the grid's x index `i` (gx of them, a multiple of 8): the
+// XCD i mod 8 takes a run of gx / 8 neighbouring groups.  The runs rotate over
+// the XCDs with the view and the row band, because outer columns have shorter
+// rays.
+__device__ __forceinline__ int sid_group(uint32_t i, uint32_t gx, uint32_t pg, uint32_t views, uint32_t bz) {
+    const uint32_t run = (i + pg * 8u / views + bz) & 7u;
+    return (int)(run * (gx / 8u) + i / 8u);
 }
 
 // Forward clean Siddon.  Each lane takes the segments of the per-ray
 // traversal (same operations, same order), so results are bit-identical to
-// it.  What changes is the schedule and the memory layout: when every ray of
-// the wave has the same dominant in-plane axis A (|d_A| >= the other two
-// components) and the same direction along it, the wave walks the slabs of A
-// together.  The 64 rays of a wave are a 32-column x 2-row detector block, spread
-// across the other in-plane axis, so at a given slab they read voxels that
-// are contiguous when that other axis varies fastest: x-fastest (the caller's
-// layout) for y-slabs, a y-fastest copy for x-slabs.  Waves that mix axes
-// (views near 45 degrees) step per lane on the x-fastest volume.
-// Grid: x = detector column group, y = view, z = detector row group.  Blocks
-// are dispatched x fastest and spread over the XCDs round robin, so the chip
-// works through every view of one row band before the next band: the rays of
-// a row band stay in a thin z band of the volume, which the L2 and the
-// Infinity Cache hold, instead of streaming the whole volume from HBM once
-// per view.
+// it.  What changes is the schedule and the memory layout (see above).
+// A wave is `rows` (64, 32 or 16) detector rows of 64 / rows columns; a
+// workgroup is these cells in kSidViews consecutive views, whose rays run
+// through nearly the same columns of the volume at the same time (512^3 / 512
+// views: 33.1 ms with four neighbouring column groups of one view per
+// workgroup, 31.7 ms with four views; 1024^3 / 720 views, bound by the lines
+// that miss L2: 238 and 182 ms).  Grid: x = column group, y = view group, z =
+// row group: the chip works through every view of one row band before the
+// next band, whose rays stay in a z band of the volume.  Workgroups go to the
+// XCDs round robin; sid_group gives each XCD neighbouring column groups, so that
+// its L2 meets the columns of one view again in the next ones (512^3: 38.1 ms
+// without it, at four columns of one view per workgroup).
 template <typename TV, typename TS, bool BUF>
-__device__ __forceinline__ void siddon_tile(const DevGeom& g, const TV* __restrict__ qx, const TV* __restrict__ qy,
-                                            unsigned qx_bytes, unsigned qy_bytes, float vol_inv,
-                                            TS* __restrict__ sino, float sino_scale, int bx, int p, int bz) {
-    const int m = bx * BX + threadIdx.x;
-    const int n = bz * BY + threadIdx.y;
-    const bool inside = m < g.nu && n < g.nv;
-    SidRay r;
-    r.ok = false;
+__device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __restrict__ cols, float vol_inv,
+                                            TS* __restrict__ sino, float sino_scale, int rows, int bx, int pg, int bz) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int per = 64 / rows;  // columns of a wave
+    const int p = pg * kSidViews + wv;
+    const int m = bx * per + lane / rows;
+    const int n = bz * rows + lane % rows;
+    const bool inside = p < g.nphi && m < g.nu && n < g.nv;
+    SidRay r{};
     if (inside) r = sid_setup(g, p, m, n);
     const bool ok = r.ok && r.tmax > 0.0f;
-    // Slab code of this ray: 0/1 = x axis up/down, 2/3 = y axis up/down, when
-    // the crossings of the other two axes are spaced farther apart than the
-    // slabs by more than two ulps of tmax (inc = delta/|d|), and the first
-    // slab is no longer than the others.  A FOV entry outside the grid along
-    // the slab axis (the cylinder is wider than the grid when ny < nx) clamps
-    // the first voxel and makes the first slab long; such rays step per lane.
-    int code = -1;
-    if (ok) {
-        const float big = 3.0e38f, margin = 1.0e-6f * r.tmax;
-        const float ix = r.step[0] ? r.inc[0] : big, iy = r.step[1] ? r.inc[1] : big;
-        const float iz = r.step[2] ? r.inc[2] : big;
-        if (r.step[0] != 0 && iy > ix + margin && iz > ix + margin && r.first[0] <= ix)
-            code = r.step[0] > 0 ? 0 : 1;
-        else if (r.step[1] != 0 && ix > iy + margin && iz > iy + margin && r.first[1] <= iy)
-            code = r.step[1] > 0 ? 2 : 3;
-    }
-    const unsigned long long okmask = __ballot(ok);
-    int mode = -1;
-    if (okmask != 0ull) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (__ballot(ok && code == c) == okmask) mode = c;
-    }
-    // one z direction per wave (its rows on one side of the detector centre), or none
-    const bool zneg_all = __ballot(ok && r.step[2] > 0) == 0ull;
-    const bool zpos_all = __ballot(ok && r.step[2] < 0) == 0ull;
-    if (!zneg_all && !zpos_all) mode = -1;
-    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    // The z crossings of the ray are spaced farther apart than the longest
+    // stretch in one cell, by more than two ulps of tmax; else the wave takes
+    // the general step.
+    const float big = 3.0e38f;
+    const float ix = r.step[0] ? r.inc[0] : big, iy = r.step[1] ? r.inc[1] : big, iz = r.step[2] ? r.inc[2] : big;
+    const float cell = fmaxf(fminf(ix, iy), fminf(fminf(r.first[0], r.first[1]), r.tmax));
+    const bool walk = __ballot(ok && !(iz > cell + 1.0e-6f * r.tmax)) == 0ull;
+    const int ny = g.ny, nz = g.nz;
+    const uint32_t pz = zcol_pitch(nz, sizeof(TV)), py = pz * (uint32_t)ny;
+    using CR = ColumnReader<TV, BUF>;
+    constexpr uint32_t u = CR::kUnit;
+    CR rd;
+    if constexpr (BUF) rd.r = buffer_rsrc(cols, (uint32_t)(zcol_words(g.nx, ny, nz, sizeof(TV)) * 4u));
+    rd.p = cols;
     float acc = 0.0f;
-    if (mode < 0) {
-        // Per-lane traversal on the y-slab copy, where voxel (x, y, z) is
-        // element 2(x+1) + 2(nx+2)(z+1) + 2(nx+2)(nz+1) y (z-pair index of
-        // corner (x, z) on plane y, first of the pair).
-        const auto rd = make_reader<TV, BUF>(qy, qy_bytes, 1.0f);
+    const uint32_t lin = ok ? (uint32_t)r.idx[0] * py + (uint32_t)r.idx[1] * pz + (uint32_t)(r.idx[2] + 1) : 0u;
+    if (walk) {
+        ColumnRay w;
+        w.fx = r.first[0];
+        w.ix = r.inc[0];
+        w.fy = r.first[1];
+        w.iy = r.inc[1];
+        w.fz = r.first[2];
+        w.iz = r.inc[2];
+        w.tmax = ok ? r.tmax : 0.0f;
+        w.down = r.step[2] < 0;
+        w.e = (lin - (w.down ? 1u : 0u)) * u;
+        w.dX = (uint32_t)r.step[0] * py * u;
+        w.dY = (uint32_t)r.step[1] * pz * u;
+        w.dZ = (uint32_t)r.step[2] * u;
+        // The wave's iterations, counted once (a scalar loop instead of a vote
+        // per cell): the x and y crossings up to tmax, from rounded quotients
+        // of two FP32 times that are off by less than one each, with a margin.
+        int cells = 0;
+        if (ok) {
+            const float qx = r.step[0] ? (w.tmax - w.fx) * __builtin_amdgcn_rcpf(w.ix) : 0.0f;
+            const float qy = r.step[1] ? (w.tmax - w.fy) * __builtin_amdgcn_rcpf(w.iy) : 0.0f;
+            cells = (int)(fminf(fmaxf(qx, 0.0f), 1.0e6f) + fminf(fmaxf(qy, 0.0f), 1.0e6f)) + 6;
+        }
+        const int trips = __builtin_amdgcn_readfirstlane(min(wave_max(cells), g.nx + ny + 6));
+        const bool any_down = __ballot(ok && w.down) != 0ull, any_up = __ballot(ok && !w.down) != 0ull;
+        if (!any_down) acc = sid_walk_columns<0>(w, rd, trips);
+        else if (!any_up) acc = sid_walk_columns<1>(w, rd, trips);
+        else acc = sid_walk_columns<2>(w, rd, trips);
+    } else {
         SidState s;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -482,27 +407,18 @@ __device__ __forceinline__ void siddon_tile(const DevGeom& g, const TV* __restri
         }
         // The copy holds fewer than 2^32 elements (checked by the launcher):
         // the index and its signed steps wrap correctly in 32-bit unsigned.
-        const unsigned sz = 2u * (unsigned)(nx + 2), sy = sz * (unsigned)(nz + 1);
-        s.lin = ok ? 2u * (unsigned)(r.idx[0] + 1) + sz * (unsigned)(r.idx[2] + 1) + sy * (unsigned)r.idx[1] : 0u;
-        s.dlin[0] = 2u * (unsigned)r.step[0];
-        s.dlin[1] = (unsigned)r.step[1] * sy;
-        s.dlin[2] = (unsigned)r.step[2] * sz;
+        s.lin = lin * u;
+        s.dlin[0] = (uint32_t)r.step[0] * py * u;
+        s.dlin[1] = (uint32_t)r.step[1] * pz * u;
+        s.dlin[2] = (uint32_t)r.step[2] * u;
         s.t = 0.0f;
         s.acc = 0.0f;
         s.live = ok;
         // Every step moves one axis toward the grid exit that bounds tmax;
         // the cap only bounds the loop.
-        int guard = nx + ny + nz + 4;
-        while (s.live && guard-- > 0) sid_step(s, r, rd);
+        int guard = g.nx + ny + nz + 4;
+        while (s.live && guard-- > 0) sid_step(s, r, [&](unsigned o) { return rd.one(o); });
         acc = s.acc;
-    } else if (mode < 2) {
-        const auto rq = make_quad_reader<TV, BUF>(qx, qx_bytes, 1.0f);
-        if (zneg_all && !zpos_all) sid_walk_quads_b<0, true>(r, rq, nx, ny, nz, ok, acc);
-        else sid_walk_quads_b<0, false>(r, rq, nx, ny, nz, ok, acc);
-    } else {
-        const auto rq = make_quad_reader<TV, BUF>(qy, qy_bytes, 1.0f);
-        if (zneg_all && !zpos_all) sid_walk_quads_b<1, true>(r, rq, ny, nx, nz, ok, acc);
-        else sid_walk_quads_b<1, false>(r, rq, ny, nx, nz, ok, acc);
     }
     // 16-bit volumes are read unscaled; the sum is linear in them, so the
     // storage scale applies once here (FP32 storage has no scale).
@@ -817,41 +733,35 @@ __global__ __launch_bounds__(BX* BY, 5) void siddon_staged_kernel(DevGeom g, con
 }
 
 template <typename TV, typename TS, bool BUF>
-__global__ __launch_bounds__(BX* BY) void siddon_kernel(DevGeom g, const TV* __restrict__ qx,
-                                                      const TV* __restrict__ qy, unsigned qx_bytes,
-                                                      unsigned qy_bytes, float vol_inv, TS* __restrict__ sino,
-                                                      float sino_scale) {
-    siddon_tile<TV, TS, BUF>(g, qx, qy, qx_bytes, qy_bytes, vol_inv, sino, sino_scale, blockIdx.x, blockIdx.y,
-                             blockIdx.z);
+__global__ __launch_bounds__(64 * kSidViews) void siddon_kernel(DevGeom g, const uint32_t* __restrict__ cols, float vol_inv,
+                                                     TS* __restrict__ sino, float sino_scale, int rows) {
+    siddon_tile<TV, TS, BUF>(g, cols, vol_inv, sino, sino_scale, rows,
+                             sid_group(blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, blockIdx.z), blockIdx.y, blockIdx.z);
 }
 
 // Shared launch: tiles are the single-problem grid's workgroups (column
-// group fastest, then view, then row group); FP32 or BF16 (kItemBF16) z-pair
+// group fastest, then view, then row group); FP32 or BF16 (kItemBF16) z-column
 // copies, FP32 sinograms.
-__global__ __launch_bounds__(BX* BY) void siddon_batch_kernel(const BatchTable* __restrict__ t, uint32_t* __restrict__ next) {
+__global__ __launch_bounds__(64 * kSidViews) void siddon_batch_kernel(const BatchTable* __restrict__ t, uint32_t* __restrict__ next) {
     TOMO_BATCH_CLAIMED(t, next) {
         const BatchItem& it = t->item[batch_find(t, tile)];
         const uint32_t local = tile - it.begin;
-        const uint32_t bx = local % it.gx, rest = local / it.gx;
+        const uint32_t rest = local / it.gx;
         const int by = (int)(rest % it.gy), bz = (int)(rest / it.gy);
+        const int bx = sid_group(local % it.gx, it.gx, (uint32_t)by, it.gy, (uint32_t)bz);
         const bool bf = (it.flags & kItemBF16) != 0;
-        const uint64_t es = bf ? 2ull : 4ull;
-        const uint64_t qxb = zpair_elems_x(it.g.nx, it.g.ny, it.g.nz) * es;
-        const uint64_t qyb = zpair_elems_y(it.g.nx, it.g.ny, it.g.nz) * es;
-        const bool buf = qxb < kSidOutside && qyb < kSidOutside;
+        const bool buf = zcol_words(it.g.nx, it.g.ny, it.g.nz, bf ? 2 : 4) * 4u < kSidOutside;
+        const int rows = sid_wave_rows(it.g.nv);
+        const uint32_t* cols = (const uint32_t*)it.in;
         using BF = __hip_bfloat16;
         if (bf && buf)
-            siddon_tile<BF, float, true>(it.g, (const BF*)it.in, (const BF*)it.in2, (unsigned)qxb, (unsigned)qyb, 1.0f,
-                                         (float*)it.out, 1.0f, (int)bx, by, bz);
+            siddon_tile<BF, float, true>(it.g, cols, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else if (bf)
-            siddon_tile<BF, float, false>(it.g, (const BF*)it.in, (const BF*)it.in2, 0u, 0u, 1.0f, (float*)it.out,
-                                          1.0f, (int)bx, by, bz);
+            siddon_tile<BF, float, false>(it.g, cols, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else if (buf)
-            siddon_tile<float, float, true>(it.g, (const float*)it.in, (const float*)it.in2, (unsigned)qxb,
-                                            (unsigned)qyb, 1.0f, (float*)it.out, 1.0f, (int)bx, by, bz);
+            siddon_tile<float, float, true>(it.g, cols, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else
-            siddon_tile<float, float, false>(it.g, (const float*)it.in, (const float*)it.in2, 0u, 0u, 1.0f,
-                                             (float*)it.out, 1.0f, (int)bx, by, bz);
+            siddon_tile<float, float, false>(it.g, cols, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
     }
 }
 
@@ -999,38 +909,37 @@ int launch_siddon(const tomo_geom* g, int compat, Buf vol, MutBuf sino, hipStrea
         TOMO_HIP(fe);
         return TOMO_OK;
     }
-    // z-pair copies of the volume for x slabs and y slabs (stream-ordered
-    // pool allocations, released after the projection on the same stream).
+    // z-column copy of the volume (a stream-ordered pool allocation, released
+    // after the projection on the same stream)
     const size_t es = vol.dtype == TOMO_F32 ? 4 : 2;
-    const size_t qx_elems = zpair_elems_x(d.nx, d.ny, d.nz), qy_elems = zpair_elems_y(d.nx, d.ny, d.nz);
-    if (qx_elems >= (1ull << 32) || qy_elems >= (1ull << 32))
+    if (zpair_elems_x(d.nx, d.ny, d.nz) >= (1ull << 32) || zpair_elems_y(d.nx, d.ny, d.nz) >= (1ull << 32))
         return fail(TOMO_ERR_UNSUPPORTED, "volume too large for the 32-bit traversal index of the Siddon projector");
-    const size_t qx_bytes = qx_elems * es, qy_bytes = qy_elems * es;
-    ZPairs zp;
-    hipError_t le = zp.alloc(vol.p, es, d.nx, d.ny, d.nz, s, x);
+    ZColumns zc;
+    hipError_t le = zc.alloc(vol.p, es, d.nx, d.ny, d.nz, s, x);
     if (le == hipSuccess) {
-        const bool buf = qx_bytes < kSidOutside && qy_bytes < kSidOutside && !x.index_reads;
+        const bool buf = zcol_words(d.nx, d.ny, d.nz, es) * 4u < kSidOutside && !x.index_reads;
+        const int rows = sid_wave_rows(d.nv);
+        const dim3 cgrid(sid_groups(d.nu, rows), ceil_div(d.nphi, kSidViews), ceil_div(d.nv, rows));
         TOMO_DISPATCH_STORAGE(vol.dtype, TV, {
             TOMO_DISPATCH_STORAGE(sino.dtype, TS, {
                 if (buf)
-                    hipLaunchKernelGGL((siddon_kernel<TV, TS, true>), grid, dim3(BX, BY), 0, s, d, (const TV*)zp.qx,
-                                       (const TV*)zp.qy, (unsigned)qx_bytes, (unsigned)qy_bytes, inv, (TS*)sino.p,
-                                       sino.scale);
+                    hipLaunchKernelGGL((siddon_kernel<TV, TS, true>), cgrid, dim3(64 * kSidViews), 0, s, d, zc.p, inv,
+                                       (TS*)sino.p, sino.scale, rows);
                 else
-                    hipLaunchKernelGGL((siddon_kernel<TV, TS, false>), grid, dim3(BX, BY), 0, s, d, (const TV*)zp.qx,
-                                       (const TV*)zp.qy, 0u, 0u, inv, (TS*)sino.p, sino.scale);
+                    hipLaunchKernelGGL((siddon_kernel<TV, TS, false>), cgrid, dim3(64 * kSidViews), 0, s, d, zc.p, inv,
+                                       (TS*)sino.p, sino.scale, rows);
             });
         });
         le = hipGetLastError();
     }
-    const hipError_t fe = zp.release(s);
+    const hipError_t fe = zc.release(s);
     TOMO_HIP(le);
     TOMO_HIP(fe);
     return TOMO_OK;
 }
 
 hipError_t launch_batch_siddon(BatchTable* t, hipStream_t s) {
-    hipLaunchKernelGGL(siddon_batch_kernel, dim3(kBatchGrid), dim3(BX, BY), 0, s, t, t->next);
+    hipLaunchKernelGGL(siddon_batch_kernel, dim3(kBatchGrid), dim3(64 * kSidViews), 0, s, t, t->next);
     return hipGetLastError();
 }
 

@@ -378,6 +378,57 @@ __global__ __launch_bounds__(256) void zpair_x_kernel(const T* __restrict__ in, 
     }
 }
 
+// z-column copy (zpair.hpp): the tile of 64 x and 64 words of each of their
+// columns at row y, transposed through LDS (65 planes for the 16-bit pairs).
+// TI: float or uint32_t (bits) for FP32 words; uint16_t (bits) or float (rounded
+// to BF16) for PAIR words.  One row of y per tile keeps even a 64^3 volume's
+// copy spread over the chip.
+constexpr int kColLds = 65;
+template <typename TI, bool PAIR>
+__device__ __forceinline__ void zcol_tile(const TI* __restrict__ in, uint32_t* __restrict__ out, int nx, int ny, int nz,
+                                          int bx, int y, int bz, uint32_t (*tile)[kColLds]) {
+    using T = typename std::conditional<PAIR, uint16_t, uint32_t>::type;
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4
+    const int x = bx * kColTile + tx, z0 = bz * kColTile - 1;  // plane of the tile's first row
+    const TI* col = in + (size_t)min(x, nx - 1) + (size_t)nx * y;
+    const size_t zs = (size_t)nx * ny;
+    // clamped addresses and masks (the elements are integers), so that no load is a branch
+    auto fetch = [&](int r) {
+        const int z = z0 + r;
+        uint32_t m = 0u - (uint32_t)((z >= 0) & (z < nz));
+        asm("" : "+v"(m));
+        return (uint32_t)(copy_cvt<T>(col[zs * (size_t)min(max(z, 0), nz - 1)])) & m;
+    };
+    uint32_t v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = fetch(ty + 4 * j);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) tile[ty + 4 * j][tx] = v[j];
+    if (PAIR && ty == 0) tile[64][tx] = fetch(64);
+    __syncthreads();
+    const int pz = (int)zcol_pitch(nz, PAIR ? 2 : 4);
+    const int zz = bz * kColTile + tx;
+    if (zz < pz) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int r = ty + 4 * j, xo = bx * kColTile + r;
+            const uint32_t w = PAIR ? tile[tx][r] | (tile[tx + 1][r] << 16) : tile[tx][r];
+            if (xo < nx) out[((size_t)xo * ny + y) * (size_t)pz + zz] = w;
+        }
+    }
+}
+
+// One workgroup per tile, tiles in (x, y, z) order.
+template <typename TI, bool PAIR>
+__global__ __launch_bounds__(256) void zcol_kernel(const TI* __restrict__ in, uint32_t* __restrict__ out, int nx, int ny,
+                                                 int nz) {
+    __shared__ uint32_t tile[kColTile + 1][kColLds];
+    const uint32_t gx = (uint32_t)(nx + kColTile - 1) / kColTile;
+    const uint32_t b = blockIdx.x, rest = b / gx;
+    zcol_tile<TI, PAIR>(in, out, nx, ny, nz, (int)(b % gx), (int)(rest % (uint32_t)ny), (int)(rest / (uint32_t)ny),
+                        tile);
+}
+
 // One A-pair group (four 16-bit elements at an index that is a multiple of
 // four) as one aligned 8-byte store.
 __device__ __forceinline__ void store_group(uint16_t* __restrict__ out, size_t o, uint16_t a, uint16_t b, uint16_t c,
@@ -485,6 +536,7 @@ __global__ __launch_bounds__(256) void zpair_x_batch_kernel(const BatchTable* __
     __shared__ uint32_t tile_lds[2][32][33];
     __shared__ uint16_t tile_lds16[2][32][33];
     __shared__ uint16_t tile_ap[2][32][34];
+    __shared__ uint32_t tile_col[kColTile + 1][kColLds];
     TOMO_BATCH_STRIDED(t) {
         const BatchItem& it = t->item[batch_find(t, tile)];
         int bx, by, bz;
@@ -492,6 +544,12 @@ __global__ __launch_bounds__(256) void zpair_x_batch_kernel(const BatchTable* __
         if (it.flags & kItemApair)
             apair_x_tile<float>((const float*)it.in, (uint16_t*)it.out, it.g.nx, it.g.ny, it.g.nz, bx, by, bz,
                                 tile_ap);
+        else if ((it.flags & kItemZcol) && (it.flags & kItemBF16))
+            zcol_tile<float, true>((const float*)it.in, (uint32_t*)it.out, it.g.nx, it.g.ny, it.g.nz, bx, by, bz,
+                                   tile_col);
+        else if (it.flags & kItemZcol)
+            zcol_tile<uint32_t, false>((const uint32_t*)it.in, (uint32_t*)it.out, it.g.nx, it.g.ny, it.g.nz, bx, by, bz,
+                                       tile_col);
         else if (it.flags & kItemBF16)
             zpair_x_tile<float, uint16_t>((const float*)it.in, (uint16_t*)it.out, it.g.nx, it.g.ny, it.g.nz, bx, by,
                                           bz, tile_lds16);
@@ -688,6 +746,17 @@ hipError_t launch_apair(const void* vol, void* qx, void* qy, int nx, int ny, int
     const dim3 gy(ceil_div((size_t)nx + 2, 256), ny + 1, nz + 1);
     hipLaunchKernelGGL(apair_x_kernel, gx, dim3(256), 0, s, (const uint16_t*)vol, (uint16_t*)qx, nx, ny, nz);
     hipLaunchKernelGGL(apair_y_kernel, gy, dim3(256), 0, s, (const uint16_t*)vol, (uint16_t*)qy, nx, ny, nz);
+    return hipGetLastError();
+}
+
+hipError_t launch_zcol(const void* vol, uint32_t* out, size_t es, int nx, int ny, int nz, hipStream_t s) {
+    const size_t tiles = (size_t)ceil_div(nx, kColTile) * ny * ceil_div(zcol_pitch(nz, es), kColTile);
+    if (es == 4)
+        hipLaunchKernelGGL((zcol_kernel<uint32_t, false>), dim3((unsigned)tiles), dim3(256), 0, s, (const uint32_t*)vol,
+                           out, nx, ny, nz);
+    else
+        hipLaunchKernelGGL((zcol_kernel<uint16_t, true>), dim3((unsigned)tiles), dim3(256), 0, s, (const uint16_t*)vol,
+                           out, nx, ny, nz);
     return hipGetLastError();
 }
 

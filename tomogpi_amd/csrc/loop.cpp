@@ -44,8 +44,8 @@ struct PoolBuf {
     }
 };
 
-// The projector's two copies (z-pair, or A-pair for RS on 16-bit volumes:
-// RS loops size them for the larger), allocated once for a loop's run and
+// The projector's copies (z-columns for Siddon; z-pair, or A-pair on 16-bit
+// volumes, for RS, sized for the larger), allocated once for a loop's run and
 // passed to each of its projections (which otherwise take them from the
 // stream-ordered pool per call: two volume-sized allocations per projection,
 // whose pool allocations stalled the host for up to seconds now and then
@@ -63,8 +63,8 @@ struct LoopCopies {
             return TOMO_OK;
         const size_t es = storage == TOMO_F32 ? 4 : 2;
         const bool rs = pr.pair != TOMO_PAIR_SIDDONVI;
-        TOMO_HIP(qx.alloc(rs ? proj_copy_bytes_x(nx, ny, nz, es) : zpair_elems_x(nx, ny, nz) * es, s));
-        TOMO_HIP(qy.alloc(rs ? proj_copy_bytes_y(nx, ny, nz, es) : zpair_elems_y(nx, ny, nz) * es, s));
+        TOMO_HIP(qx.alloc(rs ? proj_copy_bytes_x(nx, ny, nz, es) : zcol_words(nx, ny, nz, es) * 4, s));
+        if (rs) TOMO_HIP(qy.alloc(proj_copy_bytes_y(nx, ny, nz, es), s));
         extra.qx = qx.p;
         extra.qy = qy.p;
         return TOMO_OK;

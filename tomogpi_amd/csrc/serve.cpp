@@ -150,9 +150,11 @@ Layout layout_of(const tomo_geom& g, const tomo_gd_params& gd, int algo, size_t 
     sizes[i++] = (lam || sirt) ? nv * 4 : 0;                             // 4 t1 (SIRT: volume weight C)
     sizes[i++] = lam ? nv * 4 : 0;                                       // 5 t2
     sizes[i++] = lam ? nv * 4 : 0;                                       // 6 t3
-    const bool ap = apair_copies(d, gd, ces);
-    sizes[i++] = (ap ? apair_elems_x(d.nx, d.ny, d.nz) : zpair_elems_x(d.nx, d.ny, d.nz)) * ces;  // 7 qx
-    sizes[i++] = (ap ? apair_elems_y(d.nx, d.ny, d.nz) : zpair_elems_y(d.nx, d.ny, d.nz)) * ces;  // 8 qy
+    const bool ap = apair_copies(d, gd, ces), sid = gd.pair == TOMO_PAIR_SIDDONVI;
+    sizes[i++] = sid ? zcol_words(d.nx, d.ny, d.nz, ces) * 4             // 7 qx (Siddon: the z-column copy)
+                     : (ap ? apair_elems_x(d.nx, d.ny, d.nz) : zpair_elems_x(d.nx, d.ny, d.nz)) * ces;
+    sizes[i++] = sid ? 0                                                 // 8 qy
+                     : (ap ? apair_elems_y(d.nx, d.ny, d.nz) : zpair_elems_y(d.nx, d.ny, d.nz)) * ces;
     sizes[i++] = ns * 4;                                                 // 9 y
     sizes[i++] = ns * 4;                                                 // 10 px
     sizes[i++] = ns * 4;                                                 // 11 r
@@ -292,6 +294,18 @@ void build_tables(tomo_server* srv, int set, const std::vector<Request*>& runnin
         const bool ap = apair_copies(d, gd, q.bf16 ? 2 : 4);
         const int32_t cflag = (q.bf16 ? kItemBF16 : 0) | (ap ? kItemApair : 0);  // operator copies
         auto add_projection = [&](const float* vol, float* out, int opx, int opy, int ops, int opr) {
+            if (sid) {
+                BatchItem& z = tb[opx].add(d, cdiv(d.nx, kColTile), d.ny, cdiv(zcol_pitch(d.nz, q.bf16 ? 2 : 4), kColTile));
+                z.in = vol;
+                z.out = q.qx;
+                z.flags = cflag | kItemZcol;
+                const int rows = sid_wave_rows(d.nv);
+                BatchItem& p = tb[ops].add(d, sid_groups(d.nu, rows), cdiv(d.nphi, kSidViews), cdiv(d.nv, rows));
+                p.in = q.qx;
+                p.out = out;
+                p.flags = cflag;
+                return;
+            }
             BatchItem& zx = ap ? tb[opx].add(d, cdiv(d.nx + 1, 32), cdiv(d.ny + 2, 32), d.nz + 1)
                                : tb[opx].add(d, cdiv(d.nx, 32), cdiv(d.ny + 2, 32), d.nz + 1);
             zx.in = vol;
@@ -301,7 +315,7 @@ void build_tables(tomo_server* srv, int set, const std::vector<Request*>& runnin
             zy.in = vol;
             zy.out = q.qy;
             zy.flags = cflag;
-            BatchItem& p = tb[sid ? ops : opr].add(d, pgx, d.nphi, pgz);
+            BatchItem& p = tb[opr].add(d, pgx, d.nphi, pgz);
             p.in = q.qx;
             p.in2 = q.qy;
             p.out = out;

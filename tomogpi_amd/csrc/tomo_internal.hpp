@@ -70,6 +70,28 @@ namespace tomo {
 // slabs (qy): nA * (nz+1) * (nB+2) pairs.
 __host__ __device__ inline size_t zpair_elems_x(int nx, int ny, int nz) { return (size_t)nx * (nz + 1) * (ny + 2) * 2; }
 __host__ __device__ inline size_t zpair_elems_y(int nx, int ny, int nz) { return (size_t)ny * (nz + 1) * (nx + 2) * 2; }
+// z-column copy of a volume of es-byte elements (zpair.hpp): 4-byte words per
+// (x, y) column, and of the whole copy.
+__host__ __device__ inline uint32_t zcol_pitch(int nz, size_t es) { return (uint32_t)nz + (es == 4 ? 2u : 1u); }
+__host__ __device__ inline size_t zcol_words(int nx, int ny, int nz, size_t es) {
+    return (size_t)nx * ny * zcol_pitch(nz, es);
+}
+// Detector rows of a Siddon wave (64, 32 or 16, by 64 / rows columns): the most
+// that leave no more than an eighth of the row groups' lanes idle.  Fewer rows
+// read shorter runs of z per cell, idle lanes read none.
+__host__ __device__ inline int sid_wave_rows(int nv) {
+    for (int r = 64; r > 16; r >>= 1)
+        if (((nv + r - 1) / r * r - nv) * 8 <= nv) return r;
+    return 16;
+}
+// A Siddon workgroup: one wave's detector cells in kSidViews consecutive views.
+constexpr int kSidViews = 4;
+// Column groups (workgroups) of a row band, rounded up to a multiple of the 8
+// XCDs.
+inline uint32_t sid_groups(int nu, int rows) {
+    const uint32_t cols = 64u / (uint32_t)rows;
+    return ((uint32_t)nu + 8u * cols - 1u) / (8u * cols) * 8u;
+}
 // Element counts of the A-pair copies (16-bit volumes, RS): (nA+1) * (nz+1)
 // * (nB+2) groups of four elements (zpair.hpp).
 __host__ __device__ inline size_t apair_elems_x(int nx, int ny, int nz) { return (size_t)(nx + 1) * (nz + 1) * (ny + 2) * 4; }

@@ -18,6 +18,12 @@
 // (planes -1 and nA are 0), B varying fastest; two neighbouring groups are the
 // eight taps of a sample with lower corner (ap-1, bb-1, zz-1), one 16-byte
 // load.  Each copy holds (nA+1) * (nz+1) * (nB+2) * 4 elements.
+//
+// The z-column copy (read by the Siddon projector) has z fastest, then y, then
+// x.  FP32: word (x, y, zz), zz in [0, nz+1], is f(x, y, zz-1), 0 for the
+// planes -1 and nz; two neighbouring words are a voxel and the one above it.
+// 16-bit volumes: word (x, y, zz), zz in [0, nz], holds f(x, y, zz-1) in its low
+// half and f(x, y, zz) in its high half, so that one aligned word is the two.
 #pragma once
 
 #include "device_common.hpp"
@@ -35,6 +41,33 @@ __device__ __forceinline__ size_t apair_index(int ap, int zz, int bb, int nz, in
 
 // Fills qx and qy from an x-fastest volume of es-byte elements (es 4 or 2).
 hipError_t launch_zpair(const void* vol, void* qx, void* qy, size_t es, int nx, int ny, int nz, hipStream_t s);
+
+// Fills the z-column copy at `out` from an x-fastest volume of es-byte elements.
+hipError_t launch_zcol(const void* vol, uint32_t* out, size_t es, int nx, int ny, int nz, hipStream_t s);
+
+// The z-column copy for the duration of one operator call: alloc() then
+// release() on the same stream.  The memory comes from the stream-ordered
+// pool, or is the caller's (ProjExtra::qx).
+struct ZColumns {
+    uint32_t* p = nullptr;
+    bool owned = false;
+    hipError_t alloc(const void* vol, size_t es, int nx, int ny, int nz, hipStream_t s, const ProjExtra& x) {
+        hipError_t e = hipSuccess;
+        p = (uint32_t*)x.qx;
+        if (!p) {
+            owned = true;
+            e = hipMallocAsync((void**)&p, zcol_words(nx, ny, nz, es) * 4, s);
+        }
+        if (e == hipSuccess) e = launch_zcol(vol, p, es, nx, ny, nz, s);
+        return e;
+    }
+    hipError_t release(hipStream_t s) {
+        const hipError_t e = owned && p ? hipFreeAsync(p, s) : hipSuccess;
+        p = nullptr;
+        owned = false;
+        return e;
+    }
+};
 
 // Fills the A-pair copies qx and qy from an x-fastest 16-bit volume.
 hipError_t launch_apair(const void* vol, void* qx, void* qy, int nx, int ny, int nz, hipStream_t s);
