@@ -59,3 +59,13 @@ def test_siddon_steep_rays(ctx, nz):
 def test_siddon_column_runs(ctx):
     """A detector wide enough that each of the eight column runs holds several groups, row bands and view groups."""
     _check(ctx, scaled_geometry(48, 37, nu=150, nv=70), "siddon", "f32")
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 31), (31, 64), (64, 63)])
+def test_siddon_narrow_grid(ctx, nx, ny):
+    """A grid narrower than the FOV in y: rays enter the FOV outside it, cross
+    several z planes before their first x or y plane (the border voxel's
+    stretch), and do so in their second cell where the first crossing is x's."""
+    g = Geometry(fod=80.0, fdd=160.0, nphi=48, su=64 * 2.0, sv=64 * 2.4, nu=64, nv=64, sx=float(nx), sy=float(ny),
+                 sz=70.0, nx=nx, ny=ny, nz=70, num_start=0.0, den_start=1.0, num_stop=2.0, den_stop=1.0)
+    _check(ctx, g, "siddon", "f32")

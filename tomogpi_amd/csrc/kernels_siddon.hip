@@ -356,10 +356,12 @@ __device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __
     const bool ok = r.ok && r.tmax > 0.0f;
     // The z crossings of the ray are spaced farther apart than the longest
     // stretch in one cell, by more than two ulps of tmax; else the wave takes
-    // the general step.
+    // the general step.  The crossings of x (y) are ix (iy) apart, but the first
+    // may come later: a FOV entry outside a grid narrower than the FOV is
+    // clamped to the border voxel.
     const float big = 3.0e38f;
     const float ix = r.step[0] ? r.inc[0] : big, iy = r.step[1] ? r.inc[1] : big, iz = r.step[2] ? r.inc[2] : big;
-    const float cell = fmaxf(fminf(ix, iy), fminf(fminf(r.first[0], r.first[1]), r.tmax));
+    const float cell = fminf(fminf(fmaxf(ix, r.first[0]), fmaxf(iy, r.first[1])), r.tmax);
     const bool walk = __ballot(ok && !(iz > cell + 1.0e-6f * r.tmax)) == 0ull;
     const int ny = g.ny, nz = g.nz;
     const uint32_t pz = zcol_pitch(nz, sizeof(TV)), py = pz * (uint32_t)ny;
