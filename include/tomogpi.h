@@ -79,7 +79,7 @@ extern "C" {
                                         34-35): f = sum_p W_p bilinear(g_p),
                                         W_p = alphaC (FDD/du) / w^2 /
                                         sqrt(betaC + u'^2 + v'^2), no delta   */
-#define TOMO_FLAG_INDEX_READS   0x10 /* RS, clean Siddon: read the z-pair copies
+#define TOMO_FLAG_INDEX_READS   0x10 /* RS, clean Siddon: read the volume's copy
                                         through 64-bit element indices, the
                                         form every copy of 4 GiB or more
                                         takes (1024^3 in FP32 or 16-bit),
@@ -91,7 +91,7 @@ extern "C" {
                                         rays cross, a window of slabs at a
                                         time, in LDS and reads its taps there
                                         instead of gathering them per lane
-                                        from the z-pair copies; same results */
+                                        from a copy of the volume; same results */
 
 typedef struct tomo_ctx  tomo_ctx;
 typedef struct tomo_geom tomo_geom;
@@ -385,7 +385,7 @@ typedef struct tomo_serve_request {
     float*       volume;        /* result, written when the request is done */
     int32_t      algorithm;     /* TOMO_ALGO_*                              */
     int32_t      storage;       /* element type of the operator copies (the
-                                   z-pair copies the projectors read):
+                                   copies the projectors read):
                                    TOMO_F32 (0) or TOMO_BF16, rounded from
                                    the FP32 state each time they are made;
                                    VI reads the FP32 residual, and the

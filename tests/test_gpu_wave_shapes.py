@@ -46,6 +46,19 @@ def test_siddon_wave_shapes(ctx, nv, nu, nphi, nz, dt):
     _check(ctx, g, "siddon", dt)
 
 
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("op", ["rs", "rs_cube"])
+@pytest.mark.parametrize("nv,nu,nphi,nz,ny", [
+    (1, 5, 1, 1, 33), (15, 9, 3, 62, 37), (28, 8, 5, 63, 12), (29, 17, 4, 64, 37), (33, 65, 7, 65, 40), (70, 10, 6, 126, 37),
+])
+def test_rs_wave_shapes(ctx, nv, nu, nphi, nz, ny, op, dt):
+    """Waves of 16 and 32 rows; volumes narrower than the FOV in y (samples off
+    the grid, tested one by one) and not (untested up to the shortest ray)."""
+    g = Geometry(fod=90.0, fdd=180.0, nphi=nphi, su=nu * 2.0, sv=nv * 1.6, nu=nu, nv=nv, sx=37.0, sy=float(ny),
+                 sz=float(nz), nx=37, ny=ny, nz=nz, num_start=1.0, den_start=7.0, num_stop=15.0, den_stop=8.0)
+    _check(ctx, g, op, dt)
+
+
 @pytest.mark.parametrize("nz", [40, 41])
 def test_siddon_steep_rays(ctx, nz):
     """Rays up to 70 degrees off the mid plane: several z planes per in-plane

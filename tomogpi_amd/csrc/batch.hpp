@@ -51,21 +51,19 @@ struct ViBox {
 inline size_t vi_box_count(const DevGeom& d) {
     return (size_t)((d.nx + kViStageX - 1) / kViStageX) * ((d.ny + kViStageY - 1) / kViStageY) * d.nphi;
 }
-// Projector workgroup (RS, Siddon): kProjTileU detector columns x kProjTileV
-// rows of one view; a wave is 32 columns x 2 rows, rays close enough to
-// enter and leave the FOV within a few slabs of each other (the waves walk
-// slabs or samples in lockstep).
+// Workgroup of the projectors' LDS-staged forms, transposes and counters:
+// kProjTileU detector columns x kProjTileV rows of one view.
 constexpr int kProjTileU = 32, kProjTileV = 8;
-// Tile of the z-column copies: kColTile x by kColTile words of their columns, one y.
+// Tile of the projectors' copies: kColTile x by kColTile words of their columns, one y.
 constexpr int kColTile = 64;
 
 struct BatchItem {
     DevGeom g;
     const void* in;   // operator input / first element-wise operand
-    const void* in2;  // second input (z-pair qy, element-wise operand b)
+    const void* in2;  // second input (element-wise operand b)
     const void* in3;  // per-element weight of the element-wise ops (SIRT), or null
     void* out;        // output
-    void* aux;        // second output (z-pair qy) or FP64 partial sums (one per tile)
+    void* aux;        // second input (VI box table) or FP64 partial sums (one per tile)
     double* slot;     // per-problem FP64 scalars
     uint64_t n;       // element count (element-wise ops)
     uint32_t begin, tiles;
@@ -86,16 +84,11 @@ struct BatchTable {
 };
 static_assert(kBatchGrid % kBatchXcds == 0, "every XCD starts with the same number of workgroups");
 
-// Item flag bit of the projector launches: the operator copies (z-pairs) are
+// Item flag bit of the copy and projector launches: the operator copies are
 // BF16, converted from the FP32 state by the copy launches.  RS keeps bit 0
 // for the cube FOV.
 constexpr int32_t kItemBF16 = 0x10;
-// Item flag bit of the BF16 copy and RS launches: the copies are A-pair
-// copies (zpair.hpp), read with one load per RS sample.
-constexpr int32_t kItemApair = 0x20;
-
-// Item flag bit of the copy launches: the z-column copy (one item; BF16 pairs
-// with kItemBF16).
+// Item flag bit of the copy launches: the z-column copy instead of the RS copy.
 constexpr int32_t kItemZcol = 0x40;
 
 // Per-problem scalars of the gradient loop, FP64, in `slot`.
@@ -147,10 +140,9 @@ __device__ __forceinline__ int batch_find(const BatchTable* t, uint32_t tile) {
 
 // Shared launches (stream-ordered; `t` is a device copy of the table).
 // The state is FP32 throughout; operator copies are FP32 or BF16 (kItemBF16).
-hipError_t launch_batch_zpair_x(const BatchTable* t, hipStream_t s);   // in volume -> out qx (FP32/BF16)
-hipError_t launch_batch_zpair_y(const BatchTable* t, hipStream_t s);   // in volume -> out qy (FP32/BF16)
+hipError_t launch_batch_copy(const BatchTable* t, hipStream_t s);      // in volume -> out copy (FP32/BF16)
 hipError_t launch_batch_siddon(BatchTable* t, hipStream_t s);          // in z-column copy -> out sinogram
-hipError_t launch_batch_rs(BatchTable* t, hipStream_t s);              // in qx, in2 qy -> out; flags bit0 cube
+hipError_t launch_batch_rs(BatchTable* t, hipStream_t s);              // in RS copy -> out; flags bit0 cube
 // Grids of the shared launches whose workgroups take more registers than
 // kBatchGrid resident workgroups allow (RS): the number the device holds at
 // once, a multiple of kBatchXcds.  Called at context creation, before any

@@ -16,9 +16,10 @@
 // for rays parallel to y; the arc-length form here is well conditioned), the
 // samples and the sum are FP32.  The output is overwritten.
 #include <atomic>
+#include <climits>
 #include <type_traits>
 
-#include "zpair.hpp"
+#include "proj_copy.hpp"
 #include "batch.hpp"
 #include "stage_box.hpp"
 
@@ -99,195 +100,6 @@ __device__ __forceinline__ RsRay rs_setup(const DevGeom& g, int cube, int p, int
     return r;
 }
 
-// The trilinear blend of a sample's eight taps, given as the (B, z) quads of
-// its two A planes: u on plane floor(A), w on floor(A) + 1, each ordered
-// (b, z), (b, z+1), (b+1, z), (b+1, z+1).  Interpolated along x, then y, then
-// z with explicit fmaf.
-template <int A>
-__device__ __forceinline__ float trilinear_taps(float u0, float u1, float u2, float u3, float w0, float w1, float w2,
-                                                float w3, float fx, float fy, float fz) {
-    float t000, t100, t010, t110, t001, t101, t011, t111;
-    if (A == 0) {
-        t000 = u0; t001 = u1; t010 = u2; t011 = u3;
-        t100 = w0; t101 = w1; t110 = w2; t111 = w3;
-    } else {
-        t000 = u0; t001 = u1; t100 = u2; t101 = u3;
-        t010 = w0; t011 = w1; t110 = w2; t111 = w3;
-    }
-    const float c00 = fmaf(fx, t100 - t000, t000), c10 = fmaf(fx, t110 - t010, t010);
-    const float c01 = fmaf(fx, t101 - t001, t001), c11 = fmaf(fx, t111 - t011, t011);
-    const float c0 = fmaf(fy, c10 - c00, c00), c1 = fmaf(fy, c11 - c01, c01);
-    return fmaf(fz, c1 - c0, c0);
-}
-
-// Trilinear interpolation of f at (x, y, z) (voxel units), taps outside the
-// grid 0, interpolated along x, then y, then z with explicit fmaf.  The eight
-// taps come from two z-pair quads of the slab axis A: the (B, z) block of the
-// planes A = floor(A) and floor(A) + 1.  A = 0 reads qx (B = y), A = 1 reads
-// qy (B = x).  Outside the copy's corner range (B or z corner = n) the block
-// is entirely outside the grid and the quad is 0.
-template <int A, typename TV>
-__device__ __forceinline__ float trilinear_quads(const TV* __restrict__ q, int nx, int ny, int nz, float x, float y,
-                                                 float z, float inv) {
-    const float xf = floorf(x), yf = floorf(y), zf = floorf(z);
-    if (!(xf >= -1.0f && xf <= (float)nx && yf >= -1.0f && yf <= (float)ny && zf >= -1.0f && zf <= (float)nz))
-        return 0.0f;
-    const int ix = (int)xf, iy = (int)yf, iz = (int)zf;
-    const float fx = x - xf, fy = y - yf, fz = z - zf;
-    const int ia = A == 0 ? ix : iy, ib = A == 0 ? iy : ix;
-    const int nA = A == 0 ? nx : ny, nB = A == 0 ? ny : nx;
-    const bool blk = ib < nB && iz < nz;  // ib, iz >= -1 from the range test
-    const bool p0 = blk && ia >= 0 && ia < nA, p1 = blk && ia + 1 < nA;
-    const int bq = min(ib, nB - 1) + 1, zq = min(iz, nz - 1) + 1;
-    const float4 u = Storage<TV>::load4(q, zpair_index(min(max(ia, 0), nA - 1), zq, bq, nz, nB), inv);
-    const float4 w = Storage<TV>::load4(q, zpair_index(min(ia + 1, nA - 1), zq, bq, nz, nB), inv);
-    // u, w = (b, z), (b, z+1), (b+1, z), (b+1, z+1) on planes ia, ia+1
-    const float u0 = p0 ? u.x : 0.0f, u1 = p0 ? u.y : 0.0f, u2 = p0 ? u.z : 0.0f, u3 = p0 ? u.w : 0.0f;
-    const float w0 = p1 ? w.x : 0.0f, w1 = p1 ? w.y : 0.0f, w2 = p1 ? w.z : 0.0f, w3 = p1 ? w.w : 0.0f;
-    return trilinear_taps<A>(u0, u1, u2, u3, w0, w1, w2, w3, fx, fy, fz);
-}
-
-// Buffer-path sampler, for copies below 4 GiB whose A-plane stride is below
-// 2^24 bytes: 32-bit byte offsets from 24-bit multiply-adds, loads
-// issued unconditionally.  A buffer load at an offset past the copy's end
-// returns 0 and never faults, so an absent plane (outside the grid along A),
-// a sample whose cell has no voxel in the grid, or an inactive one (act
-// false) reads from kOutside: its taps are 0 and the interpolation gives +0,
-// the value the index forms return for it.  Corners are clamped before the integer conversion, which
-// keeps every offset well defined.  Same taps and arithmetic as above.
-constexpr uint32_t kOutside = 0xfffffff0u;
-
-struct CopyBuf {
-    __amdgpu_buffer_rsrc_t r;
-    uint32_t sa, sz;  // bytes per A plane and per z row
-};
-
-template <int A, typename TV>
-__device__ __forceinline__ float trilinear_quads_buf(const CopyBuf& q, int nx, int ny, int nz, float x, float y,
-                                                     float z, bool act) {
-    constexpr uint32_t es = sizeof(TV);  // a z-pair element is 2 es bytes
-    const float xf = floorf(x), yf = floorf(y), zf = floorf(z);
-    const float xc = __builtin_amdgcn_fmed3f(xf, -1.0f, (float)nx);
-    const float yc = __builtin_amdgcn_fmed3f(yf, -1.0f, (float)ny);
-    const float zc = __builtin_amdgcn_fmed3f(zf, -1.0f, (float)nz);
-    const bool in = act & (xc == xf) & (yc == yf) & (zc == zf);
-    const int ix = (int)xc, iy = (int)yc, iz = (int)zc;
-    const float fx = x - xf, fy = y - yf, fz = z - zf;
-    const int ia = A == 0 ? ix : iy, ib = A == 0 ? iy : ix;
-    const int nA = A == 0 ? nx : ny, nB = A == 0 ? ny : nx;
-    const bool blk = in & (ib < nB) & (iz < nz);
-    const bool p0 = blk & (ia >= 0) & (ia < nA), p1 = blk & (ia + 1 < nA);
-    const uint32_t bq = (uint32_t)(min(ib, nB - 1) + 1), zq = (uint32_t)(min(iz, nz - 1) + 1);
-    const uint32_t inner = __umul24(zq, q.sz) + bq * (2u * es);
-    const uint32_t o0 = p0 ? __umul24((uint32_t)max(ia, 0), q.sa) + inner : kOutside;
-    const uint32_t o1 = p1 ? __umul24((uint32_t)(ia + 1), q.sa) + inner : kOutside;
-    // u, w = (b, z), (b, z+1), (b+1, z), (b+1, z+1) on planes ia, ia+1
-    float u0, u1, u2, u3, w0, w1, w2, w3;
-    if constexpr (es == 4) {
-        const auto u = __builtin_amdgcn_raw_buffer_load_b128(q.r, (int)o0, 0, 0);
-        const auto w = __builtin_amdgcn_raw_buffer_load_b128(q.r, (int)o1, 0, 0);
-        u0 = __uint_as_float(u[0]); u1 = __uint_as_float(u[1]); u2 = __uint_as_float(u[2]); u3 = __uint_as_float(u[3]);
-        w0 = __uint_as_float(w[0]); w1 = __uint_as_float(w[1]); w2 = __uint_as_float(w[2]); w3 = __uint_as_float(w[3]);
-    } else {
-        using U = Unpack16<TV>;
-        const auto u = __builtin_amdgcn_raw_buffer_load_b64(q.r, (int)o0, 0, 0);
-        const auto w = __builtin_amdgcn_raw_buffer_load_b64(q.r, (int)o1, 0, 0);
-        u0 = U::lo(u[0]); u1 = U::hi(u[0]); u2 = U::lo(u[1]); u3 = U::hi(u[1]);
-        w0 = U::lo(w[0]); w1 = U::hi(w[0]); w2 = U::lo(w[1]); w3 = U::hi(w[1]);
-    }
-    return trilinear_taps<A>(u0, u1, u2, u3, w0, w1, w2, w3, fx, fy, fz);
-}
-
-// A-pair sampler through 64-bit element indices (16-bit volumes whose A-pair
-// copies are 4 GiB or more): one 16-byte load per sample, as below; a sample
-// outside the grid or whose block is returns 0, as trilinear_quads does.
-template <typename TV>
-__device__ __forceinline__ void apair_unpack(const uint32_t (&d)[4], float& u0, float& u1, float& u2, float& u3,
-                                             float& w0, float& w1, float& w2, float& w3) {
-    using U = Unpack16<TV>;
-    // d[0], d[1] = (a, b, z), (a, b, z+1), (a+1, b, z), (a+1, b, z+1); d[2], d[3]: the same at b + 1
-    u0 = U::lo(d[0]); u1 = U::hi(d[0]); w0 = U::lo(d[1]); w1 = U::hi(d[1]);
-    u2 = U::lo(d[2]); u3 = U::hi(d[2]); w2 = U::lo(d[3]); w3 = U::hi(d[3]);
-    if constexpr (std::is_same<TV, __half>::value) {
-        // Keep the FP16 taps as converted FP32 registers: otherwise the
-        // compiler folds their conversions into v_fma_mix_f32 operands, the
-        // same numbers at more issue time (RS at 512^3 / 512 views: 81.4 ms
-        // folded, 76.3 ms not).  An empty statement: it emits no instruction.
-        asm("" : "+v"(u0), "+v"(u1), "+v"(u2), "+v"(u3), "+v"(w0), "+v"(w1), "+v"(w2), "+v"(w3));
-    }
-}
-
-template <int A, typename TV>
-__device__ __forceinline__ float trilinear_apair(const TV* __restrict__ q, int nx, int ny, int nz, float x, float y,
-                                                 float z) {
-    static_assert(sizeof(TV) == 2, "A-pair copies hold 16-bit volumes");
-    const float xf = floorf(x), yf = floorf(y), zf = floorf(z);
-    if (!(xf >= -1.0f && xf <= (float)nx && yf >= -1.0f && yf <= (float)ny && zf >= -1.0f && zf <= (float)nz))
-        return 0.0f;
-    const int ix = (int)xf, iy = (int)yf, iz = (int)zf;
-    const float fx = x - xf, fy = y - yf, fz = z - zf;
-    const int ia = A == 0 ? ix : iy, ib = A == 0 ? iy : ix;
-    const int nA = A == 0 ? nx : ny, nB = A == 0 ? ny : nx;
-    if (!(ib < nB && iz < nz && ia < nA)) return 0.0f;  // every tap 0: the blend gives +0
-    const unsigned char* p =
-        (const unsigned char*)__builtin_assume_aligned(q + apair_index(ia + 1, iz + 1, ib + 1, nz, nB), 8);
-    uint32_t d[4];
-    __builtin_memcpy(d, p, 16);
-    float u0, u1, u2, u3, w0, w1, w2, w3;
-    apair_unpack<TV>(d, u0, u1, u2, u3, w0, w1, w2, w3);
-    return trilinear_taps<A>(u0, u1, u2, u3, w0, w1, w2, w3, fx, fy, fz);
-}
-
-// A-pair sampler (16-bit volumes, copies below 4 GiB): the eight taps are two
-// neighbouring groups of the A-pair copy (zpair.hpp), one 16-byte load where
-// the z-pair copy takes two.  Its planes -1 and nA are zeros of the copy, so
-// only a block outside the grid (B or z corner = n, A corner = nA) or an
-// inactive sample reads from kOutside.  Same taps and arithmetic as above.
-struct ApairShape {
-    uint64_t bytes_x, bytes_y;
-    uint32_t sa_x, sz_x, sa_y, sz_y;
-    bool buf;
-};
-__host__ __device__ __forceinline__ ApairShape rs_apair_shape(int nx, int ny, int nz) {
-    ApairShape c;
-    c.sz_x = (uint32_t)(ny + 2) * 8u;
-    c.sz_y = (uint32_t)(nx + 2) * 8u;
-    c.bytes_x = apair_elems_x(nx, ny, nz) * 2u;
-    c.bytes_y = apair_elems_y(nx, ny, nz) * 2u;
-    c.sa_x = c.sz_x * (uint32_t)(nz + 1);
-    c.sa_y = c.sz_y * (uint32_t)(nz + 1);
-    c.buf = apair_buffer_path(nx, ny, nz);
-    return c;
-}
-
-template <int A, typename TV>
-__device__ __forceinline__ float trilinear_apair_buf(const CopyBuf& q, int nx, int ny, int nz, float x, float y,
-                                                     float z, bool act) {
-    static_assert(sizeof(TV) == 2, "A-pair copies hold 16-bit volumes");
-    const float xf = floorf(x), yf = floorf(y), zf = floorf(z);
-    const float xc = __builtin_amdgcn_fmed3f(xf, -1.0f, (float)nx);
-    const float yc = __builtin_amdgcn_fmed3f(yf, -1.0f, (float)ny);
-    const float zc = __builtin_amdgcn_fmed3f(zf, -1.0f, (float)nz);
-    const bool in = act & (xc == xf) & (yc == yf) & (zc == zf);
-    const int ix = (int)xc, iy = (int)yc, iz = (int)zc;
-    const float fx = x - xf, fy = y - yf, fz = z - zf;
-    const int ia = A == 0 ? ix : iy, ib = A == 0 ? iy : ix;
-    const int nA = A == 0 ? nx : ny, nB = A == 0 ? ny : nx;
-    const bool blk = in & (ib < nB) & (iz < nz) & (ia < nA);  // ia >= -1 from the clamp
-    const uint32_t bq = (uint32_t)(min(ib, nB - 1) + 1), zq = (uint32_t)(min(iz, nz - 1) + 1);
-    const uint32_t ap = (uint32_t)(min(ia, nA - 1) + 1);
-    // kOutside unless blk, as a mask: a select of the offset would let the
-    // compiler move its arithmetic into a branch, which splits the unrolled
-    // samples and serialises their loads
-    const uint32_t keep = 0u - (uint32_t)blk;
-    const uint32_t o = ((__umul24(ap, q.sa) + __umul24(zq, q.sz) + bq * 8u) & keep) | (kOutside & ~keep);
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(q.r, (int)o, 0, 0);
-    const uint32_t d[4] = {v[0], v[1], v[2], v[3]};
-    float u0, u1, u2, u3, w0, w1, w2, w3;
-    apair_unpack<TV>(d, u0, u1, u2, u3, w0, w1, w2, w3);
-    return trilinear_taps<A>(u0, u1, u2, u3, w0, w1, w2, w3, fx, fy, fz);
-}
-
 __device__ __forceinline__ int wave_min(int v) {
     for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
     return v;
@@ -297,178 +109,229 @@ __device__ __forceinline__ int wave_max(int v) {
     return v;
 }
 
-__device__ __forceinline__ float wave_minf(float v) {
-    for (int off = 32; off > 0; off >>= 1) v = fminf(v, __shfl_xor(v, off, 64));
-    return v;
-}
+// Reads of the RS copy (proj_copy.hpp): 8-byte elements, z fastest; the element of
+// the lower corner (floor x, floor y, floor z) and the next one are 16 bytes.
+// FP32 elements are x pairs, so the eight taps are two 16-byte loads, at rows y
+// and y + 1; 16-bit ones hold the four voxels of a (x, y) cell: one load.
+// BUF: by 32-bit byte offset through a buffer resource; an offset past its end
+// reads 0 without touching memory.  Otherwise by 64-bit element index, and a
+// sample that is not reads element 0, a border element.
+constexpr uint32_t kOutside = 0xfffffff0u;
 
-// Samples of one lane, taken one per iteration k of the wave's loop: sample
-// s = k - k0 for k0 <= k < k0 + lr.  Same positions (fma(s, d, entry)) and
-// the same order of the sum as the per-ray loop.
-// q is the z-pair copy of A (FP32 or 16-bit, as stored); BUF reads it
-// through qb (see the buffer-path samplers); AP (16-bit volumes) reads the
-// A-pair copy of A instead, through qb or 64-bit indices.  The buffer path
-// has no branch: RS_UNROLL samples per iteration, their loads in flight
-// together, an inactive sample (s outside [0, lr)) adding +0 in its place,
-// which leaves the sum unchanged (it starts at +0 and is never -0).
-#ifndef RS_UNROLL
-#define RS_UNROLL 4
-#endif
-template <int A, typename TV, bool BUF, bool AP>
-__device__ __forceinline__ float rs_samples(const RsRay& r, const void* __restrict__ q, const CopyBuf& qb, int nx,
-                                            int ny, int nz, int k0, int kend) {
-    float acc = 0.0f;
-    if constexpr (BUF) {
-        for (int k = 0; k < kend; k += RS_UNROLL) {
-            float v[RS_UNROLL];
-#pragma unroll
-            for (int j = 0; j < RS_UNROLL; ++j) {
-                const int s = k + j - k0;
-                const float sf = (float)s;
-                const float x = fmaf(sf, r.dx, r.ex), y = fmaf(sf, r.dy, r.ey), z = fmaf(sf, r.dz, r.ez);
-                const bool act = (s >= 0) & (s < r.lr);
-                if constexpr (AP) v[j] = trilinear_apair_buf<A, TV>(qb, nx, ny, nz, x, y, z, act);
-                else v[j] = trilinear_quads_buf<A, TV>(qb, nx, ny, nz, x, y, z, act);
-            }
-#pragma unroll
-            for (int j = 0; j < RS_UNROLL; ++j) acc += v[j];
-        }
-    } else {
-        for (int k = 0; k < kend; ++k) {
-            const int s = k - k0;
-            if (s >= 0 && s < r.lr) {
-                const float sf = (float)s;
-                const float x = fmaf(sf, r.dx, r.ex), y = fmaf(sf, r.dy, r.ey), z = fmaf(sf, r.dz, r.ez);
-                if constexpr (AP) acc += trilinear_apair<A, TV>((const TV*)q, nx, ny, nz, x, y, z);
-                else acc += trilinear_quads<A>((const TV*)q, nx, ny, nz, x, y, z, 1.0f);
-            }
+// The corner's taps interpolated along x: c00 at (y, z), c10 at (y+1, z), c01 at
+// (y, z+1), c11 at (y+1, z+1).
+struct RsRows {
+    float c00, c10, c01, c11;
+};
+
+template <typename TV, bool BUF> struct RsReader {
+    __amdgpu_buffer_rsrc_t r;
+    const uint2* p;
+    uint32_t sx, sy;  // elements per x and y step; BUF: bytes
+    float syf, mz;    // BUF: sy, and 2^23 + the offset of floors (0, 0) from (-1, -1) in (y, z)
+    size_t base;      // index of the element of floors (0, 0, 0)
+    using Off = typename std::conditional<BUF, uint32_t, size_t>::type;
+    // Offset of the element of the floors, each in [-1, n - 1].  BUF: the
+    // (y, z) part as exact FP32 integers below 2^24 (sx < 2^23), whose bits
+    // hold them above 2^23, and a 24-bit multiply-add for x: fused
+    // multiply-adds issue at twice the rate of conversions.
+    __device__ __forceinline__ Off at(float xf, float yf, float zf) const {
+        if constexpr (BUF) {
+            const uint32_t yz = __float_as_uint(fmaf(yf, syf, fmaf(zf, 8.0f, mz)));
+            const uint32_t x1 = __float_as_uint(xf + 8388609.0f);
+            return __umul24(x1, sx) + yz - 0x4b000000u;
+        } else {
+            return (size_t)((int64_t)(int)xf * (int64_t)sx + (int64_t)(int)yf * (int64_t)sy + (int)zf) + base;
         }
     }
-    return acc;
+    // What a sample that is not reads.  BUF: as a mask, since a select of the
+    // offset would let the compiler move its arithmetic into a branch, which
+    // splits the unrolled samples and serialises their loads.
+    __device__ __forceinline__ Off only(bool in, Off o) const {
+        if constexpr (BUF) {
+            const uint32_t keep = 0u - (uint32_t)in;
+            return (o & keep) | (kOutside & ~keep);
+        } else {
+            return in ? o : 0;
+        }
+    }
+    struct Taps {
+        uint32_t d[sizeof(TV) == 4 ? 8 : 4];
+    };
+    __device__ __forceinline__ Taps load(Off o) const {
+        Taps t;
+        if constexpr (BUF) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)o, 0, 0);
+            t.d[0] = v[0]; t.d[1] = v[1]; t.d[2] = v[2]; t.d[3] = v[3];
+            if constexpr (sizeof(TV) == 4) {
+                const auto w = __builtin_amdgcn_raw_buffer_load_b128(r, (int)o, (int)sy, 0);
+                t.d[4] = w[0]; t.d[5] = w[1]; t.d[6] = w[2]; t.d[7] = w[3];
+            }
+        } else {
+            __builtin_memcpy(t.d, p + o, 16);
+            if constexpr (sizeof(TV) == 4) __builtin_memcpy(t.d + 4, p + o + sy, 16);
+        }
+        return t;
+    }
+};
+
+// One x row of a cell from a word of two FP16 voxels, lo + fx (hi - lo): the
+// difference and the blend each one v_fma_mix_f32, which takes the halves as
+// they are (exact conversions, one rounding: the FP32 operations' results).
+// Converted first, the eight taps cost eight conversions more.
+__device__ __forceinline__ float mix_lerp(uint32_t w, float fx) {
+    float t, c;
+    asm("v_fma_mix_f32 %0, 1.0, %1, -%1 op_sel:[0,1,0] op_sel_hi:[0,1,1]" : "=v"(t) : "v"(w));
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[0,0,1]" : "=v"(c) : "v"(fx), "v"(t), "v"(w));
+    return c;
 }
 
-// Byte strides of the copy read by the buffer path, and whether it applies.
-struct CopyShape {
-    uint64_t bytes_x, bytes_y;
-    uint32_t sa_x, sz_x, sa_y, sz_y;
-    bool buf;
-};
-__host__ __device__ __forceinline__ CopyShape rs_copy_shape(int nx, int ny, int nz, uint32_t es) {
-    CopyShape c;
-    c.sz_x = (uint32_t)(ny + 2) * 2u * es;
-    c.sz_y = (uint32_t)(nx + 2) * 2u * es;
-    c.bytes_x = zpair_elems_x(nx, ny, nz) * es;
-    c.bytes_y = zpair_elems_y(nx, ny, nz) * es;
-    const uint64_t sax = (uint64_t)c.sz_x * (uint64_t)(nz + 1), say = (uint64_t)c.sz_y * (uint64_t)(nz + 1);
-    c.sa_x = (uint32_t)sax;
-    c.sa_y = (uint32_t)say;
-    c.buf = c.bytes_x < kOutside && c.bytes_y < kOutside && sax < (1ull << 24) && say < (1ull << 24);
-    return c;
+template <typename TV, bool BUF>
+__device__ __forceinline__ RsRows rs_rows(const typename RsReader<TV, BUF>::Taps& t, float fx) {
+    auto lerp = [&](float a, float b) { return fmaf(fx, b - a, a); };
+    if constexpr (sizeof(TV) == 4) {
+        auto f = [&](int k) { return __uint_as_float(t.d[k]); };
+        return RsRows{lerp(f(0), f(1)), lerp(f(4), f(5)), lerp(f(2), f(3)), lerp(f(6), f(7))};
+    } else if constexpr (std::is_same<TV, __half>::value) {
+        return RsRows{mix_lerp(t.d[0], fx), mix_lerp(t.d[1], fx), mix_lerp(t.d[2], fx), mix_lerp(t.d[3], fx)};
+    } else {
+        using U = Unpack16<TV>;
+        auto row = [&](uint32_t w) { return lerp(U::lo(w), U::hi(w)); };
+        return RsRows{row(t.d[0]), row(t.d[1]), row(t.d[2]), row(t.d[3])};
+    }
+}
+
+template <typename TV, bool BUF>
+__device__ __forceinline__ RsReader<TV, BUF> make_rs_reader(const void* copy, int nx, int ny, int nz) {
+    RsReader<TV, BUF> q;
+    const RsCopyShape c = rs_copy_shape(nx, ny, nz, sizeof(TV));
+    q.p = (const uint2*)copy;
+    q.sx = c.sx * (BUF ? 8u : 1u);
+    q.sy = c.sy * (BUF ? 8u : 1u);
+    q.syf = (float)q.sy;
+    q.mz = 8388608.0f + (float)(q.sy + 8u);
+    q.base = (size_t)c.sx + c.sy + 1u;
+    if constexpr (BUF) q.r = buffer_rsrc(copy, (uint32_t)(c.elems * 8u));
+    return q;
+}
+
+// Samples of one lane in order: sample s at fma(s, d, entry), s < lr, the
+// trilinear blend of its taps (along x, then y, then z, with explicit fmaf),
+// taps outside the grid 0.  kRsUnroll samples per iteration, their loads in
+// flight together.  INNER: the wave's first and last samples lie in cells with
+// a voxel in the grid on every axis; positions are monotone in s, so every
+// sample does and none is tested; up to sample kall
+// every ray of the wave has one.  A sample that is not (s >= lr, or its cell
+// has no voxel in the grid) adds +0, which leaves the sum unchanged (it starts
+// at +0 and is never -0).
+//
+// FP32 is bound by the texture path: two 16-byte gathers a sample, 33 of its
+// cycles at best (four lanes a cycle), 512^3 / 512 views in 54.7 ms where
+// (B, z) quads of two slab planes along the detector rows took 91.4; with 8 in
+// flight 52.6 there, slower at 256^3 and 1024^3.  16-bit volumes take one gather
+// and are bound by VALU issue (FP16 37.1 ms, 76.6 before; with 4 in flight 44.6).
+template <typename TV> constexpr int kRsUnroll = sizeof(TV) == 4 ? 4 : 2;
+template <bool INNER, typename TV, bool BUF>
+__device__ __forceinline__ float rs_samples(const RsRay& r, const RsReader<TV, BUF>& q, int nx, int ny, int nz,
+                                            int kall, int kend) {
+    constexpr int U = kRsUnroll<TV>;
+    float acc = 0.0f, sf = 0.0f;
+    const float lrf = (float)r.lr;
+    auto samples = [&](auto tested) __attribute__((always_inline)) {
+        constexpr bool TEST = decltype(tested)::value;
+        typename RsReader<TV, BUF>::Taps t[U];
+        float fx[U], fy[U], fz[U];
+        bool in[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const float s = sf + (float)j;  // below 2^24: exact
+            const float x = fmaf(s, r.dx, r.ex), y = fmaf(s, r.dy, r.ey), z = fmaf(s, r.dz, r.ez);
+            float xf = floorf(x), yf = floorf(y), zf = floorf(z);
+            fx[j] = x - xf;
+            fy[j] = y - yf;
+            fz[j] = z - zf;
+            in[j] = true;
+            if constexpr (TEST) in[j] = s < lrf;
+            if constexpr (!INNER) {
+                const float xc = __builtin_amdgcn_fmed3f(xf, -1.0f, (float)(nx - 1));
+                const float yc = __builtin_amdgcn_fmed3f(yf, -1.0f, (float)(ny - 1));
+                const float zc = __builtin_amdgcn_fmed3f(zf, -1.0f, (float)(nz - 1));
+                in[j] = in[j] & (xc == xf) & (yc == yf) & (zc == zf);
+                xf = xc;
+                yf = yc;
+                zf = zc;
+            }
+            const auto o = q.at(xf, yf, zf);
+            t[j] = q.load(TEST || !INNER ? q.only(in[j], o) : o);
+        }
+        float v[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const RsRows c = rs_rows<TV, BUF>(t[j], fx[j]);
+            const float c0 = fmaf(fy[j], c.c10 - c.c00, c.c00), c1 = fmaf(fy[j], c.c11 - c.c01, c.c01);
+            v[j] = fmaf(fz[j], c1 - c0, c0);
+            if constexpr (!BUF && (TEST || !INNER)) v[j] = in[j] ? v[j] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < U; ++j) acc += v[j];
+        sf += (float)U;
+    };
+    int k = 0;
+    if constexpr (INNER)
+        for (; k + U <= kall; k += U) samples(std::false_type{});
+    for (; k < kend; k += U) samples(std::true_type{});
+    return acc;
 }
 
 // Forward RS projector.  Samples, taps and the order of the sum are those of
 // the per-ray loop (sample s at fma(s, d, entry), trilinear interpolation,
-// acc += in s order), so results are unchanged; what changes is the
-// schedule.  When every ray of the wave has the same dominant in-plane axis
-// A (|d_A| >= the other two) and direction, each lane starts its samples k0
-// iterations after the wave's first entry along A, k0 = its entry's distance
-// behind that one in samples (|d_A| per sample): at iteration k every lane
-// samples near the same A plane, one sample per lane per iteration.  Its 64
-// rays (a 32 x 2 block of detector cells) then read neighbouring quads of the
-// z-pair copy of A, two loads per sample (16 bytes each for FP32 storage,
-// 8 for 16-bit), or (AP, 16-bit volumes) the A-pair copy of A, one 16-byte
-// load per sample.  Other waves sample from k = 0 on the y-slab copy.  Grid: x = column group, y = view, z = row group
-// (every view of a row band before the next band).
-template <typename TV, typename TS, bool BUF, bool AP = false>
-__device__ __forceinline__ void rs_tile(const DevGeom& g, int cube, const void* __restrict__ qx,
-                                        const void* __restrict__ qy, float vol_inv, TS* __restrict__ sino,
-                                        float sino_scale, int bx, int p, int bz) {
-    const int m = bx * BX + threadIdx.x;
-    const int n = bz * BY + threadIdx.y;
-    const bool inside = m < g.nu && n < g.nv;
+// acc += in s order), so results are unchanged; what changes is the schedule
+// and the layout.  A wave is `rows` detector rows of 64 / rows columns and takes
+// sample s of its rays together.  The rays of a column enter the FOV at the
+// same in-plane point and stay close in plane at equal s (their in-plane steps
+// differ by the cosine of the cone angle), so the taps of neighbouring rows are
+// neighbours along z, the fastest axis of the copy.
+template <typename TV, typename TS, bool BUF>
+__device__ __forceinline__ void rs_tile(const DevGeom& g, int cube, const void* __restrict__ copy, float vol_inv,
+                                        TS* __restrict__ sino, float sino_scale, int rows, int bx, int pg, int bz) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int per = 64 / rows;  // columns of a wave
+    const int p = pg * kProjViews + wv;
+    const int m = bx * per + lane / rows;
+    const int n = bz * rows + lane % rows;
+    const bool inside = p < g.nphi && m < g.nu && n < g.nv;
     RsRay r{0, 0, 0, 0, 0, 0, 0};
     if (inside) r = rs_setup(g, cube, p, m, n);
     const bool ok = r.lr > 0;
-    int code = -1;
-    if (ok) {
-        const float ax = fabsf(r.dx), ay = fabsf(r.dy), az = fabsf(r.dz);
-        if (ax > 0.0f && ax >= ay && ax >= az) code = r.dx > 0.0f ? 0 : 1;
-        else if (ay > 0.0f && ay >= ax && ay >= az) code = r.dy > 0.0f ? 2 : 3;
-    }
-    const unsigned long long okmask = __ballot(ok);
-    int mode = -1;
-    if (okmask != 0ull) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (__ballot(ok && code == c) == okmask) mode = c;
-    }
-    int k0 = 0;
-    if (mode >= 0) {
-        const bool xs = mode < 2;
-        const float pa = (mode & 1) ? -(xs ? r.ex : r.ey) : (xs ? r.ex : r.ey);  // entry along the travel direction
-        const float da = fabsf(xs ? r.dx : r.dy);                                  // >= 1/sqrt(3) for admitted rays
-        const float pmin = wave_minf(ok ? pa : 3.0e38f);
-        // Entries are inside the volume's bounding box, so k0 <= sqrt(3) N.
-        if (ok) k0 = (int)((pa - pmin) / da + 0.5f);
-    }
-    const int kend = wave_max(ok ? k0 + r.lr : 0);
     const int nx = g.nx, ny = g.ny, nz = g.nz;
-    float acc;
+    auto within = [](float a, float b, int n1) {
+        const float fa = floorf(a), fb = floorf(b);
+        return (fa >= -1.0f) & (fa <= (float)(n1 - 1)) & (fb >= -1.0f) & (fb <= (float)(n1 - 1));
+    };
+    const float sl = (float)(r.lr - 1);
+    const bool inner = within(r.ex, fmaf(sl, r.dx, r.ex), nx) & within(r.ey, fmaf(sl, r.dy, r.ey), ny) &
+                       within(r.ez, fmaf(sl, r.dz, r.ez), nz);
+    const int kend = __builtin_amdgcn_readfirstlane(wave_max(ok ? r.lr : 0));
+    // a lane without a ray samples cell (0, 0, 0); its sum is dropped
+    const int kall = __builtin_amdgcn_readfirstlane(min(wave_min(ok ? r.lr : INT_MAX), kend));
+    const auto q = make_rs_reader<TV, BUF>(copy, nx, ny, nz);
+    float acc = __ballot(ok && !inner) == 0ull ? rs_samples<true>(r, q, nx, ny, nz, kall, kend)
+                                               : rs_samples<false>(r, q, nx, ny, nz, kall, kend);
     // 16-bit volumes are read unscaled; the sum is linear in them, so the
     // storage scale applies once to it (FP32 storage has no scale).
-    CopyBuf qb{};
-    if constexpr (BUF) {
-        const bool xs = mode >= 0 && mode < 2;
-        if constexpr (AP) {
-            const ApairShape cs = rs_apair_shape(nx, ny, nz);
-            qb.r = buffer_rsrc(xs ? qx : qy, (uint32_t)(xs ? cs.bytes_x : cs.bytes_y));
-            qb.sa = xs ? cs.sa_x : cs.sa_y;
-            qb.sz = xs ? cs.sz_x : cs.sz_y;
-        } else {
-            const CopyShape cs = rs_copy_shape(nx, ny, nz, sizeof(TV));
-            qb.r = buffer_rsrc(xs ? qx : qy, (uint32_t)(xs ? cs.bytes_x : cs.bytes_y));
-            qb.sa = xs ? cs.sa_x : cs.sa_y;
-            qb.sz = xs ? cs.sz_x : cs.sz_y;
-        }
-    }
-    if (mode >= 0 && mode < 2) acc = rs_samples<0, TV, BUF, AP>(r, qx, qb, nx, ny, nz, k0, kend);
-    else acc = rs_samples<1, TV, BUF, AP>(r, qy, qb, nx, ny, nz, k0, kend);
     if (sizeof(TV) == 2) acc *= vol_inv;
     if (inside) {
         const size_t o = (size_t)m + (size_t)g.nu * ((size_t)n + (size_t)g.nv * p);
-        Storage<TS>::store(sino, o, r.lr > 0 ? acc * g.delta : 0.0f, sino_scale);
+        Storage<TS>::store(sino, o, ok ? acc * g.delta : 0.0f, sino_scale);
     }
 }
 
-template <typename TV, typename TS, bool BUF, bool AP>
-__global__ __launch_bounds__(BX* BY) void rs_kernel(DevGeom g, int cube, const void* __restrict__ qx,
-                                                  const void* __restrict__ qy, float vol_inv, TS* __restrict__ sino,
-                                                  float sino_scale) {
-    rs_tile<TV, TS, BUF, AP>(g, cube, qx, qy, vol_inv, sino, sino_scale, blockIdx.x, blockIdx.y, blockIdx.z);
-}
-
-// The gather form's launch: A-pair copies (16-bit volumes) when ap, else the
-// z-pair copies; through the buffer path when buf, else 64-bit indices.
-template <typename TV, typename TS>
-void launch_rs_gathers(bool ap, bool buf, dim3 grid, hipStream_t s, const DevGeom& d, int cube, const void* cx,
-                       const void* cy, float inv, TS* sino, float sino_scale) {
-    if constexpr (sizeof(TV) == 2) {
-        if (ap) {
-            if (buf)
-                hipLaunchKernelGGL((rs_kernel<TV, TS, true, true>), grid, dim3(BX, BY), 0, s, d, cube, cx, cy, inv,
-                                   sino, sino_scale);
-            else
-                hipLaunchKernelGGL((rs_kernel<TV, TS, false, true>), grid, dim3(BX, BY), 0, s, d, cube, cx, cy, inv,
-                                   sino, sino_scale);
-            return;
-        }
-    }
-    if (buf)
-        hipLaunchKernelGGL((rs_kernel<TV, TS, true, false>), grid, dim3(BX, BY), 0, s, d, cube, cx, cy, inv, sino,
-                           sino_scale);
-    else
-        hipLaunchKernelGGL((rs_kernel<TV, TS, false, false>), grid, dim3(BX, BY), 0, s, d, cube, cx, cy, inv, sino,
-                           sino_scale);
+template <typename TV, typename TS, bool BUF>
+__global__ __launch_bounds__(64 * kProjViews) void rs_kernel(DevGeom g, int cube, const void* __restrict__ copy,
+                                                             float vol_inv, TS* __restrict__ sino, float sino_scale,
+                                                             int rows) {
+    rs_tile<TV, TS, BUF>(g, cube, copy, vol_inv, sino, sino_scale, rows,
+                         proj_group(blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, blockIdx.z), blockIdx.y, blockIdx.z);
 }
 
 // ---------------------------------------------------------------------------
@@ -753,34 +616,30 @@ __global__ __launch_bounds__(BX* BY, 5) void rs_staged_kernel(DevGeom g, int cub
     }
 }
 
-// Shared launch (FP32 or BF16 (kItemBF16) z-pair copies, or BF16 A-pair
-// copies (kItemApair), FP32 sinograms); item flags bit 0 selects the cube
-// FOV.  No minimum-waves bound: under one
-// (8 or 6 waves per SIMD, 52 or 74 VGPRs) the compiler waits for each
-// sample's two gathers before it issues the next sample's, where unbounded
-// (86 VGPRs, 5 waves per SIMD) it issues the eight gathers of four samples
-// together, as rs_kernel does; the serialised form took 27% longer per
-// 512^3 projection.  Its grid is what the chip holds at once
-// (batch_grids_init), so every workgroup is resident from the start.
-__global__ __launch_bounds__(BX* BY) void rs_batch_kernel(const BatchTable* __restrict__ t, uint32_t* __restrict__ next) {
+// Shared launch (FP32 or BF16 (kItemBF16) RS copies, FP32 sinograms); item
+// flags bit 0 selects the cube FOV.  No minimum-waves bound: under one the
+// compiler waits for each sample's gathers before it issues the next
+// sample's.  Its grid is what the chip holds at once (batch_grids_init), so
+// every workgroup is resident from the start.
+__global__ __launch_bounds__(64 * kProjViews) void rs_batch_kernel(const BatchTable* __restrict__ t, uint32_t* __restrict__ next) {
     TOMO_BATCH_CLAIMED(t, next) {
         const BatchItem& it = t->item[batch_find(t, tile)];
         const uint32_t local = tile - it.begin;
-        const uint32_t bx = local % it.gx, rest = local / it.gx;
+        const uint32_t rest = local / it.gx;
         const int by = (int)(rest % it.gy), bz = (int)(rest / it.gy), cube = it.flags & 1;
+        const int bx = proj_group(local % it.gx, it.gx, (uint32_t)by, it.gy, (uint32_t)bz);
         const bool bf = (it.flags & kItemBF16) != 0;
-        const bool buf = rs_copy_shape(it.g.nx, it.g.ny, it.g.nz, bf ? 2u : 4u).buf;
+        const bool buf = rs_copy_shape(it.g.nx, it.g.ny, it.g.nz, bf ? 2 : 4).buf;
+        const int rows = rs_wave_rows(it.g.nv);
         using BF = __hip_bfloat16;
-        if (it.flags & kItemApair)
-            rs_tile<BF, float, true, true>(it.g, cube, it.in, it.in2, 1.0f, (float*)it.out, 1.0f, (int)bx, by, bz);
-        else if (bf && buf)
-            rs_tile<BF, float, true>(it.g, cube, it.in, it.in2, 1.0f, (float*)it.out, 1.0f, (int)bx, by, bz);
+        if (bf && buf)
+            rs_tile<BF, float, true>(it.g, cube, it.in, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else if (bf)
-            rs_tile<BF, float, false>(it.g, cube, it.in, it.in2, 1.0f, (float*)it.out, 1.0f, (int)bx, by, bz);
+            rs_tile<BF, float, false>(it.g, cube, it.in, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else if (buf)
-            rs_tile<float, float, true>(it.g, cube, it.in, it.in2, 1.0f, (float*)it.out, 1.0f, (int)bx, by, bz);
+            rs_tile<float, float, true>(it.g, cube, it.in, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else
-            rs_tile<float, float, false>(it.g, cube, it.in, it.in2, 1.0f, (float*)it.out, 1.0f, (int)bx, by, bz);
+            rs_tile<float, float, false>(it.g, cube, it.in, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
     }
 }
 
@@ -852,25 +711,28 @@ int launch_rs(const tomo_geom* g, int cube, Buf vol, MutBuf sino, hipStream_t s,
         return TOMO_OK;
     }
     const float inv = 1.0f / vol.scale;
-    const uint32_t es = vol.dtype == TOMO_F32 ? 4u : 2u;
-    // 16-bit volumes take one load per sample from A-pair copies (the taps are
-    // the same numbers), through the buffer path where those fit it
-    const bool ap = es == 2;
-    ZPairs zp;
-    hipError_t le = zp.alloc(vol.p, es, d.nx, d.ny, d.nz, s, x, ap);
-    const void* cx = zp.qx;
-    const void* cy = zp.qy;
+    const size_t es = vol.dtype == TOMO_F32 ? 4 : 2;
+    const RsCopyShape cs = rs_copy_shape(d.nx, d.ny, d.nz, es);
+    ProjCopy pc;
+    hipError_t le = pc.alloc(cs.elems * 8, s, x);
+    if (le == hipSuccess) le = launch_rs_copy(vol.p, pc.p, es, d.nx, d.ny, d.nz, s);
     if (le == hipSuccess) {
-        const bool buf = !x.index_reads && (ap ? apair_buffer_path(d.nx, d.ny, d.nz)
-                                               : rs_copy_shape(d.nx, d.ny, d.nz, es).buf);
+        const bool buf = cs.buf && !x.index_reads;
+        const int rows = rs_wave_rows(d.nv);
+        const dim3 cgrid(proj_groups(d.nu, rows), ceil_div(d.nphi, kProjViews), ceil_div(d.nv, rows));
         TOMO_DISPATCH_STORAGE(vol.dtype, TV, {
             TOMO_DISPATCH_STORAGE(sino.dtype, TS, {
-                launch_rs_gathers<TV, TS>(ap, buf, grid, s, d, cube, cx, cy, inv, (TS*)sino.p, sino.scale);
+                if (buf)
+                    hipLaunchKernelGGL((rs_kernel<TV, TS, true>), cgrid, dim3(64 * kProjViews), 0, s, d, cube, pc.p,
+                                       inv, (TS*)sino.p, sino.scale, rows);
+                else
+                    hipLaunchKernelGGL((rs_kernel<TV, TS, false>), cgrid, dim3(64 * kProjViews), 0, s, d, cube, pc.p,
+                                       inv, (TS*)sino.p, sino.scale, rows);
             });
         });
         le = hipGetLastError();
     }
-    const hipError_t fe = zp.release(s);
+    const hipError_t fe = pc.release(s);
     TOMO_HIP(le);
     TOMO_HIP(fe);
     return TOMO_OK;
@@ -882,7 +744,7 @@ std::atomic<int> g_rs_batch_grid{kBatchGrid};
 
 int batch_grids_init(int device) {
     int per_cu = 0, cus = 0;
-    TOMO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, rs_batch_kernel, BX * BY, 0));
+    TOMO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, rs_batch_kernel, 64 * kProjViews, 0));
     TOMO_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     int grid = per_cu * cus;
     grid -= grid % kBatchXcds;
@@ -891,7 +753,7 @@ int batch_grids_init(int device) {
 }
 
 hipError_t launch_batch_rs(BatchTable* t, hipStream_t s) {
-    hipLaunchKernelGGL(rs_batch_kernel, dim3(g_rs_batch_grid.load()), dim3(BX, BY), 0, s, t, t->next);
+    hipLaunchKernelGGL(rs_batch_kernel, dim3(g_rs_batch_grid.load()), dim3(64 * kProjViews), 0, s, t, t->next);
     return hipGetLastError();
 }
 

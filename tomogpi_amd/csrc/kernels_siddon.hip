@@ -16,7 +16,7 @@
 // evaluation order and quirks: source on the +FOD side (mirror of RS/VI),
 // first voxel half a voxel behind the entry, last chord not clipped, indices
 // % 256 with unsigned wrap, no z clip.  Defined for 256^3 volumes only.
-#include "zpair.hpp"
+#include "proj_copy.hpp"
 #include "batch.hpp"
 #include "stage_box.hpp"
 
@@ -208,7 +208,7 @@ __device__ __forceinline__ void sid_step(SidState& s, const SidRay& r, const RD&
     s.live = s.t < r.tmax;
 }
 
-// Column walk on the z-column copy (zpair.hpp: z varies fastest).  A lane walks
+// Column walk on the z-column copy (proj_copy.hpp: z varies fastest).  A lane walks
 // the in-plane cells (x, y) its ray crosses, one per iteration; a cell's
 // segments are
 //   [t, c1] V(z),  [c1, te] V(z + dz)
@@ -319,27 +319,18 @@ __device__ __forceinline__ float sid_walk_columns(const ColumnRay& r, const CR& 
     return acc;
 }
 
-// The column group of the grid's x index `i` (gx of them, a multiple of 8): the
-// XCD i mod 8 takes a run of gx / 8 neighbouring groups.  The runs rotate over
-// the XCDs with the view and the row band, because outer columns have shorter
-// rays.
-__device__ __forceinline__ int sid_group(uint32_t i, uint32_t gx, uint32_t pg, uint32_t views, uint32_t bz) {
-    const uint32_t run = (i + pg * 8u / views + bz) & 7u;
-    return (int)(run * (gx / 8u) + i / 8u);
-}
-
 // Forward clean Siddon.  Each lane takes the segments of the per-ray
 // traversal (same operations, same order), so results are bit-identical to
 // it.  What changes is the schedule and the memory layout (see above).
 // A wave is `rows` (64, 32 or 16) detector rows of 64 / rows columns; a
-// workgroup is these cells in kSidViews consecutive views, whose rays run
+// workgroup is these cells in kProjViews consecutive views, whose rays run
 // through nearly the same columns of the volume at the same time (512^3 / 512
 // views: 33.1 ms with four neighbouring column groups of one view per
 // workgroup, 31.7 ms with four views; 1024^3 / 720 views, bound by the lines
 // that miss L2: 238 and 182 ms).  Grid: x = column group, y = view group, z =
 // row group: the chip works through every view of one row band before the
 // next band, whose rays stay in a z band of the volume.  Workgroups go to the
-// XCDs round robin; sid_group gives each XCD neighbouring column groups, so that
+// XCDs round robin; proj_group gives each XCD neighbouring column groups, so that
 // its L2 meets the columns of one view again in the next ones (512^3: 38.1 ms
 // without it, at four columns of one view per workgroup).
 template <typename TV, typename TS, bool BUF>
@@ -347,7 +338,7 @@ __device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __
                                             TS* __restrict__ sino, float sino_scale, int rows, int bx, int pg, int bz) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int per = 64 / rows;  // columns of a wave
-    const int p = pg * kSidViews + wv;
+    const int p = pg * kProjViews + wv;
     const int m = bx * per + lane / rows;
     const int n = bz * rows + lane % rows;
     const bool inside = p < g.nphi && m < g.nu && n < g.nv;
@@ -440,7 +431,7 @@ __device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __
 // boundary planes wlo - 1/2 and whi + 1/2, the voxel round(B) and its
 // neighbours, likewise in z), and each slab's quad -- the current
 // voxel, its B neighbour, its z neighbour and the diagonal one -- is two
-// ds_read2_b32 there instead of one 16-byte gather from a z-pair copy.  The
+// ds_read2_b32 there instead of a gather per lane.  The
 // per-slab arithmetic is sid_walk_quads', so every lane takes the segments
 // of the per-ray traversal in its order: results are bit-identical to it.
 // A wave whose rays go up and down in z copies its share of rows and keeps
@@ -735,22 +726,22 @@ __global__ __launch_bounds__(BX* BY, 5) void siddon_staged_kernel(DevGeom g, con
 }
 
 template <typename TV, typename TS, bool BUF>
-__global__ __launch_bounds__(64 * kSidViews) void siddon_kernel(DevGeom g, const uint32_t* __restrict__ cols, float vol_inv,
+__global__ __launch_bounds__(64 * kProjViews) void siddon_kernel(DevGeom g, const uint32_t* __restrict__ cols, float vol_inv,
                                                      TS* __restrict__ sino, float sino_scale, int rows) {
     siddon_tile<TV, TS, BUF>(g, cols, vol_inv, sino, sino_scale, rows,
-                             sid_group(blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, blockIdx.z), blockIdx.y, blockIdx.z);
+                             proj_group(blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, blockIdx.z), blockIdx.y, blockIdx.z);
 }
 
 // Shared launch: tiles are the single-problem grid's workgroups (column
 // group fastest, then view, then row group); FP32 or BF16 (kItemBF16) z-column
 // copies, FP32 sinograms.
-__global__ __launch_bounds__(64 * kSidViews) void siddon_batch_kernel(const BatchTable* __restrict__ t, uint32_t* __restrict__ next) {
+__global__ __launch_bounds__(64 * kProjViews) void siddon_batch_kernel(const BatchTable* __restrict__ t, uint32_t* __restrict__ next) {
     TOMO_BATCH_CLAIMED(t, next) {
         const BatchItem& it = t->item[batch_find(t, tile)];
         const uint32_t local = tile - it.begin;
         const uint32_t rest = local / it.gx;
         const int by = (int)(rest % it.gy), bz = (int)(rest / it.gy);
-        const int bx = sid_group(local % it.gx, it.gx, (uint32_t)by, it.gy, (uint32_t)bz);
+        const int bx = proj_group(local % it.gx, it.gx, (uint32_t)by, it.gy, (uint32_t)bz);
         const bool bf = (it.flags & kItemBF16) != 0;
         const bool buf = zcol_words(it.g.nx, it.g.ny, it.g.nz, bf ? 2 : 4) * 4u < kSidOutside;
         const int rows = sid_wave_rows(it.g.nv);
@@ -914,21 +905,24 @@ int launch_siddon(const tomo_geom* g, int compat, Buf vol, MutBuf sino, hipStrea
     // z-column copy of the volume (a stream-ordered pool allocation, released
     // after the projection on the same stream)
     const size_t es = vol.dtype == TOMO_F32 ? 4 : 2;
-    if (zpair_elems_x(d.nx, d.ny, d.nz) >= (1ull << 32) || zpair_elems_y(d.nx, d.ny, d.nz) >= (1ull << 32))
+    if (!sid_volume_fits(d.nx, d.ny, d.nz))
         return fail(TOMO_ERR_UNSUPPORTED, "volume too large for the 32-bit traversal index of the Siddon projector");
-    ZColumns zc;
-    hipError_t le = zc.alloc(vol.p, es, d.nx, d.ny, d.nz, s, x);
+    ProjCopy zc;
+    hipError_t le = zc.alloc(zcol_words(d.nx, d.ny, d.nz, es) * 4, s, x);
+    if (le == hipSuccess) le = launch_zcol(vol.p, (uint32_t*)zc.p, es, d.nx, d.ny, d.nz, s);
     if (le == hipSuccess) {
         const bool buf = zcol_words(d.nx, d.ny, d.nz, es) * 4u < kSidOutside && !x.index_reads;
         const int rows = sid_wave_rows(d.nv);
-        const dim3 cgrid(sid_groups(d.nu, rows), ceil_div(d.nphi, kSidViews), ceil_div(d.nv, rows));
+        const dim3 cgrid(proj_groups(d.nu, rows), ceil_div(d.nphi, kProjViews), ceil_div(d.nv, rows));
         TOMO_DISPATCH_STORAGE(vol.dtype, TV, {
             TOMO_DISPATCH_STORAGE(sino.dtype, TS, {
                 if (buf)
-                    hipLaunchKernelGGL((siddon_kernel<TV, TS, true>), cgrid, dim3(64 * kSidViews), 0, s, d, zc.p, inv,
+                    hipLaunchKernelGGL((siddon_kernel<TV, TS, true>), cgrid, dim3(64 * kProjViews), 0, s, d,
+                                       (const uint32_t*)zc.p, inv,
                                        (TS*)sino.p, sino.scale, rows);
                 else
-                    hipLaunchKernelGGL((siddon_kernel<TV, TS, false>), cgrid, dim3(64 * kSidViews), 0, s, d, zc.p, inv,
+                    hipLaunchKernelGGL((siddon_kernel<TV, TS, false>), cgrid, dim3(64 * kProjViews), 0, s, d,
+                                       (const uint32_t*)zc.p, inv,
                                        (TS*)sino.p, sino.scale, rows);
             });
         });
@@ -941,7 +935,7 @@ int launch_siddon(const tomo_geom* g, int compat, Buf vol, MutBuf sino, hipStrea
 }
 
 hipError_t launch_batch_siddon(BatchTable* t, hipStream_t s) {
-    hipLaunchKernelGGL(siddon_batch_kernel, dim3(kBatchGrid), dim3(64 * kSidViews), 0, s, t, t->next);
+    hipLaunchKernelGGL(siddon_batch_kernel, dim3(kBatchGrid), dim3(64 * kProjViews), 0, s, t, t->next);
     return hipGetLastError();
 }
 

@@ -10,7 +10,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "zpair.hpp"
+#include "proj_copy.hpp"
 #include "batch.hpp"
 
 namespace tomo {
@@ -209,95 +209,6 @@ __device__ __forceinline__ TO copy_cvt(TI v) {
     else return __bfloat16_as_ushort(__float2bfloat16(v));
 }
 
-// One z-pair (the two elements at an even index o) as one aligned store: the
-// copies start on 256-byte boundaries, so out + o is aligned to the pair.
-template <typename T>
-__device__ __forceinline__ void store_pair(T* __restrict__ out, size_t o, T a, T b) {
-    typedef T T2 __attribute__((ext_vector_type(2)));
-    T2 v;
-    v.x = a;
-    v.y = b;
-    *reinterpret_cast<T2*>(out + o) = v;
-}
-
-// z-pair copy for y slabs (A = y, B = x): B is also the input's fastest axis,
-// a direct pass.  Grid (ceil((nx+2)/256), ny, nz+1).
-template <typename TI, typename T>
-__device__ __forceinline__ void zpair_y_tile(const TI* __restrict__ in, T* __restrict__ out, int nx, int ny, int nz,
-                                             int bx, int y, int zz) {
-    const int bb = bx * 256 + threadIdx.x;
-    if (bb > nx + 1) return;
-    const int x = bb - 1;
-    T v[2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int z = zz - 1 + c;
-        __builtin_memset(&v[c], 0, sizeof(T));
-        if (x >= 0 && x < nx && z >= 0 && z < nz)
-            v[c] = copy_cvt<T>(in[(size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * z)]);
-    }
-    store_pair(out, zpair_index(y, zz, bb, nz, nx), v[0], v[1]);
-}
-
-// z-pair copy for x slabs (A = x, B = y): a 32x32 (x, B) tile transpose of
-// two z planes through LDS.  Grid (ceil(nx/32), ceil((ny+2)/32), nz+1).
-template <typename TI, typename T>
-__device__ __forceinline__ void zpair_x_tile(const TI* __restrict__ in, T* __restrict__ out, int nx, int ny, int nz,
-                                             int bx, int by, int zz, T (*tile)[32][33]) {
-    const int x0 = bx * 32, b0 = by * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-    for (int r = ty; r < 32; r += 8) {
-        const int x = x0 + tx, y = b0 + r - 1;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int z = zz - 1 + c;
-            T v;
-            __builtin_memset(&v, 0, sizeof(T));
-            if (x < nx && y >= 0 && y < ny && z >= 0 && z < nz)
-                v = copy_cvt<T>(in[(size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * z)]);
-            tile[c][r][tx] = v;
-        }
-    }
-    __syncthreads();
-    for (int r = ty; r < 32; r += 8) {
-        const int x = x0 + r, bb = b0 + tx;
-        if (x < nx && bb <= ny + 1) {
-            store_pair(out, zpair_index(x, zz, bb, nz, ny), tile[0][tx][r], tile[1][tx][r]);
-        }
-    }
-}
-
-// Single-problem z-pair copy for y slabs: a thread walks kZChunk z pairs of
-// one (y, bb) column, reading each input row once (a pair's upper voxel is
-// the next pair's lower one), where a tile of one pair reads both.  Grid
-// (ceil((nx+2)/256), ny, ceil((nz+1)/kZChunk)).
-constexpr int kZChunk = 32;
-template <typename T>
-__global__ __launch_bounds__(256) void zpair_y_kernel(const T* __restrict__ in, T* __restrict__ out, int nx, int ny,
-                                                    int nz) {
-    const int bb = blockIdx.x * 256 + threadIdx.x;
-    if (bb > nx + 1) return;
-    const int x = bb - 1, y = blockIdx.y;
-    const int z0 = blockIdx.z * kZChunk, z1 = min(z0 + kZChunk, nz + 1);
-    const bool xin = x >= 0 && x < nx;
-    const T* col = in + (size_t)(xin ? x : 0) + (size_t)nx * y;  // (x, y, z) at col[nx ny z]
-    const size_t zs = (size_t)nx * ny;
-    // Clamped address (always in the volume), then a mask (the element types
-    // are integers): a conditional load, or a select the compiler turns into
-    // one, is a branch per pair that waits for each load before the next.
-    auto voxel = [&](int z) {
-        const T v = col[zs * (size_t)min(max(z, 0), nz - 1)];
-        return (T)(v & (T)(0u - (unsigned)(xin && z >= 0 && z < nz)));
-    };
-    T lo = voxel(z0 - 1);
-#pragma unroll 8
-    for (int zz = z0; zz < z1; ++zz) {
-        const T hi = voxel(zz);
-        store_pair(out, zpair_index(y, zz, bb, nz, nx), lo, hi);
-        lo = hi;
-    }
-}
-
 // out[y + nyp (x + nx z)] = in[x + nx (y + ny z)], 0 for ny <= y < nyp: the
 // volume with y fastest and zero-padded rows, one 32 x 32 (x, y) tile of one
 // z plane per workgroup, through LDS.
@@ -328,57 +239,7 @@ __global__ __launch_bounds__(256) void row_pad_kernel(const float* __restrict__ 
     }
 }
 
-// Single-problem z-pair copy for x slabs: a workgroup takes one 32 x 32
-// (x, B) tile through kZChunk z pairs, each input plane of the tile read once
-// into LDS (a pair's upper plane is the next pair's lower one); the next
-// plane's loads are issued before the current pairs are written.  Grid
-// (ceil(nx/32), ceil((ny+2)/32), ceil((nz+1)/kZChunk)).
-template <typename T>
-__global__ __launch_bounds__(256) void zpair_x_kernel(const T* __restrict__ in, T* __restrict__ out, int nx, int ny,
-                                                    int nz) {
-    __shared__ T tile[2][32][33];  // [plane][B row][x]
-    const int x0 = blockIdx.x * 32, b0 = blockIdx.y * 32;
-    const int z0 = blockIdx.z * kZChunk, z1 = min(z0 + kZChunk, nz + 1);
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-    const int x = x0 + tx;
-    // rows r = ty + 8 j of plane z, as in zpair_y_kernel: clamped addresses
-    // (the loads stay unconditional) and masks of the voxels in the grid,
-    // applied when the rows go to LDS so that nothing waits for the loads
-    // before then
-    auto fetch = [&](int z, T (&v)[4], T (&m)[4]) {
-        const int zc = min(max(z, 0), nz - 1);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int y = b0 + ty + 8 * j - 1;
-            const bool ok = x < nx && y >= 0 && y < ny && z >= 0 && z < nz;
-            const size_t o = (size_t)min(x, nx - 1) + (size_t)nx * ((size_t)min(max(y, 0), ny - 1) + (size_t)ny * zc);
-            v[j] = in[o];
-            m[j] = (T)(0u - (unsigned)ok);
-        }
-    };
-    auto put = [&](const T (&v)[4], const T (&m)[4], int c) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) tile[c][ty + 8 * j][tx] = (T)(v[j] & m[j]);
-    };
-    T v[4], m[4];
-    fetch(z0 - 1, v, m);
-    put(v, m, 0);
-    fetch(z0, v, m);
-    for (int zz = z0; zz < z1; ++zz) {
-        const int cur = (zz - z0 + 1) & 1, prev = cur ^ 1;  // planes zz and zz - 1
-        put(v, m, cur);
-        __syncthreads();
-        if (zz + 1 < z1) fetch(zz + 1, v, m);
-        for (int r = ty; r < 32; r += 8) {
-            const int xo = x0 + r, bb = b0 + tx;
-            if (xo < nx && bb <= ny + 1)
-                store_pair(out, zpair_index(xo, zz, bb, nz, ny), tile[prev][tx][r], tile[cur][tx][r]);
-        }
-        __syncthreads();  // every pair of this z is written before its lower plane is overwritten
-    }
-}
-
-// z-column copy (zpair.hpp): the tile of 64 x and 64 words of each of their
+// z-column copy (proj_copy.hpp): the tile of 64 x and 64 words of each of their
 // columns at row y, transposed through LDS (65 planes for the 16-bit pairs).
 // TI: float or uint32_t (bits) for FP32 words; uint16_t (bits) or float (rounded
 // to BF16) for PAIR words.  One row of y per tile keeps even a 64^3 volume's
@@ -429,84 +290,55 @@ __global__ __launch_bounds__(256) void zcol_kernel(const TI* __restrict__ in, ui
                         tile);
 }
 
-// One A-pair group (four 16-bit elements at an index that is a multiple of
-// four) as one aligned 8-byte store.
-__device__ __forceinline__ void store_group(uint16_t* __restrict__ out, size_t o, uint16_t a, uint16_t b, uint16_t c,
-                                            uint16_t d) {
-    typedef uint16_t U4 __attribute__((ext_vector_type(4)));
-    U4 v;
-    v.x = a;
-    v.y = b;
-    v.z = c;
-    v.w = d;
-    *reinterpret_cast<U4*>(out + o) = v;
-}
-
-// A voxel of an x-fastest volume as a 16-bit copy element (0 outside the
-// grid): a bit copy of a 16-bit volume, or an FP32 voxel rounded to BF16.
-// Read at the clamped address (always in the volume), then masked: a load
-// guarded by the bounds test is a branch, which waits for it before the
-// next.  The empty statement keeps the compiler from seeing that the mask is
-// 0 or ~0 (it would turn the AND back into a select, and that into the
-// branch); it emits no instruction.
-template <typename TI>
-__device__ __forceinline__ uint16_t voxel16(const TI* __restrict__ in, int x, int y, int z, int nx, int ny, int nz) {
-    const bool ok = (x >= 0) & (x < nx) & (y >= 0) & (y < ny) & (z >= 0) & (z < nz);
-    const size_t o = (size_t)min(max(x, 0), nx - 1) +
-                     (size_t)nx * ((size_t)min(max(y, 0), ny - 1) + (size_t)ny * min(max(z, 0), nz - 1));
-    uint32_t m = 0u - (uint32_t)ok;
-    asm("" : "+v"(m));
-    return (uint16_t)(copy_cvt<uint16_t>(in[o]) & m);
-}
-
-// A-pair copy for x slabs (A = x, B = y): a tile of 32 plane pairs x 32 B
-// columns of one z pair through LDS (the input runs along x, the copy along
-// y).  Grid (ceil((nx+1)/32), ceil((ny+2)/32), nz+1).
-template <typename TI>
-__device__ __forceinline__ void apair_x_tile(const TI* __restrict__ in, uint16_t* __restrict__ out, int nx, int ny,
-                                             int nz, int bx, int by, int zz, uint16_t (*tile)[32][34]) {
-    // tile[z - (zz-1)][bb - b0][x - (ap0-1)]
-    const int ap0 = bx * 32, b0 = by * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-    for (int r = ty; r < 32; r += 8) {
-        const int y = b0 + r - 1;
-        for (int c = tx; c < 34; c += 32) {
-            tile[0][r][c] = voxel16(in, ap0 - 1 + c, y, zz - 1, nx, ny, nz);
-            tile[1][r][c] = voxel16(in, ap0 - 1 + c, y, zz, nx, ny, nz);
+// RS copy (proj_copy.hpp): the tile of 64 xx and 64 elements of each of their
+// columns at row yy, through LDS: the words of the 65 x it pairs, in FP32 one
+// voxel, in 16 bits (QUAD) the voxels of rows yy-1 and yy.
+template <typename TI, bool QUAD>
+__device__ __forceinline__ void rs_copy_tile(const TI* __restrict__ in, uint2* __restrict__ out, int nx, int ny, int nz,
+                                             int bx, int yy, int bz, uint32_t (*tile)[kColLds]) {
+    using T = typename std::conditional<QUAD, uint16_t, uint32_t>::type;
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4
+    const int x0 = bx * kColTile - 1, z0 = bz * kColTile - 1;  // voxel of the tile's first column and row
+    auto voxel = [&](int x, int y, int z) {
+        uint32_t m = 0u - (uint32_t)((x >= 0) & (x < nx) & (y >= 0) & (y < ny) & (z >= 0) & (z < nz));
+        asm("" : "+v"(m));
+        const size_t o = (size_t)min(max(x, 0), nx - 1) +
+                         (size_t)nx * ((size_t)min(max(y, 0), ny - 1) + (size_t)ny * min(max(z, 0), nz - 1));
+        return (uint32_t)copy_cvt<T>(in[o]) & m;
+    };
+    auto word = [&](int c, int r) {
+        const uint32_t lo = voxel(x0 + c, yy - 1, z0 + r);
+        if constexpr (QUAD) return lo | (voxel(x0 + c, yy, z0 + r) << 16);
+        else return lo;
+    };
+    uint32_t v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = word(tx, ty + 4 * j);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) tile[ty + 4 * j][tx] = v[j];
+    if (ty == 0) tile[tx][64] = word(64, tx);
+    __syncthreads();
+    const RsCopyShape cs = rs_copy_shape(nx, ny, nz, QUAD ? 2 : 4);
+    const int zz = bz * kColTile + tx;
+    if (zz <= nz + 1) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int r = ty + 4 * j, xx = bx * kColTile + r;
+            const uint32_t a = tile[tx][r], b = tile[tx][r + 1];
+            const uint2 e = QUAD ? make_uint2((a & 0xffffu) | (b << 16), (a >> 16) | (b & 0xffff0000u)) : make_uint2(a, b);
+            if (xx <= nx) out[(size_t)xx * cs.sx + (size_t)yy * cs.sy + zz] = e;
         }
     }
-    __syncthreads();
-    for (int r = ty; r < 32; r += 8) {
-        const int ap = ap0 + r, bb = b0 + tx;
-        if (ap <= nx && bb <= ny + 1)
-            store_group(out, apair_index(ap, zz, bb, nz, ny), tile[0][tx][r], tile[1][tx][r], tile[0][tx][r + 1],
-                        tile[1][tx][r + 1]);
-    }
 }
 
-// A-pair copy for y slabs (A = y, B = x): B is the input's fastest axis, a
-// direct pass.  Grid (ceil((nx+2)/256), ny+1, nz+1): group (ap, zz, bb) with
-// bb = 256 bx + thread.
-template <typename TI>
-__device__ __forceinline__ void apair_y_tile(const TI* __restrict__ in, uint16_t* __restrict__ out, int nx, int ny,
-                                             int nz, int bx, int ap, int zz) {
-    const int bb = bx * 256 + threadIdx.x;
-    if (bb > nx + 1) return;
-    const int x = bb - 1;
-    store_group(out, apair_index(ap, zz, bb, nz, nx), voxel16(in, x, ap - 1, zz - 1, nx, ny, nz),
-                voxel16(in, x, ap - 1, zz, nx, ny, nz), voxel16(in, x, ap, zz - 1, nx, ny, nz),
-                voxel16(in, x, ap, zz, nx, ny, nz));
-}
-
-__global__ __launch_bounds__(256) void apair_x_kernel(const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
-                                                    int nx, int ny, int nz) {
-    __shared__ uint16_t tile[2][32][34];
-    apair_x_tile<uint16_t>(in, out, nx, ny, nz, blockIdx.x, blockIdx.y, blockIdx.z, tile);
-}
-
-__global__ __launch_bounds__(256) void apair_y_kernel(const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
-                                                    int nx, int ny, int nz) {
-    apair_y_tile<uint16_t>(in, out, nx, ny, nz, blockIdx.x, blockIdx.y, blockIdx.z);
+// One workgroup per tile, tiles in (x, y, z) order.
+template <typename TI, bool QUAD>
+__global__ __launch_bounds__(256) void rs_copy_kernel(const TI* __restrict__ in, uint2* __restrict__ out, int nx, int ny,
+                                                    int nz) {
+    __shared__ uint32_t tile[kColTile + 1][kColLds];
+    const uint32_t gx = (uint32_t)nx / kColTile + 1, gy = (uint32_t)ny + (QUAD ? 1 : 2);
+    const uint32_t b = blockIdx.x, rest = b / gx;
+    rs_copy_tile<TI, QUAD>(in, out, nx, ny, nz, (int)(b % gx), (int)(rest % gy), (int)(rest / gy), tile);
 }
 
 // ---- shared launches of the gradient loop (FP32).  Element-wise tiles
@@ -530,54 +362,24 @@ __device__ __forceinline__ void batch_coords(const BatchItem& it, uint32_t tile,
     bz = (int)(rest / it.gy);
 }
 
-// z-pair copies of FP32 volumes: FP32 (bit copy) or BF16 (kItemBF16), or
-// BF16 A-pair copies (kItemApair, the item's grid is then the A-pair one).
-__global__ __launch_bounds__(256) void zpair_x_batch_kernel(const BatchTable* __restrict__ t) {
-    __shared__ uint32_t tile_lds[2][32][33];
-    __shared__ uint16_t tile_lds16[2][32][33];
-    __shared__ uint16_t tile_ap[2][32][34];
-    __shared__ uint32_t tile_col[kColTile + 1][kColLds];
-    TOMO_BATCH_STRIDED(t) {
-        const BatchItem& it = t->item[batch_find(t, tile)];
-        int bx, by, bz;
-        batch_coords(it, tile, bx, by, bz);
-        if (it.flags & kItemApair)
-            apair_x_tile<float>((const float*)it.in, (uint16_t*)it.out, it.g.nx, it.g.ny, it.g.nz, bx, by, bz,
-                                tile_ap);
-        else if ((it.flags & kItemZcol) && (it.flags & kItemBF16))
-            zcol_tile<float, true>((const float*)it.in, (uint32_t*)it.out, it.g.nx, it.g.ny, it.g.nz, bx, by, bz,
-                                   tile_col);
-        else if (it.flags & kItemZcol)
-            zcol_tile<uint32_t, false>((const uint32_t*)it.in, (uint32_t*)it.out, it.g.nx, it.g.ny, it.g.nz, bx, by, bz,
-                                       tile_col);
-        else if (it.flags & kItemBF16)
-            zpair_x_tile<float, uint16_t>((const float*)it.in, (uint16_t*)it.out, it.g.nx, it.g.ny, it.g.nz, bx, by,
-                                          bz, tile_lds16);
-        else
-            zpair_x_tile<uint32_t, uint32_t>((const uint32_t*)it.in, (uint32_t*)it.out, it.g.nx, it.g.ny, it.g.nz, bx,
-                                             by, bz, tile_lds);
-        __syncthreads();
-    }
-}
-
-// A tile is a whole (y, z pair) row of nx + 2 pairs, in chunks of 256 (the
-// single-problem grid's tiles of one row): tiles of one chunk left half the
-// launch's workgroups nearly empty at 256^3 (258 pairs a row) and paid the
-// table lookup for each.
-__global__ __launch_bounds__(256) void zpair_y_batch_kernel(const BatchTable* __restrict__ t) {
+// The projectors' copies of FP32 volumes: z-columns (kItemZcol) or RS copies, in
+// FP32 (bit copy) or BF16 (kItemBF16).
+__global__ __launch_bounds__(256) void copy_batch_kernel(const BatchTable* __restrict__ t) {
+    __shared__ uint32_t lds[kColTile + 1][kColLds];
     TOMO_BATCH_STRIDED(t) {
         const BatchItem& it = t->item[batch_find(t, tile)];
         int bx, by, bz;
         batch_coords(it, tile, bx, by, bz);
         const int nx = it.g.nx, ny = it.g.ny, nz = it.g.nz;
-        for (int c = 0; c * 256 < nx + 2; ++c) {
-            if (it.flags & kItemApair)  // by: the plane pair
-                apair_y_tile<float>((const float*)it.in, (uint16_t*)it.out, nx, ny, nz, c, by, bz);
-            else if (it.flags & kItemBF16)
-                zpair_y_tile<float, uint16_t>((const float*)it.in, (uint16_t*)it.out, nx, ny, nz, c, by, bz);
-            else
-                zpair_y_tile<uint32_t, uint32_t>((const uint32_t*)it.in, (uint32_t*)it.out, nx, ny, nz, c, by, bz);
+        const bool bf = (it.flags & kItemBF16) != 0;
+        if (it.flags & kItemZcol) {
+            if (bf) zcol_tile<float, true>((const float*)it.in, (uint32_t*)it.out, nx, ny, nz, bx, by, bz, lds);
+            else zcol_tile<uint32_t, false>((const uint32_t*)it.in, (uint32_t*)it.out, nx, ny, nz, bx, by, bz, lds);
+        } else {
+            if (bf) rs_copy_tile<float, true>((const float*)it.in, (uint2*)it.out, nx, ny, nz, bx, by, bz, lds);
+            else rs_copy_tile<uint32_t, false>((const uint32_t*)it.in, (uint2*)it.out, nx, ny, nz, bx, by, bz, lds);
         }
+        __syncthreads();
     }
 }
 
@@ -741,14 +543,6 @@ unsigned grid_for(size_t n) {
 
 }  // namespace
 
-hipError_t launch_apair(const void* vol, void* qx, void* qy, int nx, int ny, int nz, hipStream_t s) {
-    const dim3 gx(ceil_div((size_t)nx + 1, 32), ceil_div((size_t)ny + 2, 32), nz + 1);
-    const dim3 gy(ceil_div((size_t)nx + 2, 256), ny + 1, nz + 1);
-    hipLaunchKernelGGL(apair_x_kernel, gx, dim3(256), 0, s, (const uint16_t*)vol, (uint16_t*)qx, nx, ny, nz);
-    hipLaunchKernelGGL(apair_y_kernel, gy, dim3(256), 0, s, (const uint16_t*)vol, (uint16_t*)qy, nx, ny, nz);
-    return hipGetLastError();
-}
-
 hipError_t launch_zcol(const void* vol, uint32_t* out, size_t es, int nx, int ny, int nz, hipStream_t s) {
     const size_t tiles = (size_t)ceil_div(nx, kColTile) * ny * ceil_div(zcol_pitch(nz, es), kColTile);
     if (es == 4)
@@ -760,20 +554,14 @@ hipError_t launch_zcol(const void* vol, uint32_t* out, size_t es, int nx, int ny
     return hipGetLastError();
 }
 
-hipError_t launch_zpair(const void* vol, void* qx, void* qy, size_t es, int nx, int ny, int nz, hipStream_t s) {
-    const dim3 gx(ceil_div(nx, 32), ceil_div((size_t)ny + 2, 32), ceil_div((size_t)nz + 1, kZChunk));
-    const dim3 gy(ceil_div((size_t)nx + 2, 256), ny, ceil_div((size_t)nz + 1, kZChunk));
-    if (es == 4) {
-        hipLaunchKernelGGL((zpair_x_kernel<uint32_t>), gx, dim3(256), 0, s, (const uint32_t*)vol, (uint32_t*)qx, nx,
-                           ny, nz);
-        hipLaunchKernelGGL((zpair_y_kernel<uint32_t>), gy, dim3(256), 0, s, (const uint32_t*)vol, (uint32_t*)qy, nx,
-                           ny, nz);
-    } else {
-        hipLaunchKernelGGL((zpair_x_kernel<uint16_t>), gx, dim3(256), 0, s, (const uint16_t*)vol, (uint16_t*)qx, nx,
-                           ny, nz);
-        hipLaunchKernelGGL((zpair_y_kernel<uint16_t>), gy, dim3(256), 0, s, (const uint16_t*)vol, (uint16_t*)qy, nx,
-                           ny, nz);
-    }
+hipError_t launch_rs_copy(const void* vol, void* out, size_t es, int nx, int ny, int nz, hipStream_t s) {
+    const size_t tiles = ((size_t)nx / kColTile + 1) * ((size_t)ny + (es == 4 ? 2 : 1)) * ceil_div((size_t)nz + 2, kColTile);
+    if (es == 4)
+        hipLaunchKernelGGL((rs_copy_kernel<uint32_t, false>), dim3((unsigned)tiles), dim3(256), 0, s,
+                           (const uint32_t*)vol, (uint2*)out, nx, ny, nz);
+    else
+        hipLaunchKernelGGL((rs_copy_kernel<uint16_t, true>), dim3((unsigned)tiles), dim3(256), 0, s,
+                           (const uint16_t*)vol, (uint2*)out, nx, ny, nz);
     return hipGetLastError();
 }
 
@@ -789,12 +577,8 @@ hipError_t launch_row_pad(const float* vol, float* out, int nx, int nxp, size_t 
     return hipGetLastError();
 }
 
-hipError_t launch_batch_zpair_x(const BatchTable* t, hipStream_t s) {
-    hipLaunchKernelGGL(zpair_x_batch_kernel, dim3(kBatchGrid), dim3(256), 0, s, t);
-    return hipGetLastError();
-}
-hipError_t launch_batch_zpair_y(const BatchTable* t, hipStream_t s) {
-    hipLaunchKernelGGL(zpair_y_batch_kernel, dim3(kBatchGrid), dim3(256), 0, s, t);
+hipError_t launch_batch_copy(const BatchTable* t, hipStream_t s) {
+    hipLaunchKernelGGL(copy_batch_kernel, dim3(kBatchGrid), dim3(256), 0, s, t);
     return hipGetLastError();
 }
 hipError_t launch_batch_diff_sq(const BatchTable* t, hipStream_t s) {

@@ -44,29 +44,22 @@ struct PoolBuf {
     }
 };
 
-// The projector's copies (z-columns for Siddon; z-pair, or A-pair on 16-bit
-// volumes, for RS, sized for the larger), allocated once for a loop's run and
-// passed to each of its projections (which otherwise take them from the
-// stream-ordered pool per call: two volume-sized allocations per projection,
-// whose pool allocations stalled the host for up to seconds now and then
-// between the loop's synchronisations).  The compat Siddon reads the volume
-// itself and takes none; a Siddon volume beyond its 32-bit traversal index
-// takes none either, so that the projector reports it as unsupported.
+// The projector's copy of the volume, allocated once for a loop's run and passed
+// to each of its projections (which otherwise take it from the stream-ordered
+// pool per call, whose allocations stalled the host for up to seconds now and
+// then between the loop's synchronisations).  The compat Siddon reads the volume
+// itself and takes none; a Siddon volume beyond its 32-bit traversal index takes
+// none either, so that the projector reports it as unsupported.
 struct LoopCopies {
-    PoolBuf qx, qy;
+    PoolBuf buf;
     ProjExtra extra;
     int alloc(const tomo_geom* g, const tomo_gd_params& pr, int storage, hipStream_t s) {
         const int nx = g->info.nx, ny = g->info.ny, nz = g->info.nz;
-        if (pr.pair == TOMO_PAIR_SIDDONVI &&
-            ((pr.flags & TOMO_FLAG_SIDDON_COMPAT) || zpair_elems_x(nx, ny, nz) >= (1ull << 32) ||
-             zpair_elems_y(nx, ny, nz) >= (1ull << 32)))
-            return TOMO_OK;
+        const bool sid = pr.pair == TOMO_PAIR_SIDDONVI;
+        if (sid && ((pr.flags & TOMO_FLAG_SIDDON_COMPAT) || !sid_volume_fits(nx, ny, nz))) return TOMO_OK;
         const size_t es = storage == TOMO_F32 ? 4 : 2;
-        const bool rs = pr.pair != TOMO_PAIR_SIDDONVI;
-        TOMO_HIP(qx.alloc(rs ? proj_copy_bytes_x(nx, ny, nz, es) : zcol_words(nx, ny, nz, es) * 4, s));
-        if (rs) TOMO_HIP(qy.alloc(proj_copy_bytes_y(nx, ny, nz, es), s));
-        extra.qx = qx.p;
-        extra.qy = qy.p;
+        TOMO_HIP(buf.alloc(sid ? zcol_words(nx, ny, nz, es) * 4 : rs_copy_shape(nx, ny, nz, es).elems * 8, s));
+        extra.copy = buf.p;
         return TOMO_OK;
     }
 };

@@ -6,7 +6,7 @@
 // (or a fixed budget) and a slot is free (no reordering, so a large request
 // is never overtaken indefinitely).  Admission carves one stream-ordered
 // allocation into the request's resident state (view tables, volume x,
-// gradient dJ, Laplacian work volumes, z-pair copies, sinograms y / P x /
+// gradient dJ, Laplacian work volumes, the projector's copy, sinograms y / P x /
 // residual / P dJ, the VI box table, FP64 partial sums, loop scalars) and
 // stages its inputs.
 //
@@ -46,7 +46,7 @@ uint32_t cdiv(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
 // Operators of one round, in launch order.  Each has its own table.
 enum Op {
-    OP_ZPX_X, OP_ZPY_X, OP_SID_X, OP_RS_X,  // P x (direct form)
+    OP_COPY_X, OP_SID_X, OP_RS_X,           // P x (direct form)
     OP_LAP_X, OP_LAP_LX,                    // t1 = L x, t2 = L t1 (direct form)
     OP_AXPY_PX, OP_AXPY_LLX,                // recurrent form: px += alpha pd, t2 += alpha t3
     OP_DIFF,                                // r = y - px, partials of r^2
@@ -55,7 +55,7 @@ enum Op {
     OP_AXPY_REG,                            // dJ += 2 lambda t2
     OP_LAP_DJ, OP_FIN_REG,                  // t1 = L dJ, sum t1^2
     OP_LAP_LDJ,                             // recurrent form: t3 = L t1
-    OP_ZPX_D, OP_ZPY_D, OP_SID_D, OP_RS_D,  // pd = P dJ
+    OP_COPY_D, OP_SID_D, OP_RS_D,           // pd = P dJ
     OP_SQ_DJ, OP_SQ_PD, OP_FIN_DJ, OP_FIN_PD,
     OP_STEP, OP_UPDATE,                     // alpha; x += alpha dJ
     OP_COUNT
@@ -74,7 +74,8 @@ struct Request {
     // resident state (valid while admitted)
     void* block = nullptr;
     float *x = nullptr, *dj = nullptr, *t1 = nullptr, *t2 = nullptr, *t3 = nullptr;
-    float *qx = nullptr, *qy = nullptr, *y = nullptr, *px = nullptr, *r = nullptr, *pd = nullptr, *tq = nullptr;
+    void* copy = nullptr;  // the projector's copy of x or dJ
+    float *y = nullptr, *px = nullptr, *r = nullptr, *pd = nullptr, *tq = nullptr;
     double *part_res = nullptr, *part_vol = nullptr, *part_reg = nullptr, *part_pd = nullptr;
     double *slot = nullptr, *hist = nullptr;
     bool bf16 = false;      // BF16 operator copies
@@ -129,13 +130,6 @@ namespace {
 uint32_t vec_tiles(uint64_t n) { return cdiv(n, kVecTile); }
 uint32_t lap_tiles(const DevGeom& d) { return cdiv(d.nx, 64) * cdiv(d.ny, 4) * (uint32_t)d.nz; }
 
-// Whether a request's operator copies are A-pair copies: BF16 copies (ces 2)
-// of an RS request whose A-pair copies take the buffer path (one load per
-// sample); otherwise z-pair copies (FP32 or BF16).
-bool apair_copies(const DevGeom& d, const tomo_gd_params& gd, size_t ces) {
-    return ces == 2 && gd.pair != TOMO_PAIR_SIDDONVI && apair_buffer_path(d.nx, d.ny, d.nz);
-}
-
 Layout layout_of(const tomo_geom& g, const tomo_gd_params& gd, int algo, size_t ces) {
     const DevGeom& d = g.dev;
     const size_t nv = g.nvox(), ns = g.nsino();
@@ -150,11 +144,9 @@ Layout layout_of(const tomo_geom& g, const tomo_gd_params& gd, int algo, size_t 
     sizes[i++] = (lam || sirt) ? nv * 4 : 0;                             // 4 t1 (SIRT: volume weight C)
     sizes[i++] = lam ? nv * 4 : 0;                                       // 5 t2
     sizes[i++] = lam ? nv * 4 : 0;                                       // 6 t3
-    const bool ap = apair_copies(d, gd, ces), sid = gd.pair == TOMO_PAIR_SIDDONVI;
-    sizes[i++] = sid ? zcol_words(d.nx, d.ny, d.nz, ces) * 4             // 7 qx (Siddon: the z-column copy)
-                     : (ap ? apair_elems_x(d.nx, d.ny, d.nz) : zpair_elems_x(d.nx, d.ny, d.nz)) * ces;
-    sizes[i++] = sid ? 0                                                 // 8 qy
-                     : (ap ? apair_elems_y(d.nx, d.ny, d.nz) : zpair_elems_y(d.nx, d.ny, d.nz)) * ces;
+    sizes[i++] = gd.pair == TOMO_PAIR_SIDDONVI ? zcol_words(d.nx, d.ny, d.nz, ces) * 4
+                                               : rs_copy_shape(d.nx, d.ny, d.nz, ces).elems * 8;  // 7 projector's copy
+    sizes[i++] = 0;                                                      // 8 (unused)
     sizes[i++] = ns * 4;                                                 // 9 y
     sizes[i++] = ns * 4;                                                 // 10 px
     sizes[i++] = ns * 4;                                                 // 11 r
@@ -195,8 +187,7 @@ int admit(tomo_server* srv, Request& q) {
     q.t1 = (lam || sirt) ? (float*)at(4) : nullptr;
     q.t2 = lam ? (float*)at(5) : nullptr;
     q.t3 = lam ? (float*)at(6) : nullptr;
-    q.qx = (float*)at(7);
-    q.qy = (float*)at(8);
+    q.copy = at(7);
     q.y = (float*)at(9);
     q.px = (float*)at(10);
     q.r = (float*)at(11);
@@ -288,41 +279,24 @@ void build_tables(tomo_server* srv, int set, const std::vector<Request*>& runnin
         const tomo_gd_params& gd = q.req.gd;
         const size_t nv = q.geom.nvox(), ns = q.geom.nsino();
         const int k = q.k;  // 1-based iteration of this set
-        const uint32_t pgx = cdiv(d.nu, kProjTileU), pgz = cdiv(d.nv, kProjTileV);
         const bool sid = gd.pair == TOMO_PAIR_SIDDONVI;
         const int cube = (gd.flags & TOMO_FLAG_RS_FOV_CUBE) ? 1 : 0;
-        const bool ap = apair_copies(d, gd, q.bf16 ? 2 : 4);
-        const int32_t cflag = (q.bf16 ? kItemBF16 : 0) | (ap ? kItemApair : 0);  // operator copies
-        auto add_projection = [&](const float* vol, float* out, int opx, int opy, int ops, int opr) {
-            if (sid) {
-                BatchItem& z = tb[opx].add(d, cdiv(d.nx, kColTile), d.ny, cdiv(zcol_pitch(d.nz, q.bf16 ? 2 : 4), kColTile));
-                z.in = vol;
-                z.out = q.qx;
-                z.flags = cflag | kItemZcol;
-                const int rows = sid_wave_rows(d.nv);
-                BatchItem& p = tb[ops].add(d, sid_groups(d.nu, rows), cdiv(d.nphi, kSidViews), cdiv(d.nv, rows));
-                p.in = q.qx;
-                p.out = out;
-                p.flags = cflag;
-                return;
-            }
-            BatchItem& zx = ap ? tb[opx].add(d, cdiv(d.nx + 1, 32), cdiv(d.ny + 2, 32), d.nz + 1)
-                               : tb[opx].add(d, cdiv(d.nx, 32), cdiv(d.ny + 2, 32), d.nz + 1);
-            zx.in = vol;
-            zx.out = q.qx;
-            zx.flags = cflag;
-            BatchItem& zy = tb[opy].add(d, 1, ap ? d.ny + 1 : d.ny, d.nz + 1);  // whole rows
-            zy.in = vol;
-            zy.out = q.qy;
-            zy.flags = cflag;
-            BatchItem& p = tb[opr].add(d, pgx, d.nphi, pgz);
-            p.in = q.qx;
-            p.in2 = q.qy;
+        auto add_projection = [&](const float* vol, float* out, int opc, int ops, int opr) {
+            const size_t ces = q.bf16 ? 2 : 4;
+            const int32_t cflag = q.bf16 ? kItemBF16 : 0;
+            BatchItem& z = sid ? tb[opc].add(d, cdiv(d.nx, kColTile), d.ny, cdiv(zcol_pitch(d.nz, ces), kColTile))
+                               : tb[opc].add(d, cdiv(d.nx + 1, kColTile), d.ny + (q.bf16 ? 1 : 2), cdiv(d.nz + 2, kColTile));
+            z.in = vol;
+            z.out = q.copy;
+            z.flags = cflag | (sid ? kItemZcol : 0);
+            const int rows = sid ? sid_wave_rows(d.nv) : rs_wave_rows(d.nv);
+            BatchItem& p = tb[sid ? ops : opr].add(d, proj_groups(d.nu, rows), cdiv(d.nphi, kProjViews), cdiv(d.nv, rows));
+            p.in = q.copy;
             p.out = out;
             p.flags = cube | cflag;
         };
         if (q.req.algorithm == TOMO_ALGO_SIRT) {
-            add_projection(q.x, q.px, OP_ZPX_X, OP_ZPY_X, OP_SID_X, OP_RS_X);
+            add_projection(q.x, q.px, OP_COPY_X, OP_SID_X, OP_RS_X);
             BatchItem& df = tb[OP_DIFF].add_vec(d, ns);
             df.in = q.y;
             df.in2 = q.px;
@@ -358,7 +332,7 @@ void build_tables(tomo_server* srv, int set, const std::vector<Request*>& runnin
         const bool rec = recurrent_server && !gd.positivity && (k == 1 || q.prev_opt);
         const bool rec_zero = rec && k == 1;
         if (!rec) {
-            add_projection(q.x, q.px, OP_ZPX_X, OP_ZPY_X, OP_SID_X, OP_RS_X);
+            add_projection(q.x, q.px, OP_COPY_X, OP_SID_X, OP_RS_X);
             if (lam) {
                 BatchItem& l1 = tb[OP_LAP_X].add(d, cdiv(d.nx, 64), cdiv(d.ny, 4), d.nz);
                 l1.in = q.x;
@@ -433,7 +407,7 @@ void build_tables(tomo_server* srv, int set, const std::vector<Request*>& runnin
             }
         }
         if (opt) {
-            add_projection(q.dj, q.pd, OP_ZPX_D, OP_ZPY_D, OP_SID_D, OP_RS_D);
+            add_projection(q.dj, q.pd, OP_COPY_D, OP_SID_D, OP_RS_D);
             BatchItem& s1 = tb[OP_SQ_DJ].add_vec(d, nv);
             s1.in = q.dj;
             s1.aux = q.part_vol;
@@ -473,8 +447,7 @@ int launch_round(tomo_server* srv, int set) {
     hipError_t e = hipSuccess;
 #define TOMO_STEP(call) \
     if ((e = (call)) != hipSuccess) return hip_fail(e, #call)
-    TOMO_STEP(launch_batch_zpair_x(T + OP_ZPX_X, s));
-    TOMO_STEP(launch_batch_zpair_y(T + OP_ZPY_X, s));
+    TOMO_STEP(launch_batch_copy(T + OP_COPY_X, s));
     TOMO_STEP(launch_batch_siddon(T + OP_SID_X, s));
     TOMO_STEP(launch_batch_rs(T + OP_RS_X, s));
     TOMO_STEP(launch_batch_laplacian(T + OP_LAP_X, s));
@@ -488,8 +461,7 @@ int launch_round(tomo_server* srv, int set) {
     TOMO_STEP(launch_batch_laplacian(T + OP_LAP_DJ, s));
     TOMO_STEP(launch_batch_finish(T + OP_FIN_REG, s));
     TOMO_STEP(launch_batch_laplacian(T + OP_LAP_LDJ, s));
-    TOMO_STEP(launch_batch_zpair_x(T + OP_ZPX_D, s));
-    TOMO_STEP(launch_batch_zpair_y(T + OP_ZPY_D, s));
+    TOMO_STEP(launch_batch_copy(T + OP_COPY_D, s));
     TOMO_STEP(launch_batch_siddon(T + OP_SID_D, s));
     TOMO_STEP(launch_batch_rs(T + OP_RS_D, s));
     TOMO_STEP(launch_batch_sq(T + OP_SQ_DJ, s));
@@ -822,7 +794,7 @@ extern "C" int tomo_serve_submit(tomo_server* srv, const tomo_serve_request* req
     int rc = derive_geometry(req->geom, &q->geom);
     if (rc) return rc;
     const tomo_geom_info& gi = q->geom.info;
-    if (zpair_elems_x(gi.nx, gi.ny, gi.nz) >= (1ull << 32) || zpair_elems_y(gi.nx, gi.ny, gi.nz) >= (1ull << 32))
+    if (!sid_volume_fits(gi.nx, gi.ny, gi.nz))
         return fail(TOMO_ERR_UNSUPPORTED, "volume too large for the Siddon traversal index");
     std::lock_guard<std::mutex> lk(srv->mu);
     if (srv->broken) return fail(TOMO_ERR_HIP, "server stopped after a device failure");

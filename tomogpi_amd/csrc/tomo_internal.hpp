@@ -66,11 +66,14 @@ struct tomo_geom {
 
 namespace tomo {
 
-// Element counts of the z-pair copies of a volume for x slabs (qx) and y
-// slabs (qy): nA * (nz+1) * (nB+2) pairs.
-__host__ __device__ inline size_t zpair_elems_x(int nx, int ny, int nz) { return (size_t)nx * (nz + 1) * (ny + 2) * 2; }
-__host__ __device__ inline size_t zpair_elems_y(int nx, int ny, int nz) { return (size_t)ny * (nz + 1) * (nx + 2) * 2; }
-// z-column copy of a volume of es-byte elements (zpair.hpp): 4-byte words per
+// Volumes the Siddon projector takes: its offsets into the z-column copy, and
+// their steps, are 32-bit (a copy of up to 2^32 words; this bound is half of it
+// and a border).
+inline bool sid_volume_fits(int nx, int ny, int nz) {
+    const size_t z2 = 2 * ((size_t)nz + 1);
+    return (size_t)nx * z2 * ((size_t)ny + 2) < (1ull << 32) && (size_t)ny * z2 * ((size_t)nx + 2) < (1ull << 32);
+}
+// z-column copy of a volume of es-byte elements (proj_copy.hpp): 4-byte words per
 // (x, y) column, and of the whole copy.
 __host__ __device__ inline uint32_t zcol_pitch(int nz, size_t es) { return (uint32_t)nz + (es == 4 ? 2u : 1u); }
 __host__ __device__ inline size_t zcol_words(int nx, int ny, int nz, size_t es) {
@@ -84,39 +87,38 @@ __host__ __device__ inline int sid_wave_rows(int nv) {
         if (((nv + r - 1) / r * r - nv) * 8 <= nv) return r;
     return 16;
 }
-// A Siddon workgroup: one wave's detector cells in kSidViews consecutive views.
-constexpr int kSidViews = 4;
+// A projector workgroup: one wave's detector cells in kProjViews consecutive views.
+constexpr int kProjViews = 4;
 // Column groups (workgroups) of a row band, rounded up to a multiple of the 8
 // XCDs.
-inline uint32_t sid_groups(int nu, int rows) {
+inline uint32_t proj_groups(int nu, int rows) {
     const uint32_t cols = 64u / (uint32_t)rows;
     return ((uint32_t)nu + 8u * cols - 1u) / (8u * cols) * 8u;
 }
-// Element counts of the A-pair copies (16-bit volumes, RS): (nA+1) * (nz+1)
-// * (nB+2) groups of four elements (zpair.hpp).
-__host__ __device__ inline size_t apair_elems_x(int nx, int ny, int nz) { return (size_t)(nx + 1) * (nz + 1) * (ny + 2) * 4; }
-__host__ __device__ inline size_t apair_elems_y(int nx, int ny, int nz) { return (size_t)(ny + 1) * (nz + 1) * (nx + 2) * 4; }
-// Whether RS reads the A-pair copies through 32-bit buffer offsets: each copy
-// below 2^32 - 16 bytes (the offset of a read that returns zeros lies past
-// it) and its plane stride below 2^24 bytes (24-bit multiplies); otherwise
-// 16-bit RS reads the z-pair copies.
-__host__ __device__ inline bool apair_buffer_path(int nx, int ny, int nz) {
-    const uint64_t plane_x = (uint64_t)(ny + 2) * 8u * (uint64_t)(nz + 1);
-    const uint64_t plane_y = (uint64_t)(nx + 2) * 8u * (uint64_t)(nz + 1);
-    return apair_elems_x(nx, ny, nz) * 2u < 0xfffffff0ull && apair_elems_y(nx, ny, nz) * 2u < 0xfffffff0ull &&
-           plane_x < (1ull << 24) && plane_y < (1ull << 24);
+// RS copy of a volume of es-byte elements (proj_copy.hpp): 8-byte elements per x
+// and y step and in all, and whether RS reads it through 32-bit byte offsets
+// (below 2^32 - 16 bytes, where the offset of a read that returns 0 lies, and
+// its steps in signed 24 bits, for 24-bit multiplies).
+struct RsCopyShape {
+    size_t elems;
+    uint32_t sx, sy;
+    bool buf;
+};
+__host__ __device__ inline RsCopyShape rs_copy_shape(int nx, int ny, int nz, size_t es) {
+    RsCopyShape c;
+    const size_t sy = (size_t)nz + 2, sx = sy * ((size_t)ny + (es == 4 ? 2 : 1));
+    c.elems = sx * ((size_t)nx + 1);
+    c.sx = (uint32_t)sx;
+    c.sy = (uint32_t)sy;
+    c.buf = c.elems * 8 < 0xfffffff0ull && sx * 8 < (1ull << 23) && nz < (1 << 23);
+    return c;
 }
-// Bytes of the largest copy any projector form reads for slabs along x (y)
-// from a volume of es-byte elements: what a caller that hands copies to every
-// projection (ProjExtra) allocates.
-inline size_t proj_copy_bytes_x(int nx, int ny, int nz, size_t es) {
-    const size_t z = zpair_elems_x(nx, ny, nz) * es;
-    return es == 2 ? std::max(z, apair_elems_x(nx, ny, nz) * es) : z;
-}
-inline size_t proj_copy_bytes_y(int nx, int ny, int nz, size_t es) {
-    const size_t z = zpair_elems_y(nx, ny, nz) * es;
-    return es == 2 ? std::max(z, apair_elems_y(nx, ny, nz) * es) : z;
-}
+// Detector rows of an RS wave: 32, or 16 where that leaves fewer lanes idle.  At
+// equal sample index the rows of a column drift apart in plane with the cosine
+// of the cone angle, so longer waves touch more columns at once (512^3 / 512
+// views: 68.6 ms at 64 rows, 55.3 at 32, 54.6 at 16); shorter ones read shorter
+// runs of z (1024^3, 96 views: 82, 87, 101 ms).
+__host__ __device__ inline int rs_wave_rows(int nv) { return ((nv + 31) / 32 * 32 - nv) * 8 <= nv ? 32 : 16; }
 
 // Derives the geometry exactly as the reference constructors do.
 int derive_geometry(const tomo_geom_desc& d, tomo_geom* g);
@@ -139,16 +141,15 @@ struct MutBuf {
 int launch_vi(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t s, int fdk = 0);
 int launch_vi_adjoint(const tomo_geom* g, Buf vol, MutBuf sino, hipStream_t s);
 // Projector options beyond the FOV / compat mode.  index_reads: read the
-// z-pair copies through 64-bit element indices even where 32-bit buffer
-// offsets apply (the form every copy of 4 GiB or more takes).  qx, qy: the
-// projector's copies in memory the caller provides (proj_copy_bytes_x / _y
-// bytes each, for the volume's element size); null: the launcher allocates
-// them from the stream-ordered pool for the call.
+// copies through 64-bit element indices even where 32-bit buffer
+// offsets apply (the form every copy of 4 GiB or more takes).  copy: memory of
+// the caller for the projector's copy of the volume (rs_copy_shape or
+// zcol_words, for the volume's element size); null: the launcher allocates it
+// from the stream-ordered pool for the call.
 struct ProjExtra {
     bool index_reads = false;
     bool staged = false;  // RS, Siddon (FP32 volumes): LDS-staged taps instead of per-lane gathers
-    void* qx = nullptr;
-    void* qy = nullptr;
+    void* copy = nullptr;
 };
 int launch_rs(const tomo_geom* g, int cube, Buf vol, MutBuf sino, hipStream_t s, const ProjExtra& x = ProjExtra{});
 int launch_rs_adjoint(const tomo_geom* g, int cube, Buf sino, MutBuf vol, hipStream_t s);
