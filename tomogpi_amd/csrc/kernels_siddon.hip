@@ -16,6 +16,9 @@
 // evaluation order and quirks: source on the +FOD side (mirror of RS/VI),
 // first voxel half a voxel behind the entry, last chord not clipped, indices
 // % 256 with unsigned wrap, no z clip.  Defined for 256^3 volumes only.
+#include <algorithm>
+#include <cmath>
+
 #include "proj_copy.hpp"
 #include "batch.hpp"
 #include "stage_box.hpp"
@@ -758,6 +761,253 @@ __global__ __launch_bounds__(64 * kProjViews) void siddon_batch_kernel(const Bat
     }
 }
 
+// ---------------------------------------------------------------------------
+// Transpose of the clean Siddon as a gather: f(i,j,k) = sum over rays of chord
+// times g, every voxel summed by one lane, written once.
+//
+// In terms of tau, the fraction of the way from the source to the detector
+// cell, all rows n of a detector column m run over the same in-plane line:
+// x(tau) = Sx + tau rx, y(tau) = Sy + tau ry, z(tau) = tau t_n.  So the stretch
+// [tau0, tau1] that column m spends over the column (i, j) of voxels is found
+// once per (view, m) for all z, and a ray's chord in voxel k is its length from
+// source to cell times the part of that stretch in which z(tau) lies between the
+// voxel's planes.  A wave owns the voxel column: its lanes first find the
+// stretches of 64 views at a time, one view each, in FP64 (the columns m whose
+// lines can meet it are those between the projections of its corners), then it
+// takes them one by one, a lane per voxel (K of them, 64 apart), over the rows
+// that can meet it.  The rows of a lane are read with one 16-byte load from a
+// copy of the sinogram with v fastest, already times the ray's length.
+//
+// VALU issue bounds it: about 13 cycles a row, 2-3 rows a voxel, 1.3 columns a
+// view.  256^3 / 256 views: 5.6 ms (6.3 without the bound of 64 registers, which
+// spills some of the FP64 part; 11.6 with one 16-byte load in flight a lane),
+// rel-L2 8e-8 off 64 bits; scattering the chords with FP32 atomics from one
+// lane per ray took 126 ms and was 6e-7 off.  (LDS accumulation is no way
+// out: ds_add_f32 took 190 cycles a wave instruction.)
+constexpr int kSidTWaves = 8;  // waves per workgroup: voxel columns next to each other in x
+constexpr int kSidTPad = 4;    // zero rows at both ends of a column of the sinogram copy
+
+__host__ __device__ inline size_t sid_t_pitch(int nv) { return (size_t)nv + 2 * kSidTPad; }
+
+// out[(p nu + m) pitch + pad + n] = g(p, n, m) |D - S|, 0 for the pad rows; one
+// 64 x 64 tile of one view per workgroup, tiles in (u, v, view) order.
+template <typename TS>
+__global__ __launch_bounds__(256) void siddon_t_prepare_kernel(DevGeom g, const TS* __restrict__ sino, float sino_inv,
+                                                               float* __restrict__ out) {
+    __shared__ float tile[64][65];
+    const int pitch = (int)sid_t_pitch(g.nv);
+    const uint32_t gx = (uint32_t)(g.nu + 63) / 64, gy = (uint32_t)(pitch + 63) / 64;
+    const uint32_t bx = blockIdx.x % gx, rest = blockIdx.x / gx, by = rest % gy;
+    const size_t p = rest / gy;
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const int m = (int)bx * 64 + tx, r0 = (int)by * 64;
+    const double s = ((double)m - (double)g.cu) * (double)g.du;
+    for (int r = ty; r < 64; r += 4) {
+        const int n = r0 + r - kSidTPad;
+        float v = 0.0f;
+        if (m < g.nu && n >= 0 && n < g.nv) {
+            const double t = ((double)n - (double)g.cv) * (double)g.dv;
+            const float gv = Storage<TS>::load(sino, (size_t)m + (size_t)g.nu * ((size_t)n + (size_t)g.nv * p), sino_inv);
+            v = (float)((double)gv * sqrt((g.fdd * g.fdd + s * s) + t * t));
+        }
+        tile[r][tx] = v;
+    }
+    __syncthreads();
+    const int row = r0 + tx;
+    if (row < pitch)
+        for (int r = ty; r < 64; r += 4) {
+            const int mo = (int)bx * 64 + r;
+            if (mo < g.nu) out[(p * (size_t)g.nu + mo) * pitch + row] = tile[tx][r];
+        }
+}
+
+__device__ __forceinline__ double read_lane(double v, int l) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, l);
+    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
+    return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
+}
+__device__ __forceinline__ float read_lane(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// views: the np views of `gt`, from view p0; add: to what vol holds.  Grid: x =
+// (column group, j), y = z block of 64 K voxels.  TIE: an odd number of detector
+// rows over an even number of slices: the middle row's rays run along the plane
+// between two slices, and belong to the upper one, as the projector's; its height
+// is then taken exactly at each row instead of carried on from the first.
+template <int K, bool TIE>
+__global__ __launch_bounds__(64 * kSidTWaves, 8) void siddon_t_kernel(DevGeom g, const float* __restrict__ gt, int p0,
+                                                                   int np, int add, float* __restrict__ vol) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t gx = (uint32_t)(g.nx + kSidTWaves - 1) / kSidTWaves;
+    const int i = (int)(blockIdx.x % gx) * kSidTWaves + wv, j = (int)(blockIdx.x / gx);
+    if (i >= g.nx) return;
+    const int kb = (int)blockIdx.y * 64 * K;
+    const double dl = (double)g.delta, inf = __builtin_inf();
+    // The voxel column's cell in the plane (mm).  The cylinder may be wider than
+    // the grid in y (ny < nx): a ray that comes from outside walks along the
+    // border row until it reaches the grid, so the border cells reach out to
+    // the cylinder for rays that enter on their side.
+    const double Rm = 0.5 * (double)g.nx * dl;
+    const double xa = ((double)i - 0.5 - (double)g.cx) * dl, xb = ((double)i + 0.5 - (double)g.cx) * dl;
+    const double ya = ((double)j - 0.5 - (double)g.cy) * dl, yb = ((double)j + 0.5 - (double)g.cy) * dl;
+    const double ylo = j == 0 ? fmin(ya, -Rm) : ya, yhi = j == g.ny - 1 ? fmax(yb, Rm) : yb;
+    // a cell inside the cylinder needs no cut by it
+    const double fx = fmax(fabs(xa), fabs(xb)), fy = fmax(fabs(ylo), fabs(yhi));
+    const bool cut = !(fx * fx + fy * fy < Rm * Rm * (1.0 - 1e-12));
+    float acc[K];
+#pragma unroll
+    for (int c = 0; c < K; ++c) acc[c] = 0.0f;
+    // lower plane of the lane's first voxel; the next ones lie zstep apart
+    const double zlo = ((double)(kb + lane) - 0.5 - (double)g.cz) * dl, zstep64 = 64.0 * dl;
+    const float zl0 = (float)zlo, zstep = (float)zstep64;
+    const float zabs =
+        (float)(fmax(fabs(((double)kb - 0.5 - (double)g.cz)), fabs((double)min(kb + 64 * K, g.nz) - 0.5 - (double)g.cz)) * dl);
+    const int nu = g.nu, nv = g.nv;
+    const size_t pitch = sid_t_pitch(nv);
+    const float dvf = g.dv, dlf = g.delta, cvf = g.cv;
+    for (int pb = 0; pb < np; pb += 64) {
+        // ---- one view per lane: the columns m that can meet the cell
+        const int pl = pb + lane;
+        int m0 = 0, cnt = 0;
+        double ca = 1.0, sa = 0.0;
+        if (pl < np) {
+            const double* vw = g.view + (size_t)(p0 + pl) * kViewStride;
+            ca = vw[0];
+            sa = vw[1];
+            double u0 = inf, u1 = -inf;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const double X = q & 1 ? xb : xa, Y = q & 2 ? yhi : ylo;
+                const double u = (ca * Y - sa * X) * g.fdd / ((ca * X + sa * Y) + g.fod);
+                u0 = fmin(u0, u);
+                u1 = fmax(u1, u);
+            }
+            const double eps = 1e-6;
+            const double lo = ceil(u0 / (double)g.du + (double)g.cu - eps), hi = floor(u1 / (double)g.du + (double)g.cu + eps);
+            m0 = (int)fmax(lo, 0.0);
+            cnt = max(0, (int)fmin(hi, (double)(nu - 1)) - m0 + 1);
+        }
+        const int most = __builtin_amdgcn_readfirstlane(wave_max(cnt));
+        for (int q = 0; q < most; ++q) {
+            // ---- the stretch of column m0 + q over the cell
+            double tau0 = 0.0;
+            float span = 0.0f, inv0 = 0.0f, inv1 = 0.0f;
+            int rows = 0;
+            const int m = m0 + q;
+            if (q < cnt) {
+                const double s = ((double)m - (double)g.cu) * (double)g.du;
+                const double rx = ca * g.fdd - s * sa, ry = sa * g.fdd + s * ca;
+                const double Sx = -g.fod * ca, Sy = -g.fod * sa;
+                double t0 = 0.0, t1 = 1.0;
+                const double a = rx * rx + ry * ry, b = Sx * rx + Sy * ry, disc = b * b - a * ((Sx * Sx + Sy * Sy) - Rm * Rm);
+                bool ok = disc > 0.0;
+                if (cut && ok) {
+                    const double sq = sqrt(disc);
+                    t0 = (-b - sq) / a;
+                    t1 = (-b + sq) / a;
+                }
+                // A line along an axis keeps its voxel index on the other one,
+                // floor(position + 1/2) where it enters, as the projector's.
+                const double flat = 1e-9 * g.fdd;
+                if (fabs(rx) < flat) {
+                    ok = ok && floor((Sx + t0 * rx) / dl + (double)g.cx + 0.5) == (double)i;
+                } else {
+                    const double c0 = (xa - Sx) / rx, c1 = (xb - Sx) / rx;
+                    t0 = fmax(t0, fmin(c0, c1));
+                    t1 = fmin(t1, fmax(c0, c1));
+                }
+                if (fabs(ry) < flat) {
+                    const double at = floor((Sy + t0 * ry) / dl + (double)g.cy + 0.5);
+                    ok = ok && fmin(fmax(at, 0.0), (double)(g.ny - 1)) == (double)j;
+                } else {
+                    const double c0 = ((ry > 0.0 ? ylo : ya) - Sy) / ry, c1 = ((ry < 0.0 ? yhi : yb) - Sy) / ry;
+                    t0 = fmax(t0, fmin(c0, c1));
+                    t1 = fmin(t1, fmax(c0, c1));
+                }
+                if (ok && t1 > t0) {
+                    tau0 = t0;
+                    span = (float)(t1 - t0);
+                    // rows per mm of height at both ends; the most rows that meet one voxel
+                    inv0 = (float)(1.0 / (t0 * (double)g.dv));
+                    inv1 = (float)(1.0 / (t1 * (double)g.dv));
+                    rows = (int)(dlf * inv0 + zabs * (inv0 - inv1) + 4e-3f) + 1;
+                }
+            }
+            // ---- every voxel of the column, one stretch at a time; the 64 views'
+            // parts are summed apart, which keeps the sum's rounding near one
+            // of a few dozen terms
+            float part[K];
+#pragma unroll
+            for (int c = 0; c < K; ++c) part[c] = 0.0f;
+            for (uint64_t todo = __ballot(rows > 0); todo != 0ull; todo &= todo - 1) {
+                const int l = __builtin_ctzll(todo);
+                const double step = read_lane(tau0, l) * (double)g.dv;  // z per row at tau0
+                const float dt = read_lane(span, l), i0 = read_lane(inv0, l), i1 = read_lane(inv1, l);
+                const int most_rows = __builtin_amdgcn_readlane(rows, l), ml = __builtin_amdgcn_readlane(m, l);
+                const float* col = gt + ((size_t)(pb + l) * nu + ml) * pitch + kSidTPad;
+                const float stepf = (float)step;
+float nf[K];
+#pragma unroll
+                for (int c = 0; c < K; ++c) {
+                    // first row that can reach the voxel
+                    const float zl = zl0 + zstep * (float)c;
+                    nf[c] = ceilf(fmaf(zl, zl > 0.0f ? i1 : i0, cvf) - 2e-3f);
+                }
+                for (int left = most_rows; left > 0; left -= 4) {
+                    float4 gv[K];
+#pragma unroll
+                    for (int c = 0; c < K; ++c) {
+                        nf[c] = __builtin_amdgcn_fmed3f(nf[c], (float)-kSidTPad, (float)nv);  // within the padded column
+                        __builtin_memcpy(&gv[c], col + (int)nf[c], 16);
+                    }
+#pragma unroll
+                    for (int c = 0; c < K; ++c) {
+                        // The rows are whole before the branches on their number:
+                        // sunk into them, their loads met at a common last one
+                        // whose address the compiler (clang 22 of ROCm 7.2) left
+                        // undefined for four rows.  An empty statement.
+                        asm volatile("" : "+v"(gv[c].x), "+v"(gv[c].y), "+v"(gv[c].z), "+v"(gv[c].w));
+                        // height of row nf at tau0 above the voxel's lower plane
+                        const double zl = zlo + zstep64 * (double)c;
+                        float z0 = (float)fma(step, (double)(nf[c] - cvf), -zl);
+                        auto row = [&](float gn, bool first) __attribute__((always_inline)) {
+                            if (TIE && !first) z0 = (float)fma(step, (double)(nf[c] - cvf), -zl);
+                            const float t = (nf[c] - cvf) * dvf + 1e-30f;
+                            const float rt = __builtin_amdgcn_rcpf(t);
+                            // where the row crosses the voxel's planes, from tau0
+                            const float a = -z0 * rt, b = fmaf(dlf, rt, a);
+                            const float in = fminf(fmaxf(a, b), dt) - fmaxf(fminf(a, b), 0.0f);
+                            part[c] = fmaf(in, in > 0.0f ? gn : 0.0f, part[c]);
+                            nf[c] += 1.0f;
+                            if (!TIE) z0 += stepf;
+                        };
+                        row(gv[c].x, true);
+                        if (left > 1) {
+                            row(gv[c].y, false);
+                            if (left > 2) {
+                                row(gv[c].z, false);
+                                if (left > 3) row(gv[c].w, false);
+                            }
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < K; ++c) acc[c] += part[c];
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+        const int k = kb + 64 * c + lane;
+        if (k < g.nz) {
+            float* o = vol + ((size_t)i + (size_t)g.nx * ((size_t)j + (size_t)g.ny * k));
+            *o = add ? *o + acc[c] : acc[c];
+        }
+    }
+}
+
 template <typename TS>
 __global__ __launch_bounds__(BX* BY) void siddon_adjoint_kernel(DevGeom g, const TS* __restrict__ sino,
                                                               float sino_inv, float* __restrict__ vol) {
@@ -939,13 +1189,67 @@ hipError_t launch_batch_siddon(BatchTable* t, hipStream_t s) {
     return hipGetLastError();
 }
 
+// The gather needs every voxel column in front of the source in every view (its
+// corners project onto the detector plane); a geometry with the source inside
+// the cylinder's bounding square scatters.  So do the smallest problems, whose
+// few chords cost less than the gather's extra launch and its FP64 chain: 24^3 /
+// 16 views 18.8 us against 28.8, 24^3 / 32 views 32.3 and 34.7, 32^3 / 16 views
+// 30.0 and 28.6, 32^3 / 32 views 50.0 and 34.6, 64^3 / 64 views 669 and 70.
+static bool sid_t_gathers(const DevGeom& d) {
+    const double half = 0.5 * (double)d.delta * (double)std::max(d.nx, d.ny);
+    const double chords = (double)d.nu * d.nv * d.nphi * std::max(d.nx, d.ny);
+    return d.fod > 1.01 * std::sqrt(2.0) * half && chords >= 8e5;
+}
+
+template <int K>
+static void launch_siddon_t(const DevGeom& d, const float* gt, int p0, int np, float* vol, hipStream_t s) {
+    const dim3 grid(ceil_div(d.nx, kSidTWaves) * (unsigned)d.ny, ceil_div(d.nz, 64 * K));
+    if (d.nv % 2 == 1 && d.nz % 2 == 0)
+        hipLaunchKernelGGL((siddon_t_kernel<K, true>), grid, dim3(64 * kSidTWaves), 0, s, d, gt, p0, np, p0 > 0, vol);
+    else
+        hipLaunchKernelGGL((siddon_t_kernel<K, false>), grid, dim3(64 * kSidTWaves), 0, s, d, gt, p0, np, p0 > 0, vol);
+}
+
 int launch_siddon_adjoint(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t s) {
     if (vol.dtype != TOMO_F32) return fail(TOMO_ERR_UNSUPPORTED, "adjoint output must be F32");
     const DevGeom& d = g->dev;
+    const float inv = 1.0f / sino.scale;
+    // the sinogram copy, at most 1 GiB of views at a time; without the memory the chords scatter
+    const size_t view = (size_t)d.nu * sid_t_pitch(d.nv) * sizeof(float);
+    const int chunk = (int)std::min<size_t>((size_t)d.nphi, std::max<size_t>(1, ((size_t)1 << 30) / view));
+    float* gt = nullptr;
+    if (sid_t_gathers(d) && hipMallocAsync((void**)&gt, view * (size_t)chunk, s) != hipSuccess) {
+        (void)hipGetLastError();
+        gt = nullptr;
+    }
+    if (gt) {
+        hipError_t e = hipSuccess;
+        for (int p0 = 0; p0 < d.nphi && e == hipSuccess; p0 += chunk) {
+            const int np = std::min(chunk, d.nphi - p0);
+            const size_t skip = (size_t)p0 * d.nu * d.nv;
+            const unsigned tiles = ceil_div(d.nu, 64) * ceil_div(sid_t_pitch(d.nv), 64) * (unsigned)np;
+            TOMO_DISPATCH_STORAGE(sino.dtype, TS, {
+                hipLaunchKernelGGL((siddon_t_prepare_kernel<TS>), dim3(tiles), dim3(256), 0, s, d,
+                                   (const TS*)sino.p + skip, inv, gt);
+            });
+            // K 64-voxel steps per lane: the fewest z blocks that K <= 4 allows
+            const int steps = (int)ceil_div(d.nz, 64), blocks = (int)ceil_div(steps, 4);
+            switch (ceil_div(steps, blocks)) {
+                case 1: launch_siddon_t<1>(d, gt, p0, np, (float*)vol.p, s); break;
+                case 2: launch_siddon_t<2>(d, gt, p0, np, (float*)vol.p, s); break;
+                case 3: launch_siddon_t<3>(d, gt, p0, np, (float*)vol.p, s); break;
+                default: launch_siddon_t<4>(d, gt, p0, np, (float*)vol.p, s); break;
+            }
+            e = hipGetLastError();
+        }
+        const hipError_t f = hipFreeAsync(gt, s);
+        TOMO_HIP(e);
+        TOMO_HIP(f);
+        return TOMO_OK;
+    }
     int rc = launch_fill((float*)vol.p, 0.0f, g->nvox(), s);
     if (rc) return rc;
     const dim3 grid(ceil_div(d.nu, BX), d.nphi, ceil_div(d.nv, BY));
-    const float inv = 1.0f / sino.scale;
     TOMO_DISPATCH_STORAGE(sino.dtype, TS, {
         hipLaunchKernelGGL((siddon_adjoint_kernel<TS>), grid, dim3(BX, BY), 0, s, d, (const TS*)sino.p, inv,
                            (float*)vol.p);
