@@ -95,3 +95,92 @@ def test_siddon_transpose_infinity(ctx):
         assert np.isinf(got[hit]).mean() > 0.99  # a chord of rounding length may count as none
     finally:
         G.close()
+
+
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("nx,ny,nz,nu,nv,nphi,pixel", [
+    (30, 30, 30, 40, 63, 20, 2.0), (30, 31, 33, 41, 64, 21, 2.0), (31, 30, 40, 42, 65, 20, 2.0),  # one, two steps of rows
+    (33, 17, 129, 17, 190, 31, 2.0), (16, 16, 200, 24, 256, 20, 2.0),  # three, four; partial column groups
+    (16, 16, 180, 19, 257, 20, 2.0), (64, 20, 24, 64, 33, 40, 2.0),    # two row blocks; a narrow grid
+    (20, 20, 20, 90, 90, 12, 0.3), (40, 40, 60, 9, 11, 30, 9.0),       # many cells a voxel, many voxels a cell
+    (40, 40, 61, 30, 34, 30, 4.0), (33, 1, 1, 50, 7, 70, 1.0), (1, 1, 40, 9, 60, 30, 1.0),  # one slice, one column
+    (20, 20, 20, 1, 1, 8, 3.0),
+])
+def test_vi_transpose(ctx, nx, ny, nz, nu, nv, nphi, pixel, dt):
+    g = _geom(nx, ny, nz, nu, nv, nphi, pixel)
+    G = _geometry(ctx, g)
+    try:
+        x = dev(np.random.default_rng(nz).random(g.vol_shape, dtype=np.float32))
+        if dt != "f32":
+            x = x.to(torch.bfloat16 if dt == "bf16" else torch.float16)
+        ref = Oracle(g).vi_T(x.float().cpu().numpy())
+        out = torch.full(g.sino_shape, np.nan, dtype=torch.float32, device="cuda")
+        G.backproject_adjoint(x, out)
+        assert rel_l2(out.cpu().numpy(), ref) <= 1e-6
+    finally:
+        G.close()
+
+
+def test_vi_transpose_source_inside(ctx):
+    """A source inside the volume's bounding square (the scatter form)."""
+    g = _geom(40, 40, 30, 40, 40, 24, pixel=1.0, fod=0.6)
+    G = _geometry(ctx, g)
+    try:
+        x = np.random.default_rng(3).random(g.vol_shape, dtype=np.float32)
+        out = torch.empty(g.sino_shape, dtype=torch.float32, device="cuda")
+        G.backproject_adjoint(dev(x), out)
+        assert rel_l2(out.cpu().numpy(), Oracle(g).vi_T(x)) <= 1e-5
+    finally:
+        G.close()
+
+
+def test_vi_transpose_infinity(ctx):
+    """An infinite voxel reaches the cells around its projections and no other."""
+    g = _geom(32, 32, 40, 48, 70, 20)
+    G = _geometry(ctx, g)
+    try:
+        x = np.random.default_rng(8).random(g.vol_shape, dtype=np.float32)
+        one = np.zeros_like(x)
+        one[17, 30, 20] = 1.0
+        hit = Oracle(g).vi_T(one) > 0.0
+        x[17, 30, 20] = np.inf
+        out = torch.empty(g.sino_shape, dtype=torch.float32, device="cuda")
+        G.backproject_adjoint(dev(x), out)
+        got = out.cpu().numpy()
+        assert np.isfinite(got[~hit]).all()
+        assert np.isinf(got[hit]).mean() > 0.99  # a weight of rounding size may count as none
+    finally:
+        G.close()
+
+
+@pytest.mark.parametrize("op", ["siddon", "vi"])
+def test_transpose_under_capture(ctx, op):
+    """A captured transpose allocates nothing: the scatter form, replayed with new
+    inputs against the eager call (1e-5: two FP32 sums of the same terms)."""
+    g = _geom(48, 48, 48, 48, 48, 40)
+    G = _geometry(ctx, g)
+    try:
+        a, b = (g.sino_shape, g.vol_shape) if op == "siddon" else (g.vol_shape, g.sino_shape)
+        x, y = torch.rand(a, device="cuda"), torch.empty(b, device="cuda")
+
+        def run(out):
+            if op == "siddon":
+                G.project_adjoint(x, out, lib.PROJ_SIDDON)
+            else:
+                G.backproject_adjoint(x, out)
+
+        run(y)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            run(y)
+        for _ in range(4):
+            x.uniform_()
+            y.fill_(np.nan)
+            graph.replay()
+            eager = torch.empty_like(y)
+            run(eager)
+            torch.cuda.synchronize()
+            assert rel_l2(y.cpu().numpy(), eager.cpu().numpy()) <= 1e-5
+    finally:
+        G.close()

@@ -119,6 +119,15 @@ __device__ __forceinline__ float tap(const T* p, int64_t idx, bool ok, float inv
     return ok ? v : 0.0f;
 }
 
+// Whether work given to the stream is being captured into a graph.
+inline bool stream_captures(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
 inline unsigned ceil_div(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
 
 // Dispatch a templated launcher on a TOMO_F32/F16/BF16 code.

@@ -1214,11 +1214,13 @@ int launch_siddon_adjoint(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t 
     if (vol.dtype != TOMO_F32) return fail(TOMO_ERR_UNSUPPORTED, "adjoint output must be F32");
     const DevGeom& d = g->dev;
     const float inv = 1.0f / sino.scale;
-    // the sinogram copy, at most 1 GiB of views at a time; without the memory the chords scatter
+    // the sinogram copy, at most 1 GiB of views at a time; without the memory, or in a stream
+    // capture, which is left free of allocations, the chords scatter
     const size_t view = (size_t)d.nu * sid_t_pitch(d.nv) * sizeof(float);
     const int chunk = (int)std::min<size_t>((size_t)d.nphi, std::max<size_t>(1, ((size_t)1 << 30) / view));
     float* gt = nullptr;
-    if (sid_t_gathers(d) && hipMallocAsync((void**)&gt, view * (size_t)chunk, s) != hipSuccess) {
+    if (!stream_captures(s) && sid_t_gathers(d) &&
+        hipMallocAsync((void**)&gt, view * (size_t)chunk, s) != hipSuccess) {
         (void)hipGetLastError();
         gt = nullptr;
     }

@@ -504,6 +504,234 @@ __global__ __launch_bounds__(TX* TY) void vi_adjoint_kernel(DevGeom g, const TV*
     }
 }
 
+// ---------------------------------------------------------------------------
+// VI^T as a gather: g_p(n, m) = sum over voxels of their bilinear weight at the
+// cell times delta f, every cell summed by one lane, written once.
+//
+// A column (i, j) of voxels projects onto one u for all z, between the detector
+// columns floor(u) and floor(u) + 1, and its voxels onto v = fma(z', A, cv).  A
+// wave owns M neighbouring detector columns of a view and 64 K rows, a
+// lane per row (K of them, 64 apart).  The voxel columns that project between
+// its outer neighbours lie in a strip; it is walked along the in-plane axis the
+// strip is steeper to, 64 slabs at a time: each lane finds its slab's cells (the
+// crossings of the two outer lines) and their FP64 column terms, then the wave
+// takes the voxel columns one by one: the column's voxels go through the wave's
+// piece of LDS (one 16-byte load per lane, the next column's in flight), and a
+// lane sums its two or three with the weights 1 - |v - n|; the sum goes to the
+// detector columns on both sides of u.  v - n is one fused operation from the
+// exact cv - n, and the fraction of u is taken in FP64: v and u are never
+// rounded to the FP32 of a large coordinate.
+//
+// VALU issue takes about half of its time, waits on the columns most of the rest
+// (they come from the memory-side cache: 256^3 and 256 views read 6 GB).  201 x
+// 187 x 149, 229 x 173, 131 views: 10.0 -> 1.10 ms against the scatter below;
+// 256^3 and 256 views 71.9 -> 3.44 ms.
+constexpr int kViTPad = 4;
+constexpr int kViTWords = 512;  // voxels of a column a wave stages, two loads of 64 x 4
+__host__ __device__ inline size_t vi_t_pitch(int nz) { return (size_t)(nz + 3) / 4 * 4 + 2 * kViTPad; }
+
+// out[(x ny + y) pitch + pad + z] = delta f(x, y, z), 0 for the pad; one tile of
+// 64 x and 64 words of their columns at one y per workgroup.
+template <typename TV>
+__global__ __launch_bounds__(256) void vi_t_prepare_kernel(DevGeom g, const TV* __restrict__ vol, float vol_inv,
+                                                           float* __restrict__ out) {
+    __shared__ float tile[64][65];
+    const int pitch = (int)vi_t_pitch(g.nz);
+    const uint32_t gx = (uint32_t)(g.nx + 63) / 64;
+    const uint32_t bx = blockIdx.x % gx, rest = blockIdx.x / gx, y = rest % (uint32_t)g.ny, bz = rest / (uint32_t)g.ny;
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const int x = (int)bx * 64 + tx, r0 = (int)bz * 64;
+    for (int r = ty; r < 64; r += 4) {
+        const int z = r0 + r - kViTPad;
+        float v = 0.0f;
+        if (x < g.nx && z >= 0 && z < g.nz)
+            v = Storage<TV>::load(vol, (size_t)x + (size_t)g.nx * ((size_t)y + (size_t)g.ny * z), vol_inv) * g.delta;
+        tile[r][tx] = v;
+    }
+    __syncthreads();
+    const int row = r0 + tx;
+    if (row < pitch)
+        for (int r = ty; r < 64; r += 4) {
+            const int xo = (int)bx * 64 + r;
+            if (xo < g.nx) out[((size_t)xo * g.ny + y) * pitch + row] = tile[tx][r];
+        }
+}
+
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// Grid: x = (view, column group), views first; y = row block of 64 K rows.  One
+// wave per workgroup: nothing is shared, and the strips differ in length.
+template <int K, int M>
+__global__ __launch_bounds__(64, 5) void vi_t_kernel(DevGeom g, const float* __restrict__ vt, float* __restrict__ sino) {
+    typedef float V4 __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) float stage[kViTWords + 8];
+    const int lane = threadIdx.x;
+    const int p = (int)(blockIdx.x % (uint32_t)g.nphi), m0 = (int)(blockIdx.x / (uint32_t)g.nphi) * M;
+    const int nb = (int)blockIdx.y * 64 * K;
+    typedef const __attribute__((address_space(4))) double* ConstView;
+    const ConstView vw = (ConstView)(g.view + (size_t)p * kViewStride);
+    double cvt[kViewStride];
+#pragma unroll
+    for (int e = 0; e < kViewStride; ++e) cvt[e] = vw[e];
+    const double ca = cvt[0], sa = cvt[1], dl = (double)g.delta;
+    const double Sx = -g.fod * ca, Sy = -g.fod * sa;
+    auto line = [&](double col, double& rx, double& ry) {
+        const double s = (col - (double)g.cu) * (double)g.du;
+        rx = ca * g.fdd - s * sa;
+        ry = sa * g.fdd + s * ca;
+    };
+    double rx, ry, ax, ay, bx, by;
+    line((double)m0 + 0.5 * (M - 1), rx, ry);
+    line((double)(m0 - 1), ax, ay);
+    line((double)(m0 + M), bx, by);
+    const bool alongy = fabs(ry) >= fabs(rx);
+    const int nA = alongy ? g.ny : g.nx, nB = alongy ? g.nx : g.ny;
+    const double cA = alongy ? (double)g.cy : (double)g.cx, cB = alongy ? (double)g.cx : (double)g.cy;
+    const double SA = alongy ? Sy : Sx, SB = alongy ? Sx : Sy;
+    const double ta = alongy ? ax / ay : ay / ax, tb = alongy ? bx / by : by / bx;  // B per A along the outer lines
+    const float row0 = (float)(nb + lane) - g.cv, first = (float)nb - g.cv;  // exact: cv is a multiple of 1/2
+    const float czf = g.cz, czs = czf - 2e-3f;
+    const int quads = (g.nz + 3) / 4;
+    const size_t pitch = vi_t_pitch(g.nz);
+    float acc[M][K];
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+#pragma unroll
+        for (int e = 0; e < M; ++e) acc[e][c] = 0.0f;
+    // first voxel that can reach a row: the rounding of these coordinates is
+    // below the 2e-3, whose voxel has a weight of that size at most
+    auto first_voxel = [&](float row, float inv) __attribute__((always_inline)) {
+        return ceilf(fmaf(row - 1.0f, inv, czs));
+    };
+    for (int ab = 0; ab < nA; ab += 64) {
+        // ---- one slab per lane: its cells between the outer lines
+        const int a = ab + lane;
+        int b0 = 0, cnt = 0;
+        if (a < nA) {
+            const double at = ((double)a - cA) * dl - SA;
+            const double pa = (SB + at * ta) / dl + cB, pb = (SB + at * tb) / dl + cB;
+            const double lo = ceil(fmin(pa, pb) - 1e-6), hi = floor(fmax(pa, pb) + 1e-6);
+            b0 = (int)fmax(lo, 0.0);
+            cnt = max(0, (int)fmin(hi, (double)(nB - 1)) - b0 + 1);
+        }
+        const int most = __builtin_amdgcn_readfirstlane(wave_max(cnt));
+        for (int q = 0; q < most; ++q) {
+            const int b = b0 + q;
+            const int i = alongy ? b : a, j = alongy ? a : b;
+            const double xp = (double)i - (double)g.cx, yp = (double)j - (double)g.cy;
+            const double iw = 1.0 / fma(cvt[2], xp, fma(cvt[3], yp, g.fod));
+            const double u = fma(fma(cvt[4], xp, cvt[5] * yp), iw, (double)g.cu), uf = floor(u);
+            const double e0 = uf - (double)m0;  // the detector column floor(u), from m0
+            const float lwu = (float)(u - uf), lA = (float)(cvt[6] * iw), linv = 1.0f / lA;
+            const float lstart = floorf(first_voxel(first, linv) * 0.25f), reach = floorf(2.0f * linv + 4e-3f) + 1.0f;
+            // the column's words from lstart on that the rows reach: a second load where they exceed 64 quads
+            const float words = first_voxel(first + (float)(64 * K - 1), linv) + reach - 4.0f * lstart;
+            const int far = words > 256.0f ? 1 : 0;
+            const bool on = q < cnt && e0 >= -1.0 && e0 <= (double)(M - 1) && lA > 0.0f &&
+                            lstart < (float)(quads + 1) && words <= (float)kViTWords;
+            const int lquad = (int)fmaxf(lstart, -1048576.0f), lcol = i * g.ny + j;
+            const int lhow = ((int)e0 + 1) | far << 4 | (int)reach << 8;
+            uint64_t todo = __ballot(on);
+            if (todo == 0ull) continue;
+            V4 f0, f1;
+            auto load = [&](int l) __attribute__((always_inline)) {
+                const float* zc = vt + (size_t)(uint32_t)__builtin_amdgcn_readlane(lcol, l) * pitch;
+                const int at = __builtin_amdgcn_readlane(lquad, l) + lane;
+                // quads before and after the column are 0, as its pads are
+                f0 = *(const V4*)((const char*)zc + (uint32_t)(min(max(at, -1), quads) + 1) * 16u);
+                if (__builtin_amdgcn_readlane(lhow, l) >> 4 & 1)
+                    f1 = *(const V4*)((const char*)zc + (uint32_t)(min(max(at + 64, -1), quads) + 1) * 16u);
+            };
+            f0 = f1 = (V4)0.0f;
+            load(__builtin_ctzll(todo));
+            do {
+                const int l = __builtin_ctzll(todo);
+                const int how = __builtin_amdgcn_readlane(lhow, l);
+                todo &= todo - 1;
+                *(V4*)(stage + 4 * lane) = f0;
+                if (how >> 4 & 1) *(V4*)(stage + 256 + 4 * lane) = f1;
+                if (todo != 0ull) load(__builtin_ctzll(todo));
+                const float A = lane_value(lA, l), inv = lane_value(linv, l), wu = lane_value(lwu, l);
+                const float start = 4.0f * lane_value(lstart, l);
+                const int voxels = how >> 8;
+                const float* at[K];
+                float t0[K], part[K];
+#pragma unroll
+                for (int c = 0; c < K; ++c) {
+                    const float row = row0 + (float)(64 * c), k = first_voxel(row, inv);
+                    at[c] = stage + (uint32_t)(k - start);
+                    t0[c] = fmaf(k - czf, A, -row);
+                }
+                // The lane's voxels.  A weight of 0 takes nothing from its voxel, whatever it
+                // holds: a sum that is not finite is taken again with that test (FINITE off).
+                auto sum = [&](auto finite) __attribute__((always_inline)) {
+                    float t[K];
+                    auto voxel = [&](int c, float fk) __attribute__((always_inline)) {
+                        const float w = __builtin_amdgcn_fmed3f(1.0f - fabsf(t[c]), 0.0f, 1.0f);
+                        if constexpr (decltype(finite)::value)
+                            part[c] = fmaf(w, fk, part[c]);
+                        else
+                            part[c] = w > 0.0f ? fmaf(w, fk, part[c]) : part[c];
+                        t[c] += A;
+                    };
+#pragma unroll
+                    for (int c = 0; c < K; ++c) {
+                        t[c] = t0[c];
+                        part[c] = 0.0f;
+                    }
+                    // read in threes, the second and third also where only the first counts
+                    for (int k = 0; k < voxels; k += 3) {
+                        float f[3][K];
+#pragma unroll
+                        for (int c = 0; c < K; ++c)
+#pragma unroll
+                            for (int h = 0; h < 3; ++h) f[h][c] = at[c][k + h];
+#pragma unroll
+                        for (int c = 0; c < K; ++c) voxel(c, f[0][c]);
+                        if (k + 1 < voxels) {
+#pragma unroll
+                            for (int c = 0; c < K; ++c) voxel(c, f[1][c]);
+                        }
+                        if (k + 2 < voxels) {
+#pragma unroll
+                            for (int c = 0; c < K; ++c) voxel(c, f[2][c]);
+                        }
+                    }
+                };
+                sum(std::true_type{});
+                bool odd = false;
+#pragma unroll
+                for (int c = 0; c < K; ++c) odd |= !__builtin_isfinite(part[c]);
+                if (__ballot(odd) != 0ull) sum(std::false_type{});
+                const int e = (how & 15) - 1;
+#pragma unroll
+                for (int d = -1; d < M; ++d)
+                    if (e == d) {
+                        // a branch, not selects over all columns (empty statement)
+                        asm volatile("" : "+v"(part[0]));
+#pragma unroll
+                        for (int c = 0; c < K; ++c) {
+                            if (d >= 0) acc[d < 0 ? 0 : d][c] = fmaf(1.0f - wu, part[c], acc[d < 0 ? 0 : d][c]);
+                            if (d + 1 < M) acc[d + 1 < M ? d + 1 : 0][c] = fmaf(wu, part[c], acc[d + 1 < M ? d + 1 : 0][c]);
+                        }
+                    }
+            } while (todo != 0ull);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+        const int n = nb + 64 * c + lane;
+        if (n < g.nv) {
+            float* o = sino + ((size_t)m0 + (size_t)g.nu * ((size_t)n + (size_t)g.nv * p));
+#pragma unroll
+            for (int d = 0; d < M; ++d)
+                if (m0 + d < g.nu) o[d] = acc[d][c];
+        }
+    }
+}
+
 }  // namespace
 
 // Voxels per thread column of the staged kernel.
@@ -605,13 +833,74 @@ hipError_t launch_batch_vi(BatchTable* t, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Row steps per lane of the gather, the fewest row blocks that K <= 4 allows;
+// 0 where it does not apply and the voxels scatter: a voxel column behind or
+// beside the source, a wave's outer lines too far apart (detector columns as
+// wide as a 20th of the distance to them), or 64 rows that reach more than
+// kViTWords voxels of a column (7.8 voxels to a row).  There is no lower limit:
+// 17^3 and 16 views take 33 us here and 108 scattered.
+static int vi_t_steps(const DevGeom& d) {
+    const double half = 0.5 * (double)d.delta * (double)std::max(d.nx, d.ny);
+    const double far = d.fod + std::sqrt(2.0) * half;
+    const double inv = far * (double)d.dv / ((double)d.delta * d.fdd);  // most voxels to a row
+    if (!(d.fod > 1.01 * std::sqrt(2.0) * half && (double)d.du * (4 + 1) < 0.25 * d.fdd)) return 0;
+    // FP32 voxel coordinates within 1e-3, 32-bit column numbers
+    if (d.nv * inv + d.nz > 8192.0 || (double)d.nx * d.ny > 2147483647.0) return 0;
+    const int steps = (int)ceil_div(d.nv, 64), most = std::min(4, (int)(((kViTWords - 6) / (1.001 * inv) - 1.0) / 64.0));
+    return most < 1 ? 0 : (int)ceil_div(steps, ceil_div(steps, most));
+}
+
+template <int K>
+static void launch_vi_t(const DevGeom& d, const float* vt, float* sino, hipStream_t s) {
+    // Columns per wave: wide strips share their voxel columns, M + 1 reads for M
+    // columns; narrow ones are more waves (1024 SIMDs).  Waves at M = 4, us at
+    // M = 1 / 2 / 4: 1024 (64^3, 64 views) 81 / 103 / 172; 1152 (96^3, 48) 160 /
+    // 197 / 311; 4096 (128^3, 128) 484 / 416 / 454; 7598 (201 x 187 x 149, 131)
+    // 1253 / 1128 / 1104; 16384 (256^3, 256) 4636 / 3689 / 3445.
+    const size_t waves = (size_t)ceil_div(d.nu, 4) * d.nphi * ceil_div(d.nv, 64 * K);
+    const int cols = waves < 2048 ? 1 : waves < 6144 ? 2 : 4;
+    const dim3 grid(ceil_div(d.nu, cols) * (unsigned)d.nphi, ceil_div(d.nv, 64 * K));
+    if (cols == 1)
+        hipLaunchKernelGGL((vi_t_kernel<K, 1>), grid, dim3(64), 0, s, d, vt, sino);
+    else if (cols == 2)
+        hipLaunchKernelGGL((vi_t_kernel<K, 2>), grid, dim3(64), 0, s, d, vt, sino);
+    else
+        hipLaunchKernelGGL((vi_t_kernel<K, 4>), grid, dim3(64), 0, s, d, vt, sino);
+}
+
 int launch_vi_adjoint(const tomo_geom* g, Buf vol, MutBuf sino, hipStream_t s) {
     if (sino.dtype != TOMO_F32) return fail(TOMO_ERR_UNSUPPORTED, "adjoint output must be F32");
     const DevGeom& d = g->dev;
+    const float inv = 1.0f / vol.scale;
+    float* vt = nullptr;
+    // without the copy's memory, or in a stream capture, which is left free of
+    // allocations, the voxels scatter
+    const int steps = stream_captures(s) ? 0 : vi_t_steps(d);
+    if (steps > 0 &&
+        hipMallocAsync((void**)&vt, (size_t)d.nx * d.ny * vi_t_pitch(d.nz) * sizeof(float), s) != hipSuccess) {
+        (void)hipGetLastError();
+        vt = nullptr;
+    }
+    if (vt) {
+        const unsigned tiles = ceil_div(d.nx, 64) * (unsigned)d.ny * ceil_div(vi_t_pitch(d.nz), 64);
+        TOMO_DISPATCH_STORAGE(vol.dtype, TV, {
+            hipLaunchKernelGGL((vi_t_prepare_kernel<TV>), dim3(tiles), dim3(256), 0, s, d, (const TV*)vol.p, inv, vt);
+        });
+        switch (steps) {
+            case 1: launch_vi_t<1>(d, vt, (float*)sino.p, s); break;
+            case 2: launch_vi_t<2>(d, vt, (float*)sino.p, s); break;
+            case 3: launch_vi_t<3>(d, vt, (float*)sino.p, s); break;
+            default: launch_vi_t<4>(d, vt, (float*)sino.p, s); break;
+        }
+        const hipError_t e = hipGetLastError();
+        const hipError_t f = hipFreeAsync(vt, s);
+        TOMO_HIP(e);
+        TOMO_HIP(f);
+        return TOMO_OK;
+    }
     int rc = launch_fill((float*)sino.p, 0.0f, g->nsino(), s);
     if (rc) return rc;
     dim3 grid(ceil_div(d.nx, TX), ceil_div(d.ny, TY), ceil_div(d.nz, ZB));
-    const float inv = 1.0f / vol.scale;
     TOMO_DISPATCH_STORAGE(vol.dtype, TV, {
         hipLaunchKernelGGL((vi_adjoint_kernel<TV>), grid, dim3(TX * TY), 0, s, d, (const TV*)vol.p, inv,
                            (float*)sino.p);
