@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "device_common.hpp"
+#include "fdk_weight.hpp"
 #include "batch.hpp"
 
 namespace tomo {
@@ -33,6 +34,16 @@ struct ColumnView {
     float num, base;  // FDK weight terms (FDK only)
 };
 
+// 1 / w: the hardware's reciprocal (2^-24) and two Newton steps, correctly
+// rounded but for a few mantissas next to 2, which come out an ulp off (of
+// 1.1e10 values none other); half the instructions of the division.  w = 0 gives
+// NaN where the division gives an infinity: a column-view that is dropped either way.
+__device__ __forceinline__ double recip64(double w) {
+    double r = __builtin_amdgcn_rcp(w);
+    r = fma(fma(-w, r, 1.0), r, r);
+    return fma(fma(-w, r, 1.0), r, r);
+}
+
 // Per (column, view) terms in FP64.  FDK (back_fdk,
 // K/BackProjector/FDK3D_kernel_16reg.cuh:71-88; constants C/BackProjector.cu:
 // 34-35) adds num = alphaC (FDD/du) / w^2 and base = betaC + u'^2, u' = u - cu
@@ -42,7 +53,7 @@ struct ColumnView {
 template <bool FDK>
 __device__ __forceinline__ ColumnView column_view(const DevGeom& g, const double* c, double xp, double yp) {
     const double w = fma(c[2], xp, fma(c[3], yp, g.fod));
-    const double inv = 1.0 / w;
+    const double inv = recip64(w);
     const double un = fma(c[4], xp, c[5] * yp);
     ColumnView r;
     r.u = (float)fma(un, inv, (double)g.cu);
@@ -54,7 +65,13 @@ __device__ __forceinline__ ColumnView column_view(const DevGeom& g, const double
         const double ku = g.fdd / (double)g.du;
         const double alpha_c = (double)(float)(M_PI * g.fod * g.fdd / (double)g.nphi);
         const double up = un * inv;
-        r.num = (float)(alpha_c * ku / (w * w));
+        // alphaC ku / w^2: a Newton step on 1 / w^2 and a residual step, correctly
+        // rounded for each of 1.1e10 random pairs
+        const double w2 = w * w, a = alpha_c * ku;
+        double i2 = inv * inv;
+        i2 = fma(fma(-w2, i2, 1.0), i2, i2);
+        const double n = a * i2;
+        r.num = (float)fma(fma(-w2, n, a), i2, n);
         r.base = (float)(ku * ku + up * up);
     }
     if (!fin) {
@@ -70,38 +87,50 @@ __device__ __forceinline__ ColumnView column_view(const DevGeom& g, const double
 // A workgroup owns SX x SY voxel columns of ZS voxels.  For each view it
 // copies the detector taps its voxels read into LDS with coalesced loads
 // (taps off the detector as 0), and each voxel-view update reads its four
-// taps from there with two ds_read2_b32 instead of one 16-byte gather from
-// the tap-quad copy; the arithmetic is vi_tile's.  The taps are the box of
+// taps from there with two ds_read2_b32.  The taps are the box of
 // rows [v0, v1 + 1] and columns [u0, u1 + 1] with (u0, u1) the extreme
 // clamped cell corners floor(u) of the tile's columns and (v0, v1) the
 // extreme floor(v) of its voxels.  A table holds, per (column tile, view),
 // u0, u1 and the extreme A of the tile's columns (vi_box_kernel, the same
 // FP64 column terms); since v = fmaf(z', A, cv) is monotone in z' and in A,
 // the row extremes are the floors at the four (z', A) corners, so the box is
-// exact.  The rows are not clamped as in vi_tile: a row off the detector
-// holds zeros in the box, as the clamped cell it stands for.  View p is
-// staged in buffer p & 1, so one barrier per view separates the copy from
-// the reads.  A view whose box exceeds the buffer reads the taps directly.
+// exact.  A row off the detector holds zeros in the box.  Groups of 1, 2 or 4
+// views (ZS 16, 8, 4) alternate between two buffers, so one barrier per group
+// separates the copies from the reads.  A group with a box that exceeds its
+// buffer reads the taps directly.
+//
+// Per wave and view, 16 voxels are about 500 VALU cycles of a SIMD, the FP64
+// column terms 120 and the copies and plans 40; the LDS reads are 128 cycles of
+// the CU, 85% of the time at 512^3 and 512 views, where that binds (and the
+// clock falls to 2.05 GHz): 22.3 -> 19.7 ms with the plans made by lane, the
+// direct views in a loop of their own, 16-byte copies and the short reciprocal.
+// FDK (256^3, 360 views) is bound by VALU: 5.93 -> 3.96 ms, most of it from
+// fdk_weight.
 constexpr int SX = kViStageX, SY = kViStageY;  // voxel columns per workgroup; a wave is 8 x 8 columns
 // Floats per staged row.  A wave's 64 lanes read taps (u, r) at word
 // r * pitch + u; lanes spread over about 20 columns and a few rows, so two
 // lanes share a bank when their row and column offsets satisfy
-// dr * pitch + du = 0 mod 32.  With 8 x 8 waves a pitch of 75 (11 mod 32)
-// keeps such pairs rare at 512^3 / 512 views; with 32 x 2 waves (40 columns,
-// past the 32 banks) and a pitch of 65 (1 mod 32) a ds_read2_b32 took 2.6
-// extra cycles on bank conflicts.
-constexpr int kStagePitch = 75;
+// dr * pitch + du = 0 mod 32.  With 8 x 8 waves a pitch of 76 (12 mod 32, and
+// whole 16-byte pieces) keeps such pairs rare at 512^3 / 512 views, 2% of the
+// LDS cycles; with 32 x 2 waves (40 columns, past the 32 banks) and a pitch of
+// 65 (1 mod 32) a ds_read2_b32 took 2.6 extra cycles on bank conflicts.
+constexpr int kStagePitch = 76;
 
-// Staging buffer of a workgroup of 16-voxel columns: up to 38 rows of 64
-// taps (at 512^3 / 512 views about 0.1% of the boxes need 39 or 40 and read
-// their taps directly); two of them are 22.8 KB of LDS, 7 workgroups per CU
-// (FDK: 6, its VGPRs).
+// Staging buffers of a workgroup of ZS-voxel columns: `rows` rows of 64 taps for
+// each of `views` views, twice, in whole pieces of 256 words (one 16-byte load
+// per lane).  16: up to 37 rows (at 512^3 / 512 views about 0.1% of the boxes
+// need more and read their taps directly), 22.5 KB of LDS, 7 workgroups per CU.
+// Shorter columns stage several views between two barriers: there are few waves
+// then to wait for the taps, and the boxes are small.
 template <int ZS>
 struct StageShape {
-    static_assert(ZS == 16, "staging buffer sized for 16-voxel columns");
+    static_assert(ZS == 16 || ZS == 8 || ZS == 4, "staging buffers sized for 16, 8 and 4 voxels");
     static_assert(SX == 32 && SY == 8, "four 8 x 8 waves per workgroup");
-    static constexpr int rows = 38;                  // staged rows per view
-    static constexpr int taps = rows * kStagePitch;  // floats per buffer
+    static constexpr int rows = ZS == 16 ? 37 : ZS == 8 ? 26 : 16;      // staged rows per view
+    static constexpr int views = ZS == 16 ? 1 : ZS == 8 ? 2 : 4;        // views between two barriers
+    static constexpr int pieces = (rows * kStagePitch + 255) / 256;     // of a view
+    static constexpr int taps = pieces * 256;                           // floats per view
+    static constexpr int words = 2 * views * taps;
 };
 
 __device__ __forceinline__ int wave_min(int v) { return __reduce_min_sync(~0ull, v); }
@@ -164,42 +193,31 @@ __global__ __launch_bounds__(SX* SY) void vi_box_kernel(DevGeom g, ViBox* __rest
 }
 
 // Per-view staging plan of a workgroup: the box of taps (rows from v0,
-// columns from u0) and whether it fits the buffer.  Wave w copies box rows
-// w, w + 4, ..., one column per lane, so a box is at most 64 columns wide.
+// columns from u0), no rows where it does not fit the buffer.  Wave w copies box
+// rows w, w + 4, ..., one column per lane, so a box is at most 64 columns wide.
+// Each lane makes the plan of one of 64 views, which the wave then reads lane by
+// lane: made by every lane for every view it was an eighth of the instructions.
 struct StagePlan {
-    int u0, v0, cols, rows;
-    bool fits;
+    int u0, v0, rows;
+    bool quads;  // 16-byte loads: no tap of the box is off the detector's left or right end
 };
 
-// The box rows from the four (z', A) corners; with A >= 0 (a wave-uniform
-// sign test on the table's bits) the lowest row is at z' = zp0 with the
-// largest A when zp0 < 0 (the smallest otherwise) and the highest at z' = zp1
-// with the largest A when zp1 > 0, the same values with two fmas.
+// The box rows from the four (z', A) corners; v0 and the number of rows as v0 * 256
+// + rows, 0 where the box does not fit.
 template <int ZS>
-__device__ __forceinline__ StagePlan stage_plan(const ViBox& bb, float zp0, float cv, bool lo_amax, bool hi_amax) {
+__device__ __forceinline__ int stage_rows(const ViBox& bb, float zp0, float cv, int rl, int nv) {
     const float zp1 = zp0 + (float)(ZS - 1);
-    float vlo, vhi;
-    if (__float_as_int(bb.amin) >= 0) {
-        vlo = fmaf(zp0, lo_amax ? bb.amax : bb.amin, cv);
-        vhi = fmaf(zp1, hi_amax ? bb.amax : bb.amin, cv);
-    } else {
-        const float va = fmaf(zp0, bb.amin, cv), vb = fmaf(zp0, bb.amax, cv);
-        const float vc = fmaf(zp1, bb.amin, cv), vd = fmaf(zp1, bb.amax, cv);
-        vlo = fminf(fminf(va, vb), fminf(vc, vd));
-        vhi = fmaxf(fmaxf(va, vb), fmaxf(vc, vd));
-    }
-    vlo = floorf(vlo);
-    vhi = floorf(vhi);
-    StagePlan s;
-    s.u0 = bb.u0;
-    s.cols = bb.u1 - bb.u0 + 2;
+    const float va = fmaf(zp0, bb.amin, cv), vb = fmaf(zp0, bb.amax, cv);
+    const float vc = fmaf(zp1, bb.amin, cv), vd = fmaf(zp1, bb.amax, cv);
+    const float vlo = floorf(fminf(fminf(va, vb), fminf(vc, vd)));
+    const float vhi = floorf(fmaxf(fmaxf(va, vb), fmaxf(vc, vd)));
     const bool fits = vlo >= -32768.0f && vhi <= 32768.0f && vhi - vlo + 2.0f <= (float)StageShape<ZS>::rows &&
-                      s.cols <= 64;
-    // wave-uniform: keep the plan in scalar registers
-    s.fits = __builtin_amdgcn_readfirstlane((int)fits) != 0;
-    s.v0 = __builtin_amdgcn_readfirstlane(s.fits ? (int)vlo : 0);
-    s.rows = __builtin_amdgcn_readfirstlane(s.fits ? (int)(vhi - vlo) + 2 : 0);
-    return s;
+                      bb.u1 - bb.u0 + 2 <= 64;
+    // a lane's four taps start at a tap of the box and end on its row; the 32-bit
+    // offsets of rows off the detector do not come round to it
+    const bool quads = bb.u0 >= 0 && bb.u1 + 1 + 3 < rl && (int)vlo >= -64 && (int)vlo <= nv &&
+                       (uint64_t)(nv + 128) * (uint32_t)rl < (1u << 29);
+    return fits ? (int)vlo * 256 + (quads ? 128 : 0) + (int)(vhi - vlo) + 2 : 0;
 }
 
 // FP16 u-weights (1 - w, w) of a column-view, w = fu rounded to a multiple of
@@ -246,7 +264,8 @@ __device__ __forceinline__ void pair_sample4(const uint32_t (&p0)[4], const uint
 
 // PAIR: `sino` holds u-pair words (vi_pair_kernel; nu + 1 per row) instead of
 // FP32 taps; the box copy and the tap offsets are the same, one word per row.
-template <typename TV, bool FDK, int ZS, bool PAIR = false>
+// FDK: 0 VI, 1 FDK, 2 FDK whose weights are within fdk_weight's bounds.
+template <typename TV, int FDK, int ZS, bool PAIR = false>
 __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __restrict__ sino,
                                                const ViBox* __restrict__ boxes, TV* __restrict__ vol,
                                                float vol_scale, float post, int bx, int by, int bz,
@@ -261,27 +280,25 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     const int i = bx * SX + wv * 8 + (lane & 7);
     const int j = by * SY + (lane >> 3);
     const int k0 = bz * ZS;
-    const bool active = i < g.nx && j < g.ny;
-    const double xp = (double)i - (double)g.cx, yp = (double)j - (double)g.cy;
+    // a lane past the volume's edge works on the edge column, and stores nothing
+    const double xp = (double)min(i, g.nx - 1) - (double)g.cx, yp = (double)min(j, g.ny - 1) - (double)g.cy;
     const float zp0 = (float)((double)k0 - (double)g.cz);
     const float cv = g.cv;
     const float fnu = (float)g.nu;
     const int nu = g.nu, nv = g.nv;
     const int rl = PAIR ? nu + 1 : nu;  // words per detector row
     const size_t plane = (size_t)rl * nv;
-    // The box and view tables are read-only here and indexed by wave-uniform
-    // values: read through the constant address space they come in with scalar
-    // loads, and the staging plan's branches are uniform.
-    typedef const __attribute__((address_space(4))) ViBox* ConstBox;
+    // The view table is read-only here and indexed by wave-uniform values: read
+    // through the constant address space it comes in with scalar loads.
     typedef const __attribute__((address_space(4))) double* ConstView;
-    const ConstBox bt = (ConstBox)(boxes + (size_t)(by * ((g.nx + SX - 1) / SX) + bx) * g.nphi);
+    const ViBox* const bt = boxes + (size_t)(by * ((g.nx + SX - 1) / SX) + bx) * g.nphi;
     float acc[ZS];
 #pragma unroll
     for (int k = 0; k < ZS; ++k) acc[k] = 0.0f;
     auto add = [&](const ColumnView& cvw, int k, float r) {
         if (FDK) {
-            const float vp = (zp0 + (float)k) * cvw.A;
-            const float wt = cvw.num / sqrtf(fmaf(vp, vp, cvw.base));
+            const float vp = (zp0 + (float)k) * cvw.A, q = fmaf(vp, vp, cvw.base);
+            const float wt = FDK == 2 ? fdk_weight(cvw.num, q) : cvw.num / sqrtf(q);
             acc[k] += wt * r;
         } else {
             acc[k] += r;
@@ -295,18 +312,43 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
         const float b = fmaf(fu, t11 - t01, t01);
         add(cvw, k, fmaf(fv, b - a, a));
     };
-    // Copy of view p's box into buffer b: wave wv copies box rows wv + q NW,
-    // lane l column l, straight from memory into LDS (buffer_load ... lds).
-    // Each row is read through a buffer resource of that detector row (of no
-    // bytes for a row off the detector), so a tap off the detector reads past
-    // the resource's end, which writes 0; the lane offsets are the same for
-    // every row.
+    const uint32_t view_bytes = (uint32_t)(plane * sizeof(float));
+    // Byte offset in the view of a lane's four taps of the wave's q-th piece, from
+    // the box's first: word w of the buffer is tap (w / pitch, w mod pitch).
+    constexpr int kPieces = (SS::pieces + NW - 1) / NW;
+    uint32_t piece[kPieces];
+#pragma unroll
+    for (int q = 0; q < kPieces; ++q) {
+        const int w = 256 * (wv + q * NW) + 4 * lane, row = w / kStagePitch;
+        piece[q] = (uint32_t)(row * rl + (w - row * kStagePitch)) * 4u;
+    }
+    // Copy of view p's box into view buffer b, straight from memory into LDS
+    // (buffer_load ... lds); a tap off the detector's upper or lower edge is
+    // outside the view's bytes, which writes 0.  Words past the box hold taps
+    // that nothing reads.  One 16-byte load per lane brings 3.4 rows; by rows, a
+    // 4-byte load each, the copies kept the data return 80% busy at 512^3.
+    //
+    // Boxes at the detector's left and right ends go by rows: wave wv copies box
+    // rows wv + q NW, lane l column l, each row read through a buffer resource of
+    // that detector row (of no bytes for a row off the detector), so that a tap
+    // off the row reads past the resource's end.
     auto copy_box = [&](const StagePlan& s, int p, int b) {
-        if (!s.fits) return;
         const float* view = sino + (size_t)p * plane;
+        float* dst = stage + b * SS::taps;
+        if (s.quads) {
+            const __amdgpu_buffer_rsrc_t rr = buffer_rsrc(view, view_bytes);
+            const uint32_t at = (uint32_t)(s.v0 * rl + s.u0) * 4u;
+            const int words = s.rows * kStagePitch;
+#pragma unroll
+            for (int q = 0; q < kPieces; ++q)
+                if (256 * (wv + q * NW) < words)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                        rr, (__attribute__((address_space(3))) void*)(dst + 256 * (wv + q * NW)), 16,
+                        (int)(at + piece[q]), 0, 0, 0);
+            return;
+        }
         // past the row's end unless 0 <= u < nu (FP32) or the pair index u + 1 <= nu
-        const uint32_t loff = (uint32_t)(s.u0 + (PAIR ? 1 : 0) + lane) * 4u;
-        float* dst = stage + b * SS::taps + wv * kStagePitch;
+        const uint32_t loff = (uint32_t)(s.u0 + lane) * 4u;
 #pragma unroll
         for (int q = 0; q < kSlots; ++q) {
             if (wv + q * NW < s.rows) {
@@ -315,101 +357,150 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
                 const __amdgpu_buffer_rsrc_t rr =
                     buffer_rsrc(view + (size_t)(vin ? v : 0) * rl, vin ? (uint32_t)rl * 4u : 0u);
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    rr, (__attribute__((address_space(3))) void*)(dst + q * NW * kStagePitch), 4, loff, 0, 0, 0);
+                    rr, (__attribute__((address_space(3))) void*)(dst + (wv + q * NW) * kStagePitch), 4, loff, 0, 0, 0);
             }
         }
     };
-    const bool lo_amax = zp0 < 0.0f, hi_amax = zp0 + (float)(ZS - 1) > 0.0f;
-    const uint32_t view_bytes = (uint32_t)(plane * sizeof(float));
-    auto box_of = [&](int p) { return ViBox{bt[p].u0, bt[p].u1, bt[p].amin, bt[p].amax}; };
-    StagePlan nxt = stage_plan<ZS>(box_of(0), zp0, cv, lo_amax, hi_amax);
-    copy_box(nxt, 0, 0);
-    for (int p = 0; p < g.nphi; ++p) {
-        // this wave's copies of view p have landed; every wave is done with view p - 1
+    int plan_u0 = 0, plan_v = 0;  // of view (p & ~63) + lane
+    auto plan_of = [&](int p) {
+        const int v = __builtin_amdgcn_readlane(plan_v, p & 63);
+        return StagePlan{__builtin_amdgcn_readlane(plan_u0, p & 63), v >> 8, v & 127, (v & 128) != 0};
+    };
+    // Plans and copies of the group of G views from p on; rows is 0 if one of its
+    // boxes does not fit, and all of the group's taps are then read directly.
+    constexpr int G = SS::views;
+    struct Group {
+        int u0[G], v0[G], rows;
+    };
+    auto stage_group = [&](int p, int half) {
+        Group r;
+        r.rows = 1;
+        if ((p & 63) == 0 && p + lane < g.nphi) {  // G divides 64
+            ViBox bb = bt[p + lane];
+            bb.u0 += PAIR;  // word index of tap pair (u, u + 1)
+            bb.u1 += PAIR;
+            plan_v = stage_rows<ZS>(bb, zp0, cv, rl, nv);
+            plan_u0 = (plan_v & 128) ? bb.u0 & ~3 : bb.u0;  // rows of a multiple of 4 taps: aligned loads
+        }
+#pragma unroll
+        for (int t = 0; t < G; ++t) {
+            const StagePlan s = p + t < g.nphi ? plan_of(p + t) : StagePlan{0, 0, 0, false};
+            r.u0[t] = s.u0;
+            r.v0[t] = s.v0;
+            if (p + t < g.nphi) {
+                if (s.rows == 0) r.rows = 0;
+                copy_box(s, p + t, half * G + t);
+            }
+        }
+        return r;
+    };
+    auto view_terms = [&](int p) {
+        const ConstView vt = (ConstView)(g.view + (size_t)p * kViewStride);
+        double c[kViewStride];
+#pragma unroll
+        for (int e = 0; e < kViewStride; ++e) c[e] = vt[e];
+        return column_view<FDK != 0>(g, c, xp, yp);
+    };
+    Group now, nxt = stage_group(0, 0);
+    int p = 0, half = 0;
+    // the copies of the group at p have landed (this wave's, then all); every wave is done with the group before
+    auto next_group = [&]() {
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        const StagePlan now = nxt;
-        if (p + 1 < g.nphi) {
-            nxt = stage_plan<ZS>(box_of(p + 1), zp0, cv, lo_amax, hi_amax);
-            copy_box(nxt, p + 1, (p + 1) & 1);
-        }
-        if (active) {
-            const ConstView vt = (ConstView)(g.view + (size_t)p * kViewStride);
-            double c[kViewStride];
+        now = nxt;
+        if (p + G < g.nphi) nxt = stage_group(p + G, half ^ 1);
+    };
+    do {
+        // The staged views in a loop of their own: as one branch of two in it, the
+        // sums changed registers for every view (16 moves, 6% of the instructions).
+        while (p < g.nphi && nxt.rows > 0) {
+            next_group();
 #pragma unroll
-            for (int e = 0; e < kViewStride; ++e) c[e] = vt[e];
-            const ColumnView cvw = column_view<FDK>(g, c, xp, yp);
-            const float uf = floorf(cvw.u);
-            const float fu = cvw.u - uf;
-            const float uc = __builtin_amdgcn_fmed3f(uf, -2.0f, fnu);
-            const uint32_t pw = PAIR ? pair_weights(fu) : 0u;
-            if (now.fits) {
+            for (int t = 0; t < G; ++t) {
+                if (t > 0 && p + t >= g.nphi) break;
+                const ColumnView cvw = view_terms(p + t);
+                const float uf = floorf(cvw.u);
+                const float fu = cvw.u - uf;
+                const float uc = __builtin_amdgcn_fmed3f(uf, -2.0f, fnu);
                 // byte offset in the buffer of tap (uc, vf): ((vf - v0) pitch + uc - u0) 4,
-                // one exact fma of small integers
-                const float colb =
-                    (float)(((int)uc - now.u0 - now.v0 * kStagePitch + (p & 1) * SS::taps) * 4);
+                // one exact fma of small integers on top of 2^23, whose low bits are then the
+                // offset: an and (0.6 cycles per wave and CU) for a conversion (1.1)
+                const float colb = (float)(((int)uc + PAIR - now.u0[t] - now.v0[t] * kStagePitch + (half * G + t) * SS::taps) * 4) +
+                                   0x1p23f;
                 if constexpr (PAIR) {
                     static_assert(ZS % 4 == 0, "u-pair samples go four voxels at a time");
+                    const uint32_t pw = pair_weights(fu);
 #pragma unroll
                     for (int k4 = 0; k4 < ZS; k4 += 4) {
                         uint32_t p0[4], p1[4];
                         float fv[4], r0[4], dr[4];
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) {
-                            const float v = fmaf(zp0 + (float)(k4 + t), cvw.A, cv);
+                        for (int e = 0; e < 4; ++e) {
+                            const float v = fmaf(zp0 + (float)(k4 + e), cvw.A, cv);
                             const float vf = floorf(v);
-                            const uint32_t off = (uint32_t)fmaf(vf, (float)(kStagePitch * 4), colb);
+                            const uint32_t off = __float_as_uint(fmaf(vf, (float)(kStagePitch * 4), colb)) & 0x7fffffu;
                             const uint32_t* qw = (const uint32_t*)((const char*)stage + off);
-                            p0[t] = qw[0];
-                            p1[t] = qw[kStagePitch];
-                            fv[t] = v - vf;
+                            p0[e] = qw[0];
+                            p1[e] = qw[kStagePitch];
+                            fv[e] = v - vf;
                         }
                         pair_sample4(p0, p1, pw, r0, dr);
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) add(cvw, k4 + t, fmaf(fv[t], dr[t], r0[t]));
+                        for (int e = 0; e < 4; ++e) add(cvw, k4 + e, fmaf(fv[e], dr[e], r0[e]));
                     }
                 } else {
 #pragma unroll
                     for (int k = 0; k < ZS; ++k) {
                         const float v = fmaf(zp0 + (float)k, cvw.A, cv);
                         const float vf = floorf(v);
-                        const uint32_t off = (uint32_t)fmaf(vf, (float)(kStagePitch * 4), colb);
+                        const uint32_t off = __float_as_uint(fmaf(vf, (float)(kStagePitch * 4), colb)) & 0x7fffffu;
                         const float* q = (const float*)((const char*)stage + off);
                         term(cvw, fu, k, v, vf, q[0], q[kStagePitch], q[1], q[kStagePitch + 1]);
                     }
                 }
-            } else {
-                // box larger than the buffer: the four taps straight from the view, one voxel at a time
-                const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(sino + (size_t)p * plane, view_bytes);
-                const int iu = (int)uc;
-                const bool u0ok = (unsigned)iu < (unsigned)nu, u1ok = (unsigned)(iu + 1) < (unsigned)nu;
-                const bool pok = (unsigned)(iu + 1) <= (unsigned)nu;  // pair word iu + 1 exists
-                ColumnView cw = cvw;
-                asm volatile("" : "+v"(cw.A));  // this path's rows are its own, not hoisted above the branch
-                auto rd = [&](bool ok, int v, int u) {
-                    const uint32_t off = ok ? (uint32_t)(v * rl + u) * 4u : 0xfffffff0u;
-                    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)off, 0, 0));
-                };
+            }
+            p += G;
+            half ^= 1;
+        }
+        if (p >= g.nphi) break;
+        // a box larger than the buffer: the four taps straight from the views, one voxel at a time
+        next_group();
+#pragma clang loop unroll(disable)
+        for (int pd = p; pd < min(p + G, g.nphi); ++pd) {
+            const ColumnView cvw = view_terms(pd);
+            const float uf = floorf(cvw.u);
+            const float fu = cvw.u - uf;
+            const float uc = __builtin_amdgcn_fmed3f(uf, -2.0f, fnu);
+            const uint32_t pw = PAIR ? pair_weights(fu) : 0u;
+            const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(sino + (size_t)pd * plane, view_bytes);
+            const int iu = (int)uc;
+            const bool u0ok = (unsigned)iu < (unsigned)nu, u1ok = (unsigned)(iu + 1) < (unsigned)nu;
+            const bool pok = (unsigned)(iu + 1) <= (unsigned)nu;  // pair word iu + 1 exists
+            auto rd = [&](bool ok, int v, int u) {
+                const uint32_t off = ok ? (uint32_t)(v * rl + u) * 4u : 0xfffffff0u;
+                return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)off, 0, 0));
+            };
 #pragma unroll
-                for (int k = 0; k < ZS; ++k) {
-                    const float v = fmaf(zp0 + (float)k, cw.A, cv);
-                    const float vf = floorf(v);
-                    const int iv = (int)__builtin_amdgcn_fmed3f(vf, -2.0f, (float)nv);
-                    const bool v0ok = (unsigned)iv < (unsigned)nv, v1ok = (unsigned)(iv + 1) < (unsigned)nv;
-                    if constexpr (PAIR) {
-                        const uint32_t p0 = __builtin_bit_cast(uint32_t, rd(pok && v0ok, iv, iu + 1));
-                        const uint32_t p1 = __builtin_bit_cast(uint32_t, rd(pok && v1ok, iv + 1, iu + 1));
-                        add(cw, k, pair_sample(p0, p1, pw, v - vf));
-                    } else {
-                        term(cw, fu, k, v, vf, rd(u0ok && v0ok, iv, iu), rd(u0ok && v1ok, iv + 1, iu),
-                             rd(u1ok && v0ok, iv, iu + 1), rd(u1ok && v1ok, iv + 1, iu + 1));
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+            for (int k = 0; k < ZS; ++k) {
+                const float v = fmaf(zp0 + (float)k, cvw.A, cv);
+                const float vf = floorf(v);
+                const int iv = (int)__builtin_amdgcn_fmed3f(vf, -2.0f, (float)nv);
+                const bool v0ok = (unsigned)iv < (unsigned)nv, v1ok = (unsigned)(iv + 1) < (unsigned)nv;
+                if constexpr (PAIR) {
+                    const uint32_t p0 = __builtin_bit_cast(uint32_t, rd(pok && v0ok, iv, iu + 1));
+                    const uint32_t p1 = __builtin_bit_cast(uint32_t, rd(pok && v1ok, iv + 1, iu + 1));
+                    add(cvw, k, pair_sample(p0, p1, pw, v - vf));
+                } else {
+                    term(cvw, fu, k, v, vf, rd(u0ok && v0ok, iv, iu), rd(u0ok && v1ok, iv + 1, iu),
+                         rd(u1ok && v0ok, iv, iu + 1), rd(u1ok && v1ok, iv + 1, iu + 1));
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-    }
-    if (!active) return;
+        p += G;
+        half ^= 1;
+    } while (p < g.nphi);
+    if (i >= g.nx || j >= g.ny) return;
     const size_t sxy = (size_t)g.nx * g.ny;
     const size_t base = (size_t)i + (size_t)g.nx * j;
 #pragma unroll
@@ -419,12 +510,15 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
                                vol_scale);
 }
 
+// Waves per SIMD that a kernel's registers are held to.
+constexpr int vi_waves(int fdk, int zs, bool pair) { return !pair ? 7 : fdk == 1 ? 5 : 6; }
+
 // post: 1 for FP32 taps, 1 / storage scale for FP16 u-pairs.
-template <typename TV, bool FDK, int ZS, bool PAIR>
-__global__ __launch_bounds__(SX* SY, FDK ? 6 : 7) void vi_staged_kernel(DevGeom g, const float* __restrict__ sino,
+template <typename TV, int FDK, int ZS, bool PAIR>
+__global__ __launch_bounds__(SX* SY, vi_waves(FDK, ZS, PAIR)) void vi_staged_kernel(DevGeom g, const float* __restrict__ sino,
                                                          const ViBox* __restrict__ boxes, TV* __restrict__ vol,
                                                          float vol_scale, float post) {
-    __shared__ float stage[2 * StageShape<ZS>::taps];
+    __shared__ __align__(16) float stage[StageShape<ZS>::words];
     vi_staged_tile<TV, FDK, ZS, PAIR>(g, sino, boxes, vol, vol_scale, post, blockIdx.x, blockIdx.y, blockIdx.z,
                                       stage);
 }
@@ -448,13 +542,13 @@ __global__ __launch_bounds__(256) void vi_pair_kernel(const uint16_t* __restrict
 // ceil(ny/SY), ceil(nz/16)) on the sinogram `in` with the problem's box table
 // `aux` (launch_vi_boxes); the stored value is (delta * sum) * a.
 __global__ __launch_bounds__(SX* SY, 7) void vi_batch_kernel(const BatchTable* __restrict__ t, uint32_t* __restrict__ next) {
-    __shared__ float stage[2 * StageShape<kViTileZ>::taps];
+    __shared__ __align__(16) float stage[StageShape<kViTileZ>::words];
     TOMO_BATCH_CLAIMED(t, next) {
         const BatchItem& it = t->item[batch_find(t, tile)];
         const uint32_t local = tile - it.begin;
         const uint32_t bx = local % it.gx, rest = local / it.gx;
         const int by = (int)(rest % it.gy), bz = (int)(rest / it.gy);
-        vi_staged_tile<float, false, kViTileZ>(it.g, (const float*)it.in, (const ViBox*)it.aux, (float*)it.out, 1.0f,
+        vi_staged_tile<float, 0, kViTileZ>(it.g, (const float*)it.in, (const ViBox*)it.aux, (float*)it.out, 1.0f,
                                                it.a, (int)bx, by, bz, stage);
     }
 }
@@ -734,8 +828,27 @@ __global__ __launch_bounds__(64, 5) void vi_t_kernel(DevGeom g, const float* __r
 
 }  // namespace
 
-// Voxels per thread column of the staged kernel.
-constexpr int kStagedZ = kViTileZ;
+// Whether every FDK weight of the geometry is within fdk_weight's bounds: the
+// source is outside the volume's square, so that w is within fod +- its half
+// diagonal, and the extreme terms of that range are.
+static bool fdk_in_bounds(const DevGeom& d) {
+    const double half = 0.5 * std::sqrt(2.0) * (double)d.delta * (double)std::max(d.nx, d.ny);
+    const double w0 = d.fod - half, w1 = d.fod + half;
+    if (!(w0 > 0.01 * d.fod)) return false;
+    const double ku = d.fdd / (double)d.du, alpha = M_PI * d.fod * d.fdd / (double)d.nphi;
+    const double up = half / w0 * ku, vp = 0.5 * (double)d.nz * (double)d.delta * d.fdd / ((double)d.dv * w0);
+    const double num0 = alpha * ku / (w1 * w1), num1 = alpha * ku / (w0 * w0);
+    return num0 >= 2.0 * kFdkLeast && num1 <= 0.5 * kFdkMost && ku * ku >= 2.0 * kFdkLeast &&
+           ku * ku + up * up + vp * vp <= 0.5 * kFdkMost;
+}
+
+template <typename TV, int FDK, int ZS, bool PAIR>
+static void launch_vi_tiles(const DevGeom& d, const float* sino, const ViBox* boxes, void* vol, float vol_scale,
+                            float post, hipStream_t s) {
+    const dim3 grid(ceil_div(d.nx, SX), ceil_div(d.ny, SY), ceil_div(d.nz, ZS));
+    hipLaunchKernelGGL((vi_staged_kernel<TV, FDK, ZS, PAIR>), grid, dim3(SX * SY), 0, s, d, sino, boxes, (TV*)vol,
+                       vol_scale, post);
+}
 
 // The staged kernel on an FP32 sinogram, with the geometry's box table
 // (`boxes`) or, when null, one made for this call from the stream-ordered
@@ -753,13 +866,26 @@ static hipError_t launch_vi_staged(const DevGeom& d, int fdk, const float* sino,
         boxes = own;
     }
     if (e == hipSuccess) {
-        const dim3 grid(ntx, nty, ceil_div(d.nz, kStagedZ));
-        if (fdk)
-            hipLaunchKernelGGL((vi_staged_kernel<TV, true, kStagedZ, PAIR>), grid, dim3(SX * SY), 0, s, d, sino,
-                               (const ViBox*)boxes, (TV*)vol, vol_scale, post);
+        // Columns of 16 voxels share a column-view's terms best; below two or three
+        // workgroups per CU the views' latency decides, and shorter columns are more
+        // workgroups that wait for several views at once.  VI, us at 4 / 8 / 16
+        // voxels by workgroups of 16: 64 (64^3, 64 views) 39 / 50 / 75; 150 (80^3)
+        // 58 / 62 / 93; 216 (96^3) 80 / 77 / 112; 512 (128^3, 180 views) 270 / 191 /
+        // 217; 765 (136^3) 272 / 220 / 203; 1000 (160^3, 180 views) 464 / 342 / 287.
+        const size_t tiles = (size_t)ntx * nty * ceil_div(d.nz, kViTileZ);
+        const int zs = tiles < 192 ? 4 : tiles < 640 ? 8 : 16;
+        const ViBox* bt = (const ViBox*)boxes;
+        if (fdk && !fdk_in_bounds(d))
+            launch_vi_tiles<TV, 1, kViTileZ, PAIR>(d, sino, bt, vol, vol_scale, post, s);
+        else if (zs == kViTileZ)
+            fdk ? launch_vi_tiles<TV, 2, kViTileZ, PAIR>(d, sino, bt, vol, vol_scale, post, s)
+                : launch_vi_tiles<TV, 0, kViTileZ, PAIR>(d, sino, bt, vol, vol_scale, post, s);
+        else if (zs == 8)
+            fdk ? launch_vi_tiles<TV, 2, 8, PAIR>(d, sino, bt, vol, vol_scale, post, s)
+                : launch_vi_tiles<TV, 0, 8, PAIR>(d, sino, bt, vol, vol_scale, post, s);
         else
-            hipLaunchKernelGGL((vi_staged_kernel<TV, false, kStagedZ, PAIR>), grid, dim3(SX * SY), 0, s, d, sino,
-                               (const ViBox*)boxes, (TV*)vol, vol_scale, post);
+            fdk ? launch_vi_tiles<TV, 2, 4, PAIR>(d, sino, bt, vol, vol_scale, post, s)
+                : launch_vi_tiles<TV, 0, 4, PAIR>(d, sino, bt, vol, vol_scale, post, s);
         e = hipGetLastError();
     }
     if (own) {
@@ -807,15 +933,15 @@ int launch_vi(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t s, int fdk) 
     }
     const float post = pair ? 1.0f / sino.scale : 1.0f;
     hipError_t e = hipSuccess;
-#define TOMO_VI_STAGED(TV)                                                                              \
+#define TOMO_VI_LAUNCH(TV)                                                                              \
     e = pair ? launch_vi_staged<TV, true>(d, fdk, taps, g->d_vi_boxes, vol.p, vol.scale, post, s)     \
              : launch_vi_staged<TV, false>(d, fdk, taps, g->d_vi_boxes, vol.p, vol.scale, post, s)
     switch (vol.dtype) {
-        case TOMO_F32: TOMO_VI_STAGED(float); break;
-        case TOMO_F16: TOMO_VI_STAGED(__half); break;
-        default: TOMO_VI_STAGED(__hip_bfloat16); break;
+        case TOMO_F32: TOMO_VI_LAUNCH(float); break;
+        case TOMO_F16: TOMO_VI_LAUNCH(__half); break;
+        default: TOMO_VI_LAUNCH(__hip_bfloat16); break;
     }
-#undef TOMO_VI_STAGED
+#undef TOMO_VI_LAUNCH
     if (wide) TOMO_HIP(hipFreeAsync(wide, s));
     TOMO_HIP(e);
     return TOMO_OK;
