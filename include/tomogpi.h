@@ -280,7 +280,8 @@ typedef struct tomo_gd_iter_stat {
 /* Runs the loop on device-resident data (or host data with TOMO_HOST_PTR in
  * params->flags).  `volume` holds the initial estimate on entry and the
  * result on exit.  stats (may be NULL) receives gradient_iteration_nb
- * records.  Synchronous (the step rule needs the norms on the host).        */
+ * records.  Synchronous (it returns when the volume and the records are
+ * there; the step rule runs on the device).                                  */
 int tomo_gd_run(tomo_ctx* ctx, const tomo_geom* geom, const tomo_gd_params* params,
                 const float* sinogram, float* volume, tomo_gd_iter_stat* stats,
                 void* stream);

@@ -17,7 +17,7 @@ namespace tomo {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kReduceBlocks = 2048;
+constexpr int kReduceBlocks = kLoopPartials;
 
 __global__ __launch_bounds__(kBlock) void fill_kernel(float* x, float v, size_t n) {
     for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) x[i] = v;
@@ -40,17 +40,12 @@ __global__ __launch_bounds__(kBlock) void axpy_kernel(float* y, const float* x, 
 
 // SIRT element-wise steps (FP32, no fused multiply-add):
 //   weights  w = s > 0 ? a / s : 0
-//   residual d = y - e; out = d * w
 //   update   x = x + c * b, clamped at 0 with positivity
 __global__ __launch_bounds__(kBlock) void recip_weight_kernel(const float* s_in, float a, float* w, size_t n) {
     for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
         const float v = s_in[i];
         w[i] = v > 0.0f ? a / v : 0.0f;
     }
-}
-__global__ __launch_bounds__(kBlock) void mul_kernel(float* x, const float* w, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock)
-        x[i] = x[i] * w[i];
 }
 __global__ __launch_bounds__(kBlock) void waxpy_kernel(float* x, const float* c, const float* b, int positive,
                                                      size_t n) {
@@ -157,6 +152,155 @@ __device__ __forceinline__ float laplacian_tile(const float* __restrict__ x, flo
 __global__ __launch_bounds__(kBlock) void laplacian_kernel(const float* __restrict__ x, float* __restrict__ y, int nx,
                                                          int ny, int nz) {
     (void)laplacian_tile(x, y, nx, ny, nz, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// ---- the loops' steps.  What a loop's iteration does besides its operators is a
+// dozen passes of a few microseconds at 128^3, where a launch costs as much as
+// the pass: neighbouring passes are one kernel, with the operations and the order
+// of every sum as in the kernels above, and the scalars stay in device memory.
+
+// o = d (or d w with w set), d = a - b; partial sums of d^2 when partial is set.
+__global__ __launch_bounds__(kBlock) void diff_sq_kernel(const float* a, const float* b, const float* w, float* o,
+                                                         size_t n, double* partial) {
+    double s = 0.0;
+    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
+        const float d = a[i] - b[i];
+        o[i] = w ? d * w[i] : d;
+        s += (double)d * (double)d;
+    }
+    if (!partial) return;
+    const double r = block_sum(s);
+    if (threadIdx.x == 0) partial[blockIdx.x] = r;
+}
+
+__device__ __forceinline__ float laplacian_at(const float* __restrict__ x, int nx, int ny, int nz, uint32_t o) {
+    const uint32_t row = o / (uint32_t)nx, k = row / (uint32_t)ny;
+    const int i = (int)(o - row * (uint32_t)nx), j = (int)(row - k * (uint32_t)ny);
+    const size_t sy = (size_t)nx, sz = (size_t)nx * ny;
+    const float c = x[o], c2 = c + c;
+    const float xm = i > 0 ? x[o - 1] : 0.0f, xp = i < nx - 1 ? x[(size_t)o + 1] : 0.0f;
+    const float ym = j > 0 ? x[o - sy] : 0.0f, yp = j < ny - 1 ? x[o + sy] : 0.0f;
+    const float zm = k > 0 ? x[o - sz] : 0.0f, zp = (int)k < nz - 1 ? x[o + sz] : 0.0f;
+    const float h = (c2 - xm) - xp, v = (c2 - ym) - yp, p = (c2 - zm) - zp;
+    return (h + v) + p;
+}
+
+// Partial sums of (L x)^2, with y = L x when y is set and partial sums of x^2
+// when partial_x is set.  Threads take the elements that sq_partial_kernel's do.
+__global__ __launch_bounds__(kBlock) void laplacian_sq_kernel(const float* __restrict__ x, float* __restrict__ y, int nx,
+                                                              int ny, int nz, double* partial, double* partial_x) {
+    const size_t n = (size_t)nx * ny * nz;
+    double s = 0.0, t = 0.0;
+    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
+        const float v = laplacian_at(x, nx, ny, nz, (uint32_t)i);
+        if (y) y[i] = v;
+        s += (double)v * (double)v;
+        const double c = (double)x[i];
+        t += c * c;
+    }
+    const double r = block_sum(s);
+    if (threadIdx.x == 0) partial[blockIdx.x] = r;
+    if (!partial_x) return;
+    __syncthreads();
+    const double q = block_sum(t);
+    if (threadIdx.x == 0) partial_x[blockIdx.x] = q;
+}
+
+// d = d scale + a (L x)
+__global__ __launch_bounds__(kBlock) void scale_laplacian_kernel(const float* __restrict__ x, float* __restrict__ d,
+                                                                 float scale, float a, int nx, int ny, int nz) {
+    const int i = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6), k = blockIdx.z;
+    if (i >= nx || j >= ny) return;
+    const size_t sy = (size_t)nx, sz = (size_t)nx * ny;
+    const size_t o = (size_t)i + sy * j + sz * k;
+    const float c = x[o], c2 = c + c;
+    const float xm = i > 0 ? x[o - 1] : 0.0f, xp = i < nx - 1 ? x[o + 1] : 0.0f;
+    const float ym = j > 0 ? x[o - sy] : 0.0f, yp = j < ny - 1 ? x[o + sy] : 0.0f;
+    const float zm = k > 0 ? x[o - sz] : 0.0f, zp = k < nz - 1 ? x[o + sz] : 0.0f;
+    const float h = (c2 - xm) - xp, v = (c2 - ym) - yp, p = (c2 - zm) - zp;
+    d[o] = d[o] * scale + a * ((h + v) + p);
+}
+
+// y = y + (float)*a x, clamped at 0 with positivity
+__global__ __launch_bounds__(kBlock) void axpy_scalar_kernel(float* y, const float* x, const double* a, int positive,
+                                                             size_t n) {
+    const float f = (float)*a;
+    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
+        float v = y[i] + f * x[i];
+        if (positive && v < 0.0f) v = 0.0f;
+        y[i] = v;
+    }
+}
+
+// d = g (beta null) or d (float)*beta + g; partial sums of g d.
+__global__ __launch_bounds__(kBlock) void direction_kernel(const float* g, float* d, const double* beta, size_t n,
+                                                           double* partial) {
+    const float f = beta ? (float)*beta : 0.0f;
+    double s = 0.0;
+    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
+        const float gi = g[i];
+        const float v = beta ? d[i] * f + gi : gi;
+        d[i] = v;
+        s += (double)gi * (double)v;
+    }
+    const double r = block_sum(s);
+    if (threadIdx.x == 0) partial[blockIdx.x] = r;
+}
+
+// Ends the iteration's sums (one block, each as final_sum_kernel) and applies
+// the step rule to the iteration's statistics.
+__global__ __launch_bounds__(kBlock) void loop_step_kernel(LoopStep a) {
+    // all loads first: one after the other they took 13 us
+    double s[kLoopSums], v[kLoopSums][kReduceBlocks / kBlock];
+#pragma unroll
+    for (int q = 0; q < kLoopSums; ++q)
+#pragma unroll
+        for (int t = 0; t < kReduceBlocks / kBlock; ++t) {
+            const int i = threadIdx.x + t * kBlock;
+            v[q][t] = i < a.blocks[q] ? a.partial[q * kReduceBlocks + i] : 0.0;
+        }
+#pragma unroll
+    for (int q = 0; q < kLoopSums; ++q) {
+        s[q] = 0.0;
+#pragma unroll
+        for (int t = 0; t < kReduceBlocks / kBlock; ++t) s[q] += v[q][t];
+    }
+#pragma unroll
+    for (int q = 0; q < kLoopSums; ++q) {
+        if (a.blocks[q] == 0) continue;
+        s[q] = block_sum(s[q]);
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    if (a.rule == kRuleResidual) {
+        a.stat->residual_sq = s[kLoopResidual];
+        return;
+    }
+    tomo_gd_iter_stat st = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (!a.begins) st = *a.stat;
+    if (a.blocks[kLoopResidual]) st.residual_sq = s[kLoopResidual];
+    if (a.blocks[kLoopReg]) st.j_reg = s[kLoopReg];
+    const double norm_reg = a.blocks[kLoopDirReg] ? 2.0 * s[kLoopDirReg] : 0.0;
+    const double proj = 2.0 * s[kLoopProj] + a.lambda * norm_reg;
+    double state = a.first ? a.init : *a.state;
+    if (a.rule == kRuleOptimal) {
+        st.norm_dj = s[kLoopDir];
+        st.norm_dj_proj = proj;
+        st.alpha = -s[kLoopDir] / proj;
+        state = fmax(st.alpha, state);
+    } else if (a.rule == kRuleFixed) {
+        st.alpha = state;
+    } else if (a.rule == kRuleBeta) {
+        st.norm_dj = s[kLoopDir];
+        if (!a.first) st.beta = s[kLoopDir] / state;
+        state = s[kLoopDir];
+    } else {  // kRuleConjugate; its kLoopDir is g . d, and the state stays |g|^2
+        st.norm_dj_proj = proj;
+        st.alpha = -s[kLoopDir] / proj;
+        state = *a.state;
+    }
+    *a.stat = st;
+    *a.state = state;
 }
 
 // Ellipsoid phantoms; 16 doubles per ellipsoid: rotation (9, row-major),
@@ -635,11 +779,6 @@ int launch_recip_weight(const float* s_in, float a, float* w, size_t n, hipStrea
     TOMO_HIP(hipGetLastError());
     return TOMO_OK;
 }
-int launch_mul(float* x, const float* w, size_t n, hipStream_t s) {
-    hipLaunchKernelGGL(mul_kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, x, w, n);
-    TOMO_HIP(hipGetLastError());
-    return TOMO_OK;
-}
 int launch_waxpy(float* x, const float* c, const float* b, int positive, size_t n, hipStream_t s) {
     hipLaunchKernelGGL(waxpy_kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, x, c, b, positive, n);
     TOMO_HIP(hipGetLastError());
@@ -653,6 +792,49 @@ int launch_convert(Buf in, MutBuf out, size_t n, hipStream_t s) {
                                (TO*)out.p, out.scale, n);
         });
     });
+    TOMO_HIP(hipGetLastError());
+    return TOMO_OK;
+}
+
+unsigned loop_blocks(size_t n) {
+    const unsigned b = grid_for(n);
+    return b > (unsigned)kReduceBlocks ? (unsigned)kReduceBlocks : b;
+}
+int launch_loop_sq(const float* x, size_t n, double* partial, hipStream_t s) {
+    hipLaunchKernelGGL((sq_partial_kernel<float>), dim3(loop_blocks(n)), dim3(kBlock), 0, s, x, 1.0f, n, partial);
+    TOMO_HIP(hipGetLastError());
+    return TOMO_OK;
+}
+int launch_diff_sq(const float* a, const float* b, const float* w, float* o, size_t n, double* partial, hipStream_t s) {
+    hipLaunchKernelGGL(diff_sq_kernel, dim3(loop_blocks(n)), dim3(kBlock), 0, s, a, b, w, o, n, partial);
+    TOMO_HIP(hipGetLastError());
+    return TOMO_OK;
+}
+int launch_laplacian_sq(const float* x, float* y, int nx, int ny, int nz, double* partial, double* partial_x,
+                        hipStream_t s) {
+    hipLaunchKernelGGL(laplacian_sq_kernel, dim3(loop_blocks((size_t)nx * ny * nz)), dim3(kBlock), 0, s, x, y, nx, ny, nz,
+                       partial, partial_x);
+    TOMO_HIP(hipGetLastError());
+    return TOMO_OK;
+}
+int launch_scale_laplacian(const float* x, float* d, float scale, float a, int nx, int ny, int nz, hipStream_t s) {
+    dim3 grid(ceil_div(nx, 64), ceil_div(ny, 4), nz);
+    hipLaunchKernelGGL(scale_laplacian_kernel, grid, dim3(kBlock), 0, s, x, d, scale, a, nx, ny, nz);
+    TOMO_HIP(hipGetLastError());
+    return TOMO_OK;
+}
+int launch_axpy_scalar(float* y, const float* x, const double* a, int positive, size_t n, hipStream_t s) {
+    hipLaunchKernelGGL(axpy_scalar_kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, y, x, a, positive, n);
+    TOMO_HIP(hipGetLastError());
+    return TOMO_OK;
+}
+int launch_direction(const float* g, float* d, const double* beta, size_t n, double* partial, hipStream_t s) {
+    hipLaunchKernelGGL(direction_kernel, dim3(loop_blocks(n)), dim3(kBlock), 0, s, g, d, beta, n, partial);
+    TOMO_HIP(hipGetLastError());
+    return TOMO_OK;
+}
+int launch_loop_step(const LoopStep& a, hipStream_t s) {
+    hipLaunchKernelGGL(loop_step_kernel, dim3(1), dim3(kBlock), 0, s, a);
     TOMO_HIP(hipGetLastError());
     return TOMO_OK;
 }
@@ -702,10 +884,7 @@ static int launch_sq_partial(Buf x, size_t n, unsigned blocks, double* part, hip
     return TOMO_OK;
 }
 
-static unsigned reduce_blocks(size_t n) {
-    const unsigned b = grid_for(n);
-    return b > (unsigned)kReduceBlocks ? (unsigned)kReduceBlocks : b;
-}
+static unsigned reduce_blocks(size_t n) { return loop_blocks(n); }
 
 int reduce_sq_norm(tomo_ctx* ctx, Buf x, size_t n, double* out, hipStream_t s) {
     (void)ctx;

@@ -166,9 +166,33 @@ int launch_diff(const float* a, const float* b, float* out, size_t n, hipStream_
 int launch_scale(float* x, float v, size_t n, hipStream_t s);
 int launch_axpy(float* y, const float* x, float a, int positive, size_t n, hipStream_t s);
 int launch_laplacian(const float* x, float* y, int nx, int ny, int nz, hipStream_t s);
-// SIRT element-wise steps: w = s > 0 ? a / s : 0; x *= w; x = x + c * b (+clamp).
+
+// The loops' steps: fused passes with partial sums (kLoopPartials doubles per
+// sum at most, one per block of loop_blocks(n)), and the kernel that ends the
+// sums and applies the step rule to the iteration's statistics on the device.
+constexpr int kLoopPartials = 2048;
+enum LoopSum { kLoopResidual, kLoopReg, kLoopDirReg, kLoopDir, kLoopProj, kLoopSums };
+enum LoopRule { kRuleOptimal, kRuleFixed, kRuleBeta, kRuleConjugate, kRuleResidual };
+struct LoopStep {
+    const double* partial;    // kLoopSums x kLoopPartials
+    int blocks[kLoopSums];    // 0: not summed
+    tomo_gd_iter_stat* stat;  // of the iteration, device memory (kRuleResidual: its first field only)
+    double* state;            // smallest step (gd), last |g|^2 (cg)
+    double init;              // state before the first iteration
+    double lambda;
+    int rule, first, begins;  // first iteration of the run; first call of the iteration
+};
+unsigned loop_blocks(size_t n);
+int launch_loop_sq(const float* x, size_t n, double* partial, hipStream_t s);
+int launch_diff_sq(const float* a, const float* b, const float* w, float* o, size_t n, double* partial, hipStream_t s);
+int launch_laplacian_sq(const float* x, float* y, int nx, int ny, int nz, double* partial, double* partial_x,
+                        hipStream_t s);
+int launch_scale_laplacian(const float* x, float* d, float scale, float a, int nx, int ny, int nz, hipStream_t s);
+int launch_axpy_scalar(float* y, const float* x, const double* a, int positive, size_t n, hipStream_t s);
+int launch_direction(const float* g, float* d, const double* beta, size_t n, double* partial, hipStream_t s);
+int launch_loop_step(const LoopStep& a, hipStream_t s);
+// SIRT element-wise steps: w = s > 0 ? a / s : 0; x = x + c * b (+clamp).
 int launch_recip_weight(const float* s_in, float a, float* w, size_t n, hipStream_t s);
-int launch_mul(float* x, const float* w, size_t n, hipStream_t s);
 int launch_waxpy(float* x, const float* c, const float* b, int positive, size_t n, hipStream_t s);
 int reduce_sq_norm(tomo_ctx* ctx, Buf x, size_t n, double* out, hipStream_t s);
 int reduce_dot(tomo_ctx* ctx, const float* a, const float* b, size_t n, double* out, hipStream_t s);
