@@ -153,21 +153,21 @@ def test_vi_transpose_infinity(ctx):
         G.close()
 
 
-@pytest.mark.parametrize("op", ["siddon", "vi"])
+@pytest.mark.parametrize("op", ["siddon", "vi", "rs"])
 def test_transpose_under_capture(ctx, op):
     """A captured transpose allocates nothing: the scatter form, replayed with new
     inputs against the eager call (1e-5: two FP32 sums of the same terms)."""
     g = _geom(48, 48, 48, 48, 48, 40)
     G = _geometry(ctx, g)
     try:
-        a, b = (g.sino_shape, g.vol_shape) if op == "siddon" else (g.vol_shape, g.sino_shape)
+        a, b = (g.vol_shape, g.sino_shape) if op == "vi" else (g.sino_shape, g.vol_shape)
         x, y = torch.rand(a, device="cuda"), torch.empty(b, device="cuda")
 
         def run(out):
-            if op == "siddon":
-                G.project_adjoint(x, out, lib.PROJ_SIDDON)
-            else:
+            if op == "vi":
                 G.backproject_adjoint(x, out)
+            else:
+                G.project_adjoint(x, out, lib.PROJ_RS if op == "rs" else lib.PROJ_SIDDON)
 
         run(y)
         torch.cuda.synchronize()
@@ -182,5 +182,83 @@ def test_transpose_under_capture(ctx, op):
             run(eager)
             torch.cuda.synchronize()
             assert rel_l2(y.cpu().numpy(), eager.cpu().numpy()) <= 1e-5
+    finally:
+        G.close()
+
+
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("cube", [False, True])
+@pytest.mark.parametrize("nx,ny,nz,nu,nv,nphi,pixel", [
+    (30, 30, 63, 40, 40, 20, 2.0), (30, 31, 64, 40, 41, 65, 2.0),   # one step of z; views past 64
+    (31, 30, 65, 40, 60, 64, 2.0), (17, 33, 129, 33, 90, 31, 2.0),  # two, three steps; a grid narrower than the FOV
+    (16, 16, 257, 24, 140, 20, 2.0), (64, 20, 24, 64, 33, 40, 2.0),  # two z blocks; much narrower
+    (20, 20, 20, 90, 90, 12, 0.45), (24, 24, 24, 12, 9, 16, 5.0),   # many rows and columns a voxel, few
+    (33, 1, 1, 50, 7, 70, 1.0), (1, 1, 40, 9, 60, 30, 1.0),         # one slice, one column
+])
+def test_rs_transpose(ctx, nx, ny, nz, nu, nv, nphi, pixel, cube, dt):
+    g = _geom(nx, ny, nz, nu, nv, nphi, pixel)
+    G = _geometry(ctx, g)
+    try:
+        y = dev(np.random.default_rng(nz).random(g.sino_shape, dtype=np.float32))
+        if dt != "f32":
+            y = y.to(torch.bfloat16 if dt == "bf16" else torch.float16)
+        ref = Oracle(g).rs_T(y.float().cpu().numpy(), cube=cube)
+        out = torch.full(g.vol_shape, np.nan, dtype=torch.float32, device="cuda")
+        G.project_adjoint(y, out, lib.PROJ_RS, lib.FLAG_RS_FOV_CUBE if cube else 0)
+        got = out.cpu().numpy()
+        if not ref.any():
+            assert not got.any()
+        else:
+            assert rel_l2(got, ref) <= 1e-6
+    finally:
+        G.close()
+
+
+def test_rs_transpose_source_inside(ctx):
+    """A source inside the volume's bounding square (the scatter form)."""
+    g = _geom(40, 40, 30, 40, 40, 24, pixel=1.0, fod=0.6)
+    G = _geometry(ctx, g)
+    try:
+        y = np.random.default_rng(3).random(g.sino_shape, dtype=np.float32)
+        out = torch.empty(g.vol_shape, dtype=torch.float32, device="cuda")
+        G.project_adjoint(dev(y), out, lib.PROJ_RS)
+        assert rel_l2(out.cpu().numpy(), Oracle(g).rs_T(y)) <= 1e-5
+    finally:
+        G.close()
+
+
+def test_rs_transpose_view_chunks(ctx):
+    """More than 1 GiB of the rays' table: the views go in two chunks that add
+    (<A x, y> = <x, A^T y> within 1e-5)."""
+    g = _geom(24, 24, 24, 1024, 1024, 80, pixel=0.08)
+    G = _geometry(ctx, g)
+    try:
+        gen = torch.Generator(device="cuda").manual_seed(5)
+        x = torch.rand(g.vol_shape, generator=gen, device="cuda")
+        y = torch.rand(g.sino_shape, generator=gen, device="cuda")
+        ax, aty = torch.empty_like(y), torch.empty_like(x)
+        G.project(x, ax, lib.PROJ_RS)
+        G.project_adjoint(y, aty, lib.PROJ_RS)
+        lhs, rhs = lib.dot(ctx, ax, y), lib.dot(ctx, x, aty)
+        assert abs(lhs - rhs) <= 1e-5 * abs(rhs), (lhs, rhs)
+    finally:
+        G.close()
+
+
+def test_rs_transpose_infinity(ctx):
+    """An infinite sinogram cell reaches the voxels around its samples and no other."""
+    g = _geom(32, 32, 40, 48, 48, 20)
+    G = _geometry(ctx, g)
+    try:
+        y = np.random.default_rng(8).random(g.sino_shape, dtype=np.float32)
+        one = np.zeros_like(y)
+        one[7, 30, 20] = 1.0
+        hit = Oracle(g).rs_T(one) > 0.0
+        y[7, 30, 20] = np.inf
+        out = torch.empty(g.vol_shape, dtype=torch.float32, device="cuda")
+        G.project_adjoint(dev(y), out, lib.PROJ_RS)
+        got = out.cpu().numpy()
+        assert np.isfinite(got[~hit]).all()
+        assert np.isinf(got[hit]).mean() > 0.99  # a weight of rounding size may count as none
     finally:
         G.close()
