@@ -104,8 +104,8 @@ __device__ __forceinline__ ColumnView column_view(const DevGeom& g, const double
 // the CU, 85% of the time at 512^3 and 512 views, where that binds (and the
 // clock falls to 2.05 GHz): 22.3 -> 19.7 ms with the plans made by lane, the
 // direct views in a loop of their own, 16-byte copies and the short reciprocal.
-// FDK (256^3, 360 views) is bound by VALU: 5.93 -> 3.96 ms, most of it from
-// fdk_weight.
+// FDK (256^3, 360 views) is bound by VALU: 5.93 -> 3.25 ms, most of it from
+// fdk_weight and its sharing between mirrored voxels.
 constexpr int SX = kViStageX, SY = kViStageY;  // voxel columns per workgroup; a wave is 8 x 8 columns
 // Floats per staged row.  A wave's 64 lanes read taps (u, r) at word
 // r * pitch + u; lanes spread over about 20 columns and a few rows, so two
@@ -122,15 +122,19 @@ constexpr int kStagePitch = 76;
 // need more and read their taps directly), 22.5 KB of LDS, 7 workgroups per CU.
 // Shorter columns stage several views between two barriers: there are few waves
 // then to wait for the taps, and the boxes are small.
-template <int ZS>
+// MIRROR: a column is two halves at opposite heights, each with a box of its own.
+template <int ZS, bool MIRROR = false>
 struct StageShape {
     static_assert(ZS == 16 || ZS == 8 || ZS == 4, "staging buffers sized for 16, 8 and 4 voxels");
     static_assert(SX == 32 && SY == 8, "four 8 x 8 waves per workgroup");
-    static constexpr int rows = ZS == 16 ? 37 : ZS == 8 ? 26 : 16;      // staged rows per view
+    static_assert(!MIRROR || ZS >= 8, "halves of 8 and 4 voxels");
+    static constexpr int boxes = MIRROR ? 2 : 1;                        // per view
+    static constexpr int height = ZS / boxes;                           // voxels of a box
+    static constexpr int rows = MIRROR ? (ZS == 16 ? 20 : 16) : ZS == 16 ? 37 : ZS == 8 ? 26 : 16;  // rows of a box
     static constexpr int views = ZS == 16 ? 1 : ZS == 8 ? 2 : 4;        // views between two barriers
-    static constexpr int pieces = (rows * kStagePitch + 255) / 256;     // of a view
-    static constexpr int taps = pieces * 256;                           // floats per view
-    static constexpr int words = 2 * views * taps;
+    static constexpr int pieces = (rows * kStagePitch + 255) / 256;     // of a box
+    static constexpr int taps = pieces * 256;                           // floats per box
+    static constexpr int words = 2 * views * boxes * taps;
 };
 
 __device__ __forceinline__ int wave_min(int v) { return __reduce_min_sync(~0ull, v); }
@@ -204,14 +208,14 @@ struct StagePlan {
 
 // The box rows from the four (z', A) corners; v0 and the number of rows as v0 * 256
 // + rows, 0 where the box does not fit.
-template <int ZS>
+template <typename SS>
 __device__ __forceinline__ int stage_rows(const ViBox& bb, float zp0, float cv, int rl, int nv) {
-    const float zp1 = zp0 + (float)(ZS - 1);
+    const float zp1 = zp0 + (float)(SS::height - 1);
     const float va = fmaf(zp0, bb.amin, cv), vb = fmaf(zp0, bb.amax, cv);
     const float vc = fmaf(zp1, bb.amin, cv), vd = fmaf(zp1, bb.amax, cv);
     const float vlo = floorf(fminf(fminf(va, vb), fminf(vc, vd)));
     const float vhi = floorf(fmaxf(fmaxf(va, vb), fmaxf(vc, vd)));
-    const bool fits = vlo >= -32768.0f && vhi <= 32768.0f && vhi - vlo + 2.0f <= (float)StageShape<ZS>::rows &&
+    const bool fits = vlo >= -32768.0f && vhi <= 32768.0f && vhi - vlo + 2.0f <= (float)SS::rows &&
                       bb.u1 - bb.u0 + 2 <= 64;
     // a lane's four taps start at a tap of the box and end on its row; the 32-bit
     // offsets of rows off the detector do not come round to it
@@ -264,13 +268,18 @@ __device__ __forceinline__ void pair_sample4(const uint32_t (&p0)[4], const uint
 
 // PAIR: `sino` holds u-pair words (vi_pair_kernel; nu + 1 per row) instead of
 // FP32 taps; the box copy and the tap offsets are the same, one word per row.
-// FDK: 0 VI, 1 FDK, 2 FDK whose weights are within fdk_weight's bounds.
+// FDK: 0 VI, 1 FDK, 2 FDK whose weights are within fdk_weight's bounds, 3 the same
+// on mirrored columns: the weight depends on z'^2, so a voxel at z' and the one at
+// -z' share it.  A column is then ZS / 2 voxels from k0 = bz ZS / 2 on and their
+// mirror images nz - 1 - k.  256^3 and 360 views: 3.95 ms without, 3.25 with.
 template <typename TV, int FDK, int ZS, bool PAIR = false>
 __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __restrict__ sino,
                                                const ViBox* __restrict__ boxes, TV* __restrict__ vol,
                                                float vol_scale, float post, int bx, int by, int bz,
                                                float* __restrict__ stage) {
-    using SS = StageShape<ZS>;
+    constexpr bool MIRROR = FDK == 3;
+    using SS = StageShape<ZS, MIRROR>;
+    constexpr int H = SS::height, B = SS::boxes;
     constexpr int NT = SX * SY;
     constexpr int NW = NT / 64;                             // waves per workgroup
     constexpr int kSlots = (SS::rows + NW - 1) / NW;        // box rows per wave at most
@@ -279,7 +288,7 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     // wave wv covers columns x in [8 wv, 8 wv + 8), y in [0, 8)
     const int i = bx * SX + wv * 8 + (lane & 7);
     const int j = by * SY + (lane >> 3);
-    const int k0 = bz * ZS;
+    const int k0 = bz * H;
     // a lane past the volume's edge works on the edge column, and stores nothing
     const double xp = (double)min(i, g.nx - 1) - (double)g.cx, yp = (double)min(j, g.ny - 1) - (double)g.cy;
     const float zp0 = (float)((double)k0 - (double)g.cz);
@@ -295,22 +304,19 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     float acc[ZS];
 #pragma unroll
     for (int k = 0; k < ZS; ++k) acc[k] = 0.0f;
-    auto add = [&](const ColumnView& cvw, int k, float r) {
-        if (FDK) {
-            const float vp = (zp0 + (float)k) * cvw.A, q = fmaf(vp, vp, cvw.base);
-            const float wt = FDK == 2 ? fdk_weight(cvw.num, q) : cvw.num / sqrtf(q);
-            acc[k] += wt * r;
-        } else {
-            acc[k] += r;
-        }
+    // z' of voxel k; the second half is the first's mirror image, exactly (cz is (nz - 1) / 2)
+    auto height = [&](int k) { return k < H ? zp0 + (float)k : -(zp0 + (float)(k - H)); };
+    auto weight = [&](const ColumnView& cvw, int k) {
+        const float vp = height(k) * cvw.A, q = fmaf(vp, vp, cvw.base);
+        return FDK >= 2 ? fdk_weight(cvw.num, q) : cvw.num / sqrtf(q);
     };
-    auto term = [&](const ColumnView& cvw, float fu, int k, float v, float vf, float t00, float t01, float t10,
-                    float t11) {
+    auto add = [&](float wt, int k, float r) { acc[k] += FDK ? wt * r : r; };
+    auto bilinear = [&](float fu, float v, float vf, float t00, float t01, float t10, float t11) {
         // t00 = (u, v), t01 = (u, v+1), t10 = (u+1, v), t11 = (u+1, v+1)
         const float fv = v - vf;
         const float a = fmaf(fu, t10 - t00, t00);
         const float b = fmaf(fu, t11 - t01, t01);
-        add(cvw, k, fmaf(fv, b - a, a));
+        return fmaf(fv, b - a, a);
     };
     const uint32_t view_bytes = (uint32_t)(plane * sizeof(float));
     // Byte offset in the view of a lane's four taps of the wave's q-th piece, from
@@ -322,7 +328,7 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
         const int w = 256 * (wv + q * NW) + 4 * lane, row = w / kStagePitch;
         piece[q] = (uint32_t)(row * rl + (w - row * kStagePitch)) * 4u;
     }
-    // Copy of view p's box into view buffer b, straight from memory into LDS
+    // Copy of a box of view p into buffer b, straight from memory into LDS
     // (buffer_load ... lds); a tap off the detector's upper or lower edge is
     // outside the view's bytes, which writes 0.  Words past the box hold taps
     // that nothing reads.  One 16-byte load per lane brings 3.4 rows; by rows, a
@@ -361,16 +367,16 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
             }
         }
     };
-    int plan_u0 = 0, plan_v = 0;  // of view (p & ~63) + lane
-    auto plan_of = [&](int p) {
-        const int v = __builtin_amdgcn_readlane(plan_v, p & 63);
-        return StagePlan{__builtin_amdgcn_readlane(plan_u0, p & 63), v >> 8, v & 127, (v & 128) != 0};
+    int plan_u0[B] = {}, plan_v[B] = {};  // of view (p & ~63) + lane
+    auto plan_of = [&](int p, int b) {
+        const int v = __builtin_amdgcn_readlane(plan_v[b], p & 63);
+        return StagePlan{__builtin_amdgcn_readlane(plan_u0[b], p & 63), v >> 8, v & 127, (v & 128) != 0};
     };
     // Plans and copies of the group of G views from p on; rows is 0 if one of its
     // boxes does not fit, and all of the group's taps are then read directly.
     constexpr int G = SS::views;
     struct Group {
-        int u0[G], v0[G], rows;
+        int u0[G][B], v0[G][B], rows;
     };
     auto stage_group = [&](int p, int half) {
         Group r;
@@ -379,19 +385,24 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
             ViBox bb = bt[p + lane];
             bb.u0 += PAIR;  // word index of tap pair (u, u + 1)
             bb.u1 += PAIR;
-            plan_v = stage_rows<ZS>(bb, zp0, cv, rl, nv);
-            plan_u0 = (plan_v & 128) ? bb.u0 & ~3 : bb.u0;  // rows of a multiple of 4 taps: aligned loads
-        }
 #pragma unroll
-        for (int t = 0; t < G; ++t) {
-            const StagePlan s = p + t < g.nphi ? plan_of(p + t) : StagePlan{0, 0, 0, false};
-            r.u0[t] = s.u0;
-            r.v0[t] = s.v0;
-            if (p + t < g.nphi) {
-                if (s.rows == 0) r.rows = 0;
-                copy_box(s, p + t, half * G + t);
+            for (int b = 0; b < B; ++b) {
+                plan_v[b] = stage_rows<SS>(bb, b ? -(zp0 + (float)(H - 1)) : zp0, cv, rl, nv);
+                plan_u0[b] = (plan_v[b] & 128) ? bb.u0 & ~3 : bb.u0;  // rows of a multiple of 4 taps: aligned loads
             }
         }
+#pragma unroll
+        for (int t = 0; t < G; ++t)
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                const StagePlan s = p + t < g.nphi ? plan_of(p + t, b) : StagePlan{0, 0, 0, false};
+                r.u0[t][b] = s.u0;
+                r.v0[t][b] = s.v0;
+                if (p + t < g.nphi) {
+                    if (s.rows == 0) r.rows = 0;
+                    copy_box(s, p + t, (half * G + t) * B + b);
+                }
+            }
         return r;
     };
     auto view_terms = [&](int p) {
@@ -425,37 +436,52 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
                 // byte offset in the buffer of tap (uc, vf): ((vf - v0) pitch + uc - u0) 4,
                 // one exact fma of small integers on top of 2^23, whose low bits are then the
                 // offset: an and (0.6 cycles per wave and CU) for a conversion (1.1)
-                const float colb = (float)(((int)uc + PAIR - now.u0[t] - now.v0[t] * kStagePitch + (half * G + t) * SS::taps) * 4) +
-                                   0x1p23f;
+                float colb[B];
+#pragma unroll
+                for (int b = 0; b < B; ++b)
+                    colb[b] = (float)(((int)uc + PAIR - now.u0[t][b] - now.v0[t][b] * kStagePitch +
+                                       ((half * G + t) * B + b) * SS::taps) * 4) + 0x1p23f;
+                auto taps = [&](float vf, int b) {
+                    const uint32_t off = __float_as_uint(fmaf(vf, (float)(kStagePitch * 4), colb[b])) & 0x7fffffu;
+                    return (const char*)stage + off;
+                };
                 if constexpr (PAIR) {
-                    static_assert(ZS % 4 == 0, "u-pair samples go four voxels at a time");
+                    static_assert(H % 4 == 0, "u-pair samples go four voxels at a time");
                     const uint32_t pw = pair_weights(fu);
 #pragma unroll
-                    for (int k4 = 0; k4 < ZS; k4 += 4) {
-                        uint32_t p0[4], p1[4];
-                        float fv[4], r0[4], dr[4];
+                    for (int k4 = 0; k4 < H; k4 += 4) {
+                        float wt[4];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float v = fmaf(zp0 + (float)(k4 + e), cvw.A, cv);
-                            const float vf = floorf(v);
-                            const uint32_t off = __float_as_uint(fmaf(vf, (float)(kStagePitch * 4), colb)) & 0x7fffffu;
-                            const uint32_t* qw = (const uint32_t*)((const char*)stage + off);
-                            p0[e] = qw[0];
-                            p1[e] = qw[kStagePitch];
-                            fv[e] = v - vf;
+                        for (int e = 0; e < 4; ++e) wt[e] = FDK ? weight(cvw, k4 + e) : 1.0f;
+#pragma unroll
+                        for (int b = 0; b < B; ++b) {
+                            uint32_t p0[4], p1[4];
+                            float fv[4], r0[4], dr[4];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const float v = fmaf(height(b * H + k4 + e), cvw.A, cv);
+                                const float vf = floorf(v);
+                                const uint32_t* qw = (const uint32_t*)taps(vf, b);
+                                p0[e] = qw[0];
+                                p1[e] = qw[kStagePitch];
+                                fv[e] = v - vf;
+                            }
+                            pair_sample4(p0, p1, pw, r0, dr);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) add(wt[e], b * H + k4 + e, fmaf(fv[e], dr[e], r0[e]));
                         }
-                        pair_sample4(p0, p1, pw, r0, dr);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) add(cvw, k4 + e, fmaf(fv[e], dr[e], r0[e]));
                     }
                 } else {
 #pragma unroll
-                    for (int k = 0; k < ZS; ++k) {
-                        const float v = fmaf(zp0 + (float)k, cvw.A, cv);
-                        const float vf = floorf(v);
-                        const uint32_t off = __float_as_uint(fmaf(vf, (float)(kStagePitch * 4), colb)) & 0x7fffffu;
-                        const float* q = (const float*)((const char*)stage + off);
-                        term(cvw, fu, k, v, vf, q[0], q[kStagePitch], q[1], q[kStagePitch + 1]);
+                    for (int k = 0; k < H; ++k) {
+                        const float wt = FDK ? weight(cvw, k) : 1.0f;
+#pragma unroll
+                        for (int b = 0; b < B; ++b) {
+                            const float v = fmaf(height(b * H + k), cvw.A, cv);
+                            const float vf = floorf(v);
+                            const float* q = (const float*)taps(vf, b);
+                            add(wt, b * H + k, bilinear(fu, v, vf, q[0], q[kStagePitch], q[1], q[kStagePitch + 1]));
+                        }
                     }
                 }
             }
@@ -482,17 +508,17 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
             };
 #pragma unroll
             for (int k = 0; k < ZS; ++k) {
-                const float v = fmaf(zp0 + (float)k, cvw.A, cv);
+                const float v = fmaf(height(k), cvw.A, cv), wt = FDK ? weight(cvw, k) : 1.0f;
                 const float vf = floorf(v);
                 const int iv = (int)__builtin_amdgcn_fmed3f(vf, -2.0f, (float)nv);
                 const bool v0ok = (unsigned)iv < (unsigned)nv, v1ok = (unsigned)(iv + 1) < (unsigned)nv;
                 if constexpr (PAIR) {
                     const uint32_t p0 = __builtin_bit_cast(uint32_t, rd(pok && v0ok, iv, iu + 1));
                     const uint32_t p1 = __builtin_bit_cast(uint32_t, rd(pok && v1ok, iv + 1, iu + 1));
-                    add(cvw, k, pair_sample(p0, p1, pw, v - vf));
+                    add(wt, k, pair_sample(p0, p1, pw, v - vf));
                 } else {
-                    term(cvw, fu, k, v, vf, rd(u0ok && v0ok, iv, iu), rd(u0ok && v1ok, iv + 1, iu),
-                         rd(u1ok && v0ok, iv, iu + 1), rd(u1ok && v1ok, iv + 1, iu + 1));
+                    add(wt, k, bilinear(fu, v, vf, rd(u0ok && v0ok, iv, iu), rd(u0ok && v1ok, iv + 1, iu),
+                                        rd(u1ok && v0ok, iv, iu + 1), rd(u1ok && v1ok, iv + 1, iu + 1)));
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -504,21 +530,23 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     const size_t sxy = (size_t)g.nx * g.ny;
     const size_t base = (size_t)i + (size_t)g.nx * j;
 #pragma unroll
-    for (int k = 0; k < ZS; ++k)
-        if (k0 + k < g.nz)
-            Storage<TV>::store(vol, base + (size_t)(k0 + k) * sxy, FDK ? acc[k] * post : (acc[k] * g.delta) * post,
-                               vol_scale);
+    for (int k = 0; k < ZS; ++k) {
+        // mirrored: the middle slice of an odd volume belongs to the first half
+        const int zk = k < H ? k0 + k : g.nz - 1 - (k0 + k - H);
+        if (MIRROR ? (k < H ? 2 * zk < g.nz : 2 * zk >= g.nz) : zk < g.nz)
+            Storage<TV>::store(vol, base + (size_t)zk * sxy, FDK ? acc[k] * post : (acc[k] * g.delta) * post, vol_scale);
+    }
 }
 
 // Waves per SIMD that a kernel's registers are held to.
-constexpr int vi_waves(int fdk, int zs, bool pair) { return !pair ? 7 : fdk == 1 ? 5 : 6; }
+constexpr int vi_waves(int fdk, int zs, bool pair) { return fdk == 3 ? 6 : !pair ? 7 : fdk == 1 ? 5 : 6; }
 
 // post: 1 for FP32 taps, 1 / storage scale for FP16 u-pairs.
 template <typename TV, int FDK, int ZS, bool PAIR>
 __global__ __launch_bounds__(SX* SY, vi_waves(FDK, ZS, PAIR)) void vi_staged_kernel(DevGeom g, const float* __restrict__ sino,
                                                          const ViBox* __restrict__ boxes, TV* __restrict__ vol,
                                                          float vol_scale, float post) {
-    __shared__ __align__(16) float stage[StageShape<ZS>::words];
+    __shared__ __align__(16) float stage[StageShape<ZS, FDK == 3>::words];
     vi_staged_tile<TV, FDK, ZS, PAIR>(g, sino, boxes, vol, vol_scale, post, blockIdx.x, blockIdx.y, blockIdx.z,
                                       stage);
 }
@@ -845,7 +873,8 @@ static bool fdk_in_bounds(const DevGeom& d) {
 template <typename TV, int FDK, int ZS, bool PAIR>
 static void launch_vi_tiles(const DevGeom& d, const float* sino, const ViBox* boxes, void* vol, float vol_scale,
                             float post, hipStream_t s) {
-    const dim3 grid(ceil_div(d.nx, SX), ceil_div(d.ny, SY), ceil_div(d.nz, ZS));
+    const dim3 grid(ceil_div(d.nx, SX), ceil_div(d.ny, SY),
+                    FDK == 3 ? ceil_div((d.nz + 1) / 2, ZS / 2) : ceil_div(d.nz, ZS));
     hipLaunchKernelGGL((vi_staged_kernel<TV, FDK, ZS, PAIR>), grid, dim3(SX * SY), 0, s, d, sino, boxes, (TV*)vol,
                        vol_scale, post);
 }
@@ -878,10 +907,10 @@ static hipError_t launch_vi_staged(const DevGeom& d, int fdk, const float* sino,
         if (fdk && !fdk_in_bounds(d))
             launch_vi_tiles<TV, 1, kViTileZ, PAIR>(d, sino, bt, vol, vol_scale, post, s);
         else if (zs == kViTileZ)
-            fdk ? launch_vi_tiles<TV, 2, kViTileZ, PAIR>(d, sino, bt, vol, vol_scale, post, s)
+            fdk ? launch_vi_tiles<TV, 3, kViTileZ, PAIR>(d, sino, bt, vol, vol_scale, post, s)
                 : launch_vi_tiles<TV, 0, kViTileZ, PAIR>(d, sino, bt, vol, vol_scale, post, s);
         else if (zs == 8)
-            fdk ? launch_vi_tiles<TV, 2, 8, PAIR>(d, sino, bt, vol, vol_scale, post, s)
+            fdk ? launch_vi_tiles<TV, 3, 8, PAIR>(d, sino, bt, vol, vol_scale, post, s)
                 : launch_vi_tiles<TV, 0, 8, PAIR>(d, sino, bt, vol, vol_scale, post, s);
         else
             fdk ? launch_vi_tiles<TV, 2, 4, PAIR>(d, sino, bt, vol, vol_scale, post, s)
