@@ -694,11 +694,11 @@ __global__ __launch_bounds__(BX* BY) void rs_adjoint_kernel(DevGeom g, int cube,
 // are relative to the point of the line next to the column, so that the weights
 // hold no rounding of a large coordinate.
 //
-// VALU issue bounds it: 8 cycles per sample, 15 per row and 20 per line of 64
-// voxels, about 300 per 64 voxels and view.  Against the scatter below, 256^3 and
-// 256 views: 684 -> 34.0 ms; 64^3 and 64 views 4.2 -> 0.30 ms; 17^3 and 16 views
-// 78 -> 72 us, so that no size goes back to it.  Four waves per SIMD, with a few
-// registers in memory at K = 4, are 8% faster than three.
+// VALU issue bounds it: 8 cycles per sample (6 with its mirror image), 15 per row
+// and 20 per line of 64 voxels.  Against the scatter below, 256^3 and 256 views:
+// 684 -> 34.0 ms, 26.5 with the mirror images; 64^3 and 64 views 4.2 -> 0.30 ms;
+// 17^3 and 16 views 78 us either way, so that no size goes back to it.  Four waves
+// per SIMD, with a few registers in memory at K = 2, are 8% faster than three.
 constexpr int kRsTWaves = 4;
 __host__ __device__ inline size_t rs_t_rows(int nv) { return (size_t)nv + 2; }  // row -1 and row nv hold no ray
 
@@ -729,8 +729,12 @@ __device__ __forceinline__ float lane_value(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
+// MIRROR: a lane takes its voxel k of the lower half and the mirror image nz - 1 - k,
+// whose samples lie on the mirrored rows with the same weights; the rays' values and
+// numbers of samples are the mirrored rows' own.
+//
 // Grid: x = (4 voxel columns along x, y), y = z block of 64 K.  Views p0 + [0, np).
-template <int K>
+template <int K, bool MIRROR>
 __global__ __launch_bounds__(64 * kRsTWaves, 4) void rs_t_kernel(DevGeom g, int cube, const float4* __restrict__ tab, int p0,
                                                              int np, int add, float* __restrict__ vol) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -743,12 +747,14 @@ __global__ __launch_bounds__(64 * kRsTWaves, 4) void rs_t_kernel(DevGeom g, int 
     const double xi = (double)i - (double)g.cx, yj = (double)j - (double)g.cy;
     const double half = 0.5 * (double)g.nx, R2 = cube ? 2.0 * (half * half) : half * half;
     const float cv = g.cv, last = (float)g.nv;
-    const float kmax = fmaxf(fabsf((float)kb - g.cz), fabsf((float)min(kb + 64 * K, g.nz) - 1.0f - g.cz));
-    float kk[K], total[K], acc[K];
+    const float kmax = fmaxf(fabsf((float)kb - g.cz), fabsf((float)min(kb + 64 * K, MIRROR ? (g.nz + 1) / 2 : g.nz) - 1.0f - g.cz));
+    constexpr int B = MIRROR ? 2 : 1;
+    float kk[K], total[B][K], acc[B][K];
 #pragma unroll
     for (int c = 0; c < K; ++c) {
         kk[c] = (float)(kb + 64 * c + lane) - g.cz;
-        total[c] = 0.0f;
+#pragma unroll
+        for (int b = 0; b < B; ++b) total[b][c] = 0.0f;
     }
     for (int pb = 0; pb < np; pb += 64) {
         // ---- one view per lane: the detector columns whose lines may cross the square
@@ -771,7 +777,9 @@ __global__ __launch_bounds__(64 * kRsTWaves, 4) void rs_t_kernel(DevGeom g, int 
         for (int h = 0; h < most; ++h) {
             // ---- one line per lane; partial sums of a line, of 64 lines, and of all
 #pragma unroll
-            for (int c = 0; c < K; ++c) acc[c] = 0.0f;
+            for (int c = 0; c < K; ++c)
+#pragma unroll
+                for (int b = 0; b < B; ++b) acc[b][c] = 0.0f;
             const int m = m0 + h;
             bool on = h < cnt;
             const double sm = ((double)m - (double)g.cu) * (double)g.du;
@@ -813,31 +821,42 @@ __global__ __launch_bounds__(64 * kRsTWaves, 4) void rs_t_kernel(DevGeom g, int 
                 const float i0 = lane_value(li0, l), i1 = lane_value(li1, l), Dlo = Dh + lane_value(llo, l);
                 const int num = __builtin_amdgcn_readlane(lnum, l), R = num >> 8, S = num & 255;
                 const float4* line = tab + (size_t)(uint32_t)__builtin_amdgcn_readlane(lbase, l) * rows + 1;
-                float row[K], part[K];
+                float row[K], part[B][K];
 #pragma unroll
                 for (int c = 0; c < K; ++c) {
-                    part[c] = 0.0f;
+#pragma unroll
+                    for (int b = 0; b < B; ++b) part[b][c] = 0.0f;
                     const float k0 = kk[c] - 1.0f;
                     row[c] = ceilf(fminf(k0 * i0, k0 * i1) + (cv - 2e-3f));  // first that may reach the voxel
                 }
                 for (int r = 0; r < R; ++r) {
                     typedef float V4 __attribute__((ext_vector_type(4)));
+                    typedef float V2 __attribute__((ext_vector_type(2)));
                     V4 e[K];
+                    V2 image[K];  // (delta g, samples) of the mirrored row
 #pragma unroll
-                    for (int c = 0; c < K; ++c)
+                    for (int c = 0; c < K; ++c) {
                         e[c] = *(const V4*)(line + (int)__builtin_amdgcn_fmed3f(row[c], -1.0f, last));
-                    float sg[K], zb[K], dt[K], rem[K], w[K];
+                        image[c] = (V2)0.0f;
+                        if (MIRROR)
+                            image[c] = *(const V2*)(line + (int)__builtin_amdgcn_fmed3f(last - 1.0f - row[c], -1.0f, last));
+                    }
+                    float sg[K], zb[K], dt[K], rem[B][K], w[B][K];
 #pragma unroll
                     for (int c = 0; c < K; ++c) {
                         // whole before the loops on the numbers (empty statement)
-                        asm volatile("" : "+v"(e[c]));
+                        asm volatile("" : "+v"(e[c]), "+v"(image[c]));
                         const float nr = row[c] - cv;
                         sg[c] = nr * qs;
                         zb[c] = fmaf(nr, Al, fmaf(nr, Ah, -kk[c]));
                         const float s0 = fmaxf(ceilf(fmaf(Dlo, __builtin_amdgcn_rcpf(e[c].z), -1e-3f)), 0.0f);
                         dt[c] = fmaf(s0, e[c].z, -Dh) + fmaf(s0, e[c].w, -Dl);
-                        rem[c] = e[c].y - s0;
-                        w[c] = 0.0f;
+                        rem[0][c] = e[c].y - s0;
+                        w[0][c] = 0.0f;
+                        if (MIRROR) {
+                            rem[B - 1][c] = image[c].y - s0;
+                            w[B - 1][c] = 0.0f;
+                        }
                         row[c] += 1.0f;
                     }
                     float ts = 0.0f;
@@ -847,29 +866,43 @@ __global__ __launch_bounds__(64 * kRsTWaves, 4) void rs_t_kernel(DevGeom g, int 
                             const float wx = __builtin_amdgcn_fmed3f(1.0f - fabsf(fmaf(dt[c], uxs, ax)), 0.0f, 1.0f);
                             const float wy = __builtin_amdgcn_fmed3f(1.0f - fabsf(fmaf(dt[c], uys, ay)), 0.0f, 1.0f);
                             const float wz = __builtin_amdgcn_fmed3f(1.0f - fabsf(fmaf(dt[c], sg[c], zb[c])), 0.0f, 1.0f);
-                            w[c] = fmaf(ts < rem[c] ? wx * wy : 0.0f, wz, w[c]);
+                            const float wxy = wx * wy;
+#pragma unroll
+                            for (int b = 0; b < B; ++b) w[b][c] = fmaf(ts < rem[b][c] ? wxy : 0.0f, wz, w[b][c]);
                             dt[c] += e[c].z;
                         }
                         ts += 1.0f;
                     }
                     // a weight of 0 takes nothing from its ray, whatever it holds
 #pragma unroll
-                    for (int c = 0; c < K; ++c) part[c] = w[c] > 0.0f ? fmaf(w[c], e[c].x, part[c]) : part[c];
+                    for (int c = 0; c < K; ++c)
+#pragma unroll
+                        for (int b = 0; b < B; ++b)
+                            part[b][c] = w[b][c] > 0.0f ? fmaf(w[b][c], b ? image[c].x : e[c].x, part[b][c]) : part[b][c];
                 }
 #pragma unroll
-                for (int c = 0; c < K; ++c) acc[c] += part[c];
+                for (int c = 0; c < K; ++c)
+#pragma unroll
+                    for (int b = 0; b < B; ++b) acc[b][c] += part[b][c];
             }
 #pragma unroll
-            for (int c = 0; c < K; ++c) total[c] += acc[c];
+            for (int c = 0; c < K; ++c)
+#pragma unroll
+                for (int b = 0; b < B; ++b) total[b][c] += acc[b][c];
         }
     }
     const size_t sxy = (size_t)g.nx * g.ny;
 #pragma unroll
     for (int c = 0; c < K; ++c) {
         const int k = kb + 64 * c + lane;
-        if (k < g.nz) {
-            float* o = vol + ((size_t)i + (size_t)g.nx * j + sxy * k);
-            *o = add ? *o + total[c] : total[c];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int z = b ? g.nz - 1 - k : k;
+            // the middle slice of an odd volume belongs to the lower half
+            if (!MIRROR ? z < g.nz : b ? 2 * z >= g.nz : 2 * z < g.nz) {
+                float* o = vol + ((size_t)i + (size_t)g.nx * j + sxy * z);
+                *o = add ? *o + total[b][c] : total[b][c];
+            }
         }
     }
 }
@@ -963,10 +996,10 @@ static bool rs_t_gathers(const DevGeom& d) {
            (size_t)d.nu * d.nphi < (1ull << 31);
 }
 
-template <int K>
+template <int K, bool MIRROR>
 static void launch_rs_t(const DevGeom& d, int cube, const float4* tab, int p0, int np, float* vol, hipStream_t s) {
-    const dim3 grid(ceil_div(d.nx, kRsTWaves) * (unsigned)d.ny, ceil_div(d.nz, 64 * K));
-    hipLaunchKernelGGL((rs_t_kernel<K>), grid, dim3(64 * kRsTWaves), 0, s, d, cube, tab, p0, np, p0 > 0, vol);
+    const dim3 grid(ceil_div(d.nx, kRsTWaves) * (unsigned)d.ny, ceil_div(MIRROR ? (d.nz + 1) / 2 : d.nz, 64 * K));
+    hipLaunchKernelGGL((rs_t_kernel<K, MIRROR>), grid, dim3(64 * kRsTWaves), 0, s, d, cube, tab, p0, np, p0 > 0, vol);
 }
 
 int launch_rs_adjoint(const tomo_geom* g, int cube, Buf sino, MutBuf vol, hipStream_t s) {
@@ -993,14 +1026,14 @@ int launch_rs_adjoint(const tomo_geom* g, int cube, Buf sino, MutBuf vol, hipStr
                 hipLaunchKernelGGL((rs_t_prepare_kernel<TS>), dim3(tiles), dim3(256), 0, s, d, cube,
                                    (const TS*)sino.p + skip, inv, p0, tab);
             });
-            // K 64-voxel steps per lane: the fewest z blocks that K <= 4 allows
-            const int steps = (int)ceil_div(d.nz, 64), blocks = (int)ceil_div(steps, 4);
-            switch (ceil_div(steps, blocks)) {
-                case 1: launch_rs_t<1>(d, cube, tab, p0, np, (float*)vol.p, s); break;
-                case 2: launch_rs_t<2>(d, cube, tab, p0, np, (float*)vol.p, s); break;
-                case 3: launch_rs_t<3>(d, cube, tab, p0, np, (float*)vol.p, s); break;
-                default: launch_rs_t<4>(d, cube, tab, p0, np, (float*)vol.p, s); break;
-            }
+            // one step of 64 voxels, or one or two of 64 and their mirror images (up to
+            // 64 slices these would leave half of the lanes idle)
+            if (d.nz <= 64)
+                launch_rs_t<1, false>(d, cube, tab, p0, np, (float*)vol.p, s);
+            else if (d.nz <= 128)
+                launch_rs_t<1, true>(d, cube, tab, p0, np, (float*)vol.p, s);
+            else
+                launch_rs_t<2, true>(d, cube, tab, p0, np, (float*)vol.p, s);
             e = hipGetLastError();
         }
         const hipError_t f = hipFreeAsync(tab, s);
