@@ -527,7 +527,7 @@ def batch_leg(ctx, n_prob, iters=20, seed=7):
             "peak_active": st["peak_active"], "rounds": st["rounds"], "identical_to_one_at_a_time": same,
             "bf16_copies": {"batched_s": round(t_bf16, 3), "speedup_vs_one_at_a_time_fp32": round(t_seq / t_bf16, 3),
                             "max_rel_l2_vs_fp32_batched": float(f"{err16:.3e}"),
-                            "note": "BF16 operator copies (z-pair; A-pair for RS problems) rounded from the FP32 state; VI, sums and state FP32"}}
+                            "note": "BF16 operator copies rounded from the FP32 state; VI, sums and state FP32"}}
 
 
 def loop_leg(G, vol, sino, iters, upd, stream):
@@ -675,10 +675,10 @@ def main():
         ops[name] = rec
     ops["siddon"]["n_seg"] = n_seg
     ops["rs"]["n_samp"] = n_samp
-    ops["rs"]["form"] = "per-lane gathers from the z-pair copies (rs_kernel)"
+    ops["rs"]["form"] = "per-lane gathers from the RS copy (rs_kernel)"
     ops["rs_staged"]["form"] = ("taps staged in LDS per window of up to 8 sample planes, copied as 16-byte "
                                 "chunks (TOMO_FLAG_STAGED, rs_staged_kernel)")
-    ops["siddon"]["form"] = "per-lane gathers from the z-pair copies (siddon_kernel)"
+    ops["siddon"]["form"] = "per-lane gathers from the z-column copy (siddon_kernel)"
     ops["siddon_staged"]["form"] = ("quads staged in LDS per window of up to 8 slabs, copied as 16-byte chunks "
                                     "(TOMO_FLAG_STAGED, siddon_staged_kernel)")
     ops["siddon_staged"]["n_seg"] = n_seg
