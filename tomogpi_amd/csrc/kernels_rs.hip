@@ -696,9 +696,10 @@ __global__ __launch_bounds__(BX* BY) void rs_adjoint_kernel(DevGeom g, int cube,
 //
 // VALU issue bounds it: 8 cycles per sample (6 with its mirror image), 15 per row
 // and 20 per line of 64 voxels.  Against the scatter below, 256^3 and 256 views:
-// 684 -> 34.0 ms, 26.5 with the mirror images; 64^3 and 64 views 4.2 -> 0.30 ms;
-// 17^3 and 16 views 78 us either way, so that no size goes back to it.  Four waves
-// per SIMD, with a few registers in memory at K = 2, are 8% faster than three.
+// 684 -> 34.0 ms, 26.5 with the mirror images, 25.0 with six waves per SIMD (a few
+// registers in memory; 128^3 and 128 views 2.32 ms at four, 2.06 at six, 2.03 at
+// seven); 64^3 and 64 views 4.2 -> 0.30 ms; 17^3 and 16 views 78 -> 73 us, so that no
+// size goes back to it.
 constexpr int kRsTWaves = 4;
 __host__ __device__ inline size_t rs_t_rows(int nv) { return (size_t)nv + 2; }  // row -1 and row nv hold no ray
 
@@ -735,7 +736,7 @@ __device__ __forceinline__ float lane_value(float v, int l) {
 //
 // Grid: x = (4 voxel columns along x, y), y = z block of 64 K.  Views p0 + [0, np).
 template <int K, bool MIRROR>
-__global__ __launch_bounds__(64 * kRsTWaves, 4) void rs_t_kernel(DevGeom g, int cube, const float4* __restrict__ tab, int p0,
+__global__ __launch_bounds__(64 * kRsTWaves, 6) void rs_t_kernel(DevGeom g, int cube, const float4* __restrict__ tab, int p0,
                                                              int np, int add, float* __restrict__ vol) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t gx = (uint32_t)(g.nx + kRsTWaves - 1) / kRsTWaves;

@@ -646,8 +646,8 @@ __global__ __launch_bounds__(TX* TY) void vi_adjoint_kernel(DevGeom g, const TV*
 //
 // VALU issue takes about half of its time, waits on the columns most of the rest
 // (they come from the memory-side cache: 256^3 and 256 views read 6 GB).  201 x
-// 187 x 149, 229 x 173, 131 views: 10.0 -> 1.10 ms against the scatter below;
-// 256^3 and 256 views 71.9 -> 3.44 ms.
+// 187 x 149, 229 x 173, 131 views: 10.0 -> 1.10 ms against the scatter below, 0.97
+// with seven waves per SIMD instead of five; 256^3 and 256 views 71.9 -> 3.27 ms.
 constexpr int kViTPad = 4;
 constexpr int kViTWords = 512;  // voxels of a column a wave stages, two loads of 64 x 4
 __host__ __device__ inline size_t vi_t_pitch(int nz) { return (size_t)(nz + 3) / 4 * 4 + 2 * kViTPad; }
@@ -686,7 +686,7 @@ __device__ __forceinline__ float lane_value(float v, int l) {
 // Grid: x = (view, column group), views first; y = row block of 64 K rows.  One
 // wave per workgroup: nothing is shared, and the strips differ in length.
 template <int K, int M>
-__global__ __launch_bounds__(64, 5) void vi_t_kernel(DevGeom g, const float* __restrict__ vt, float* __restrict__ sino) {
+__global__ __launch_bounds__(64, 7) void vi_t_kernel(DevGeom g, const float* __restrict__ vt, float* __restrict__ sino) {
     typedef float V4 __attribute__((ext_vector_type(4)));
     __shared__ __align__(16) float stage[kViTWords + 8];
     const int lane = threadIdx.x;
