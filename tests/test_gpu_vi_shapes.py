@@ -20,6 +20,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("fdk", [False, True])
 @pytest.mark.parametrize("nx,ny,nz,nu,nv,nphi,pixel,fod", [
     (33, 17, 9, 50, 20, 67, 2.0, 2.0), (64, 64, 64, 64, 64, 3, 2.0, 2.0), (40, 30, 3, 37, 5, 1, 2.0, 2.0),  # 4 voxels
+    (64, 64, 64, 64, 64, 46, 2.0, 2.0),  # 4 voxels, boxes of up to 20 rows, the buffers' last, and two views left over
     (96, 90, 90, 150, 110, 66, 2.0, 2.0), (100, 100, 101, 101, 99, 7, 2.0, 2.0),                            # 8
     (137, 136, 130, 139, 133, 65, 2.0, 2.0), (130, 150, 150, 300, 200, 9, 2.0, 2.0),                        # 16
     (64, 64, 40, 200, 200, 6, 0.4, 2.0), (96, 96, 90, 400, 300, 5, 0.5, 2.0),  # boxes past the buffers

@@ -122,6 +122,8 @@ constexpr int kStagePitch = 76;
 // need more and read their taps directly), 22.5 KB of LDS, 7 workgroups per CU.
 // Shorter columns stage several views between two barriers: there are few waves
 // then to wait for the taps, and the boxes are small.
+// 4: 20 rows, what six pieces hold; with 16, 2% of the groups at 64^3 read directly, and
+// the slowest workgroup two of twelve (64^3 and 48 views 30.0 us, 27.2 with 20).
 // MIRROR: a column is two halves at opposite heights, each with a box of its own.
 template <int ZS, bool MIRROR = false>
 struct StageShape {
@@ -130,7 +132,7 @@ struct StageShape {
     static_assert(!MIRROR || ZS >= 8, "halves of 8 and 4 voxels");
     static constexpr int boxes = MIRROR ? 2 : 1;                        // per view
     static constexpr int height = ZS / boxes;                           // voxels of a box
-    static constexpr int rows = MIRROR ? (ZS == 16 ? 20 : 16) : ZS == 16 ? 37 : ZS == 8 ? 26 : 16;  // rows of a box
+    static constexpr int rows = MIRROR ? (ZS == 16 ? 20 : 16) : ZS == 16 ? 37 : ZS == 8 ? 26 : 20;  // rows of a box
     static constexpr int views = ZS == 16 ? 1 : ZS == 8 ? 2 : 4;        // views between two barriers
     static constexpr int pieces = (rows * kStagePitch + 255) / 256;     // of a box
     static constexpr int taps = pieces * 256;                           // floats per box
@@ -282,9 +284,18 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     constexpr int H = SS::height, B = SS::boxes;
     constexpr int NT = SX * SY;
     constexpr int NW = NT / 64;                             // waves per workgroup
-    constexpr int kSlots = (SS::rows + NW - 1) / NW;        // box rows per wave at most
+    // Waves that copy a box together.  A copy's branches and resources cost each of
+    // them the same, so the boxes of short columns, whose waves are alone or two on a
+    // SIMD, are dealt out to the waves; all four on each box: 64^3 and 180 views 97 us,
+    // dealt out 86; 40^3 and 48 views 28.4 and 25.1; 80^3 and 64 views 43 and 38; at 8
+    // voxels 96^3 and 96 views 75 and 73, 128^3 and 180 views 189 and 185.  At 16 the
+    // copies are spread over more waves: 512^3 19.8 ms, FDK 256^3 dealt out 1% slower.
+    constexpr int CW = ZS == 16 ? NW : NW / (SS::views * B);
+    static_assert(CW == NW || CW * SS::views * B == NW, "a wave copies for one box");
+    constexpr int kSlots = (SS::rows + CW - 1) / CW;        // box rows per wave at most
     const int tid = threadIdx.x;
     const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int cw = wv % CW;
     // wave wv covers columns x in [8 wv, 8 wv + 8), y in [0, 8)
     const int i = bx * SX + wv * 8 + (lane & 7);
     const int j = by * SY + (lane >> 3);
@@ -321,11 +332,11 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     const uint32_t view_bytes = (uint32_t)(plane * sizeof(float));
     // Byte offset in the view of a lane's four taps of the wave's q-th piece, from
     // the box's first: word w of the buffer is tap (w / pitch, w mod pitch).
-    constexpr int kPieces = (SS::pieces + NW - 1) / NW;
+    constexpr int kPieces = (SS::pieces + CW - 1) / CW;
     uint32_t piece[kPieces];
 #pragma unroll
     for (int q = 0; q < kPieces; ++q) {
-        const int w = 256 * (wv + q * NW) + 4 * lane, row = w / kStagePitch;
+        const int w = 256 * (cw + q * CW) + 4 * lane, row = w / kStagePitch;
         piece[q] = (uint32_t)(row * rl + (w - row * kStagePitch)) * 4u;
     }
     // Copy of a box of view p into buffer b, straight from memory into LDS
@@ -334,8 +345,8 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     // that nothing reads.  One 16-byte load per lane brings 3.4 rows; by rows, a
     // 4-byte load each, the copies kept the data return 80% busy at 512^3.
     //
-    // Boxes at the detector's left and right ends go by rows: wave wv copies box
-    // rows wv + q NW, lane l column l, each row read through a buffer resource of
+    // Boxes at the detector's left and right ends go by rows: wave cw copies box
+    // rows cw + q CW, lane l column l, each row read through a buffer resource of
     // that detector row (of no bytes for a row off the detector), so that a tap
     // off the row reads past the resource's end.
     auto copy_box = [&](const StagePlan& s, int p, int b) {
@@ -347,9 +358,9 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
             const int words = s.rows * kStagePitch;
 #pragma unroll
             for (int q = 0; q < kPieces; ++q)
-                if (256 * (wv + q * NW) < words)
+                if (256 * (cw + q * CW) < words)
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                        rr, (__attribute__((address_space(3))) void*)(dst + 256 * (wv + q * NW)), 16,
+                        rr, (__attribute__((address_space(3))) void*)(dst + 256 * (cw + q * CW)), 16,
                         (int)(at + piece[q]), 0, 0, 0);
             return;
         }
@@ -357,13 +368,13 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
         const uint32_t loff = (uint32_t)(s.u0 + lane) * 4u;
 #pragma unroll
         for (int q = 0; q < kSlots; ++q) {
-            if (wv + q * NW < s.rows) {
-                const int v = s.v0 + wv + q * NW;
+            if (cw + q * CW < s.rows) {
+                const int v = s.v0 + cw + q * CW;
                 const bool vin = (unsigned)v < (unsigned)nv;
                 const __amdgpu_buffer_rsrc_t rr =
                     buffer_rsrc(view + (size_t)(vin ? v : 0) * rl, vin ? (uint32_t)rl * 4u : 0u);
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    rr, (__attribute__((address_space(3))) void*)(dst + (wv + q * NW) * kStagePitch), 4, loff, 0, 0, 0);
+                    rr, (__attribute__((address_space(3))) void*)(dst + (cw + q * CW) * kStagePitch), 4, loff, 0, 0, 0);
             }
         }
     };
@@ -400,9 +411,13 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
                 r.v0[t][b] = s.v0;
                 if (p + t < g.nphi) {
                     if (s.rows == 0) r.rows = 0;
-                    copy_box(s, p + t, (half * G + t) * B + b);
+                    if (CW == NW) copy_box(s, p + t, (half * G + t) * B + b);
                 }
             }
+        if (CW < NW) {
+            const int box = wv / CW, t = box / B;
+            if (p + t < g.nphi) copy_box(box % B ? plan_of(p + t, B - 1) : plan_of(p + t, 0), p + t, half * G * B + box);
+        }
         return r;
     };
     auto view_terms = [&](int p) {
@@ -898,9 +913,9 @@ static hipError_t launch_vi_staged(const DevGeom& d, int fdk, const float* sino,
         // Columns of 16 voxels share a column-view's terms best; below two or three
         // workgroups per CU the views' latency decides, and shorter columns are more
         // workgroups that wait for several views at once.  VI, us at 4 / 8 / 16
-        // voxels by workgroups of 16: 64 (64^3, 64 views) 39 / 50 / 75; 150 (80^3)
-        // 58 / 62 / 93; 216 (96^3) 80 / 77 / 112; 512 (128^3, 180 views) 270 / 191 /
-        // 217; 765 (136^3) 272 / 220 / 203; 1000 (160^3, 180 views) 464 / 342 / 287.
+        // voxels by workgroups of 16: 64 (64^3, 64 views) 32 / 48 / 73; 150 (80^3, 64)
+        // 39 / 48 / 73; 216 (96^3, 64) 57 / 49 / 73; 512 (128^3, 180 views) 279 / 186 /
+        // 214; 765 (136^3, 96) 204 / 155 / 142; 1000 (160^3, 180) 487 / 335 / 281.
         const size_t tiles = (size_t)ntx * nty * ceil_div(d.nz, kViTileZ);
         const int zs = tiles < 192 ? 4 : tiles < 640 ? 8 : 16;
         const ViBox* bt = (const ViBox*)boxes;
