@@ -199,17 +199,18 @@ __global__ __launch_bounds__(SX* SY) void vi_box_kernel(DevGeom g, ViBox* __rest
 }
 
 // Per-view staging plan of a workgroup: the box of taps (rows from v0,
-// columns from u0), no rows where it does not fit the buffer.  Wave w copies box
-// rows w, w + 4, ..., one column per lane, so a box is at most 64 columns wide.
+// columns from u0), no rows where it does not fit the buffer.  Boxes at the detector's
+// ends are copied one column per lane, so a box is at most 64 columns wide.
 // Each lane makes the plan of one of 64 views, which the wave then reads lane by
 // lane: made by every lane for every view it was an eighth of the instructions.
 struct StagePlan {
     int u0, v0, rows;
     bool quads;  // 16-byte loads: no tap of the box is off the detector's left or right end
+    bool near;   // 32-bit offsets in the view of the box's rows off the detector do not come round to it
 };
 
 // The box rows from the four (z', A) corners; v0 and the number of rows as v0 * 256
-// + rows, 0 where the box does not fit.
+// + rows and the flags, 0 where the box does not fit.
 template <typename SS>
 __device__ __forceinline__ int stage_rows(const ViBox& bb, float zp0, float cv, int rl, int nv) {
     const float zp1 = zp0 + (float)(SS::height - 1);
@@ -219,11 +220,11 @@ __device__ __forceinline__ int stage_rows(const ViBox& bb, float zp0, float cv, 
     const float vhi = floorf(fmaxf(fmaxf(va, vb), fmaxf(vc, vd)));
     const bool fits = vlo >= -32768.0f && vhi <= 32768.0f && vhi - vlo + 2.0f <= (float)SS::rows &&
                       bb.u1 - bb.u0 + 2 <= 64;
-    // a lane's four taps start at a tap of the box and end on its row; the 32-bit
-    // offsets of rows off the detector do not come round to it
-    const bool quads = bb.u0 >= 0 && bb.u1 + 1 + 3 < rl && (int)vlo >= -64 && (int)vlo <= nv &&
-                       (uint64_t)(nv + 128) * (uint32_t)rl < (1u << 29);
-    return fits ? (int)vlo * 256 + (quads ? 128 : 0) + (int)(vhi - vlo) + 2 : 0;
+    static_assert(SS::rows < 64, "rows below the flags");
+    const bool near = (int)vlo >= -64 && (int)vlo <= nv && (uint64_t)(nv + 128) * (uint32_t)rl < (1u << 29);
+    // a lane's four taps start at a tap of the box and end on its row
+    const bool quads = near && bb.u0 >= 0 && bb.u1 + 1 + 3 < rl;
+    return fits ? (int)vlo * 256 + (quads ? 128 : 0) + (near ? 64 : 0) + (int)(vhi - vlo) + 2 : 0;
 }
 
 // FP16 u-weights (1 - w, w) of a column-view, w = fu rounded to a multiple of
@@ -287,7 +288,7 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     // Waves that copy a box together.  A copy's branches and resources cost each of
     // them the same, so the boxes of short columns, whose waves are alone or two on a
     // SIMD, are dealt out to the waves; all four on each box: 64^3 and 180 views 97 us,
-    // dealt out 86; 40^3 and 48 views 28.4 and 25.1; 80^3 and 64 views 43 and 38; at 8
+    // dealt out 87; 40^3 and 48 views 28.4 and 25.1; 80^3 and 64 views 43 and 38; at 8
     // voxels 96^3 and 96 views 75 and 73, 128^3 and 180 views 189 and 185.  At 16 the
     // copies are spread over more waves: 512^3 19.8 ms, FDK 256^3 dealt out 1% slower.
     constexpr int CW = ZS == 16 ? NW : NW / (SS::views * B);
@@ -346,9 +347,11 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     // 4-byte load each, the copies kept the data return 80% busy at 512^3.
     //
     // Boxes at the detector's left and right ends go by rows: wave cw copies box
-    // rows cw + q CW, lane l column l, each row read through a buffer resource of
-    // that detector row (of no bytes for a row off the detector), so that a tap
-    // off the row reads past the resource's end.
+    // rows cw + q CW, lane l column l; lanes off the detector read past the view's
+    // bytes.  Far from the detector, or on one past 2^29 taps, each row is read
+    // through a buffer resource of that detector row (of no bytes for a row off the
+    // detector), which takes some 20 instructions a row instead of 5: 64^3 and 180
+    // views 90 us, 85 through the view's; 128^3 and 180 views 185 and 182.
     auto copy_box = [&](const StagePlan& s, int p, int b) {
         const float* view = sino + (size_t)p * plane;
         float* dst = stage + b * SS::taps;
@@ -364,9 +367,24 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
                         (int)(at + piece[q]), 0, 0, 0);
             return;
         }
+        if (s.near) {
+            // a lane off the detector's columns starts 2^31 bytes on, past the view's end
+            const int u = s.u0 + lane;
+            uint32_t off = (unsigned)u < (unsigned)rl ? (uint32_t)(s.v0 * rl + u) * 4u : 0x80000000u;
+            off += (uint32_t)(cw * rl) * 4u;
+            const __amdgpu_buffer_rsrc_t rr = buffer_rsrc(view, view_bytes);
+#pragma unroll
+            for (int q = 0; q < kSlots; ++q) {
+                if (cw + q * CW < s.rows)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                        rr, (__attribute__((address_space(3))) void*)(dst + (cw + q * CW) * kStagePitch), 4, off, 0, 0, 0);
+                off += (uint32_t)(CW * rl) * 4u;
+            }
+            return;
+        }
         // past the row's end unless 0 <= u < nu (FP32) or the pair index u + 1 <= nu
         const uint32_t loff = (uint32_t)(s.u0 + lane) * 4u;
-#pragma unroll
+#pragma clang loop unroll(disable)
         for (int q = 0; q < kSlots; ++q) {
             if (cw + q * CW < s.rows) {
                 const int v = s.v0 + cw + q * CW;
@@ -381,7 +399,7 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
     int plan_u0[B] = {}, plan_v[B] = {};  // of view (p & ~63) + lane
     auto plan_of = [&](int p, int b) {
         const int v = __builtin_amdgcn_readlane(plan_v[b], p & 63);
-        return StagePlan{__builtin_amdgcn_readlane(plan_u0[b], p & 63), v >> 8, v & 127, (v & 128) != 0};
+        return StagePlan{__builtin_amdgcn_readlane(plan_u0[b], p & 63), v >> 8, v & 63, (v & 128) != 0, (v & 64) != 0};
     };
     // Plans and copies of the group of G views from p on; rows is 0 if one of its
     // boxes does not fit, and all of the group's taps are then read directly.
@@ -406,7 +424,7 @@ __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __
         for (int t = 0; t < G; ++t)
 #pragma unroll
             for (int b = 0; b < B; ++b) {
-                const StagePlan s = p + t < g.nphi ? plan_of(p + t, b) : StagePlan{0, 0, 0, false};
+                const StagePlan s = p + t < g.nphi ? plan_of(p + t, b) : StagePlan{0, 0, 0, false, false};
                 r.u0[t][b] = s.u0;
                 r.v0[t][b] = s.v0;
                 if (p + t < g.nphi) {
