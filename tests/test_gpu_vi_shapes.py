@@ -25,6 +25,7 @@ pytestmark = pytest.mark.gpu
     (137, 136, 130, 139, 133, 65, 2.0, 2.0), (130, 150, 150, 300, 200, 9, 2.0, 2.0),                        # 16
     (64, 64, 40, 200, 200, 6, 0.4, 2.0), (96, 96, 90, 400, 300, 5, 0.5, 2.0),  # boxes past the buffers
     (40, 40, 30, 24, 24, 21, 9.0, 2.0), (48, 40, 30, 1, 1, 5, 3.0, 2.0),       # many voxels a tap; one tap
+    (40, 40, 200, 50, 5, 9, 2.0, 2.0), (90, 96, 260, 70, 9, 6, 2.0, 2.0),      # boxes more than 64 rows off the detector
     (64, 60, 50, 60, 50, 40, 2.0, 0.6),                                        # a source within the square
 ])
 def test_vi_shapes(ctx, nx, ny, nz, nu, nv, nphi, pixel, fod, fdk, dt):
