@@ -1,0 +1,52 @@
+"""GPU: the transposes on acquisitions other than 1 mm voxels and a detector at
+twice the source's distance, against the FP64-accumulating oracle (rel-L2 <=
+1e-6: FP32 sums of at most a few thousand terms of one sign, each within a few
+1e-7 of the oracle's).
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle_ffi import Geometry, Oracle
+from test_gpu_parity import dev, rel_l2, to_desc
+from tomogpi_amd import lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _geom(nx, ny, nz, nu, nv, nphi, pixel=2.0, fod=2.0, fdd=2.0, voxel=1.0, start=1.0 / 7.0, stop=1.875):
+    """pixel in voxels at the detector, fod in volume widths, fdd in fod."""
+    return Geometry(fod=fod * nx * voxel, fdd=fdd * fod * nx * voxel, nphi=nphi, su=nu * pixel * voxel,
+                    sv=nv * pixel * voxel, nu=nu, nv=nv, sx=nx * voxel, sy=ny * voxel, sz=nz * voxel, nx=nx, ny=ny, nz=nz,
+                    num_start=start, den_start=1.0, num_stop=stop, den_stop=1.0)
+
+
+def _check(ctx, g, op, cube=False):
+    print(f"[case] {op} {g.nx} {g.ny} {g.nz} / {g.nu} {g.nv} {g.nphi} fdd/fod {g.fdd / g.fod:.3g} voxel {g.sx / g.nx:.3g}",
+          flush=True)
+    G, o = lib.Geometry(ctx, to_desc(g)), Oracle(g)
+    try:
+        rng = np.random.default_rng(g.nz)
+        if op == "vi":
+            x = rng.random(g.vol_shape, dtype=np.float32)
+            ref, out = o.vi_T(x), torch.full(g.sino_shape, np.nan, dtype=torch.float32, device="cuda")
+            G.backproject_adjoint(dev(x), out)
+        else:
+            y = rng.random(g.sino_shape, dtype=np.float32)
+            ref = o.siddon_T(y) if op == "siddon" else o.rs_T(y, cube=cube)
+            out = torch.full(g.vol_shape, np.nan, dtype=torch.float32, device="cuda")
+            G.project_adjoint(dev(y), out, lib.PROJ_SIDDON if op == "siddon" else lib.PROJ_RS,
+                              lib.FLAG_RS_FOV_CUBE if cube else 0)
+        assert rel_l2(out.cpu().numpy(), ref) <= 1e-6
+    finally:
+        G.close()
+
+
+@pytest.mark.parametrize("voxel", [0.1, 0.4, 0.55, 0.8, 1.1])
+@pytest.mark.parametrize("nx,ny,nz,nu,nv,nphi", [(30, 31, 64, 40, 41, 65), (16, 16, 130, 24, 35, 40), (31, 30, 63, 40, 41, 30)])
+@pytest.mark.parametrize("op", ["siddon", "vi", "rs"])
+def test_voxel_size(ctx, op, nx, ny, nz, nu, nv, nphi, voxel):
+    """Voxel sizes whose products round.  An odd number of rows over an even number of
+    slices: the middle row's rays run along the plane between two slices and
+    belong to the upper one alone."""
+    _check(ctx, _geom(nx, ny, nz, nu, nv, nphi, voxel=voxel), op)

@@ -948,7 +948,7 @@ __global__ __launch_bounds__(64 * kSidTWaves, 8) void siddon_t_kernel(DevGeom g,
                 const int most_rows = __builtin_amdgcn_readlane(rows, l), ml = __builtin_amdgcn_readlane(m, l);
                 const float* col = gt + ((size_t)(pb + l) * nu + ml) * pitch + kSidTPad;
                 const float stepf = (float)step;
-float nf[K];
+                float nf[K];
 #pragma unroll
                 for (int c = 0; c < K; ++c) {
                     // first row that can reach the voxel
@@ -974,8 +974,11 @@ float nf[K];
                         float z0 = (float)fma(step, (double)(nf[c] - cvf), -zl);
                         auto row = [&](float gn, bool first) __attribute__((always_inline)) {
                             if (TIE && !first) z0 = (float)fma(step, (double)(nf[c] - cvf), -zl);
-                            const float t = (nf[c] - cvf) * dvf + 1e-30f;
-                            const float rt = __builtin_amdgcn_rcpf(t);
+                            const float t = (nf[c] - cvf) * dvf;
+                            // The middle row, t = 0, crosses no plane: a height of h ends h 2^100
+                            // away.  TIE: a and b are then exact (a power of two), so that the
+                            // lower slice's upper plane, at the row's height, ends at 0.
+                            const float rt = TIE && t == 0.0f ? 0x1p100f : __builtin_amdgcn_rcpf(t + 1e-30f);
                             // where the row crosses the voxel's planes, from tau0
                             const float a = -z0 * rt, b = fmaf(dlf, rt, a);
                             const float in = fminf(fmaxf(a, b), dt) - fmaxf(fminf(a, b), 0.0f);
