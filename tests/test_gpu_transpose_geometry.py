@@ -50,3 +50,12 @@ def test_voxel_size(ctx, op, nx, ny, nz, nu, nv, nphi, voxel):
     slices: the middle row's rays run along the plane between two slices and
     belong to the upper one alone."""
     _check(ctx, _geom(nx, ny, nz, nu, nv, nphi, voxel=voxel), op)
+
+
+@pytest.mark.parametrize("fdd", [1.05, 1.2, 1.5])
+@pytest.mark.parametrize("nx,ny,nz,nu,nv,nphi", [(30, 30, 30, 46, 46, 24), (24, 40, 33, 60, 40, 30), (40, 20, 24, 60, 33, 24)])
+@pytest.mark.parametrize("op", ["siddon", "vi", "rs", "rs_cube"])
+def test_detector_inside(ctx, op, nx, ny, nz, nu, nv, nphi, fdd):
+    """A detector plane inside the volume (a virtual detector near the isocentre):
+    the rays go on behind it, as the projector's."""
+    _check(ctx, _geom(nx, ny, nz, nu, nv, nphi, pixel=0.8 * fdd, fdd=fdd), op.split("_")[0], cube=op == "rs_cube")

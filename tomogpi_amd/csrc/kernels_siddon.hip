@@ -900,7 +900,9 @@ __global__ __launch_bounds__(64 * kSidTWaves, 8) void siddon_t_kernel(DevGeom g,
                 const double s = ((double)m - (double)g.cu) * (double)g.du;
                 const double rx = ca * g.fdd - s * sa, ry = sa * g.fdd + s * ca;
                 const double Sx = -g.fod * ca, Sy = -g.fod * sa;
-                double t0 = 0.0, t1 = 1.0;
+                // from the source on; the ray does not end at its detector cell, which may lie
+                // inside the volume (fdd < fod + Rm)
+                double t0 = 0.0, t1 = inf;
                 const double a = rx * rx + ry * ry, b = Sx * rx + Sy * ry, disc = b * b - a * ((Sx * Sx + Sy * Sy) - Rm * Rm);
                 bool ok = disc > 0.0;
                 if (cut && ok) {
