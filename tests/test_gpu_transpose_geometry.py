@@ -59,3 +59,13 @@ def test_detector_inside(ctx, op, nx, ny, nz, nu, nv, nphi, fdd):
     """A detector plane inside the volume (a virtual detector near the isocentre):
     the rays go on behind it, as the projector's."""
     _check(ctx, _geom(nx, ny, nz, nu, nv, nphi, pixel=0.8 * fdd, fdd=fdd), op.split("_")[0], cube=op == "rs_cube")
+
+
+@pytest.mark.parametrize("nx,ny,nz,nv", [(32, 32, 24, 40), (30, 28, 33, 41), (64, 64, 20, 33), (31, 32, 24, 40), (128, 128, 6, 9)])
+@pytest.mark.parametrize("voxel", [1.0, 0.55])
+def test_siddon_rays_along_planes(ctx, nx, ny, nz, nv, voxel):
+    """An odd number of detector columns over an even number of voxels: in the views
+    along the axes the middle column's rays run along a plane between voxels, up
+    to the rounding of the view's cosine, and belong to the voxels that the
+    projector gives them to."""
+    _check(ctx, _geom(nx, ny, nz, 41 if nx < 64 else 2 * (nx // 2) + 1, nv, 24, voxel=voxel, start=0.0, stop=2.0), "siddon")

@@ -821,6 +821,29 @@ __global__ __launch_bounds__(256) void siddon_t_prepare_kernel(DevGeom g, const 
         }
 }
 
+// A detector column's line along an axis (its direction's other component r is 0 but
+// for the rounding of the view's cosine or sine) has one coordinate there, S + tau
+// r at the isocentre.  Where that lies on a plane between two voxels, which of them
+// the rays belong to follows from the rounding of the projector's own setup, ray by
+// ray: they are left to the per-ray traversal.  kSidBetween: how near, in voxels; more
+// than such a line drifts on its way, less than any other lies off a plane.
+constexpr double kSidBetween = 1e-5;
+__host__ __device__ inline bool sid_line_flat(const DevGeom& g, double r) { return fabs(r) < 1e-9 * g.fdd; }
+__host__ __device__ inline double sid_line_at(const DevGeom& g, double S, double r) { return S + g.fod / g.fdd * r; }
+// The detector column whose line runs between two rows of voxels in a view, along
+// y (x = 0) or x (x = 1), -1 where none does.
+__host__ __device__ inline int sid_between_column(const DevGeom& g, const double* vw, int x) {
+    const double ca = vw[0], sa = vw[1];
+    const double at = rint((x ? -sa / ca : ca / sa) * g.fdd / (double)g.du + (double)g.cu);
+    if (!(at >= 0.0 && at < (double)g.nu)) return -1;
+    const double s = (at - (double)g.cu) * (double)g.du;
+    const double r = x ? sa * g.fdd + s * ca : ca * g.fdd - s * sa;
+    if (!sid_line_flat(g, r)) return -1;
+    const double pos = sid_line_at(g, x ? -g.fod * sa : -g.fod * ca, r) / (double)g.delta + (double)(x ? g.cy : g.cx) + 0.5;
+    const double plane = rint(pos);
+    return plane >= 1.0 && plane < (double)(x ? g.ny : g.nx) && fabs(pos - plane) <= kSidBetween ? (int)at : -1;
+}
+
 __device__ __forceinline__ double read_lane(double v, int l) {
     const uint64_t b = __builtin_bit_cast(uint64_t, v);
     const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, l);
@@ -910,19 +933,18 @@ __global__ __launch_bounds__(64 * kSidTWaves, 8) void siddon_t_kernel(DevGeom g,
                     t0 = (-b - sq) / a;
                     t1 = (-b + sq) / a;
                 }
-                // A line along an axis keeps its voxel index on the other one,
-                // floor(position + 1/2) where it enters, as the projector's.
-                const double flat = 1e-9 * g.fdd;
-                if (fabs(rx) < flat) {
-                    ok = ok && floor((Sx + t0 * rx) / dl + (double)g.cx + 0.5) == (double)i;
+                // a line along an axis stays in one row of voxels (kSidBetween)
+                if (sid_line_flat(g, rx)) {
+                    const double at = sid_line_at(g, Sx, rx);
+                    ok = ok && at - xa > kSidBetween * dl && xb - at > kSidBetween * dl;
                 } else {
                     const double c0 = (xa - Sx) / rx, c1 = (xb - Sx) / rx;
                     t0 = fmax(t0, fmin(c0, c1));
                     t1 = fmin(t1, fmax(c0, c1));
                 }
-                if (fabs(ry) < flat) {
-                    const double at = floor((Sy + t0 * ry) / dl + (double)g.cy + 0.5);
-                    ok = ok && fmin(fmax(at, 0.0), (double)(g.ny - 1)) == (double)j;
+                if (sid_line_flat(g, ry)) {
+                    const double at = sid_line_at(g, Sy, ry);
+                    ok = ok && at - ylo > kSidBetween * dl && yhi - at > kSidBetween * dl;
                 } else {
                     const double c0 = ((ry > 0.0 ? ylo : ya) - Sy) / ry, c1 = ((ry < 0.0 ? yhi : yb) - Sy) / ry;
                     t0 = fmax(t0, fmin(c0, c1));
@@ -1011,6 +1033,20 @@ __global__ __launch_bounds__(64 * kSidTWaves, 8) void siddon_t_kernel(DevGeom g,
             *o = add ? *o + acc[c] : acc[c];
         }
     }
+}
+
+// The rays that siddon_t_kernel leaves out, one per thread, added to vol.  Grid: x =
+// view, y = row block, z = axis (sid_between_column).
+template <typename TS>
+__global__ __launch_bounds__(64) void siddon_t_between_kernel(DevGeom g, const TS* __restrict__ sino, float sino_inv,
+                                                            float* __restrict__ vol) {
+    const int p = blockIdx.x, n = (int)blockIdx.y * 64 + threadIdx.x;
+    const int m = sid_between_column(g, g.view + (size_t)p * kViewStride, blockIdx.z);
+    if (m < 0 || n >= g.nv) return;
+    const float gv = Storage<TS>::load(sino, (size_t)m + (size_t)g.nu * ((size_t)n + (size_t)g.nv * p), sino_inv);
+    if (gv == 0.0f) return;
+    const SidRay r = sid_setup(g, p, m, n);
+    if (r.ok) sid_trace<1>(g, r, vol, gv, nullptr);
 }
 
 template <typename TS>
@@ -1247,6 +1283,16 @@ int launch_siddon_adjoint(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t 
                 case 3: launch_siddon_t<3>(d, gt, p0, np, (float*)vol.p, s); break;
                 default: launch_siddon_t<4>(d, gt, p0, np, (float*)vol.p, s); break;
             }
+            e = hipGetLastError();
+        }
+        bool between = false;
+        for (int p = 0; p < d.nphi && !between; ++p)
+            for (int x = 0; x < 2; ++x) between |= sid_between_column(d, g->view.data() + (size_t)p * kViewStride, x) >= 0;
+        if (between && e == hipSuccess) {
+            TOMO_DISPATCH_STORAGE(sino.dtype, TS, {
+                hipLaunchKernelGGL((siddon_t_between_kernel<TS>), dim3(d.nphi, ceil_div(d.nv, 64), 2), dim3(64), 0, s, d,
+                                   (const TS*)sino.p, inv, (float*)vol.p);
+            });
             e = hipGetLastError();
         }
         const hipError_t f = hipFreeAsync(gt, s);
