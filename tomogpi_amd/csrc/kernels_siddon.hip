@@ -243,6 +243,7 @@ constexpr uint32_t kSidOutside = 0xfffffff0u;
 template <typename TV, bool BUF> struct ColumnReader {
     static constexpr uint32_t kUnit = BUF ? 4u : 1u;
     static constexpr uint32_t kIdle = BUF ? kSidOutside : 0u;
+    static constexpr bool kZeroIdle = BUF;
     __amdgpu_buffer_rsrc_t r;
     const uint32_t* p;
     __device__ __forceinline__ float2 operator()(uint32_t o) const {
@@ -279,14 +280,17 @@ __device__ __forceinline__ float sid_walk_columns(const ColumnRay& r, const CR& 
     float tx = r.fx, ty = r.fy, tz = r.fz, k = 0.0f, cx = 0.0f, cz = 0.0f, t = 0.0f, acc = 0.0f;
     uint32_t e = r.e;
     // A lane past its last cell has t = tmax: every later time lies at tmax or
-    // beyond, so its segments have no length, and its loads go to kIdle.
+    // beyond, so its segments have no length, and its loads go to kIdle, which
+    // reads 0 (by index: a voxel, which is masked).
     struct Cell {
         float d1, d2;
         float2 v;
     };
     auto next = [&]() __attribute__((always_inline)) {
         Cell c;
-        c.v = rd(t < r.tmax ? e : CR::kIdle);
+        const bool live = t < r.tmax;
+        c.v = rd(live ? e : CR::kIdle);
+        if constexpr (!CR::kZeroIdle) c.v = live ? c.v : make_float2(0.0f, 0.0f);
         const float te = min_nn(min_nn(tx, ty), r.tmax);
         const float c1 = min_nn(tz, te);
         c.d1 = c1 - t;
@@ -394,7 +398,12 @@ __device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __
         if (!any_down) acc = sid_walk_columns<0>(w, rd, trips);
         else if (!any_up) acc = sid_walk_columns<1>(w, rd, trips);
         else acc = sid_walk_columns<2>(w, rd, trips);
-    } else {
+    }
+    // A segment of no length takes its voxel times 0, which is not 0 where the voxel
+    // is not finite: a sum that is not is taken again by the general step, which
+    // reads the voxels on the ray only.
+    const bool step = ok && (!walk || !__builtin_isfinite(acc));
+    if (__ballot(step) != 0ull) {
         SidState s;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -409,12 +418,12 @@ __device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __
         s.dlin[2] = (uint32_t)r.step[2] * u;
         s.t = 0.0f;
         s.acc = 0.0f;
-        s.live = ok;
+        s.live = step;
         // Every step moves one axis toward the grid exit that bounds tmax;
         // the cap only bounds the loop.
         int guard = g.nx + ny + nz + 4;
         while (s.live && guard-- > 0) sid_step(s, r, [&](unsigned o) { return rd.one(o); });
-        acc = s.acc;
+        if (step) acc = s.acc;
     }
     // 16-bit volumes are read unscaled; the sum is linear in them, so the
     // storage scale applies once here (FP32 storage has no scale).
