@@ -69,3 +69,12 @@ def test_siddon_rays_along_planes(ctx, nx, ny, nz, nv, voxel):
     to the rounding of the view's cosine, and belong to the voxels that the
     projector gives them to."""
     _check(ctx, _geom(nx, ny, nz, 41 if nx < 64 else 2 * (nx // 2) + 1, nv, 24, voxel=voxel, start=0.0, stop=2.0), "siddon")
+
+
+@pytest.mark.parametrize("nx,ny,nz,nu,nv,nphi,pixel", [
+    (20, 20, 20, 90, 5, 12, 0.3), (24, 24, 2, 30, 8, 20, 0.25), (20, 20, 130, 60, 3, 16, 0.5), (24, 20, 70, 300, 1, 16, 0.1),
+])
+@pytest.mark.parametrize("op", ["siddon", "vi", "rs", "rs_cube"])
+def test_few_fine_rows(ctx, op, nx, ny, nz, nu, nv, nphi, pixel):
+    """Fewer detector rows than pass one voxel."""
+    _check(ctx, _geom(nx, ny, nz, nu, nv, nphi, pixel=pixel), op.split("_")[0], cube=op == "rs_cube")

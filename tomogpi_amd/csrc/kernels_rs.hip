@@ -828,7 +828,8 @@ __global__ __launch_bounds__(64 * kRsTWaves, 6) void rs_t_kernel(DevGeom g, int 
 #pragma unroll
                     for (int b = 0; b < B; ++b) part[b][c] = 0.0f;
                     const float k0 = kk[c] - 1.0f;
-                    row[c] = ceilf(fminf(k0 * i0, k0 * i1) + (cv - 2e-3f));  // first that may reach the voxel
+                    // first that may reach the voxel; -1 before the detector, whose rows R covers
+                    row[c] = fmaxf(ceilf(fminf(k0 * i0, k0 * i1) + (cv - 2e-3f)), -1.0f);
                 }
                 for (int r = 0; r < R; ++r) {
                     typedef float V4 __attribute__((ext_vector_type(4)));
