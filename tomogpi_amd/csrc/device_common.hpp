@@ -130,6 +130,15 @@ inline bool stream_captures(hipStream_t s) {
 }
 inline unsigned ceil_div(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
 
+// A grid of `tiles` workgroups of `threads` in x and, where that would be 2^32 work
+// items or more, which HIP refuses, in y; `z` of them.  The last row may hold tiles
+// past the end.
+inline dim3 tile_grid(size_t tiles, unsigned threads, unsigned z = 1) {
+    const unsigned y = ceil_div(tiles * threads, 0xffffffffu);
+    return dim3(ceil_div(tiles, y), y, z);
+}
+__device__ __forceinline__ uint32_t tile_index() { return blockIdx.x + gridDim.x * blockIdx.y; }
+
 // Dispatch a templated launcher on a TOMO_F32/F16/BF16 code.
 #define TOMO_DISPATCH_STORAGE(code, T, ...)                        \
     switch (code) {                                                \

@@ -734,15 +734,16 @@ __device__ __forceinline__ float lane_value(float v, int l) {
 // whose samples lie on the mirrored rows with the same weights; the rays' values and
 // numbers of samples are the mirrored rows' own.
 //
-// Grid: x = (4 voxel columns along x, y), y = z block of 64 K.  Views p0 + [0, np).
+// Grid: x, y = (4 voxel columns along x, j), z = z block of 64 K.  Views p0 + [0, np).
 template <int K, bool MIRROR>
 __global__ __launch_bounds__(64 * kRsTWaves, 6) void rs_t_kernel(DevGeom g, int cube, const float4* __restrict__ tab, int p0,
                                                              int np, int add, float* __restrict__ vol) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t gx = (uint32_t)(g.nx + kRsTWaves - 1) / kRsTWaves;
-    const int i = (int)(blockIdx.x % gx) * kRsTWaves + wv, j = (int)(blockIdx.x / gx);
-    if (i >= g.nx) return;
-    const int kb = (int)blockIdx.y * 64 * K;
+    const uint32_t tile = tile_index();
+    const int i = (int)(tile % gx) * kRsTWaves + wv, j = (int)(tile / gx);
+    if (i >= g.nx || j >= g.ny) return;
+    const int kb = (int)blockIdx.z * 64 * K;
     const int rows = (int)rs_t_rows(g.nv);
     const double dl = (double)g.delta, fod = g.fod / dl;
     const double xi = (double)i - (double)g.cx, yj = (double)j - (double)g.cy;
@@ -1000,7 +1001,8 @@ static bool rs_t_gathers(const DevGeom& d) {
 
 template <int K, bool MIRROR>
 static void launch_rs_t(const DevGeom& d, int cube, const float4* tab, int p0, int np, float* vol, hipStream_t s) {
-    const dim3 grid(ceil_div(d.nx, kRsTWaves) * (unsigned)d.ny, ceil_div(MIRROR ? (d.nz + 1) / 2 : d.nz, 64 * K));
+    const dim3 grid = tile_grid((size_t)ceil_div(d.nx, kRsTWaves) * d.ny, 64 * kRsTWaves,
+                                ceil_div(MIRROR ? (d.nz + 1) / 2 : d.nz, 64 * K));
     hipLaunchKernelGGL((rs_t_kernel<K, MIRROR>), grid, dim3(64 * kRsTWaves), 0, s, d, cube, tab, p0, np, p0 > 0, vol);
 }
 

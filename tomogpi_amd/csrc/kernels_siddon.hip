@@ -863,8 +863,8 @@ __device__ __forceinline__ float read_lane(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// views: the np views of `gt`, from view p0; add: to what vol holds.  Grid: x =
-// (column group, j), y = z block of 64 K voxels.  TIE: an odd number of detector
+// views: the np views of `gt`, from view p0; add: to what vol holds.  Grid: x, y =
+// (column group, j), z = z block of 64 K voxels.  TIE: an odd number of detector
 // rows over an even number of slices: the middle row's rays run along the plane
 // between two slices, and belong to the upper one, as the projector's; its height
 // is then taken exactly at each row instead of carried on from the first.
@@ -873,9 +873,10 @@ __global__ __launch_bounds__(64 * kSidTWaves, 8) void siddon_t_kernel(DevGeom g,
                                                                    int np, int add, float* __restrict__ vol) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t gx = (uint32_t)(g.nx + kSidTWaves - 1) / kSidTWaves;
-    const int i = (int)(blockIdx.x % gx) * kSidTWaves + wv, j = (int)(blockIdx.x / gx);
-    if (i >= g.nx) return;
-    const int kb = (int)blockIdx.y * 64 * K;
+    const uint32_t tile = tile_index();
+    const int i = (int)(tile % gx) * kSidTWaves + wv, j = (int)(tile / gx);
+    if (i >= g.nx || j >= g.ny) return;
+    const int kb = (int)blockIdx.z * 64 * K;
     const double dl = (double)g.delta, inf = __builtin_inf();
     // The voxel column's cell in the plane (mm).  The cylinder may be wider than
     // the grid in y (ny < nx): a ray that comes from outside walks along the
@@ -1253,7 +1254,7 @@ static bool sid_t_gathers(const DevGeom& d) {
 
 template <int K>
 static void launch_siddon_t(const DevGeom& d, const float* gt, int p0, int np, float* vol, hipStream_t s) {
-    const dim3 grid(ceil_div(d.nx, kSidTWaves) * (unsigned)d.ny, ceil_div(d.nz, 64 * K));
+    const dim3 grid = tile_grid((size_t)ceil_div(d.nx, kSidTWaves) * d.ny, 64 * kSidTWaves, ceil_div(d.nz, 64 * K));
     if (d.nv % 2 == 1 && d.nz % 2 == 0)
         hipLaunchKernelGGL((siddon_t_kernel<K, true>), grid, dim3(64 * kSidTWaves), 0, s, d, gt, p0, np, p0 > 0, vol);
     else

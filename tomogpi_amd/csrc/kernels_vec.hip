@@ -429,7 +429,7 @@ __global__ __launch_bounds__(256) void zcol_kernel(const TI* __restrict__ in, ui
                                                  int nz) {
     __shared__ uint32_t tile[kColTile + 1][kColLds];
     const uint32_t gx = (uint32_t)(nx + kColTile - 1) / kColTile;
-    const uint32_t b = blockIdx.x, rest = b / gx;
+    const uint32_t b = tile_index(), rest = b / gx;
     zcol_tile<TI, PAIR>(in, out, nx, ny, nz, (int)(b % gx), (int)(rest % (uint32_t)ny), (int)(rest / (uint32_t)ny),
                         tile);
 }
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(256) void rs_copy_kernel(const TI* __restrict__ in,
                                                     int nz) {
     __shared__ uint32_t tile[kColTile + 1][kColLds];
     const uint32_t gx = (uint32_t)nx / kColTile + 1, gy = (uint32_t)ny + (QUAD ? 1 : 2);
-    const uint32_t b = blockIdx.x, rest = b / gx;
+    const uint32_t b = tile_index(), rest = b / gx;
     rs_copy_tile<TI, QUAD>(in, out, nx, ny, nz, (int)(b % gx), (int)(rest % gy), (int)(rest / gy), tile);
 }
 
@@ -690,10 +690,10 @@ unsigned grid_for(size_t n) {
 hipError_t launch_zcol(const void* vol, uint32_t* out, size_t es, int nx, int ny, int nz, hipStream_t s) {
     const size_t tiles = (size_t)ceil_div(nx, kColTile) * ny * ceil_div(zcol_pitch(nz, es), kColTile);
     if (es == 4)
-        hipLaunchKernelGGL((zcol_kernel<uint32_t, false>), dim3((unsigned)tiles), dim3(256), 0, s, (const uint32_t*)vol,
+        hipLaunchKernelGGL((zcol_kernel<uint32_t, false>), tile_grid(tiles, 256), dim3(256), 0, s, (const uint32_t*)vol,
                            out, nx, ny, nz);
     else
-        hipLaunchKernelGGL((zcol_kernel<uint16_t, true>), dim3((unsigned)tiles), dim3(256), 0, s, (const uint16_t*)vol,
+        hipLaunchKernelGGL((zcol_kernel<uint16_t, true>), tile_grid(tiles, 256), dim3(256), 0, s, (const uint16_t*)vol,
                            out, nx, ny, nz);
     return hipGetLastError();
 }
@@ -701,10 +701,10 @@ hipError_t launch_zcol(const void* vol, uint32_t* out, size_t es, int nx, int ny
 hipError_t launch_rs_copy(const void* vol, void* out, size_t es, int nx, int ny, int nz, hipStream_t s) {
     const size_t tiles = ((size_t)nx / kColTile + 1) * ((size_t)ny + (es == 4 ? 2 : 1)) * ceil_div((size_t)nz + 2, kColTile);
     if (es == 4)
-        hipLaunchKernelGGL((rs_copy_kernel<uint32_t, false>), dim3((unsigned)tiles), dim3(256), 0, s,
+        hipLaunchKernelGGL((rs_copy_kernel<uint32_t, false>), tile_grid(tiles, 256), dim3(256), 0, s,
                            (const uint32_t*)vol, (uint2*)out, nx, ny, nz);
     else
-        hipLaunchKernelGGL((rs_copy_kernel<uint16_t, true>), dim3((unsigned)tiles), dim3(256), 0, s,
+        hipLaunchKernelGGL((rs_copy_kernel<uint16_t, true>), tile_grid(tiles, 256), dim3(256), 0, s,
                            (const uint16_t*)vol, (uint2*)out, nx, ny, nz);
     return hipGetLastError();
 }

@@ -693,7 +693,8 @@ __global__ __launch_bounds__(256) void vi_t_prepare_kernel(DevGeom g, const TV* 
     __shared__ float tile[64][65];
     const int pitch = (int)vi_t_pitch(g.nz);
     const uint32_t gx = (uint32_t)(g.nx + 63) / 64;
-    const uint32_t bx = blockIdx.x % gx, rest = blockIdx.x / gx, y = rest % (uint32_t)g.ny, bz = rest / (uint32_t)g.ny;
+    const uint32_t tile_no = tile_index();
+    const uint32_t bx = tile_no % gx, rest = tile_no / gx, y = rest % (uint32_t)g.ny, bz = rest / (uint32_t)g.ny;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     const int x = (int)bx * 64 + tx, r0 = (int)bz * 64;
     for (int r = ty; r < 64; r += 4) {
@@ -716,15 +717,17 @@ __device__ __forceinline__ float lane_value(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// Grid: x = (view, column group), views first; y = row block of 64 K rows.  One
+// Grid: x, y = (view, column group), views first; z = row block of 64 K rows.  One
 // wave per workgroup: nothing is shared, and the strips differ in length.
 template <int K, int M>
 __global__ __launch_bounds__(64, 7) void vi_t_kernel(DevGeom g, const float* __restrict__ vt, float* __restrict__ sino) {
     typedef float V4 __attribute__((ext_vector_type(4)));
     __shared__ __align__(16) float stage[kViTWords + 8];
     const int lane = threadIdx.x;
-    const int p = (int)(blockIdx.x % (uint32_t)g.nphi), m0 = (int)(blockIdx.x / (uint32_t)g.nphi) * M;
-    const int nb = (int)blockIdx.y * 64 * K;
+    const uint32_t tile = tile_index();
+    const int p = (int)(tile % (uint32_t)g.nphi), m0 = (int)(tile / (uint32_t)g.nphi) * M;
+    if (m0 >= g.nu) return;
+    const int nb = (int)blockIdx.z * 64 * K;
     typedef const __attribute__((address_space(4))) double* ConstView;
     const ConstView vw = (ConstView)(g.view + (size_t)p * kViewStride);
     double cvt[kViewStride];
@@ -1047,7 +1050,7 @@ static void launch_vi_t(const DevGeom& d, const float* vt, float* sino, hipStrea
     // 1253 / 1128 / 1104; 16384 (256^3, 256) 4636 / 3689 / 3445.
     const size_t waves = (size_t)ceil_div(d.nu, 4) * d.nphi * ceil_div(d.nv, 64 * K);
     const int cols = waves < 2048 ? 1 : waves < 6144 ? 2 : 4;
-    const dim3 grid(ceil_div(d.nu, cols) * (unsigned)d.nphi, ceil_div(d.nv, 64 * K));
+    const dim3 grid = tile_grid((size_t)ceil_div(d.nu, cols) * d.nphi, 64, ceil_div(d.nv, 64 * K));
     if (cols == 1)
         hipLaunchKernelGGL((vi_t_kernel<K, 1>), grid, dim3(64), 0, s, d, vt, sino);
     else if (cols == 2)
@@ -1070,9 +1073,9 @@ int launch_vi_adjoint(const tomo_geom* g, Buf vol, MutBuf sino, hipStream_t s) {
         vt = nullptr;
     }
     if (vt) {
-        const unsigned tiles = ceil_div(d.nx, 64) * (unsigned)d.ny * ceil_div(vi_t_pitch(d.nz), 64);
+        const size_t tiles = (size_t)ceil_div(d.nx, 64) * d.ny * ceil_div(vi_t_pitch(d.nz), 64);
         TOMO_DISPATCH_STORAGE(vol.dtype, TV, {
-            hipLaunchKernelGGL((vi_t_prepare_kernel<TV>), dim3(tiles), dim3(256), 0, s, d, (const TV*)vol.p, inv, vt);
+            hipLaunchKernelGGL((vi_t_prepare_kernel<TV>), tile_grid(tiles, 256), dim3(256), 0, s, d, (const TV*)vol.p, inv, vt);
         });
         switch (steps) {
             case 1: launch_vi_t<1>(d, vt, (float*)sino.p, s); break;
