@@ -195,7 +195,8 @@ __device__ __forceinline__ void vi_box_tile(const DevGeom& g, ViBox* __restrict_
 
 // One workgroup per (column tile, view).
 __global__ __launch_bounds__(SX* SY) void vi_box_kernel(DevGeom g, ViBox* __restrict__ box, int ntx) {
-    vi_box_tile(g, box, ntx, blockIdx.x / (uint32_t)g.nphi, blockIdx.x % (uint32_t)g.nphi);
+    const uint32_t b = tile_index(), tile = b / (uint32_t)g.nphi;
+    if (tile < (uint32_t)ntx * (uint32_t)((g.ny + SY - 1) / SY)) vi_box_tile(g, box, ntx, tile, b % (uint32_t)g.nphi);
 }
 
 // Per-view staging plan of a workgroup: the box of taps (rows from v0,
@@ -588,8 +589,9 @@ __global__ __launch_bounds__(SX* SY, vi_waves(FDK, ZS, PAIR)) void vi_staged_ker
 // [0, nu] of the row holds taps (j - 1, j) as its low and high halves, a tap
 // off the row as 0.
 __global__ __launch_bounds__(256) void vi_pair_kernel(const uint16_t* __restrict__ sino,
-                                                      uint32_t* __restrict__ pairs, int nu) {
-    const size_t row = blockIdx.x;
+                                                      uint32_t* __restrict__ pairs, int nu, uint32_t rows) {
+    const size_t row = tile_index();
+    if (row >= rows) return;
     const uint16_t* src = sino + row * (size_t)nu;
     uint32_t* dst = pairs + row * (size_t)(nu + 1);
     for (int j = threadIdx.x; j <= nu; j += blockDim.x) {
@@ -926,7 +928,7 @@ static hipError_t launch_vi_staged(const DevGeom& d, int fdk, const float* sino,
     hipError_t e = hipSuccess;
     if (!boxes) {
         if ((e = hipMallocAsync(&own, vi_box_count(d) * sizeof(ViBox), s)) != hipSuccess) return e;
-        hipLaunchKernelGGL(vi_box_kernel, dim3((unsigned)vi_box_count(d)), dim3(SX * SY), 0, s, d, (ViBox*)own, ntx);
+        hipLaunchKernelGGL(vi_box_kernel, tile_grid(vi_box_count(d), SX * SY), dim3(SX * SY), 0, s, d, (ViBox*)own, ntx);
         e = hipGetLastError();
         boxes = own;
     }
@@ -979,8 +981,8 @@ int launch_vi(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t s, int fdk) 
         const size_t rows = (size_t)d.nv * d.nphi;
         if (rows >= (1ull << 31)) return fail(TOMO_ERR_UNSUPPORTED, "VI needs fewer than 2^31 detector rows");
         TOMO_HIP(hipMallocAsync(&wide, rows * (size_t)(d.nu + 1) * sizeof(uint32_t), s));
-        if (rows > 0) hipLaunchKernelGGL(vi_pair_kernel, dim3((unsigned)rows), dim3(256), 0, s,
-                                         (const uint16_t*)sino.p, (uint32_t*)wide, d.nu);
+        if (rows > 0) hipLaunchKernelGGL(vi_pair_kernel, tile_grid(rows, 256), dim3(256), 0, s,
+                                         (const uint16_t*)sino.p, (uint32_t*)wide, d.nu, (uint32_t)rows);
         const hipError_t le = hipGetLastError();
         if (le != hipSuccess) {
             (void)hipFreeAsync(wide, s);
@@ -1014,7 +1016,7 @@ int launch_vi(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t s, int fdk) 
 
 int launch_vi_boxes(const DevGeom& d, void* boxes, hipStream_t s) {
     const int ntx = ceil_div(d.nx, SX);
-    hipLaunchKernelGGL(vi_box_kernel, dim3((unsigned)vi_box_count(d)), dim3(SX * SY), 0, s, d, (ViBox*)boxes, ntx);
+    hipLaunchKernelGGL(vi_box_kernel, tile_grid(vi_box_count(d), SX * SY), dim3(SX * SY), 0, s, d, (ViBox*)boxes, ntx);
     TOMO_HIP(hipGetLastError());
     return TOMO_OK;
 }
