@@ -65,7 +65,10 @@ struct BatchItem {
     void* out;        // output
     void* aux;        // second input (VI box table) or FP64 partial sums (one per tile)
     double* slot;     // per-problem FP64 scalars
-    uint64_t n;       // element count (element-wise ops)
+    union {
+        uint64_t n;         // element count (element-wise ops)
+        ProjPlanes planes;  // of the projector's copy (copy launches, projectors)
+    };
     uint32_t begin, tiles;
     uint32_t gx, gy;  // tile grid of the problem (x, y); z = tiles / (gx * gy)
     int32_t flags;

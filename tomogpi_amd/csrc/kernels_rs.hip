@@ -128,10 +128,10 @@ template <typename TV, bool BUF> struct RsReader {
     __amdgpu_buffer_rsrc_t r;
     const uint2* p;
     uint32_t sx, sy;  // elements per x and y step; BUF: bytes
-    float syf, mz;    // BUF: sy, and 2^23 + the offset of floors (0, 0) from (-1, -1) in (y, z)
+    float syf, mz;    // BUF: sy, and 2^23 + the offset of floors (0, 0) from (-1, z0 - 1) in (y, z)
     size_t base;      // index of the element of floors (0, 0, 0)
     using Off = typename std::conditional<BUF, uint32_t, size_t>::type;
-    // Offset of the element of the floors, each in [-1, n - 1].  BUF: the
+    // Offset of the element of the floors, each in [-1, n - 1], z in [z0 - 1, z0 + nz - 1].  BUF: the
     // (y, z) part as exact FP32 integers below 2^24 (sx < 2^23), whose bits
     // hold them above 2^23, and a 24-bit multiply-add for x: fused
     // multiply-adds issue at twice the rate of conversions.
@@ -202,15 +202,15 @@ __device__ __forceinline__ RsRows rs_rows(const typename RsReader<TV, BUF>::Taps
 }
 
 template <typename TV, bool BUF>
-__device__ __forceinline__ RsReader<TV, BUF> make_rs_reader(const void* copy, int nx, int ny, int nz) {
+__device__ __forceinline__ RsReader<TV, BUF> make_rs_reader(const void* copy, int nx, int ny, ProjPlanes zp) {
     RsReader<TV, BUF> q;
-    const RsCopyShape c = rs_copy_shape(nx, ny, nz, sizeof(TV));
+    const RsCopyShape c = rs_copy_shape(nx, ny, zp.nz, sizeof(TV));
     q.p = (const uint2*)copy;
     q.sx = c.sx * (BUF ? 8u : 1u);
     q.sy = c.sy * (BUF ? 8u : 1u);
     q.syf = (float)q.sy;
-    q.mz = 8388608.0f + (float)(q.sy + 8u);
-    q.base = (size_t)c.sx + c.sy + 1u;
+    q.mz = 8388608.0f + ((float)(q.sy + 8u) - 8.0f * (float)zp.z0);
+    q.base = (size_t)c.sx + c.sy + 1u - (size_t)zp.z0;
     if constexpr (BUF) q.r = buffer_rsrc(copy, (uint32_t)(c.elems * 8u));
     return q;
 }
@@ -292,8 +292,9 @@ __device__ __forceinline__ float rs_samples(const RsRay& r, const RsReader<TV, B
 // differ by the cosine of the cone angle), so the taps of neighbouring rows are
 // neighbours along z, the fastest axis of the copy.
 template <typename TV, typename TS, bool BUF>
-__device__ __forceinline__ void rs_tile(const DevGeom& g, int cube, const void* __restrict__ copy, float vol_inv,
-                                        TS* __restrict__ sino, float sino_scale, int rows, int bx, int pg, int bz) {
+__device__ __forceinline__ void rs_tile(const DevGeom& g, int cube, const void* __restrict__ copy, ProjPlanes zp,
+                                        float vol_inv, TS* __restrict__ sino, float sino_scale, int rows, int bx, int pg,
+                                        int bz) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int per = 64 / rows;  // columns of a wave
     const int p = pg * kProjViews + wv;
@@ -303,6 +304,8 @@ __device__ __forceinline__ void rs_tile(const DevGeom& g, int cube, const void* 
     RsRay r{0, 0, 0, 0, 0, 0, 0};
     if (inside) r = rs_setup(g, cube, p, m, n);
     const bool ok = r.lr > 0;
+    // a lane without a ray samples the first plane's cell (0, 0); its sum is dropped
+    if (!ok) r.ez = (float)zp.z0;
     const int nx = g.nx, ny = g.ny, nz = g.nz;
     auto within = [](float a, float b, int n1) {
         const float fa = floorf(a), fb = floorf(b);
@@ -312,9 +315,8 @@ __device__ __forceinline__ void rs_tile(const DevGeom& g, int cube, const void* 
     const bool inner = within(r.ex, fmaf(sl, r.dx, r.ex), nx) & within(r.ey, fmaf(sl, r.dy, r.ey), ny) &
                        within(r.ez, fmaf(sl, r.dz, r.ez), nz);
     const int kend = __builtin_amdgcn_readfirstlane(wave_max(ok ? r.lr : 0));
-    // a lane without a ray samples cell (0, 0, 0); its sum is dropped
     const int kall = __builtin_amdgcn_readfirstlane(min(wave_min(ok ? r.lr : INT_MAX), kend));
-    const auto q = make_rs_reader<TV, BUF>(copy, nx, ny, nz);
+    const auto q = make_rs_reader<TV, BUF>(copy, nx, ny, zp);
     float acc = __ballot(ok && !inner) == 0ull ? rs_samples<true>(r, q, nx, ny, nz, kall, kend)
                                                : rs_samples<false>(r, q, nx, ny, nz, kall, kend);
     // 16-bit volumes are read unscaled; the sum is linear in them, so the
@@ -328,9 +330,9 @@ __device__ __forceinline__ void rs_tile(const DevGeom& g, int cube, const void* 
 
 template <typename TV, typename TS, bool BUF>
 __global__ __launch_bounds__(64 * kProjViews) void rs_kernel(DevGeom g, int cube, const void* __restrict__ copy,
-                                                             float vol_inv, TS* __restrict__ sino, float sino_scale,
-                                                             int rows) {
-    rs_tile<TV, TS, BUF>(g, cube, copy, vol_inv, sino, sino_scale, rows,
+                                                             ProjPlanes zp, float vol_inv, TS* __restrict__ sino,
+                                                             float sino_scale, int rows) {
+    rs_tile<TV, TS, BUF>(g, cube, copy, zp, vol_inv, sino, sino_scale, rows,
                          proj_group(blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, blockIdx.z), blockIdx.y, blockIdx.z);
 }
 
@@ -629,17 +631,17 @@ __global__ __launch_bounds__(64 * kProjViews) void rs_batch_kernel(const BatchTa
         const int by = (int)(rest % it.gy), bz = (int)(rest / it.gy), cube = it.flags & 1;
         const int bx = proj_group(local % it.gx, it.gx, (uint32_t)by, it.gy, (uint32_t)bz);
         const bool bf = (it.flags & kItemBF16) != 0;
-        const bool buf = rs_copy_shape(it.g.nx, it.g.ny, it.g.nz, bf ? 2 : 4).buf;
+        const bool buf = rs_copy_shape(it.g.nx, it.g.ny, it.planes.nz, bf ? 2 : 4).buf;
         const int rows = rs_wave_rows(it.g.nv);
         using BF = __hip_bfloat16;
         if (bf && buf)
-            rs_tile<BF, float, true>(it.g, cube, it.in, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
+            rs_tile<BF, float, true>(it.g, cube, it.in, it.planes, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else if (bf)
-            rs_tile<BF, float, false>(it.g, cube, it.in, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
+            rs_tile<BF, float, false>(it.g, cube, it.in, it.planes, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else if (buf)
-            rs_tile<float, float, true>(it.g, cube, it.in, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
+            rs_tile<float, float, true>(it.g, cube, it.in, it.planes, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else
-            rs_tile<float, float, false>(it.g, cube, it.in, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
+            rs_tile<float, float, false>(it.g, cube, it.in, it.planes, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
     }
 }
 
@@ -945,10 +947,11 @@ int launch_rs(const tomo_geom* g, int cube, Buf vol, MutBuf sino, hipStream_t s,
     }
     const float inv = 1.0f / vol.scale;
     const size_t es = vol.dtype == TOMO_F32 ? 4 : 2;
-    const RsCopyShape cs = rs_copy_shape(d.nx, d.ny, d.nz, es);
+    const ProjPlanes zp = proj_planes(d, cube);
+    const RsCopyShape cs = rs_copy_shape(d.nx, d.ny, zp.nz, es);
     ProjCopy pc;
     hipError_t le = pc.alloc(cs.elems * 8, s, x);
-    if (le == hipSuccess) le = launch_rs_copy(vol.p, pc.p, es, d.nx, d.ny, d.nz, s);
+    if (le == hipSuccess) le = launch_rs_copy(vol.p, pc.p, es, d.nx, d.ny, d.nz, zp, s);
     if (le == hipSuccess) {
         const bool buf = cs.buf && !x.index_reads;
         const int rows = rs_wave_rows(d.nv);
@@ -957,10 +960,10 @@ int launch_rs(const tomo_geom* g, int cube, Buf vol, MutBuf sino, hipStream_t s,
             TOMO_DISPATCH_STORAGE(sino.dtype, TS, {
                 if (buf)
                     hipLaunchKernelGGL((rs_kernel<TV, TS, true>), cgrid, dim3(64 * kProjViews), 0, s, d, cube, pc.p,
-                                       inv, (TS*)sino.p, sino.scale, rows);
+                                       zp, inv, (TS*)sino.p, sino.scale, rows);
                 else
                     hipLaunchKernelGGL((rs_kernel<TV, TS, false>), cgrid, dim3(64 * kProjViews), 0, s, d, cube, pc.p,
-                                       inv, (TS*)sino.p, sino.scale, rows);
+                                       zp, inv, (TS*)sino.p, sino.scale, rows);
             });
         });
         le = hipGetLastError();

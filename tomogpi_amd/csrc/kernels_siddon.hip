@@ -341,7 +341,7 @@ __device__ __forceinline__ float sid_walk_columns(const ColumnRay& r, const CR& 
 // its L2 meets the columns of one view again in the next ones (512^3: 38.1 ms
 // without it, at four columns of one view per workgroup).
 template <typename TV, typename TS, bool BUF>
-__device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __restrict__ cols, float vol_inv,
+__device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __restrict__ cols, ProjPlanes zp, float vol_inv,
                                             TS* __restrict__ sino, float sino_scale, int rows, int bx, int pg, int bz) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int per = 64 / rows;  // columns of a wave
@@ -362,14 +362,14 @@ __device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __
     const float cell = fminf(fminf(fmaxf(ix, r.first[0]), fmaxf(iy, r.first[1])), r.tmax);
     const bool walk = __ballot(ok && !(iz > cell + 1.0e-6f * r.tmax)) == 0ull;
     const int ny = g.ny, nz = g.nz;
-    const uint32_t pz = zcol_pitch(nz, sizeof(TV)), py = pz * (uint32_t)ny;
+    const uint32_t pz = zcol_pitch(zp.nz, sizeof(TV)), py = pz * (uint32_t)ny;
     using CR = ColumnReader<TV, BUF>;
     constexpr uint32_t u = CR::kUnit;
     CR rd;
-    if constexpr (BUF) rd.r = buffer_rsrc(cols, (uint32_t)(zcol_words(g.nx, ny, nz, sizeof(TV)) * 4u));
+    if constexpr (BUF) rd.r = buffer_rsrc(cols, (uint32_t)(zcol_words(g.nx, ny, zp.nz, sizeof(TV)) * 4u));
     rd.p = cols;
     float acc = 0.0f;
-    const uint32_t lin = ok ? (uint32_t)r.idx[0] * py + (uint32_t)r.idx[1] * pz + (uint32_t)(r.idx[2] + 1) : 0u;
+    const uint32_t lin = ok ? (uint32_t)r.idx[0] * py + (uint32_t)r.idx[1] * pz + (uint32_t)(r.idx[2] + 1 - zp.z0) : 0u;
     if (walk) {
         ColumnRay w;
         w.fx = r.first[0];
@@ -738,9 +738,9 @@ __global__ __launch_bounds__(BX* BY, 5) void siddon_staged_kernel(DevGeom g, con
 }
 
 template <typename TV, typename TS, bool BUF>
-__global__ __launch_bounds__(64 * kProjViews) void siddon_kernel(DevGeom g, const uint32_t* __restrict__ cols, float vol_inv,
-                                                     TS* __restrict__ sino, float sino_scale, int rows) {
-    siddon_tile<TV, TS, BUF>(g, cols, vol_inv, sino, sino_scale, rows,
+__global__ __launch_bounds__(64 * kProjViews) void siddon_kernel(DevGeom g, const uint32_t* __restrict__ cols, ProjPlanes zp,
+                                                     float vol_inv, TS* __restrict__ sino, float sino_scale, int rows) {
+    siddon_tile<TV, TS, BUF>(g, cols, zp, vol_inv, sino, sino_scale, rows,
                              proj_group(blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, blockIdx.z), blockIdx.y, blockIdx.z);
 }
 
@@ -755,18 +755,18 @@ __global__ __launch_bounds__(64 * kProjViews) void siddon_batch_kernel(const Bat
         const int by = (int)(rest % it.gy), bz = (int)(rest / it.gy);
         const int bx = proj_group(local % it.gx, it.gx, (uint32_t)by, it.gy, (uint32_t)bz);
         const bool bf = (it.flags & kItemBF16) != 0;
-        const bool buf = zcol_words(it.g.nx, it.g.ny, it.g.nz, bf ? 2 : 4) * 4u < kSidOutside;
+        const bool buf = zcol_words(it.g.nx, it.g.ny, it.planes.nz, bf ? 2 : 4) * 4u < kSidOutside;
         const int rows = sid_wave_rows(it.g.nv);
         const uint32_t* cols = (const uint32_t*)it.in;
         using BF = __hip_bfloat16;
         if (bf && buf)
-            siddon_tile<BF, float, true>(it.g, cols, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
+            siddon_tile<BF, float, true>(it.g, cols, it.planes, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else if (bf)
-            siddon_tile<BF, float, false>(it.g, cols, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
+            siddon_tile<BF, float, false>(it.g, cols, it.planes, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else if (buf)
-            siddon_tile<float, float, true>(it.g, cols, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
+            siddon_tile<float, float, true>(it.g, cols, it.planes, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
         else
-            siddon_tile<float, float, false>(it.g, cols, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
+            siddon_tile<float, float, false>(it.g, cols, it.planes, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
     }
 }
 
@@ -1209,21 +1209,23 @@ int launch_siddon(const tomo_geom* g, int compat, Buf vol, MutBuf sino, hipStrea
     if (!sid_volume_fits(d.nx, d.ny, d.nz))
         return fail(TOMO_ERR_UNSUPPORTED, "volume too large for the 32-bit traversal index of the Siddon projector");
     ProjCopy zc;
-    hipError_t le = zc.alloc(zcol_words(d.nx, d.ny, d.nz, es) * 4, s, x);
-    if (le == hipSuccess) le = launch_zcol(vol.p, (uint32_t*)zc.p, es, d.nx, d.ny, d.nz, s);
+    const ProjPlanes zp = proj_planes(d, 0);
+    const size_t words = zcol_words(d.nx, d.ny, zp.nz, es);
+    hipError_t le = zc.alloc(words * 4, s, x);
+    if (le == hipSuccess) le = launch_zcol(vol.p, (uint32_t*)zc.p, es, d.nx, d.ny, d.nz, zp, s);
     if (le == hipSuccess) {
-        const bool buf = zcol_words(d.nx, d.ny, d.nz, es) * 4u < kSidOutside && !x.index_reads;
+        const bool buf = words * 4u < kSidOutside && !x.index_reads;
         const int rows = sid_wave_rows(d.nv);
         const dim3 cgrid(proj_groups(d.nu, rows), ceil_div(d.nphi, kProjViews), ceil_div(d.nv, rows));
         TOMO_DISPATCH_STORAGE(vol.dtype, TV, {
             TOMO_DISPATCH_STORAGE(sino.dtype, TS, {
                 if (buf)
                     hipLaunchKernelGGL((siddon_kernel<TV, TS, true>), cgrid, dim3(64 * kProjViews), 0, s, d,
-                                       (const uint32_t*)zc.p, inv,
+                                       (const uint32_t*)zc.p, zp, inv,
                                        (TS*)sino.p, sino.scale, rows);
                 else
                     hipLaunchKernelGGL((siddon_kernel<TV, TS, false>), cgrid, dim3(64 * kProjViews), 0, s, d,
-                                       (const uint32_t*)zc.p, inv,
+                                       (const uint32_t*)zc.p, zp, inv,
                                        (TS*)sino.p, sino.scale, rows);
             });
         });

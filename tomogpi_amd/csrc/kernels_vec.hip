@@ -391,10 +391,10 @@ __global__ __launch_bounds__(256) void row_pad_kernel(const float* __restrict__ 
 constexpr int kColLds = 65;
 template <typename TI, bool PAIR>
 __device__ __forceinline__ void zcol_tile(const TI* __restrict__ in, uint32_t* __restrict__ out, int nx, int ny, int nz,
-                                          int bx, int y, int bz, uint32_t (*tile)[kColLds]) {
+                                          ProjPlanes zp, int bx, int y, int bz, uint32_t (*tile)[kColLds]) {
     using T = typename std::conditional<PAIR, uint16_t, uint32_t>::type;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4
-    const int x = bx * kColTile + tx, z0 = bz * kColTile - 1;  // plane of the tile's first row
+    const int x = bx * kColTile + tx, z0 = zp.z0 + bz * kColTile - 1;  // plane of the tile's first row
     const TI* col = in + (size_t)min(x, nx - 1) + (size_t)nx * y;
     const size_t zs = (size_t)nx * ny;
     // clamped addresses and masks (the elements are integers), so that no load is a branch
@@ -411,7 +411,7 @@ __device__ __forceinline__ void zcol_tile(const TI* __restrict__ in, uint32_t* _
     for (int j = 0; j < 16; ++j) tile[ty + 4 * j][tx] = v[j];
     if (PAIR && ty == 0) tile[64][tx] = fetch(64);
     __syncthreads();
-    const int pz = (int)zcol_pitch(nz, PAIR ? 2 : 4);
+    const int pz = (int)zcol_pitch(zp.nz, PAIR ? 2 : 4);
     const int zz = bz * kColTile + tx;
     if (zz < pz) {
 #pragma unroll
@@ -426,11 +426,11 @@ __device__ __forceinline__ void zcol_tile(const TI* __restrict__ in, uint32_t* _
 // One workgroup per tile, tiles in (x, y, z) order.
 template <typename TI, bool PAIR>
 __global__ __launch_bounds__(256) void zcol_kernel(const TI* __restrict__ in, uint32_t* __restrict__ out, int nx, int ny,
-                                                 int nz) {
+                                                 int nz, ProjPlanes zp) {
     __shared__ uint32_t tile[kColTile + 1][kColLds];
     const uint32_t gx = (uint32_t)(nx + kColTile - 1) / kColTile;
     const uint32_t b = tile_index(), rest = b / gx;
-    zcol_tile<TI, PAIR>(in, out, nx, ny, nz, (int)(b % gx), (int)(rest % (uint32_t)ny), (int)(rest / (uint32_t)ny),
+    zcol_tile<TI, PAIR>(in, out, nx, ny, nz, zp, (int)(b % gx), (int)(rest % (uint32_t)ny), (int)(rest / (uint32_t)ny),
                         tile);
 }
 
@@ -439,10 +439,10 @@ __global__ __launch_bounds__(256) void zcol_kernel(const TI* __restrict__ in, ui
 // voxel, in 16 bits (QUAD) the voxels of rows yy-1 and yy.
 template <typename TI, bool QUAD>
 __device__ __forceinline__ void rs_copy_tile(const TI* __restrict__ in, uint2* __restrict__ out, int nx, int ny, int nz,
-                                             int bx, int yy, int bz, uint32_t (*tile)[kColLds]) {
+                                             ProjPlanes zp, int bx, int yy, int bz, uint32_t (*tile)[kColLds]) {
     using T = typename std::conditional<QUAD, uint16_t, uint32_t>::type;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4
-    const int x0 = bx * kColTile - 1, z0 = bz * kColTile - 1;  // voxel of the tile's first column and row
+    const int x0 = bx * kColTile - 1, z0 = zp.z0 + bz * kColTile - 1;  // voxel of the tile's first column and row
     auto voxel = [&](int x, int y, int z) {
         uint32_t m = 0u - (uint32_t)((x >= 0) & (x < nx) & (y >= 0) & (y < ny) & (z >= 0) & (z < nz));
         asm("" : "+v"(m));
@@ -462,9 +462,9 @@ __device__ __forceinline__ void rs_copy_tile(const TI* __restrict__ in, uint2* _
     for (int j = 0; j < 16; ++j) tile[ty + 4 * j][tx] = v[j];
     if (ty == 0) tile[tx][64] = word(64, tx);
     __syncthreads();
-    const RsCopyShape cs = rs_copy_shape(nx, ny, nz, QUAD ? 2 : 4);
+    const RsCopyShape cs = rs_copy_shape(nx, ny, zp.nz, QUAD ? 2 : 4);
     const int zz = bz * kColTile + tx;
-    if (zz <= nz + 1) {
+    if (zz <= zp.nz + 1) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             const int r = ty + 4 * j, xx = bx * kColTile + r;
@@ -478,11 +478,11 @@ __device__ __forceinline__ void rs_copy_tile(const TI* __restrict__ in, uint2* _
 // One workgroup per tile, tiles in (x, y, z) order.
 template <typename TI, bool QUAD>
 __global__ __launch_bounds__(256) void rs_copy_kernel(const TI* __restrict__ in, uint2* __restrict__ out, int nx, int ny,
-                                                    int nz) {
+                                                    int nz, ProjPlanes zp) {
     __shared__ uint32_t tile[kColTile + 1][kColLds];
     const uint32_t gx = (uint32_t)nx / kColTile + 1, gy = (uint32_t)ny + (QUAD ? 1 : 2);
     const uint32_t b = tile_index(), rest = b / gx;
-    rs_copy_tile<TI, QUAD>(in, out, nx, ny, nz, (int)(b % gx), (int)(rest % gy), (int)(rest / gy), tile);
+    rs_copy_tile<TI, QUAD>(in, out, nx, ny, nz, zp, (int)(b % gx), (int)(rest % gy), (int)(rest / gy), tile);
 }
 
 // ---- shared launches of the gradient loop (FP32).  Element-wise tiles
@@ -516,12 +516,13 @@ __global__ __launch_bounds__(256) void copy_batch_kernel(const BatchTable* __res
         batch_coords(it, tile, bx, by, bz);
         const int nx = it.g.nx, ny = it.g.ny, nz = it.g.nz;
         const bool bf = (it.flags & kItemBF16) != 0;
+        const ProjPlanes zp = it.planes;
         if (it.flags & kItemZcol) {
-            if (bf) zcol_tile<float, true>((const float*)it.in, (uint32_t*)it.out, nx, ny, nz, bx, by, bz, lds);
-            else zcol_tile<uint32_t, false>((const uint32_t*)it.in, (uint32_t*)it.out, nx, ny, nz, bx, by, bz, lds);
+            if (bf) zcol_tile<float, true>((const float*)it.in, (uint32_t*)it.out, nx, ny, nz, zp, bx, by, bz, lds);
+            else zcol_tile<uint32_t, false>((const uint32_t*)it.in, (uint32_t*)it.out, nx, ny, nz, zp, bx, by, bz, lds);
         } else {
-            if (bf) rs_copy_tile<float, true>((const float*)it.in, (uint2*)it.out, nx, ny, nz, bx, by, bz, lds);
-            else rs_copy_tile<uint32_t, false>((const uint32_t*)it.in, (uint2*)it.out, nx, ny, nz, bx, by, bz, lds);
+            if (bf) rs_copy_tile<float, true>((const float*)it.in, (uint2*)it.out, nx, ny, nz, zp, bx, by, bz, lds);
+            else rs_copy_tile<uint32_t, false>((const uint32_t*)it.in, (uint2*)it.out, nx, ny, nz, zp, bx, by, bz, lds);
         }
         __syncthreads();
     }
@@ -687,25 +688,25 @@ unsigned grid_for(size_t n) {
 
 }  // namespace
 
-hipError_t launch_zcol(const void* vol, uint32_t* out, size_t es, int nx, int ny, int nz, hipStream_t s) {
-    const size_t tiles = (size_t)ceil_div(nx, kColTile) * ny * ceil_div(zcol_pitch(nz, es), kColTile);
+hipError_t launch_zcol(const void* vol, uint32_t* out, size_t es, int nx, int ny, int nz, ProjPlanes zp, hipStream_t s) {
+    const size_t tiles = (size_t)ceil_div(nx, kColTile) * ny * ceil_div(zcol_pitch(zp.nz, es), kColTile);
     if (es == 4)
         hipLaunchKernelGGL((zcol_kernel<uint32_t, false>), tile_grid(tiles, 256), dim3(256), 0, s, (const uint32_t*)vol,
-                           out, nx, ny, nz);
+                           out, nx, ny, nz, zp);
     else
         hipLaunchKernelGGL((zcol_kernel<uint16_t, true>), tile_grid(tiles, 256), dim3(256), 0, s, (const uint16_t*)vol,
-                           out, nx, ny, nz);
+                           out, nx, ny, nz, zp);
     return hipGetLastError();
 }
 
-hipError_t launch_rs_copy(const void* vol, void* out, size_t es, int nx, int ny, int nz, hipStream_t s) {
-    const size_t tiles = ((size_t)nx / kColTile + 1) * ((size_t)ny + (es == 4 ? 2 : 1)) * ceil_div((size_t)nz + 2, kColTile);
+hipError_t launch_rs_copy(const void* vol, void* out, size_t es, int nx, int ny, int nz, ProjPlanes zp, hipStream_t s) {
+    const size_t tiles = ((size_t)nx / kColTile + 1) * ((size_t)ny + (es == 4 ? 2 : 1)) * ceil_div((size_t)zp.nz + 2, kColTile);
     if (es == 4)
         hipLaunchKernelGGL((rs_copy_kernel<uint32_t, false>), tile_grid(tiles, 256), dim3(256), 0, s,
-                           (const uint32_t*)vol, (uint2*)out, nx, ny, nz);
+                           (const uint32_t*)vol, (uint2*)out, nx, ny, nz, zp);
     else
         hipLaunchKernelGGL((rs_copy_kernel<uint16_t, true>), tile_grid(tiles, 256), dim3(256), 0, s,
-                           (const uint16_t*)vol, (uint2*)out, nx, ny, nz);
+                           (const uint16_t*)vol, (uint2*)out, nx, ny, nz, zp);
     return hipGetLastError();
 }
 

@@ -58,7 +58,8 @@ struct LoopCopies {
         const bool sid = pr.pair == TOMO_PAIR_SIDDONVI;
         if (sid && ((pr.flags & TOMO_FLAG_SIDDON_COMPAT) || !sid_volume_fits(nx, ny, nz))) return TOMO_OK;
         const size_t es = storage == TOMO_F32 ? 4 : 2;
-        TOMO_HIP(buf.alloc(sid ? zcol_words(nx, ny, nz, es) * 4 : rs_copy_shape(nx, ny, nz, es).elems * 8, s));
+        const int planes = proj_planes(g->dev, !sid && (pr.flags & TOMO_FLAG_RS_FOV_CUBE)).nz;
+        TOMO_HIP(buf.alloc(sid ? zcol_words(nx, ny, planes, es) * 4 : rs_copy_shape(nx, ny, planes, es).elems * 8, s));
         extra.copy = buf.p;
         return TOMO_OK;
     }

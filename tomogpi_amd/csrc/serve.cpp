@@ -130,6 +130,11 @@ namespace {
 uint32_t vec_tiles(uint64_t n) { return cdiv(n, kVecTile); }
 uint32_t lap_tiles(const DevGeom& d) { return cdiv(d.nx, 64) * cdiv(d.ny, 4) * (uint32_t)d.nz; }
 
+// The planes of a request's operator copies.
+ProjPlanes copy_planes(const DevGeom& d, const tomo_gd_params& gd) {
+    return proj_planes(d, gd.pair != TOMO_PAIR_SIDDONVI && (gd.flags & TOMO_FLAG_RS_FOV_CUBE));
+}
+
 Layout layout_of(const tomo_geom& g, const tomo_gd_params& gd, int algo, size_t ces) {
     const DevGeom& d = g.dev;
     const size_t nv = g.nvox(), ns = g.nsino();
@@ -144,8 +149,9 @@ Layout layout_of(const tomo_geom& g, const tomo_gd_params& gd, int algo, size_t 
     sizes[i++] = (lam || sirt) ? nv * 4 : 0;                             // 4 t1 (SIRT: volume weight C)
     sizes[i++] = lam ? nv * 4 : 0;                                       // 5 t2
     sizes[i++] = lam ? nv * 4 : 0;                                       // 6 t3
-    sizes[i++] = gd.pair == TOMO_PAIR_SIDDONVI ? zcol_words(d.nx, d.ny, d.nz, ces) * 4
-                                               : rs_copy_shape(d.nx, d.ny, d.nz, ces).elems * 8;  // 7 projector's copy
+    const int planes = copy_planes(d, gd).nz;
+    sizes[i++] = gd.pair == TOMO_PAIR_SIDDONVI ? zcol_words(d.nx, d.ny, planes, ces) * 4
+                                               : rs_copy_shape(d.nx, d.ny, planes, ces).elems * 8;  // 7 projector's copy
     sizes[i++] = 0;                                                      // 8 (unused)
     sizes[i++] = ns * 4;                                                 // 9 y
     sizes[i++] = ns * 4;                                                 // 10 px
@@ -284,13 +290,16 @@ void build_tables(tomo_server* srv, int set, const std::vector<Request*>& runnin
         auto add_projection = [&](const float* vol, float* out, int opc, int ops, int opr) {
             const size_t ces = q.bf16 ? 2 : 4;
             const int32_t cflag = q.bf16 ? kItemBF16 : 0;
-            BatchItem& z = sid ? tb[opc].add(d, cdiv(d.nx, kColTile), d.ny, cdiv(zcol_pitch(d.nz, ces), kColTile))
-                               : tb[opc].add(d, cdiv(d.nx + 1, kColTile), d.ny + (q.bf16 ? 1 : 2), cdiv(d.nz + 2, kColTile));
+            const ProjPlanes zp = copy_planes(d, gd);
+            BatchItem& z = sid ? tb[opc].add(d, cdiv(d.nx, kColTile), d.ny, cdiv(zcol_pitch(zp.nz, ces), kColTile))
+                               : tb[opc].add(d, cdiv(d.nx + 1, kColTile), d.ny + (q.bf16 ? 1 : 2), cdiv(zp.nz + 2, kColTile));
+            z.planes = zp;
             z.in = vol;
             z.out = q.copy;
             z.flags = cflag | (sid ? kItemZcol : 0);
             const int rows = sid ? sid_wave_rows(d.nv) : rs_wave_rows(d.nv);
             BatchItem& p = tb[sid ? ops : opr].add(d, proj_groups(d.nu, rows), cdiv(d.nphi, kProjViews), cdiv(d.nv, rows));
+            p.planes = zp;
             p.in = q.copy;
             p.out = out;
             p.flags = cube | cflag;

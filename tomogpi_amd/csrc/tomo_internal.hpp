@@ -73,7 +73,22 @@ inline bool sid_volume_fits(int nx, int ny, int nz) {
     const size_t z2 = 2 * ((size_t)nz + 1);
     return (size_t)nx * z2 * ((size_t)ny + 2) < (1ull << 32) && (size_t)ny * z2 * ((size_t)nx + 2) < (1ull << 32);
 }
-// z-column copy of a volume of es-byte elements (proj_copy.hpp): 4-byte words per
+// The planes of the volume that a projector's rays can read, of which its copy is
+// made: z0 .. z0 + nz - 1.  The outermost row leaves the field of view farthest
+// from the mid plane; 3 planes more for the neighbours that a sample or a cell
+// reads and the rounding of its place.
+struct ProjPlanes {
+    int z0, nz;
+};
+inline ProjPlanes proj_planes(const DevGeom& d, int cube) {
+    const double fov = 0.5 * (double)d.nx * (double)d.delta * (cube ? 1.4143 : 1.0);
+    const double reach = (double)d.cv * (double)d.dv * (d.fod + fov) / (d.fdd * (double)d.delta) + 3.0;
+    // below 2^20 planes FP32 places are well within the margin
+    if (!(reach < (double)d.cz) || d.nz >= (1 << 20)) return ProjPlanes{0, d.nz};
+    const int z0 = (int)((double)d.cz - reach);
+    return ProjPlanes{z0, d.nz - 2 * z0};
+}
+// z-column copy of nz planes of es-byte elements (proj_copy.hpp): 4-byte words per
 // (x, y) column, and of the whole copy.
 __host__ __device__ inline uint32_t zcol_pitch(int nz, size_t es) { return (uint32_t)nz + (es == 4 ? 2u : 1u); }
 __host__ __device__ inline size_t zcol_words(int nx, int ny, int nz, size_t es) {
@@ -95,7 +110,7 @@ inline uint32_t proj_groups(int nu, int rows) {
     const uint32_t cols = 64u / (uint32_t)rows;
     return ((uint32_t)nu + 8u * cols - 1u) / (8u * cols) * 8u;
 }
-// RS copy of a volume of es-byte elements (proj_copy.hpp): 8-byte elements per x
+// RS copy of nz planes of es-byte elements (proj_copy.hpp): 8-byte elements per x
 // and y step and in all, and whether RS reads it through 32-bit byte offsets
 // (below 2^32 - 16 bytes, where the offset of a read that returns 0 lies, and
 // its steps in signed 24 bits, for 24-bit multiplies).
@@ -144,7 +159,7 @@ int launch_vi_adjoint(const tomo_geom* g, Buf vol, MutBuf sino, hipStream_t s);
 // copies through 64-bit element indices even where 32-bit buffer
 // offsets apply (the form every copy of 4 GiB or more takes).  copy: memory of
 // the caller for the projector's copy of the volume (rs_copy_shape or
-// zcol_words, for the volume's element size); null: the launcher allocates it
+// zcol_words, for its planes and the volume's element size); null: the launcher allocates it
 // from the stream-ordered pool for the call.
 struct ProjExtra {
     bool index_reads = false;
