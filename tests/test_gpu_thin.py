@@ -45,6 +45,34 @@ def test_thin_projections(ctx, nx, ny, nz, nu, nv, nphi, pixel, fod, dt):
         G.close()
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("ny,nz,nu,nv,nphi", [
+    (24, 1, 300, 1, 260), (20, 60, 300, 1, 260),     # a row a wave
+    (24, 2, 300, 2, 260), (24, 40, 260, 2, 130), (24, 2, 260, 64, 130),  # two
+    (24, 3, 290, 3, 130), (24, 5, 260, 6, 130), (24, 8, 260, 9, 130),    # four, eight
+    (24, 14, 200, 20, 90), (24, 6, 260, 70, 90), (24, 30, 130, 37, 60),  # and more; rows off the volume
+])
+def test_thin_wave_rows(ctx, ny, nz, nu, nv, nphi, dt):
+    """Enough rays for waves of few rows."""
+    g = _geom(24, ny, nz, nu, nv, nphi, fod=1.953125)
+    g.su = nu * 0.25
+    print(f"[case] {ny} {nz} / {nu} {nv} {nphi} {dt}", flush=True)
+    G, o = lib.Geometry(ctx, to_desc(g)), Oracle(g)
+    try:
+        v = dev(np.random.default_rng(nv).random(g.vol_shape, dtype=np.float32)).to(
+            torch.float32 if dt == "f32" else torch.bfloat16)
+        vol = v.float().cpu().numpy()
+        for op, cube, ref in (("siddon", 0, o.siddon(vol)), ("rs", 0, o.rs(vol)), ("rs", 1, o.rs(vol, cube=True))):
+            for extra in (0, lib.FLAG_INDEX_READS):
+                out = torch.full(g.sino_shape, np.nan, dtype=torch.float32, device="cuda")
+                G.project(v, out, lib.PROJ_SIDDON if op == "siddon" else lib.PROJ_RS,
+                          extra | (lib.FLAG_RS_FOV_CUBE if cube else 0))
+                got = out.cpu().numpy()
+                assert np.array_equal(got, ref), (op, cube, extra, rel_l2(got, ref))
+    finally:
+        G.close()
+
+
 @pytest.mark.parametrize("pair", [lib.PAIR_SIDDONVI, lib.PAIR_RSVI])
 def test_thin_loop_and_server(ctx, pair):
     """A loop and a served request of few rows over many planes, in FP32 as the
@@ -69,3 +97,28 @@ def test_thin_loop_and_server(ctx, pair):
     finally:
         srv.close()
         G.close()
+
+
+@pytest.mark.parametrize("pair", [lib.PAIR_SIDDONVI, lib.PAIR_RSVI])
+def test_thin_server_rows(ctx, pair):
+    """Served requests whose waves hold few rows, two of different shapes at once
+    (rel-L2 1e-6, the bound of the served results)."""
+    kw = dict(iters=2, kopt=3, lam=0.01)
+    print(f"[case] pair={pair}", flush=True)
+    srv, jobs = lib.Server(ctx, max_active=4), []
+    try:
+        for nz, nu, nv, nphi in ((6, 260, 6, 130), (1, 300, 1, 260)):
+            g = _geom(24, 24, nz, nu, nv, nphi, fod=1.953125)
+            g.su = nu * 0.25
+            y = np.random.default_rng(nv).random(g.sino_shape, dtype=np.float32)
+            jobs.append((g, y, dev(y), torch.empty(g.vol_shape, device="cuda")))
+        torch.cuda.synchronize()
+        ids = [srv.submit(to_desc(g), d, z, pair=pair, **kw) for g, _, d, z in jobs]
+        for i in ids:
+            srv.wait(i)
+        torch.cuda.synchronize()
+        for g, y, _, z in jobs:
+            ref, _ = Oracle(g).gd(y, pair=pair, **kw)
+            assert rel_l2(z.cpu().numpy(), ref) <= 1e-6
+    finally:
+        srv.close()

@@ -93,6 +93,8 @@ static_assert(kBatchGrid % kBatchXcds == 0, "every XCD starts with the same numb
 constexpr int32_t kItemBF16 = 0x10;
 // Item flag bit of the copy launches: the z-column copy instead of the RS copy.
 constexpr int32_t kItemZcol = 0x40;
+// First item flag bit of the log2 of the projector launches' wave rows.
+constexpr int kItemRowsShift = 8;
 
 // Per-problem scalars of the gradient loop, FP64, in `slot`.
 enum GdSlot {

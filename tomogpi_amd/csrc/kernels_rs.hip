@@ -301,6 +301,12 @@ __device__ __forceinline__ void rs_tile(const DevGeom& g, int cube, const void* 
     const int m = bx * per + lane / rows;
     const int n = bz * rows + lane % rows;
     const bool inside = p < g.nphi && m < g.nu && n < g.nv;
+    // (an entry up to half a voxel above the last slice's centre counts)
+    if (proj_rows_miss(g, (cube ? 0.70711 : 0.5) * (double)g.nx * (double)g.delta, (0.5 * g.nz + 0.5) * (double)g.delta,
+                       bz * rows, rows)) {
+        if (inside) Storage<TS>::store(sino, (size_t)m + (size_t)g.nu * ((size_t)n + (size_t)g.nv * p), 0.0f, sino_scale);
+        return;
+    }
     RsRay r{0, 0, 0, 0, 0, 0, 0};
     if (inside) r = rs_setup(g, cube, p, m, n);
     const bool ok = r.lr > 0;
@@ -632,7 +638,7 @@ __global__ __launch_bounds__(64 * kProjViews) void rs_batch_kernel(const BatchTa
         const int bx = proj_group(local % it.gx, it.gx, (uint32_t)by, it.gy, (uint32_t)bz);
         const bool bf = (it.flags & kItemBF16) != 0;
         const bool buf = rs_copy_shape(it.g.nx, it.g.ny, it.planes.nz, bf ? 2 : 4).buf;
-        const int rows = rs_wave_rows(it.g.nv);
+        const int rows = 1 << (it.flags >> kItemRowsShift);
         using BF = __hip_bfloat16;
         if (bf && buf)
             rs_tile<BF, float, true>(it.g, cube, it.in, it.planes, 1.0f, (float*)it.out, 1.0f, rows, bx, by, bz);
@@ -954,7 +960,7 @@ int launch_rs(const tomo_geom* g, int cube, Buf vol, MutBuf sino, hipStream_t s,
     if (le == hipSuccess) le = launch_rs_copy(vol.p, pc.p, es, d.nx, d.ny, d.nz, zp, s);
     if (le == hipSuccess) {
         const bool buf = cs.buf && !x.index_reads;
-        const int rows = rs_wave_rows(d.nv);
+        const int rows = rs_wave_rows(d, zp);
         const dim3 cgrid(proj_groups(d.nu, rows), ceil_div(d.nphi, kProjViews), ceil_div(d.nv, rows));
         TOMO_DISPATCH_STORAGE(vol.dtype, TV, {
             TOMO_DISPATCH_STORAGE(sino.dtype, TS, {

@@ -329,7 +329,7 @@ __device__ __forceinline__ float sid_walk_columns(const ColumnRay& r, const CR& 
 // Forward clean Siddon.  Each lane takes the segments of the per-ray
 // traversal (same operations, same order), so results are bit-identical to
 // it.  What changes is the schedule and the memory layout (see above).
-// A wave is `rows` (64, 32 or 16) detector rows of 64 / rows columns; a
+// A wave is `rows` (sid_wave_rows) detector rows of 64 / rows columns; a
 // workgroup is these cells in kProjViews consecutive views, whose rays run
 // through nearly the same columns of the volume at the same time (512^3 / 512
 // views: 33.1 ms with four neighbouring column groups of one view per
@@ -349,6 +349,10 @@ __device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __
     const int m = bx * per + lane / rows;
     const int n = bz * rows + lane % rows;
     const bool inside = p < g.nphi && m < g.nu && n < g.nv;
+    if (proj_rows_miss(g, 0.5 * (double)g.nx * (double)g.delta, 0.5 * (double)g.nz * (double)g.delta, bz * rows, rows)) {
+        if (inside) Storage<TS>::store(sino, (size_t)m + (size_t)g.nu * ((size_t)n + (size_t)g.nv * p), 0.0f, sino_scale);
+        return;
+    }
     SidRay r{};
     if (inside) r = sid_setup(g, p, m, n);
     const bool ok = r.ok && r.tmax > 0.0f;
@@ -756,7 +760,7 @@ __global__ __launch_bounds__(64 * kProjViews) void siddon_batch_kernel(const Bat
         const int bx = proj_group(local % it.gx, it.gx, (uint32_t)by, it.gy, (uint32_t)bz);
         const bool bf = (it.flags & kItemBF16) != 0;
         const bool buf = zcol_words(it.g.nx, it.g.ny, it.planes.nz, bf ? 2 : 4) * 4u < kSidOutside;
-        const int rows = sid_wave_rows(it.g.nv);
+        const int rows = 1 << (it.flags >> kItemRowsShift);
         const uint32_t* cols = (const uint32_t*)it.in;
         using BF = __hip_bfloat16;
         if (bf && buf)
@@ -1215,7 +1219,7 @@ int launch_siddon(const tomo_geom* g, int compat, Buf vol, MutBuf sino, hipStrea
     if (le == hipSuccess) le = launch_zcol(vol.p, (uint32_t*)zc.p, es, d.nx, d.ny, d.nz, zp, s);
     if (le == hipSuccess) {
         const bool buf = words * 4u < kSidOutside && !x.index_reads;
-        const int rows = sid_wave_rows(d.nv);
+        const int rows = sid_wave_rows(d, zp);
         const dim3 cgrid(proj_groups(d.nu, rows), ceil_div(d.nphi, kProjViews), ceil_div(d.nv, rows));
         TOMO_DISPATCH_STORAGE(vol.dtype, TV, {
             TOMO_DISPATCH_STORAGE(sino.dtype, TS, {

@@ -35,6 +35,14 @@ __device__ __forceinline__ int proj_group(uint32_t i, uint32_t gx, uint32_t pg, 
     return (int)(run * (gx / 8u) + i / 8u);
 }
 
+// Whether none of the rows n0 .. n0 + rows - 1 has a ray in the volume: rays enter the
+// FOV (of radius fov, mm) at fod - fov from the source's plane at the nearest, and
+// these are above or below `half` there (mm from the mid plane).
+__device__ __forceinline__ bool proj_rows_miss(const DevGeom& g, double fov, double half, int n0, int rows) {
+    const float off = fmaxf(fmaxf((float)n0 - g.cv, g.cv - (float)(n0 + rows - 1)), 0.0f);
+    return (double)off * (double)g.dv * (g.fod - fov) > half * g.fdd * (1.0 + 1e-6);
+}
+
 // Fills the z-column copy of planes zp at `out` from an x-fastest volume of es-byte elements.
 hipError_t launch_zcol(const void* vol, uint32_t* out, size_t es, int nx, int ny, int nz, ProjPlanes zp, hipStream_t s);
 

@@ -297,12 +297,12 @@ void build_tables(tomo_server* srv, int set, const std::vector<Request*>& runnin
             z.in = vol;
             z.out = q.copy;
             z.flags = cflag | (sid ? kItemZcol : 0);
-            const int rows = sid ? sid_wave_rows(d.nv) : rs_wave_rows(d.nv);
+            const int rows = sid ? sid_wave_rows(d, zp) : rs_wave_rows(d, zp);
             BatchItem& p = tb[sid ? ops : opr].add(d, proj_groups(d.nu, rows), cdiv(d.nphi, kProjViews), cdiv(d.nv, rows));
             p.planes = zp;
             p.in = q.copy;
             p.out = out;
-            p.flags = cube | cflag;
+            p.flags = cube | cflag | __builtin_ctz(rows) << kItemRowsShift;
         };
         if (q.req.algorithm == TOMO_ALGO_SIRT) {
             add_projection(q.x, q.px, OP_COPY_X, OP_SID_X, OP_RS_X);

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstddef>
 #include <string>
@@ -75,14 +76,14 @@ inline bool sid_volume_fits(int nx, int ny, int nz) {
 }
 // The planes of the volume that a projector's rays can read, of which its copy is
 // made: z0 .. z0 + nz - 1.  The outermost row leaves the field of view farthest
-// from the mid plane; 3 planes more for the neighbours that a sample or a cell
-// reads and the rounding of its place.
+// from the mid plane; 1 1/2 planes more for the neighbours that a sample or a cell
+// reads, 1/2 for the rounding of its place.
 struct ProjPlanes {
     int z0, nz;
 };
 inline ProjPlanes proj_planes(const DevGeom& d, int cube) {
     const double fov = 0.5 * (double)d.nx * (double)d.delta * (cube ? 1.4143 : 1.0);
-    const double reach = (double)d.cv * (double)d.dv * (d.fod + fov) / (d.fdd * (double)d.delta) + 3.0;
+    const double reach = (double)d.cv * (double)d.dv * (d.fod + fov) / (d.fdd * (double)d.delta) + 2.0;
     // below 2^20 planes FP32 places are well within the margin
     if (!(reach < (double)d.cz) || d.nz >= (1 << 20)) return ProjPlanes{0, d.nz};
     const int z0 = (int)((double)d.cz - reach);
@@ -93,14 +94,6 @@ inline ProjPlanes proj_planes(const DevGeom& d, int cube) {
 __host__ __device__ inline uint32_t zcol_pitch(int nz, size_t es) { return (uint32_t)nz + (es == 4 ? 2u : 1u); }
 __host__ __device__ inline size_t zcol_words(int nx, int ny, int nz, size_t es) {
     return (size_t)nx * ny * zcol_pitch(nz, es);
-}
-// Detector rows of a Siddon wave (64, 32 or 16, by 64 / rows columns): the most
-// that leave no more than an eighth of the row groups' lanes idle.  Fewer rows
-// read shorter runs of z per cell, idle lanes read none.
-__host__ __device__ inline int sid_wave_rows(int nv) {
-    for (int r = 64; r > 16; r >>= 1)
-        if (((nv + r - 1) / r * r - nv) * 8 <= nv) return r;
-    return 16;
 }
 // A projector workgroup: one wave's detector cells in kProjViews consecutive views.
 constexpr int kProjViews = 4;
@@ -128,12 +121,69 @@ __host__ __device__ inline RsCopyShape rs_copy_shape(int nx, int ny, int nz, siz
     c.buf = c.elems * 8 < 0xfffffff0ull && sx * 8 < (1ull << 23) && nz < (1 << 23);
     return c;
 }
-// Detector rows of an RS wave: 32, or 16 where that leaves fewer lanes idle.  At
-// equal sample index the rows of a column drift apart in plane with the cosine
-// of the cone angle, so longer waves touch more columns at once (512^3 / 512
-// views: 68.6 ms at 64 rows, 55.3 at 32, 54.6 at 16); shorter ones read shorter
-// runs of z (1024^3, 96 views: 82, 87, 101 ms).
-__host__ __device__ inline int rs_wave_rows(int nv) { return ((nv + 31) / 32 * 32 - nv) * 8 <= nv ? 32 : 16; }
+// Detector rows of a projector's wave (a power of two up to 64, by 64 / rows columns).
+// `tall` where many rows cross the volume, else the rows of the least
+//     sum over row groups of max(16 rows, lines) x the longest ray's part of the FOV + 1/2.
+// A gather takes 16 cycles of the texture path a wave, 64 / rows columns of it, and the
+// L2 lines of the columns' runs of z take more where the runs are short and the columns
+// lie far apart; idle rows of a group that holds a ray cost as much as the others.
+// lines: 20 + 3 (planes + 2) up to 160 for Siddon, 15 + 4 (planes + 2) up to 120 for RS, and
+// up to twice that with few views, whose rays share fewer lines: over 125 and 185 shapes
+// of 1 to 48 crossing rows 1% and 2% above the best rows' times.
+// Not below `tall` with fewer waves than SIMDs (90 views of 64 x 4 cells, RS: 71 us by 4
+// rows, 50 by 16), and one row a wave for one crossing row only (256 x 256 x 1 and 64 rows,
+// RS: 171 us by 1 row, 91 by 2).
+//
+// 512 x 512 and 360 views, us at 64 / 32 / 16 / 8 / 4 / 2 / 1 rows.  Siddon: one slice
+// and row 2658 / 1348 / 698 / 380 / 215 / 161 / 155; 8 and 8 2682 / 1371 / 714 / 394 /
+// 450 / 820 / 1852; 4 slices, 64 rows 2688 / 2676 / 1395 / 760 / 456 / 408 / 766.  RS: 4152
+// / 2149 / 1134 / 632 / 391 / 286 / 210; 4072 / 2064 / 1064 / 564 / 657 / 1180 / 2364; 4228 /
+// 4227 / 2207 / 1195 / 687 / 570 / 824.
+inline int proj_wave_rows(const DevGeom& d, double lines, int tall) {
+    constexpr int kMost = 48;  // rows that cross the volume
+    const double fov = 0.5 * (double)d.nx * (double)d.delta, nearest = d.fod - fov;
+    if (!(nearest > 0.0)) return tall;
+    // z leaves the volume at the in-plane distance edge / |n - cv|
+    const double edge = 0.5 * (double)d.nz * (double)d.delta * d.fdd / (double)d.dv;
+    const int first = std::max(0, (int)std::ceil((double)d.cv - std::min(edge / nearest, 1e9)));
+    const int crossing = d.nv - 2 * first;  // centred
+    if (crossing < 1 || crossing > kMost) return tall;
+    const double share = lines * (1.0 + std::min(1.0, 60.0 / d.nphi));
+    int best = tall;
+    double least = 0.0;
+    for (int r = 64; r >= std::min(crossing, 2); r >>= 1) {
+        const int g0 = first / r, g1 = (d.nv - 1 - first) / r;
+        if (r < tall && (size_t)d.nu * r / 64 * d.nphi * (size_t)(g1 - g0 + 1) < 1024) break;
+        double cost = 0.5 * ((d.nv + r - 1) / r - (g1 - g0 + 1));
+        for (int g = g0; g <= g1; ++g) {
+            // the group's row nearest to the mid plane
+            const double n = std::min(std::max((double)d.cv, (double)g * r), std::min((double)g * r + r, (double)d.nv) - 1.0);
+            const double off = std::fabs(n - (double)d.cv);
+            const double part = off * (d.fod + fov) <= edge ? 1.0 : (edge / off - nearest) / (2.0 * fov);
+            cost += std::max(16.0 * r, share) * part + 0.5;
+        }
+        if (r == 64 || cost <= least) {
+            least = cost;
+            best = r;
+        }
+    }
+    return best;
+}
+// Siddon.  tall: the most of 64, 32 and 16 that leave no more than an eighth of the
+// row groups' lanes idle.
+inline int sid_wave_rows(const DevGeom& d, ProjPlanes zp) {
+    int tall = 64;
+    while (tall > 16 && ((d.nv + tall - 1) / tall * tall - d.nv) * 8 > d.nv) tall >>= 1;
+    return proj_wave_rows(d, std::min(20.0 + 3.0 * (zp.nz + 2), 160.0), tall);
+}
+// RS.  tall: 32, or 16 where that leaves fewer lanes idle.  At equal sample index the rows
+// of a column drift apart in plane with the cosine of the cone angle, so longer waves
+// touch more columns at once (512^3 / 512 views: 68.6 ms at 64 rows, 55.3 at 32, 54.6 at
+// 16); shorter ones read shorter runs of z (1024^3, 96 views: 82, 87, 101 ms).
+inline int rs_wave_rows(const DevGeom& d, ProjPlanes zp) {
+    return proj_wave_rows(d, std::min(15.0 + 4.0 * (zp.nz + 2), 120.0),
+                          ((d.nv + 31) / 32 * 32 - d.nv) * 8 <= d.nv ? 32 : 16);
+}
 
 // Derives the geometry exactly as the reference constructors do.
 int derive_geometry(const tomo_geom_desc& d, tomo_geom* g);
