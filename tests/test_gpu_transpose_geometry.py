@@ -21,7 +21,7 @@ def _geom(nx, ny, nz, nu, nv, nphi, pixel=2.0, fod=2.0, fdd=2.0, voxel=1.0, star
                     num_start=start, den_start=1.0, num_stop=stop, den_stop=1.0)
 
 
-def _check(ctx, g, op, cube=False):
+def _check(ctx, g, op, cube=False, bound=1e-6):
     print(f"[case] {op} {g.nx} {g.ny} {g.nz} / {g.nu} {g.nv} {g.nphi} fdd/fod {g.fdd / g.fod:.3g} voxel {g.sx / g.nx:.3g}",
           flush=True)
     G, o = lib.Geometry(ctx, to_desc(g)), Oracle(g)
@@ -37,7 +37,7 @@ def _check(ctx, g, op, cube=False):
             out = torch.full(g.vol_shape, np.nan, dtype=torch.float32, device="cuda")
             G.project_adjoint(dev(y), out, lib.PROJ_SIDDON if op == "siddon" else lib.PROJ_RS,
                               lib.FLAG_RS_FOV_CUBE if cube else 0)
-        assert rel_l2(out.cpu().numpy(), ref) <= 1e-6
+        assert rel_l2(out.cpu().numpy(), ref) <= bound
     finally:
         G.close()
 
@@ -71,10 +71,21 @@ def test_siddon_rays_along_planes(ctx, nx, ny, nz, nv, voxel):
     _check(ctx, _geom(nx, ny, nz, 41 if nx < 64 else 2 * (nx // 2) + 1, nv, 24, voxel=voxel, start=0.0, stop=2.0), "siddon")
 
 
-@pytest.mark.parametrize("nx,ny,nz,nu,nv,nphi,pixel", [
-    (20, 20, 20, 90, 5, 12, 0.3), (24, 24, 2, 30, 8, 20, 0.25), (20, 20, 130, 60, 3, 16, 0.5), (24, 20, 70, 300, 1, 16, 0.1),
-])
+@pytest.mark.parametrize("nx,ny,nz,nu,nv,nphi", [(20, 20, 20, 24, 16, 130), (24, 20, 70, 30, 16, 130), (20, 20, 3, 30, 15, 130)])
 @pytest.mark.parametrize("op", ["siddon", "vi", "rs", "rs_cube"])
-def test_few_fine_rows(ctx, op, nx, ny, nz, nu, nv, nphi, pixel):
-    """Fewer detector rows than pass one voxel."""
-    _check(ctx, _geom(nx, ny, nz, nu, nv, nphi, pixel=pixel), op.split("_")[0], cube=op == "rs_cube")
+def test_few_fine_rows(ctx, op, nx, ny, nz, nu, nv, nphi):
+    """Fewer detector rows than pass one voxel, and rays enough for the gather."""
+    g = _geom(nx, ny, nz, nu, nv, nphi)
+    g.sv = nv * 0.2
+    _check(ctx, g, op.split("_")[0], cube=op == "rs_cube")
+
+
+@pytest.mark.parametrize("op,nx,ny,nz,nu,nv,nphi", [
+    ("siddon", 64, 64, 1, 64, 4, 64), ("siddon", 64, 64, 40, 64, 1, 300), ("rs", 64, 64, 1, 64, 16, 64),
+    ("rs", 64, 64, 100, 64, 2, 64), ("vi", 64, 64, 1, 64, 1, 700),     # scattered: few rows or slices
+    ("vi", 40, 40, 1, 40, 300, 30), ("vi", 40, 40, 2, 40, 301, 30), ("vi", 40, 40, 9, 40, 200, 30),  # rows off the volume
+])
+def test_thin(ctx, op, nx, ny, nz, nu, nv, nphi):
+    """Rel-L2 <= 1e-5: the scatter adds FP32 terms one by one."""
+    g = _geom(nx, ny, nz, nu, nv, nphi)
+    _check(ctx, g, op, bound=1e-5)

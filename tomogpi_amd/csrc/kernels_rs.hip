@@ -1000,12 +1000,27 @@ hipError_t launch_batch_rs(BatchTable* t, hipStream_t s) {
 }
 
 // The gather needs the squares around the voxel columns to be in front of the source
-// in every view, and voxel and row coordinates that FP32 holds within 1e-3.
+// in every view, and voxel and row coordinates that FP32 holds within 1e-3.  Thin
+// problems, whose lanes along z would idle, scatter: the gather costs 60 ps per voxel
+// column, view and line that may cross its square (in rounds of 64 views), and per
+// line that does 20 and 43 per row that passes a voxel, 1.4 times that for 128 voxels in
+// two halves and 2.9 for 256; the scatter 262 ps a sample, or 0.9 us and 0.35 a row
+// (of up to 8) per sample of one ray.  Scatter and gather in us, 256 x 256 and 256 views: one slice and row 2422 and
+// 9121, 4 and 4 12900 and 9150, 256 slices by 2 rows 9369 and 21496, by 8 35000 and 21700,
+// one slice by 256 rows 2712 and 10667; 64 x 64 x 16, 2 rows and 64 views 179 and 225.
 static bool rs_t_gathers(const DevGeom& d) {
     const double half = 0.5 * (double)std::max(d.nx, d.ny) + 1.0, fod = d.fod / (double)d.delta;
     if (0.5 * (double)d.nv * (double)d.dv > 50.0 * d.fdd) return false;  // at most 255 samples on a chord
-    return fod > 1.01 * std::sqrt(2.0) * half && d.nv <= 8192 && d.nz <= 8192 && fod <= 8192.0 &&
-           (size_t)d.nu * d.nphi < (1ull << 31);
+    if (!(fod > 1.01 * std::sqrt(2.0) * half && d.nv <= 8192 && d.nz <= 8192 && fod <= 8192.0 &&
+          (size_t)d.nu * d.nphi < (1ull << 31)))
+        return false;
+    const CrossingRows c(d);
+    const double mag = (double)d.delta * d.fdd / d.fod, lines = mag / (double)d.du, rows = mag / (double)d.dv;
+    const double blocks = d.nz <= 64 ? 1.0 : d.nz <= 128 ? 1.4 : 2.9 * ceil_div(d.nz, 256);
+    const double gather = 50.0 + 1e-6 * d.nx * d.ny * (60.0 * std::ceil(2.83 * lines) * 64.0 * ceil_div(d.nphi, 64) +
+                                                       2.42 * lines * (20.0 + 43.0 * (2.0 * rows + 1.0)) * blocks * d.nphi);
+    const double row = 262e-6 * crossing_columns(d, c) * d.nphi * d.nx, enough = (gather - 12.0) / row;
+    return gather - 12.0 <= (0.9 + 0.35 * c.count(d, BY)) * d.nx || c.count(d, enough) >= enough;
 }
 
 template <int K, bool MIRROR>

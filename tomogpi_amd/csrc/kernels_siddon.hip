@@ -1251,11 +1251,26 @@ hipError_t launch_batch_siddon(BatchTable* t, hipStream_t s) {
 // the cylinder's bounding square scatters.  So do the smallest problems, whose
 // few chords cost less than the gather's extra launch and its FP64 chain: 24^3 /
 // 16 views 18.8 us against 28.8, 24^3 / 32 views 32.3 and 34.7, 32^3 / 16 views
-// 30.0 and 28.6, 32^3 / 32 views 50.0 and 34.6, 64^3 / 64 views 669 and 70.
+// 30.0 and 28.6, 32^3 / 32 views 50.0 and 34.6, 64^3 / 64 views 669 and 70; and thin
+// ones.  The gather costs 21 ps per voxel column, view and line that may cross it (in
+// rounds of 64 views) and 54 ps per line and 64 voxels of it, full or not; the scatter
+// 45 ps per ray and slab, or 0.36 us per slab of one.  That picks the faster within 10%
+// at 335 of 344 shapes of 1 to 400 rows and slices, scatter and gather in us: 256 x
+// 256 and 256 views, one slice and row 799 and 1876, 4 and 4 2700 and 1874, 256 slices
+// by 4 rows 2983 and 5365, by 12 8700 and 5400, one slice by 256 rows 892 and 1983.
 static bool sid_t_gathers(const DevGeom& d) {
     const double half = 0.5 * (double)d.delta * (double)std::max(d.nx, d.ny);
     const double chords = (double)d.nu * d.nv * d.nphi * std::max(d.nx, d.ny);
-    return d.fod > 1.01 * std::sqrt(2.0) * half && chords >= 8e5;
+    if (!(d.fod > 1.01 * std::sqrt(2.0) * half && chords >= 8e5)) return false;
+    if (2 * d.ny < d.nx) return true;  // rays that run along the border row: many to a voxel
+    const CrossingRows c(d);
+    const double cols = crossing_columns(d, c), most = 3e5 / (cols * d.nphi * d.nx);
+    if (c.count(d, most) < most) return false;
+    const double lines = (double)d.delta * d.fdd / (d.fod * (double)d.du);  // columns per voxel
+    const double gather = 28.0 + 1e-6 * d.nx * d.ny * (21.5 * std::ceil(1.41 * lines) * 64.0 * ceil_div(d.nphi, 64) +
+                                                       54.0 * 1.27 * lines * d.nphi * ceil_div(d.nz, 64));
+    const double row = 45e-6 * cols * d.nphi * d.nx, enough = (gather - 16.0) / row;
+    return gather - 16.0 <= 0.36 * d.nx || c.count(d, enough) >= enough;
 }
 
 template <int K>

@@ -719,17 +719,19 @@ __device__ __forceinline__ float lane_value(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// Grid: x, y = (view, column group), views first; z = row block of 64 K rows.  One
+// Grid: x, y = (view, column group), views first; z = block of 64 K of the rows r0 ..
+// r1 - 1, which voxels can reach; the others are 0.  One
 // wave per workgroup: nothing is shared, and the strips differ in length.
 template <int K, int M>
-__global__ __launch_bounds__(64, 7) void vi_t_kernel(DevGeom g, const float* __restrict__ vt, float* __restrict__ sino) {
+__global__ __launch_bounds__(64, 7) void vi_t_kernel(DevGeom g, const float* __restrict__ vt, float* __restrict__ sino, int r0,
+                                                     int r1) {
     typedef float V4 __attribute__((ext_vector_type(4)));
     __shared__ __align__(16) float stage[kViTWords + 8];
     const int lane = threadIdx.x;
     const uint32_t tile = tile_index();
     const int p = (int)(tile % (uint32_t)g.nphi), m0 = (int)(tile / (uint32_t)g.nphi) * M;
     if (m0 >= g.nu) return;
-    const int nb = (int)blockIdx.z * 64 * K;
+    const int nb = r0 + (int)blockIdx.z * 64 * K;
     typedef const __attribute__((address_space(4))) double* ConstView;
     const ConstView vw = (ConstView)(g.view + (size_t)p * kViewStride);
     double cvt[kViewStride];
@@ -883,13 +885,20 @@ __global__ __launch_bounds__(64, 7) void vi_t_kernel(DevGeom g, const float* __r
 #pragma unroll
     for (int c = 0; c < K; ++c) {
         const int n = nb + 64 * c + lane;
-        if (n < g.nv) {
+        if (n < r1) {
             float* o = sino + ((size_t)m0 + (size_t)g.nu * ((size_t)n + (size_t)g.nv * p));
 #pragma unroll
             for (int d = 0; d < M; ++d)
                 if (m0 + d < g.nu) o[d] = acc[d][c];
         }
     }
+    if (blockIdx.z == 0)
+        for (int n = lane; n < g.nv - (r1 - r0); n += 64) {
+            const int row = n < r0 ? n : n + (r1 - r0);
+            float* o = sino + ((size_t)m0 + (size_t)g.nu * ((size_t)row + (size_t)g.nv * p));
+            for (int d = 0; d < M; ++d)
+                if (m0 + d < g.nu) o[d] = 0.0f;
+        }
 }
 
 }  // namespace
@@ -1026,12 +1035,30 @@ hipError_t launch_batch_vi(BatchTable* t, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Detector rows that voxels of a geometry with the source outside the volume's square
+// project next to, r0 .. r1 - 1 (none: r1 = r0): of a detector taller than the volume's
+// shadow only these are walked for (256 x 256 x 1, 256 rows and views 3.06 -> 1.94 ms).
+struct ViTRows {
+    int r0, r1;
+};
+static ViTRows vi_t_reach(const DevGeom& d) {
+    const double dl = d.delta, nearest = d.fod - dl * std::hypot((double)d.cx, (double)d.cy);
+    const double reach = (double)d.cz * dl * d.fdd / ((double)d.dv * nearest) * (1.0 + 1e-6) + 1.0;
+    const int r0 = reach < (double)d.cv ? (int)std::ceil((double)d.cv - reach) : 0;
+    return ViTRows{r0, std::max(r0, d.nv - r0)};
+}
+
 // Row steps per lane of the gather, the fewest row blocks that K <= 4 allows;
 // 0 where it does not apply and the voxels scatter: a voxel column behind or
 // beside the source, a wave's outer lines too far apart (detector columns as
 // wide as a 20th of the distance to them), or 64 rows that reach more than
-// kViTWords voxels of a column (7.8 voxels to a row).  There is no lower limit:
-// 17^3 and 16 views take 33 us here and 108 scattered.
+// kViTWords voxels of a column (7.8 voxels to a row).  There is no lower limit of size:
+// 17^3 and 16 views take 33 us here and 108 scattered.  Columns of which hardly a
+// voxel is on the detector scatter: 20 ps per column and view and 26 per atomic, two
+// a voxel and row, or 2.8 us a view; the gather 80 ps and 31 more per detector column of a
+// voxel.  256 x 256 and 256 views, scatter and gather in us: one slice and row 1233 and
+// 1882, two rows 1849 and 1886, 8 rows 2348 and 1880; 64 x 64 and 64 views 182 and 79; 64
+// slices, 4 rows of a quarter voxel, 90 views 541 and 658.
 static int vi_t_steps(const DevGeom& d) {
     const double half = 0.5 * (double)d.delta * (double)std::max(d.nx, d.ny);
     const double far = d.fod + std::sqrt(2.0) * half;
@@ -1039,7 +1066,12 @@ static int vi_t_steps(const DevGeom& d) {
     if (!(d.fod > 1.01 * std::sqrt(2.0) * half && (double)d.du * (4 + 1) < 0.25 * d.fdd)) return 0;
     // FP32 voxel coordinates within 1e-3, 32-bit column numbers
     if (d.nv * inv + d.nz > 8192.0 || (double)d.nx * d.ny > 2147483647.0) return 0;
-    const int steps = (int)ceil_div(d.nv, 64), most = std::min(4, (int)(((kViTWords - 6) / (1.001 * inv) - 1.0) / 64.0));
+    const double mag = (double)d.delta * d.fdd / d.fod, views = (double)d.nx * d.ny * d.nphi;
+    const double pairs = std::min((double)d.nz * std::min(d.nv, 2), 2.0 * (d.nv + 1) * (double)d.dv / mag);
+    const double scatter = std::max(1e-6 * views * (20.0 + 52.0 * pairs), 2.8 * d.nphi);
+    if (12.0 + scatter < 30.0 + 1e-6 * views * (80.0 + 31.0 * mag / (double)d.du)) return 0;
+    const ViTRows rows = vi_t_reach(d);
+    const int steps = std::max(1, (int)ceil_div(rows.r1 - rows.r0, 64)), most = std::min(4, (int)(((kViTWords - 6) / (1.001 * inv) - 1.0) / 64.0));
     return most < 1 ? 0 : (int)ceil_div(steps, ceil_div(steps, most));
 }
 
@@ -1050,15 +1082,17 @@ static void launch_vi_t(const DevGeom& d, const float* vt, float* sino, hipStrea
     // M = 1 / 2 / 4: 1024 (64^3, 64 views) 81 / 103 / 172; 1152 (96^3, 48) 160 /
     // 197 / 311; 4096 (128^3, 128) 484 / 416 / 454; 7598 (201 x 187 x 149, 131)
     // 1253 / 1128 / 1104; 16384 (256^3, 256) 4636 / 3689 / 3445.
-    const size_t waves = (size_t)ceil_div(d.nu, 4) * d.nphi * ceil_div(d.nv, 64 * K);
+    const ViTRows r = vi_t_reach(d);
+    const unsigned blocks = std::max(1u, ceil_div(r.r1 - r.r0, 64 * K));
+    const size_t waves = (size_t)ceil_div(d.nu, 4) * d.nphi * blocks;
     const int cols = waves < 2048 ? 1 : waves < 6144 ? 2 : 4;
-    const dim3 grid = tile_grid((size_t)ceil_div(d.nu, cols) * d.nphi, 64, ceil_div(d.nv, 64 * K));
+    const dim3 grid = tile_grid((size_t)ceil_div(d.nu, cols) * d.nphi, 64, blocks);
     if (cols == 1)
-        hipLaunchKernelGGL((vi_t_kernel<K, 1>), grid, dim3(64), 0, s, d, vt, sino);
+        hipLaunchKernelGGL((vi_t_kernel<K, 1>), grid, dim3(64), 0, s, d, vt, sino, r.r0, r.r1);
     else if (cols == 2)
-        hipLaunchKernelGGL((vi_t_kernel<K, 2>), grid, dim3(64), 0, s, d, vt, sino);
+        hipLaunchKernelGGL((vi_t_kernel<K, 2>), grid, dim3(64), 0, s, d, vt, sino, r.r0, r.r1);
     else
-        hipLaunchKernelGGL((vi_t_kernel<K, 4>), grid, dim3(64), 0, s, d, vt, sino);
+        hipLaunchKernelGGL((vi_t_kernel<K, 4>), grid, dim3(64), 0, s, d, vt, sino, r.r0, r.r1);
 }
 
 int launch_vi_adjoint(const tomo_geom* g, Buf vol, MutBuf sino, hipStream_t s) {

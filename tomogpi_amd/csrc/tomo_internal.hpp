@@ -121,6 +121,33 @@ __host__ __device__ inline RsCopyShape rs_copy_shape(int nx, int ny, int nz, siz
     c.buf = c.elems * 8 < 0xfffffff0ull && sx * 8 < (1ull << 23) && nz < (1 << 23);
     return c;
 }
+// The detector rows whose rays are in the volume, each by the part of its way through
+// the FOV: z leaves the volume at the in-plane distance edge / |n - cv|.  Rows are
+// counted from the middle on, until there are `enough`.
+struct CrossingRows {
+    double fov, nearest, edge;  // radius; of the FOV from the source; mm
+    explicit CrossingRows(const DevGeom& d)
+        : fov(0.5 * (double)d.nx * (double)d.delta), nearest(d.fod - fov),
+          edge(0.5 * (double)d.nz * (double)d.delta * d.fdd / (double)d.dv) {}
+    double part(double off) const {
+        return off * (nearest + 2.0 * fov) <= edge ? 1.0 : std::max(0.0, (edge / off - nearest) / (2.0 * fov));
+    }
+    double count(const DevGeom& d, double enough) const {
+        double rows = 0.0;
+        for (int n = d.nv / 2; n < d.nv && rows < enough; ++n) {
+            const double off = (double)n - (double)d.cv, p = part(off);
+            if (p == 0.0) break;
+            rows += off == 0.0 ? p : 2.0 * p;
+        }
+        return rows;
+    }
+};
+// Detector columns whose rays cross the FOV.
+inline double crossing_columns(const DevGeom& d, const CrossingRows& c) {
+    const double reach = c.nearest > 0.0 ? 2.0 * c.fov * d.fdd / std::sqrt(d.fod * d.fod - c.fov * c.fov) / (double)d.du + 1.0 : 1e30;
+    return std::min((double)d.nu, reach);
+}
+
 // Detector rows of a projector's wave (a power of two up to 64, by 64 / rows columns).
 // `tall` where many rows cross the volume, else the rows of the least
 //     sum over row groups of max(16 rows, lines) x the longest ray's part of the FOV + 1/2.
@@ -141,11 +168,9 @@ __host__ __device__ inline RsCopyShape rs_copy_shape(int nx, int ny, int nz, siz
 // 4227 / 2207 / 1195 / 687 / 570 / 824.
 inline int proj_wave_rows(const DevGeom& d, double lines, int tall) {
     constexpr int kMost = 48;  // rows that cross the volume
-    const double fov = 0.5 * (double)d.nx * (double)d.delta, nearest = d.fod - fov;
-    if (!(nearest > 0.0)) return tall;
-    // z leaves the volume at the in-plane distance edge / |n - cv|
-    const double edge = 0.5 * (double)d.nz * (double)d.delta * d.fdd / (double)d.dv;
-    const int first = std::max(0, (int)std::ceil((double)d.cv - std::min(edge / nearest, 1e9)));
+    const CrossingRows c(d);
+    if (!(c.nearest > 0.0)) return tall;
+    const int first = std::max(0, (int)std::ceil((double)d.cv - std::min(c.edge / c.nearest, 1e9)));
     const int crossing = d.nv - 2 * first;  // centred
     if (crossing < 1 || crossing > kMost) return tall;
     const double share = lines * (1.0 + std::min(1.0, 60.0 / d.nphi));
@@ -158,9 +183,7 @@ inline int proj_wave_rows(const DevGeom& d, double lines, int tall) {
         for (int g = g0; g <= g1; ++g) {
             // the group's row nearest to the mid plane
             const double n = std::min(std::max((double)d.cv, (double)g * r), std::min((double)g * r + r, (double)d.nv) - 1.0);
-            const double off = std::fabs(n - (double)d.cv);
-            const double part = off * (d.fod + fov) <= edge ? 1.0 : (edge / off - nearest) / (2.0 * fov);
-            cost += std::max(16.0 * r, share) * part + 0.5;
+            cost += std::max(16.0 * r, share) * c.part(std::fabs(n - (double)d.cv)) + 0.5;
         }
         if (r == 64 || cost <= least) {
             least = cost;
