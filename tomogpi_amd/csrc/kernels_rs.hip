@@ -365,8 +365,7 @@ __global__ __launch_bounds__(64 * kProjViews) void rs_kernel(DevGeom g, int cube
 // from the volume directly.
 constexpr int kRsWmax = 8;  // sample planes per window at most
 
-// The eight taps straight from the volume: the range and border rules and the
-// arithmetic of trilinear_quads.
+// The eight taps straight from the volume, 0 off the grid, blended as rs_samples does.
 __device__ __forceinline__ float trilinear_direct(const float* __restrict__ f, int nx, int ny, int nz, float x,
                                                   float y, float z) {
     const float xf = floorf(x), yf = floorf(y), zf = floorf(z);

@@ -447,9 +447,10 @@ __device__ __forceinline__ void siddon_tile(const DevGeom& g, const uint32_t* __
 // boundary planes wlo - 1/2 and whi + 1/2, the voxel round(B) and its
 // neighbours, likewise in z), and each slab's quad -- the current
 // voxel, its B neighbour, its z neighbour and the diagonal one -- is two
-// ds_read2_b32 there instead of a gather per lane.  The
-// per-slab arithmetic is sid_walk_quads', so every lane takes the segments
-// of the per-ray traversal in its order: results are bit-identical to it.
+// ds_read2_b32 there instead of a gather per lane.  A slab's segments run
+// to the nearer and the farther of its B and z crossings and to its end, by
+// the crossings of the per-ray traversal in its order: results are
+// bit-identical to it.
 // A wave whose rays go up and down in z copies its share of rows and keeps
 // the barriers, then steps per lane; a window whose box exceeds the buffer
 // reads the quads from the volume; a workgroup whose rays do not share A and
@@ -653,7 +654,9 @@ __global__ __launch_bounds__(BX* BY, 5) void siddon_staged_kernel(DevGeom g, con
     r.ok = false;
     if (inside) r = sid_setup(g, p, m, n);
     const bool ok = r.ok && r.tmax > 0.0f;
-    // slab code as in siddon_tile
+    // The ray's slab axis and direction: the crossings of the other axes are spaced
+    // farther apart than this one's by more than two ulps of tmax, so a slab holds at
+    // most one of each; -1 where neither x nor y is one.
     int code = -1;
     if (ok) {
         const float big = 3.0e38f, margin = 1.0e-6f * r.tmax;
@@ -692,7 +695,7 @@ __global__ __launch_bounds__(BX* BY, 5) void siddon_staged_kernel(DevGeom g, con
         const int A = mode < 2 ? 0 : 1;
         const int sAw = (mode & 1) ? -1 : 1;
         const int nA = A == 0 ? nx : ny;
-        // the workgroup's first slab, then its iteration count (as sid_walk_quads, with the workgroup's I)
+        // the workgroup's first slab I, then its iteration count: the crossings of A up to tmax from there
         const int iA = ok ? r.idx[A] : 0;
         int I = sAw > 0 ? wave_min(ok ? iA : 0x7fffffff) : wave_max(ok ? iA : -0x7fffffff);
         __syncthreads();  // every wave has read wsh[*][0]

@@ -9,7 +9,8 @@
 //   v = A z' + cv,   A = (FDD/dv) delta / w
 //   f = delta * sum_p bilinear(g_p, u, v)      (taps outside the detector = 0)
 // The output is overwritten.  As in the reference's "16reg" blocking, a
-// thread owns a column of 16 voxels that share u and A; the per-(column,view)
+// thread owns a column of voxels that share u and A (16, 8 or 4 of them, for FDK half
+// of them at the mirrored heights); the per-(column,view)
 // terms w, 1/w, u and A are evaluated in FP64 (the geometry of the FP32 form)
 // and the per-voxel v, bilinear weights and sum in FP32.  A BF16 sinogram is
 // widened to FP32 (value = stored / scale) before the same kernel; an FP16
@@ -617,7 +618,8 @@ __global__ __launch_bounds__(SX* SY, 7) void vi_batch_kernel(const BatchTable* _
 }
 
 // VI^T: g_p[tap] += delta * w_tap * f(i,j,k) (FP32 atomics, output zeroed by
-// the caller).  Same geometry and weights as vi_kernel.
+// the caller).  The geometry is the backprojector's (column_view), the weights its
+// products.
 template <typename TV>
 __global__ __launch_bounds__(TX* TY) void vi_adjoint_kernel(DevGeom g, const TV* __restrict__ vol, float vol_inv,
                                                           float* __restrict__ sino) {

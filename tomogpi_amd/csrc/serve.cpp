@@ -152,18 +152,17 @@ Layout layout_of(const tomo_geom& g, const tomo_gd_params& gd, int algo, size_t 
     const int planes = copy_planes(d, gd).nz;
     sizes[i++] = gd.pair == TOMO_PAIR_SIDDONVI ? zcol_words(d.nx, d.ny, planes, ces) * 4
                                                : rs_copy_shape(d.nx, d.ny, planes, ces).elems * 8;  // 7 projector's copy
-    sizes[i++] = 0;                                                      // 8 (unused)
-    sizes[i++] = ns * 4;                                                 // 9 y
-    sizes[i++] = ns * 4;                                                 // 10 px
-    sizes[i++] = ns * 4;                                                 // 11 r
-    sizes[i++] = ns * 4;                                                 // 12 pd (SIRT: sinogram weight R)
-    sizes[i++] = vi_box_count(d) * sizeof(ViBox);                        // 13 tq (VI box table, set at admission)
-    sizes[i++] = (size_t)vec_tiles(ns) * 8;                              // 14 part_res
-    sizes[i++] = (size_t)vec_tiles(nv) * 8;                              // 15 part_vol
-    sizes[i++] = lam ? (size_t)lap_tiles(d) * 8 : 0;                     // 16 part_reg
-    sizes[i++] = (size_t)vec_tiles(ns) * 8;                              // 17 part_pd
-    sizes[i++] = kSlotCount * 8;                                         // 18 slot
-    sizes[i++] = (size_t)std::max(gd.gradient_iteration_nb, 1) * 4 * 8;  // 19 hist
+    sizes[i++] = ns * 4;                                                 // 8 y
+    sizes[i++] = ns * 4;                                                 // 9 px
+    sizes[i++] = ns * 4;                                                 // 10 r
+    sizes[i++] = ns * 4;                                                 // 11 pd (SIRT: sinogram weight R)
+    sizes[i++] = vi_box_count(d) * sizeof(ViBox);                        // 12 tq (VI box table, set at admission)
+    sizes[i++] = (size_t)vec_tiles(ns) * 8;                              // 13 part_res
+    sizes[i++] = (size_t)vec_tiles(nv) * 8;                              // 14 part_vol
+    sizes[i++] = lam ? (size_t)lap_tiles(d) * 8 : 0;                     // 15 part_reg
+    sizes[i++] = (size_t)vec_tiles(ns) * 8;                              // 16 part_pd
+    sizes[i++] = kSlotCount * 8;                                         // 17 slot
+    sizes[i++] = (size_t)std::max(gd.gradient_iteration_nb, 1) * 4 * 8;  // 18 hist
     Layout L{};
     size_t o = 0;
     for (int j = 0; j < 24; ++j) {
@@ -194,17 +193,17 @@ int admit(tomo_server* srv, Request& q) {
     q.t2 = lam ? (float*)at(5) : nullptr;
     q.t3 = lam ? (float*)at(6) : nullptr;
     q.copy = at(7);
-    q.y = (float*)at(9);
-    q.px = (float*)at(10);
-    q.r = (float*)at(11);
-    q.pd = (float*)at(12);
-    q.tq = (float*)at(13);
-    q.part_res = (double*)at(14);
-    q.part_vol = (double*)at(15);
-    q.part_reg = lam ? (double*)at(16) : nullptr;
-    q.part_pd = (double*)at(17);
-    q.slot = (double*)at(18);
-    q.hist = (double*)at(19);
+    q.y = (float*)at(8);
+    q.px = (float*)at(9);
+    q.r = (float*)at(10);
+    q.pd = (float*)at(11);
+    q.tq = (float*)at(12);
+    q.part_res = (double*)at(13);
+    q.part_vol = (double*)at(14);
+    q.part_reg = lam ? (double*)at(15) : nullptr;
+    q.part_pd = (double*)at(16);
+    q.slot = (double*)at(17);
+    q.hist = (double*)at(18);
     const size_t ns = q.geom.nsino(), nv = q.geom.nvox();
     hipStream_t s = srv->stream;
     TOMO_HIP(hipMemcpyAsync(q.geom.d_view, q.geom.view.data(), q.geom.view.size() * sizeof(double),
