@@ -103,9 +103,9 @@ __device__ __forceinline__ ColumnView column_view(const DevGeom& g, const double
 // Per wave and view, 16 voxels are about 500 VALU cycles of a SIMD, the FP64
 // column terms 120 and the copies and plans 40; the LDS reads are 128 cycles of
 // the CU, 85% of the time at 512^3 and 512 views, where that binds (and the
-// clock falls to 2.05 GHz): 22.3 -> 19.7 ms with the plans made by lane, the
+// clock falls to 2.05 GHz): 22.0 -> 19.8 ms (20.3 on another card) with the plans made by lane, the
 // direct views in a loop of their own, 16-byte copies and the short reciprocal.
-// FDK (256^3, 360 views) is bound by VALU: 5.93 -> 3.25 ms, most of it from
+// FDK (256^3, 360 views) is bound by VALU: 5.93 -> 3.2 ms (3.5 on another card), most of it from
 // fdk_weight and its sharing between mirrored voxels.
 constexpr int SX = kViStageX, SY = kViStageY;  // voxel columns per workgroup; a wave is 8 x 8 columns
 // Floats per staged row.  A wave's 64 lanes read taps (u, r) at word
@@ -276,7 +276,7 @@ __device__ __forceinline__ void pair_sample4(const uint32_t (&p0)[4], const uint
 // FDK: 0 VI, 1 FDK, 2 FDK whose weights are within fdk_weight's bounds, 3 the same
 // on mirrored columns: the weight depends on z'^2, so a voxel at z' and the one at
 // -z' share it.  A column is then ZS / 2 voxels from k0 = bz ZS / 2 on and their
-// mirror images nz - 1 - k.  256^3 and 360 views: 3.95 ms without, 3.25 with.
+// mirror images nz - 1 - k.  256^3 and 360 views: 3.95 ms without, 3.25 with, on one card.
 template <typename TV, int FDK, int ZS, bool PAIR = false>
 __device__ __forceinline__ void vi_staged_tile(const DevGeom& g, const float* __restrict__ sino,
                                                const ViBox* __restrict__ boxes, TV* __restrict__ vol,
