@@ -656,15 +656,18 @@ __global__ __launch_bounds__(BX* BY, 5) void siddon_staged_kernel(DevGeom g, con
     const bool ok = r.ok && r.tmax > 0.0f;
     // The ray's slab axis and direction: the crossings of the other axes are spaced
     // farther apart than this one's by more than two ulps of tmax, so a slab holds at
-    // most one of each; -1 where neither x nor y is one.
+    // most one of each; -1 where neither x nor y is one.  A ray that enters a FOV wider
+    // than the grid outside it walks along the border voxels until it gets there, away
+    // from its own place, which is what is staged: its first crossing comes late.
     int code = -1;
     if (ok) {
         const float big = 3.0e38f, margin = 1.0e-6f * r.tmax;
         const float ix = r.step[0] ? r.inc[0] : big, iy = r.step[1] ? r.inc[1] : big;
         const float iz = r.step[2] ? r.inc[2] : big;
-        if (r.step[0] != 0 && iy > ix + margin && iz > ix + margin && r.first[0] <= ix)
+        const bool late = r.first[0] > ix || r.first[1] > iy;
+        if (!late && r.step[0] != 0 && iy > ix + margin && iz > ix + margin)
             code = r.step[0] > 0 ? 0 : 1;
-        else if (r.step[1] != 0 && ix > iy + margin && iz > iy + margin && r.first[1] <= iy)
+        else if (!late && r.step[1] != 0 && ix > iy + margin && iz > iy + margin)
             code = r.step[1] > 0 ? 2 : 3;
     }
     const unsigned long long okmask = __ballot(ok);
