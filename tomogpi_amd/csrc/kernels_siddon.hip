@@ -874,19 +874,28 @@ __device__ __forceinline__ float read_lane(float v, int l) {
 }
 
 // views: the np views of `gt`, from view p0; add: to what vol holds.  Grid: x, y =
-// (column group, j), z = z block of 64 K voxels.  TIE: an odd number of detector
+// (column group, j), z = z block of 64 K voxels.  The rays that enter outside a grid
+// narrower than the FOV run along its border rows: those take the views in `parts`, the
+// first rows of the grid all but one of them, and add to a cleared volume (256 x 64 x 4,
+// 4 rows and 256 views 3.3 ms with one wave a voxel column, 1.5 in parts; 256 x 1 x 1, one
+// row and 200 views 5.8 and 0.98).  TIE: an odd number of detector
 // rows over an even number of slices: the middle row's rays run along the plane
 // between two slices, and belong to the upper one, as the projector's; its height
 // is then taken exactly at each row instead of carried on from the first.
 template <int K, bool TIE>
 __global__ __launch_bounds__(64 * kSidTWaves, 8) void siddon_t_kernel(DevGeom g, const float* __restrict__ gt, int p0,
-                                                                   int np, int add, float* __restrict__ vol) {
+                                                                   int np, int add, int parts,
+                                                                   float* __restrict__ vol) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t gx = (uint32_t)(g.nx + kSidTWaves - 1) / kSidTWaves;
     const uint32_t tile = tile_index();
-    const int i = (int)(tile % gx) * kSidTWaves + wv, j = (int)(tile / gx);
+    const int ends = min(g.ny, 2), row = (int)(tile / gx) - ends * (parts - 1);
+    const int i = (int)(tile % gx) * kSidTWaves + wv, j = row >= 0 ? row : row % ends ? g.ny - 1 : 0;
     if (i >= g.nx || j >= g.ny) return;
     const int kb = (int)blockIdx.z * 64 * K;
+    const bool split = parts > 1 && (j == 0 || j == g.ny - 1);
+    const int each = split ? (np + parts - 1) / parts : np;
+    const int pbegin = row >= 0 ? 0 : ((-1 - row) / ends + 1) * each, pend = min(np, pbegin + each);
     const double dl = (double)g.delta, inf = __builtin_inf();
     // The voxel column's cell in the plane (mm).  The cylinder may be wider than
     // the grid in y (ny < nx): a ray that comes from outside walks along the
@@ -910,12 +919,12 @@ __global__ __launch_bounds__(64 * kSidTWaves, 8) void siddon_t_kernel(DevGeom g,
     const int nu = g.nu, nv = g.nv;
     const size_t pitch = sid_t_pitch(nv);
     const float dvf = g.dv, dlf = g.delta, cvf = g.cv;
-    for (int pb = 0; pb < np; pb += 64) {
+    for (int pb = pbegin; pb < pend; pb += 64) {
         // ---- one view per lane: the columns m that can meet the cell
         const int pl = pb + lane;
         int m0 = 0, cnt = 0;
         double ca = 1.0, sa = 0.0;
-        if (pl < np) {
+        if (pl < pend) {
             const double* vw = g.view + (size_t)(p0 + pl) * kViewStride;
             ca = vw[0];
             sa = vw[1];
@@ -1050,7 +1059,8 @@ __global__ __launch_bounds__(64 * kSidTWaves, 8) void siddon_t_kernel(DevGeom g,
         const int k = kb + 64 * c + lane;
         if (k < g.nz) {
             float* o = vol + ((size_t)i + (size_t)g.nx * ((size_t)j + (size_t)g.ny * k));
-            *o = add ? *o + acc[c] : acc[c];
+            if (split) unsafeAtomicAdd(o, acc[c]);
+            else *o = add ? *o + acc[c] : acc[c];
         }
     }
 }
@@ -1252,6 +1262,16 @@ hipError_t launch_batch_siddon(BatchTable* t, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Parts of np views that the border rows of a narrow grid are split into: 64 views
+// each, fewer (8 at least) where that leaves fewer than two waves a SIMD.  A border voxel
+// has the lines of up to 1 + (nx - ny) / 2 voxels; up to 8 the other rows hide it.
+static int sid_t_parts(const DevGeom& d, int np) {
+    if (d.nx - d.ny <= 16) return 1;
+    int each = 64;
+    while (each > 8 && (size_t)std::min(d.ny, 2) * d.nx * ceil_div(d.nz, 256) * ceil_div(np, each) < 2048) each >>= 1;
+    return (int)ceil_div(np, each);
+}
+
 // The gather needs every voxel column in front of the source in every view (its
 // corners project onto the detector plane); a geometry with the source inside
 // the cylinder's bounding square scatters.  So do the smallest problems, whose
@@ -1259,33 +1279,43 @@ hipError_t launch_batch_siddon(BatchTable* t, hipStream_t s) {
 // 16 views 18.8 us against 28.8, 24^3 / 32 views 32.3 and 34.7, 32^3 / 16 views
 // 30.0 and 28.6, 32^3 / 32 views 50.0 and 34.6, 64^3 / 64 views 669 and 70; and thin
 // ones.  The gather costs 21 ps per voxel column, view and line that may cross it (in
-// rounds of 64 views) and 54 ps per line and 64 voxels of it, full or not; the scatter
-// 45 ps per ray and slab, or 0.36 us per slab of one.  That picks the faster within 10%
-// at 335 of 344 shapes of 1 to 400 rows and slices, scatter and gather in us: 256 x
+// rounds of 64 views) and 54 ps per line and 64 voxels of it, full or not, and on a narrow
+// grid at least the 2.5 us a line and 0.11 more a view of one border wave; the scatter
+// 45 ps per ray and slab, or 0.36 us per slab of one, or 65 ns per ray along a border
+// voxel.  That picks the faster within 10% at 335 of 344 shapes of 1 to 400 rows and
+// slices and ny = nx, and at all but one of 62 narrow ones (128 x 32 x 1, one row and 128
+// views: 220 and 282).  Narrow ones scatter from fewer chords, as many fall on a border
+// voxel, whose sum in atomics is less exact.  Scatter and gather in us: 256 x
 // 256 and 256 views, one slice and row 799 and 1876, 4 and 4 2700 and 1874, 256 slices
 // by 4 rows 2983 and 5365, by 12 8700 and 5400, one slice by 256 rows 892 and 1983.
 static bool sid_t_gathers(const DevGeom& d) {
     const double half = 0.5 * (double)d.delta * (double)std::max(d.nx, d.ny);
     const double chords = (double)d.nu * d.nv * d.nphi * std::max(d.nx, d.ny);
     if (!(d.fod > 1.01 * std::sqrt(2.0) * half && chords >= 8e5)) return false;
-    if (2 * d.ny < d.nx) return true;  // rays that run along the border row: many to a voxel
     const CrossingRows c(d);
-    const double cols = crossing_columns(d, c), most = 3e5 / (cols * d.nphi * d.nx);
+    const double cols = crossing_columns(d, c);
+    const double most = (2 * d.ny < d.nx ? 8e4 : 3e5) / (cols * d.nphi * d.nx);
     if (c.count(d, most) < most) return false;
     const double lines = (double)d.delta * d.fdd / (d.fod * (double)d.du);  // columns per voxel
-    const double gather = 28.0 + 1e-6 * d.nx * d.ny * (21.5 * std::ceil(1.41 * lines) * 64.0 * ceil_div(d.nphi, 64) +
-                                                       54.0 * 1.27 * lines * d.nphi * ceil_div(d.nz, 64));
-    const double row = 45e-6 * cols * d.nphi * d.nx, enough = (gather - 16.0) / row;
+    const double blocks = ceil_div(d.nz, 64), outside = 0.5 * std::max(0, d.nx - d.ny);  // voxels from the border to the FOV's
+    const int parts = sid_t_parts(d, d.nphi);
+    const double rounds = 64.0 * ceil_div(d.nphi, 64), each = ceil_div(d.nphi, parts);
+    const double grid = d.nx * (double)d.ny * (21.5 * std::ceil(1.41 * lines) * rounds + 54.0 * 1.27 * lines * d.nphi * blocks);
+    const double border = 2.0 * d.nx * outside * lines * (21.5 * 1.41 * 64.0 * parts + 54.0 * 1.27 * d.nphi * blocks);
+    const double gather = 28.0 + std::max(1e-6 * (grid + border), (2.5 + 0.11 * each) * 1.27 * lines * outside * (d.ny > 1 ? 1.0 : 2.0));
+    const double shared = 0.065 * (1.0 - std::min(1.0, (double)d.ny / d.nx)) / (std::min(d.ny, 2) * std::min(d.nz, d.nv));
+    const double row = cols * d.nphi * std::max(45e-6 * d.nx, shared), enough = (gather - 16.0) / row;
     return gather - 16.0 <= 0.36 * d.nx || c.count(d, enough) >= enough;
 }
 
 template <int K>
-static void launch_siddon_t(const DevGeom& d, const float* gt, int p0, int np, float* vol, hipStream_t s) {
-    const dim3 grid = tile_grid((size_t)ceil_div(d.nx, kSidTWaves) * d.ny, 64 * kSidTWaves, ceil_div(d.nz, 64 * K));
+static void launch_siddon_t(const DevGeom& d, const float* gt, int p0, int np, int parts, float* vol, hipStream_t s) {
+    const size_t rows = (size_t)d.ny + std::min(d.ny, 2) * (parts - 1);
+    const dim3 grid = tile_grid(ceil_div(d.nx, kSidTWaves) * rows, 64 * kSidTWaves, ceil_div(d.nz, 64 * K));
     if (d.nv % 2 == 1 && d.nz % 2 == 0)
-        hipLaunchKernelGGL((siddon_t_kernel<K, true>), grid, dim3(64 * kSidTWaves), 0, s, d, gt, p0, np, p0 > 0, vol);
+        hipLaunchKernelGGL((siddon_t_kernel<K, true>), grid, dim3(64 * kSidTWaves), 0, s, d, gt, p0, np, p0 > 0, parts, vol);
     else
-        hipLaunchKernelGGL((siddon_t_kernel<K, false>), grid, dim3(64 * kSidTWaves), 0, s, d, gt, p0, np, p0 > 0, vol);
+        hipLaunchKernelGGL((siddon_t_kernel<K, false>), grid, dim3(64 * kSidTWaves), 0, s, d, gt, p0, np, p0 > 0, parts, vol);
 }
 
 int launch_siddon_adjoint(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t s) {
@@ -1303,6 +1333,14 @@ int launch_siddon_adjoint(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t 
         gt = nullptr;
     }
     if (gt) {
+        const int parts = sid_t_parts(d, chunk);
+        if (parts > 1) {
+            const int rc = launch_fill((float*)vol.p, 0.0f, g->nvox(), s);
+            if (rc) {
+                (void)hipFreeAsync(gt, s);
+                return rc;
+            }
+        }
         hipError_t e = hipSuccess;
         for (int p0 = 0; p0 < d.nphi && e == hipSuccess; p0 += chunk) {
             const int np = std::min(chunk, d.nphi - p0);
@@ -1315,10 +1353,10 @@ int launch_siddon_adjoint(const tomo_geom* g, Buf sino, MutBuf vol, hipStream_t 
             // K 64-voxel steps per lane: the fewest z blocks that K <= 4 allows
             const int steps = (int)ceil_div(d.nz, 64), blocks = (int)ceil_div(steps, 4);
             switch (ceil_div(steps, blocks)) {
-                case 1: launch_siddon_t<1>(d, gt, p0, np, (float*)vol.p, s); break;
-                case 2: launch_siddon_t<2>(d, gt, p0, np, (float*)vol.p, s); break;
-                case 3: launch_siddon_t<3>(d, gt, p0, np, (float*)vol.p, s); break;
-                default: launch_siddon_t<4>(d, gt, p0, np, (float*)vol.p, s); break;
+                case 1: launch_siddon_t<1>(d, gt, p0, np, parts, (float*)vol.p, s); break;
+                case 2: launch_siddon_t<2>(d, gt, p0, np, parts, (float*)vol.p, s); break;
+                case 3: launch_siddon_t<3>(d, gt, p0, np, parts, (float*)vol.p, s); break;
+                default: launch_siddon_t<4>(d, gt, p0, np, parts, (float*)vol.p, s); break;
             }
             e = hipGetLastError();
         }
