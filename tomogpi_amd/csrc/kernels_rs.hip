@@ -1003,10 +1003,13 @@ hipError_t launch_batch_rs(BatchTable* t, hipStream_t s) {
 // problems, whose lanes along z would idle, scatter: the gather costs 60 ps per voxel
 // column, view and line that may cross its square (in rounds of 64 views), and per
 // line that does 20 and 43 per row that passes a voxel, 1.4 times that for 128 voxels in
-// two halves and 2.9 for 256; the scatter 262 ps a sample, or 0.9 us and 0.35 a row
-// (of up to 8) per sample of one ray.  Scatter and gather in us, 256 x 256 and 256 views: one slice and row 2422 and
-// 9121, 4 and 4 12900 and 9150, 256 slices by 2 rows 9369 and 21496, by 8 35000 and 21700,
-// one slice by 256 rows 2712 and 10667; 64 x 64 x 16, 2 rows and 64 views 179 and 225.
+// two halves and 2.9 for 256; on a narrow grid (ny < nx / 2), few columns idle the chip, one
+// wave's lines, 0.1 us and 0.22 a row.  The scatter costs 262 ps a sample in the grid, 90
+// ns per tap of one voxel, or 0.9 us and 0.35 a row (of up to 8) per sample of one ray.
+// Scatter and gather in us, 256 x 256 and 256 views: one slice and row 2422 and 9121, 4
+// and 4 12900 and 9150, 256 slices by 2 rows 9369 and 21496, by 8 35000 and 21700, one
+// slice by 256 rows 2712 and 10667; 64 x 64 x 16, 2 rows and 64 views 179 and 225; 256 x
+// 64 x 1, one row and 256 views 920 and 2670.
 static bool rs_t_gathers(const DevGeom& d) {
     const double half = 0.5 * (double)std::max(d.nx, d.ny) + 1.0, fod = d.fod / (double)d.delta;
     if (0.5 * (double)d.nv * (double)d.dv > 50.0 * d.fdd) return false;  // at most 255 samples on a chord
@@ -1016,9 +1019,12 @@ static bool rs_t_gathers(const DevGeom& d) {
     const CrossingRows c(d);
     const double mag = (double)d.delta * d.fdd / d.fod, lines = mag / (double)d.du, rows = mag / (double)d.dv;
     const double blocks = d.nz <= 64 ? 1.0 : d.nz <= 128 ? 1.4 : 2.9 * ceil_div(d.nz, 256);
-    const double gather = 50.0 + 1e-6 * d.nx * d.ny * (60.0 * std::ceil(2.83 * lines) * 64.0 * ceil_div(d.nphi, 64) +
-                                                       2.42 * lines * (20.0 + 43.0 * (2.0 * rows + 1.0)) * blocks * d.nphi);
-    const double row = 262e-6 * crossing_columns(d, c) * d.nphi * d.nx, enough = (gather - 12.0) / row;
+    const double all = d.nx * (double)d.ny * (60.0 * std::ceil(2.83 * lines) * 64.0 * ceil_div(d.nphi, 64) +
+                                              2.42 * lines * (20.0 + 43.0 * (2.0 * rows + 1.0)) * blocks * d.nphi);
+    const double one = 2 * d.ny < d.nx ? 2.55 * lines * (0.1 + 0.22 * (2.0 * rows + 1.0)) * d.nphi : 0.0;
+    const double gather = 50.0 + std::max(1e-6 * all, one);
+    const double step = std::max(262e-6, 0.72 / ((double)d.nx * d.ny * d.nz));
+    const double row = step * crossing_columns(d, c) * d.nphi * std::min(d.nx, d.ny + 1), enough = (gather - 12.0) / row;
     return gather - 12.0 <= (0.9 + 0.35 * c.count(d, BY)) * d.nx || c.count(d, enough) >= enough;
 }
 
