@@ -1058,9 +1058,10 @@ static ViTRows vi_t_reach(const DevGeom& d) {
 // 17^3 and 16 views take 33 us here and 108 scattered.  Columns of which hardly a
 // voxel is on the detector scatter: 20 ps per column and view and 26 per atomic, two
 // a voxel and row, or 2.8 us a view; the gather 80 ps and 31 more per detector column of a
-// voxel.  256 x 256 and 256 views, scatter and gather in us: one slice and row 1233 and
+// voxel, and for the strips that are walked past a narrow grid.  256 x 256 and 256 views, scatter and gather in us: one slice and row 1233 and
 // 1882, two rows 1849 and 1886, 8 rows 2348 and 1880; 64 x 64 and 64 views 182 and 79; 64
-// slices, 4 rows of a quarter voxel, 90 views 541 and 658.
+// slices, 4 rows of a quarter voxel, 90 views 541 and 658; 256 x 64 x 1, one row and 256
+// views 727 and 838.
 static int vi_t_steps(const DevGeom& d) {
     const double half = 0.5 * (double)d.delta * (double)std::max(d.nx, d.ny);
     const double far = d.fod + std::sqrt(2.0) * half;
@@ -1071,7 +1072,8 @@ static int vi_t_steps(const DevGeom& d) {
     const double mag = (double)d.delta * d.fdd / d.fod, views = (double)d.nx * d.ny * d.nphi;
     const double pairs = std::min((double)d.nz * std::min(d.nv, 2), 2.0 * (d.nv + 1) * (double)d.dv / mag);
     const double scatter = std::max(1e-6 * views * (20.0 + 52.0 * pairs), 2.8 * d.nphi);
-    if (12.0 + scatter < 30.0 + 1e-6 * views * (80.0 + 31.0 * mag / (double)d.du)) return 0;
+    const double strips = std::sqrt((double)d.nx * d.ny) * std::max(d.nx, d.ny) * d.nphi;  // walked past narrow grids too
+    if (12.0 + scatter < 30.0 + 1e-6 * strips * (80.0 + 31.0 * mag / (double)d.du)) return 0;
     const ViTRows rows = vi_t_reach(d);
     const int steps = std::max(1, (int)ceil_div(rows.r1 - rows.r0, 64)), most = std::min(4, (int)(((kViTWords - 6) / (1.001 * inv) - 1.0) / 64.0));
     return most < 1 ? 0 : (int)ceil_div(steps, ceil_div(steps, most));
